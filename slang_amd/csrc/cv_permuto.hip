@@ -185,12 +185,57 @@ __global__ __launch_bounds__(1024) void permutoEncodePairsKernel(const PermutoAr
     }
 }
 
-// Reverse mode for one position: adds bary[k] * dOut to the table gradient `dTable` (global memory, or a workgroup's
-// private copy in LDS) and, if wanted, writes the position gradient.
+// Where a position's contributions to the table gradient go: nowhere (position gradients only), straight to memory, or to
+// a workgroup's copy of a part of the table in LDS.
+struct NoTable {
+    static constexpr bool kWanted = false;
+    template <int N> __device__ __forceinline__ void addEntry(uint32_t, float, const float*) const {}
+    __device__ __forceinline__ void add(uint32_t, int, float) const {}
+};
+struct TableInMemory {
+    static constexpr bool kWanted = true;
+    float* table;
+    // w * g[0..N) to the entry whose first element is idx
+    template <int N> __device__ __forceinline__ void addEntry(uint32_t idx, float w, const float* g) const
+    {
+#pragma unroll
+        for (int f = 0; f < N; ++f) add(idx, f, w * g[f]);
+    }
+    __device__ __forceinline__ void add(uint32_t idx, int f, float v) const { atomicAdd(table + idx + f, v); }
+};
+// Elements [base, base + elems) of the table.  SLICED: what lies outside belongs to another workgroup.  The features of an
+// entry are `entries` elements apart, so that one instruction's lanes, which add to the same feature of scattered entries,
+// use all banks.
+template <int FT, bool SLICED>
+struct TableInLds {
+    static constexpr bool kWanted = true;
+    double* lds;
+    uint32_t base, elems, entries, F;
+    // Odd lanes begin with the last feature: on a coarse level, where a wave's positions share a few entries, half as many
+    // lanes of an instruction meet on one address (25 entries in use: 57 -> 48 us for 2^18 positions on 8 such levels).
+    template <int N> __device__ __forceinline__ void addEntry(uint32_t idx, float w, const float* g) const
+    {
+        const uint32_t e = idx - base;
+        if (SLICED && e >= elems) return;
+        const bool odd = N > 1 && (threadIdx.x & 1u);
+        double* p = lds + e / (uint32_t)N + (odd ? (uint32_t)(N - 1) * entries : 0u);
+        const int step = odd ? -(int)entries : (int)entries;
+#pragma unroll
+        for (int f = 0; f < N; ++f, p += step) unsafeAtomicAdd(p, (double)(w * (odd ? g[N - 1 - f] : g[f])));      // ds_add_f64
+    }
+    __device__ __forceinline__ void add(uint32_t idx, int f, float v) const
+    {
+        const uint32_t e = idx - base;
+        if (!SLICED || e < elems) unsafeAtomicAdd(lds + (uint32_t)f * entries + e / F, (double)v);
+    }
+};
+
+// Reverse mode of levels [first, end) for one position: hands bary[k] * dOut to `sink` and, with POS, writes the position
+// gradient (of all levels: such calls take them all).
 // FT: the features per entry when they are 1, 2 or 4 (the loops over them unrolled, the loads of a level issued together:
 // with a run-time count every element was a load and a wait of its own), else 0.
-template <int D, int FT>
-__device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_t s, float* dTable)
+template <int D, int FT, bool POS, typename Sink>
+__device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_t s, uint32_t first, uint32_t end, const Sink& sink)
 {
     const int F = FT ? FT : a.desc.featureDimensionPerEntry;
     float pos[D], dpos[D];
@@ -198,7 +243,7 @@ __device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_
     for (int d = 0; d < D; ++d) { pos[d] = ((const float*)(a.pos + (size_t)s * a.posStride))[d]; dpos[d] = 0.f; }
     const float* table = (const float*)a.table;
     const float* g = (const float*)(a.dOut + (size_t)s * a.dOutStride);
-    for (uint32_t l = 0; l < a.desc.maxLevels; ++l) {
+    for (uint32_t l = first; l < end; ++l) {
         const CvPermutoLevelInfo& lv = a.desc.levelInfo[l];
         if ((float)lv.currentLevelIndex >= a.desc.maxLevel + 1e-3f) continue;
         float elevated[D + 1], bary[D + 2], dbary[D + 2];
@@ -214,28 +259,30 @@ __device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_
             float gv[FT], tv[D + 1][FT];
 #pragma unroll
             for (int f = 0; f < FT; ++f) gv[f] = gl[f];
+            if constexpr (POS) {
 #pragma unroll
-            for (int k = 0; k <= D; ++k)
+                for (int k = 0; k <= D; ++k)
 #pragma unroll
-                for (int f = 0; f < FT; ++f) tv[k][f] = table[idx[k] + f];
+                    for (int f = 0; f < FT; ++f) tv[k][f] = table[idx[k] + f];
+            }
 #pragma unroll
             for (int k = 0; k <= D; ++k) {
+                if constexpr (Sink::kWanted) sink.template addEntry<FT>(idx[k], bary[k], gv);    // readFeatureValueBwd, :222-238
 #pragma unroll
                 for (int f = 0; f < FT; ++f) {
-                    if (dTable) atomicAdd(dTable + idx[k] + f, bary[k] * gv[f]);    // readFeatureValueBwd, :222-238
-                    dbary[k] += tv[k][f] * gv[f];
+                    if constexpr (POS) dbary[k] += tv[k][f] * gv[f];
                 }
             }
         } else {
 #pragma unroll
             for (int k = 0; k <= D; ++k) {
                 for (int f = 0; f < F; ++f) {
-                    if (dTable) atomicAdd(dTable + idx[k] + f, bary[k] * gl[f]);    // readFeatureValueBwd, :222-238
-                    dbary[k] += table[idx[k] + f] * gl[f];
+                    if constexpr (Sink::kWanted) sink.add(idx[k], f, bary[k] * gl[f]);    // readFeatureValueBwd, :222-238
+                    if constexpr (POS) dbary[k] += table[idx[k] + f] * gl[f];
                 }
             }
         }
-        if (!a.dPos) continue;
+        if constexpr (!POS) continue;
         dbary[D + 1] += dbary[0];                                      // the wrap-around term of barycentric[0]
         float delev[D + 1];
 #pragma unroll
@@ -257,41 +304,61 @@ __device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_
             dpos[dim] += dcf * lv.scalesPerDim[dim];
         }
     }
-    if (a.dPos) {
+    if constexpr (POS) {
 #pragma unroll
         for (int d = 0; d < D; ++d) ((float*)(a.dPos + (size_t)s * a.dPosStride))[d] = dpos[d];
     }
 }
 
-template <int D, int FT>
+// Position gradients alone (TABLE false), or everything with the table's share added in memory: a table of which one level
+// alone is beyond what the LDS kernel below takes.
+template <int D, int FT, bool POS, bool TABLE>
 __global__ __launch_bounds__(256) void permutoBackwardKernel(const PermutoArgs a)
 {
     const uint32_t s = blockIdx.x * 256u + threadIdx.x;
     if (s >= a.batch) return;
-    permutoBackwardOne<D, FT>(a, s, a.dTable);
+    if constexpr (TABLE) permutoBackwardOne<D, FT, POS>(a, s, 0u, a.desc.maxLevels, TableInMemory{a.dTable});
+    else permutoBackwardOne<D, FT, POS>(a, s, 0u, a.desc.maxLevels, NoTable{});
 }
 
-// A small feature table (the reference's own test: 2 048 floats) receives every position's atomic adds on a handful of
-// addresses: 2^22 positions took 123 ms that way.  Here a workgroup accumulates into a private copy of the table in
-// LDS and adds that copy to the table gradient once, at its end: the atomic traffic to memory shrinks by the number
-// of positions per workgroup.
-// As many copies of the table as fit (a power of two, up to 16) share the lanes of a wave among them: lanes of one
-// instruction that add to the same address are served one after the other, and with 64 lanes on a level of a few hundred
-// entries that is the common case (measured: 230 cycles per LDS atomic instruction with one copy).
-template <int D, int FT>
-__global__ __launch_bounds__(1024) void permutoBackwardLdsKernel(const PermutoArgs a, uint32_t tableElems, uint32_t copies)
+// The table gradient, by parts of the table small enough for LDS: part p covers elements [base, base + elems), which
+// levels [first, end) add to.  Every position adds to a handful of entries per level; added in memory, where many positions
+// meet on few addresses, 2^18 positions in 3 dimensions on 8 levels of 2^12 two-feature entries took 6.6 ms (2.5 G additions
+// per second); here 40 us, of which a quarter is the start and the sums' way to memory.
+constexpr int kMaxTableParts = 144;      // with the encoder's description within 4 KB of kernel arguments
+struct TablePart { uint32_t base, elems, first, end; };
+struct TableParts {
+    TablePart part[kMaxTableParts];
+    uint32_t count, groups;          // parts, and workgroups to a part
+    uint32_t sliced;                 // some part is a slice of a level's entries
+};
+static_assert(sizeof(PermutoArgs) + sizeof(TableParts) <= 4096, "kernel arguments");
+
+// A workgroup owns one part and a share of the positions: it sums into LDS and adds its sums to memory once, coalesced
+// (180 G additions per second).  What bounds it: the LDS's additions and the vector instructions that find the simplex
+// (170 per position and level).  The sums are kept in double: gfx950 serves a ds_add_f64 in 8.6 ns per wave and compute
+// unit, whatever the spread of the addresses, and a ds_add_f32 in 80 (measured, random addresses, 16 waves), so the wider
+// sum is also the cheaper one and needs no copies per lane to keep equal addresses apart.
+// POS (one part that is the whole table): the position gradient in the same pass.  SLICED: some part is a slice of a level.
+template <int D, int FT, bool POS, bool SLICED>
+__global__ __launch_bounds__(1024) void permutoTableGradKernel(const PermutoArgs a, const TableParts parts)
 {
-    extern __shared__ float ldsTable[];
-    for (uint32_t i = threadIdx.x; i < tableElems * copies; i += blockDim.x) ldsTable[i] = 0.f;
+    extern __shared__ double ldsTable[];
+    // workgroup w: part w / groups, so that the workgroups of all parts that read the same positions (w % groups) sit on one
+    // die (w % 8) where groups is a multiple of 8, and find them in its L2
+    const uint32_t p = blockIdx.x / parts.groups, w = blockIdx.x - p * parts.groups;
+    const TablePart part = parts.part[p];
+    const uint32_t F = FT ? (uint32_t)FT : (uint32_t)a.desc.featureDimensionPerEntry, entries = part.elems / F;
+    for (uint32_t i = threadIdx.x; i < part.elems; i += 1024u) ldsTable[i] = 0.0;
     __syncthreads();
-    float* mine = ldsTable + (threadIdx.x & (copies - 1u)) * tableElems;
-    for (uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; s < a.batch; s += (uint64_t)gridDim.x * blockDim.x)
-        permutoBackwardOne<D, FT>(a, (uint32_t)s, mine);
+    const TableInLds<FT, SLICED> sink{ldsTable, part.base, part.elems, entries, F};
+    for (uint64_t s = (uint64_t)w * 1024u + threadIdx.x; s < a.batch; s += (uint64_t)parts.groups * 1024u)
+        permutoBackwardOne<D, FT, POS>(a, (uint32_t)s, part.first, part.end, sink);
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < tableElems; i += blockDim.x) {
-        float v = ldsTable[i];
-        for (uint32_t c = 1; c < copies; ++c) v += ldsTable[c * tableElems + i];
-        if (v != 0.f) atomicAdd(a.dTable + i, v);
+    for (uint32_t i = threadIdx.x; i < part.elems; i += 1024u) {
+        const uint32_t e = i / F, f = i - e * F;
+        const float v = (float)ldsTable[f * entries + e];
+        if (v != 0.f) atomicAdd(a.dTable + part.base + i, v);
     }
 }
 
@@ -366,45 +433,98 @@ hipError_t launchEncode(hipStream_t stream, const PermutoArgs& a)
     return hipGetLastError();
 }
 
-hipError_t launchBackward(hipStream_t stream, const PermutoArgs& a)
+// Cuts the table into parts for permutoTableGradKernel: consecutive levels as long as they fit half of a compute unit's LDS
+// together, so that two workgroups of 16 waves share it; a level beyond that by itself, up to the whole 160 KB; and a level
+// beyond those in slices of its entries, each walked by all positions of the batch.  A slice repeats the search for the
+// simplex: 2^18 positions on 8 levels of 2^16 two-feature entries, seven slices each, take 128 us, on levels of 2^17 in
+// thirteen slices 219 us, and either takes 6.3 to 6.7 ms with the additions in memory.  Sixteen slices at most, since the list of
+// parts travels with the kernel's arguments.
+// False: more parts than that, or levels that do not lie behind one another as prepareLevelInfo puts them.
+bool cutTable(const PermutoArgs& a, TableParts& t)
 {
-    const uint64_t tableElems = tableElements(a.desc);
-    const int fe = a.desc.featureDimensionPerEntry, ft = (fe == 1 || fe == 2 || fe == 4) ? fe : 0;
-    constexpr uint64_t kLdsTableBytes = 64 * 1024;
-    if (a.dTable && tableElems * 4 <= kLdsTableBytes && a.batch >= 4096u) {
-        int dev = 0, cus = 256;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-        uint32_t copies = 1;
-        while (copies < 16u && (size_t)tableElems * 4 * (copies * 2u) <= 2 * kLdsTableBytes) copies *= 2u;
-        const size_t lds = (size_t)tableElems * 4 * copies;
-        // workgroups of 16 waves, one or two to a compute unit as the copies leave room
-        const uint32_t want = (a.batch + 1023u) / 1024u, cap = (uint32_t)cus * (lds <= 80 * 1024 ? 2u : 1u);
-        const dim3 grid(want < cap ? want : cap), block(1024);
-        noteKernel(false, "permutoBackwardLdsKernel<D=%d,%u copies>", a.desc.dimensions, copies);
-        switch (a.desc.dimensions * 8 + ft) {
-#define CV_DF(N, G) case N * 8 + G: { \
-            const hipError_t e = allowDynamicLds<permutoBackwardLdsKernel<N, G>>((int)(2 * kLdsTableBytes)); \
-            if (e != hipSuccess) return e; \
-            hipLaunchKernelGGL((permutoBackwardLdsKernel<N, G>), grid, block, lds, stream, a, (uint32_t)tableElems, copies); break; }
-#define CV_D(N) CV_DF(N, 0) CV_DF(N, 1) CV_DF(N, 2) CV_DF(N, 4)
-        CV_D(1) CV_D(2) CV_D(3) CV_D(4) CV_D(5) CV_D(6) CV_D(7) CV_D(8)
-#undef CV_D
-#undef CV_DF
-        default: return hipErrorInvalidValue;
+    constexpr uint64_t kHalf = 80 * 1024 / 8, kWhole = 160 * 1024 / 8;      // elements
+    const uint64_t F = (uint64_t)a.desc.featureDimensionPerEntry;
+    t.count = 0;
+    t.sliced = 0;
+    uint64_t next = 0;
+    for (uint32_t l = 0; l < a.desc.maxLevels; ++l) {
+        const CvPermutoLevelInfo& lv = a.desc.levelInfo[l];
+        if ((uint64_t)lv.offsetOfFeatureTable * F != next) return false;
+        const uint64_t elems = (uint64_t)lv.featureTableSize * F;
+        next += elems;
+        if (next > 0xffffffffull) return false;
+        TablePart* last = t.count ? &t.part[t.count - 1] : nullptr;
+        if (last && last->end == l && (uint64_t)last->elems + elems <= kHalf) {
+            last->elems += (uint32_t)elems;
+            last->end = l + 1;
+            continue;
         }
+        const uint64_t slices = (elems + kWhole - 1) / kWhole;
+        if (slices > 16) return false;
+        if (slices > 1) t.sliced = 1;
+        const uint64_t perSlice = ((uint64_t)lv.featureTableSize + slices - 1) / (slices ? slices : 1) * F;
+        for (uint64_t at = 0; at < elems; at += perSlice) {
+            if (t.count == (uint32_t)kMaxTableParts) return false;
+            t.part[t.count++] = TablePart{(uint32_t)(next - elems + at), (uint32_t)(elems - at < perSlice ? elems - at : perSlice), l, l + 1};
+        }
+    }
+    return t.count > 0;
+}
+
+template <int D, int FT, bool POS, bool SLICED>
+hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, TableParts& t, int cus)
+{
+    uint32_t most = 0;
+    for (uint32_t p = 0; p < t.count; ++p) most = t.part[p].elems > most ? t.part[p].elems : most;
+    const size_t lds = (size_t)most * 8;
+    const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED>>(160 * 1024);
+    if (e != hipSuccess) return e;
+    // as many workgroups as the compute units hold, dealt evenly to the parts
+    const uint32_t resident = (uint32_t)cus * (lds <= 80 * 1024 ? 2u : 1u), want = (a.batch + 1023u) / 1024u;
+    const uint32_t each = resident / t.count ? resident / t.count : 1u;
+    t.groups = want < each ? want : each;
+    hipLaunchKernelGGL((permutoTableGradKernel<D, FT, POS, SLICED>), dim3(t.count * t.groups), dim3(1024), lds, stream, a, t);
+    return hipGetLastError();
+}
+
+template <int D, int FT>
+hipError_t launchBackwardSized(hipStream_t stream, const PermutoArgs& a)
+{
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+    const dim3 grid((a.batch + 255) / 256), block(256);
+    TableParts t;
+    const bool cut = a.dTable && cutTable(a, t);
+    if (cut && t.count == 1 && a.dPos) {
+        noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
+        return launchTableGrad<D, FT, true, false>(stream, a, t, cus);
+    }
+    if (cut) {
+        noteKernel(false, "permutoTableGradKernel<D=%d,%u parts>", D, t.count);
+        const hipError_t e = t.sliced ? launchTableGrad<D, FT, false, true>(stream, a, t, cus) : launchTableGrad<D, FT, false, false>(stream, a, t, cus);
+        if (e != hipSuccess || !a.dPos) return e;
+        noteKernel(true, "permutoBackwardKernel<D=%d,positions>", D);
+        hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false>), grid, block, 0, stream, a);
         return hipGetLastError();
     }
-    noteKernel(false, "permutoBackwardKernel<D=%d>", a.desc.dimensions);
-    const dim3 grid((a.batch + 255) / 256), block(256);
+    noteKernel(false, "permutoBackwardKernel<D=%d%s%s>", D, a.dPos ? ",positions" : "", a.dTable ? ",table" : "");
+    if (a.dPos && a.dTable) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, true>), grid, block, 0, stream, a);
+    else if (a.dPos) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false>), grid, block, 0, stream, a);
+    else if (a.dTable) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, false, true>), grid, block, 0, stream, a);
+    return hipGetLastError();
+}
+
+hipError_t launchBackward(hipStream_t stream, const PermutoArgs& a)
+{
+    const int fe = a.desc.featureDimensionPerEntry, ft = (fe == 1 || fe == 2 || fe == 4) ? fe : 0;
     switch (a.desc.dimensions * 8 + ft) {
-#define CV_DF(N, G) case N * 8 + G: hipLaunchKernelGGL((permutoBackwardKernel<N, G>), grid, block, 0, stream, a); break;
+#define CV_DF(N, G) case N * 8 + G: return launchBackwardSized<N, G>(stream, a);
 #define CV_D(N) CV_DF(N, 0) CV_DF(N, 1) CV_DF(N, 2) CV_DF(N, 4)
     CV_D(1) CV_D(2) CV_D(3) CV_D(4) CV_D(5) CV_D(6) CV_D(7) CV_D(8)
 #undef CV_D
 #undef CV_DF
-    default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 } // namespace

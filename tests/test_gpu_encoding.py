@@ -185,6 +185,45 @@ def test_permuto_encoder_kernel_choices(D, F, levels_n, log2):
             assert cv.lastKernelName().startswith("permutoEncodeKernel"), cv.lastKernelName()
 
 
+@pytest.mark.parametrize("D,F,levels_n,log2,B,kernel", [
+    (2, 2, 4, 8, 5000, "permutoTableGradKernel<D=2,positions>"),           # the whole table in one workgroup's LDS
+    (3, 1, 2, 6, 1, "permutoTableGradKernel<D=3,positions>"),
+    (2, 4, 3, 10, 1025, "permutoTableGradKernel<D=2,2 parts> + permutoBackwardKernel<D=2,positions>"),   # two levels, then one
+    (3, 2, 8, 12, 4099, "permutoTableGradKernel<D=3,8 parts> + permutoBackwardKernel<D=3,positions>"),   # a level to a part
+    (3, 4, 2, 12, 1023, "permutoTableGradKernel<D=3,2 parts> + permutoBackwardKernel<D=3,positions>"),   # beyond half a unit's LDS
+    (2, 5, 2, 12, 300, "permutoTableGradKernel<D=2,2 parts> + permutoBackwardKernel<D=2,positions>"),    # the LDS full to the byte
+    (2, 3, 2, 13, 2000, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),   # two slices to a level
+    (3, 2, 2, 17, 3000, "permutoTableGradKernel<D=3,26 parts> + permutoBackwardKernel<D=3,positions>"),  # thirteen slices
+    (2, 2, 1, 18, 2000, "permutoBackwardKernel<D=2,positions,table>"),     # too many slices: added in memory
+])
+def test_permuto_backward_table_parts(D, F, levels_n, log2, B, kernel):
+    # Bound: the weights of an addend are differences of single-precision values below 2, off by at most 2^-22 against the
+    # oracle's double ones, their mean is 1/(D+1), so a sum of addends is off by less than 2^-20 of its norm for D <= 3; the
+    # sums (in double, or one by one in memory: at most 2^12 addends on an entry, each rounding 2^-25) stay within 2^-16.
+    rng = np.random.default_rng(D * 1000 + F * 100 + levels_n * 10 + log2)
+    enc = cv.PermutoEncoder(D, F, log2, levels_n, baseScale=3.0, log2PerLevelScale=1.0, maxLevelRatio=1.0, seed=11)
+    levels = ob.permuto_levels(D, log2, levels_n, 3.0, 1.0, 11)
+    pos = rng.uniform(-1, 1, (B, D)).astype(np.float32)
+    table = rng.standard_normal(enc.featureTableElements).astype(np.float32)
+    g = rng.standard_normal((B, levels_n * F)).astype(np.float32)
+    r_pos, r_table = ob.permuto_encode_backward(levels, F, float(levels_n), pos, table, g)
+    start = rng.standard_normal(table.size).astype(np.float32)              # gradients are added to what is there
+    d_table = to_dev(start)
+    d_pos, _ = enc.backward(to_dev(pos), to_dev(table), to_dev(g), dFeatureTable=d_table)
+    assert cv.lastKernelName() == kernel
+    got = d_table.cpu().numpy().astype(np.float64) - start
+    rounding = 2.0 ** -23 * np.linalg.norm(start)                           # of the last sum, and of taking `start` out again
+    assert np.linalg.norm(got - r_table) <= 2.0 ** -16 * np.linalg.norm(r_table) + rounding
+    untouched = r_table == 0
+    assert np.array_equal(d_table.cpu().numpy()[untouched], start[untouched])
+    assert np.linalg.norm(d_pos.cpu().numpy() - r_pos) <= 1e-4 * np.linalg.norm(r_pos)
+    # the table gradient alone: the same sums
+    alone = torch.zeros_like(d_table)
+    none, _ = enc.backward(to_dev(pos), to_dev(table), to_dev(g), dFeatureTable=alone, wantPositionGrad=False)
+    assert none is None
+    assert np.linalg.norm(alone.cpu().numpy() - r_table) <= 2.0 ** -16 * np.linalg.norm(r_table)
+
+
 def test_encoder_feeds_the_mlp():
     # encode positions, run the decoder MLP on the fp16 features: the neural-texture shape
     rng = np.random.default_rng(8)
