@@ -762,6 +762,19 @@ CV_API CvResult cvPermutoMlpForward(void* stream, const CvPermutoDesc* desc, con
     return fromHip(e, "cvPermutoMlpForward launch");
 }
 
+// Which kernels take a training step, and the bytes of workspace they need: the fused ones for half networks of their shapes,
+// the step over rounds in LDS where the network fits, else the step over the whole batch in memory (any layer sizes).
+enum class TrainStepKind { Fused, Rounds, General };
+static TrainStepKind chooseTrainStep(const cv::MlpArgs& a, uint32_t flags, int carrierCt, int cus, size_t* bytes)
+{
+    if (!(flags & CV_FLAG_LAYERWISE_TRAINING)) {
+        if (carrierCt == CV_FLOAT16 && (*bytes = cv::trainWorkspaceBytes(a, cus)) != 0) return TrainStepKind::Fused;
+        if ((*bytes = cv::trainRoundWorkspaceBytes(a, cus, carrierCt)) != 0) return TrainStepKind::Rounds;
+    }
+    *bytes = cv::trainGeneralWorkspaceBytes(a, cus, carrierCt);
+    return TrainStepKind::General;
+}
+
 CV_API CvResult cvMlpTrainStepWorkspaceSize(const CvMlpDesc* mlp, uint32_t batch, size_t* outBytes)
 {
     if (!outBytes) return fail(CV_E_INVALID_ARG, "cvMlpTrainStepWorkspaceSize: outBytes is null");
@@ -770,7 +783,7 @@ CV_API CvResult cvMlpTrainStepWorkspaceSize(const CvMlpDesc* mlp, uint32_t batch
     memset(&a, 0, sizeof(a));
     CvResult rc = fillMlpLayers("cvMlpTrainStepWorkspaceSize", mlp, a.layers);
     if (CV_FAILED(rc)) return rc;
-    const bool f32net = mlp->weightType == CV_FLOAT32;      // a network of float: layer by layer
+    const bool f32net = mlp->weightType == CV_FLOAT32;      // a network of float
     if (mlp->weightType != CV_FLOAT16 && !f32net)
         return fail(CV_E_NOT_AVAILABLE, "cvMlpTrainStep: training needs FLOAT16 weights (or a FLOAT32 network)");
     if (mlp->numLayers < 2) return fail(CV_E_NOT_AVAILABLE, "cvMlpTrainStep: needs at least two layers");
@@ -779,9 +792,7 @@ CV_API CvResult cvMlpTrainStepWorkspaceSize(const CvMlpDesc* mlp, uint32_t batch
     a.inEncoding = mlp->inputEncoding == CV_ENCODE_XY_SQUARES ? cv::kEncodeXYSquares : cv::kEncodeNone;
     const int cus = currentDeviceCUs(&rc);
     if (CV_FAILED(rc)) return rc;
-    size_t n = ((mlp->flags & CV_FLAG_LAYERWISE_TRAINING) || f32net) ? 0 : cv::trainWorkspaceBytes(a, cus);
-    if (!n) n = cv::trainGeneralWorkspaceBytes(a, cus, f32net ? CV_FLOAT32 : CV_FLOAT16);   // no fused shape: the layer-by-layer step
-    *outBytes = n;
+    chooseTrainStep(a, mlp->flags, f32net ? CV_FLOAT32 : CV_FLOAT16, cus, outBytes);
     return CV_OK;
 }
 
@@ -795,7 +806,7 @@ static CvResult trainStep(const char* who, void* stream, const CvMlpDesc* mlp, c
     memset(&t, 0, sizeof(t));
     CvResult rc = fillMlpLayers(who, mlp, t.mlp.layers);
     if (CV_FAILED(rc)) return rc;
-    const bool f32net = mlp->weightType == CV_FLOAT32;      // a network of float: layer by layer, fp32 gradients
+    const bool f32net = mlp->weightType == CV_FLOAT32;      // a network of float: fp32 gradients
     if (mlp->weightType != CV_FLOAT16 && !f32net)
         return fail(CV_E_NOT_AVAILABLE, "%s: training needs FLOAT16 weights (or a FLOAT32 network)", who);
     if (mlp->gradType != CV_FLOAT16 && mlp->gradType != CV_FLOAT32)
@@ -854,16 +865,16 @@ static CvResult trainStep(const char* who, void* stream, const CvMlpDesc* mlp, c
     t.workspace = (float*)workspace;
     const int cus = currentDeviceCUs(&rc);
     if (CV_FAILED(rc)) return rc;
-    size_t need = ((mlp->flags & CV_FLAG_LAYERWISE_TRAINING) || f32net) ? 0 : cv::trainWorkspaceBytes(t.mlp, cus);
-    const bool fused = need != 0;
-    if (!fused) need = cv::trainGeneralWorkspaceBytes(t.mlp, cus, t.carrierCt);   // layer by layer, any layer sizes
+    size_t need = 0;
+    const TrainStepKind kind = chooseTrainStep(t.mlp, mlp->flags, t.carrierCt, cus, &need);
     if (workspaceBytes < need) {
         if (ownScratch)
             return fail(CV_E_NOT_AVAILABLE, "%s: this network needs %zu bytes of scratch, the built-in array holds %zu; "
                         "use cvMlpTrainStep with a caller-provided workspace", who, need, workspaceBytes);
         return fail(CV_E_BUFFER_TOO_SMALL, "%s: workspace of %zu bytes, %zu needed", who, workspaceBytes, need);
     }
-    if (fused) return fromHip(cv::launchMlpTrain((hipStream_t)stream, t, cus), who);
+    if (kind == TrainStepKind::Fused) return fromHip(cv::launchMlpTrain((hipStream_t)stream, t, cus), who);
+    if (kind == TrainStepKind::Rounds) return fromHip(cv::launchTrainRound((hipStream_t)stream, t, cus), who);
     const hipError_t e = cv::launchMlpTrainGeneral((hipStream_t)stream, t, cus);
     if (e == hipErrorInvalidValue)
         return fail(CV_E_NOT_AVAILABLE, "%s: a layer is wider than the matMul kernels serve (k beyond 4096)", who);

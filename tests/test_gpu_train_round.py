@@ -1,0 +1,155 @@
+"""The training steps in LDS: over rounds of 64 samples (trainRoundKernel), for half networks outside the fused kernels'
+shapes and networks of float that fit a compute unit's LDS, and with every wave by itself (trainWaveKernel), for the smaller
+of the float networks.
+
+Two bars.  Networks of small whole numbers, in which every product, sum and rounding is exact (weights of -1, 0, 1 with three
+entries to a row, so that values stay below 2048, a half's range of exact whole numbers): gradients and loss equal the
+reference bit for bit, ties of max() included.  Random networks: the bars of the other training tests, 1e-3 of a layer's
+gradient norm for half (hidden values that round the other way), 2e-5 for float."""
+import numpy as np
+import pytest
+import torch
+
+import oracle_binding as ob
+from gpu_util import DEV, as_bytes, to_dev
+from slang_amd import coopvec as cv
+from slang_amd.coopvec import Activation, CoopVecComponentType as CT, CoopVecMatrixLayout as ML, FeedForwardLayer
+from test_gpu_train import read_grads, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(specs, x, t, scale):
+    """The step in float64 with Slang's rule for max(): (dW, db, loss)."""
+    hs, zs = [x.astype(np.float64)], []
+    for s in specs:
+        z = hs[-1] @ s["W"].astype(np.float64).T + (s["b"].astype(np.float64) if s["b"] is not None else 0.0)
+        zs.append(z)
+        hs.append(np.maximum(z, 0) if s["act"] == 1 else np.maximum(z, z * s["slope"]) if s["act"] == 2 else z)
+    diff = hs[-1] - t.astype(np.float64)
+    g, dW, dB = 2.0 * diff * scale, [], []
+    for l in range(len(specs) - 1, -1, -1):
+        z, sl = zs[l], specs[l]["slope"]
+        if specs[l]["act"] == 1: g = g * np.where(z > 0, 1.0, np.where(z == 0, 0.5, 0.0))
+        if specs[l]["act"] == 2: g = g * np.where(z > 0, 1.0, np.where(z == 0, 0.5 + 0.5 * sl, sl))
+        dW.append(g.T @ hs[l]); dB.append(g.sum(axis=0))
+        g = g @ specs[l]["W"].astype(np.float64)
+    return dW[::-1], dB[::-1], float((diff ** 2).sum())
+
+
+def build(specs, ct, layout=ML.RowMajor, grad_layout=ML.TrainingOptimal, preset=0.0):
+    layers = []
+    for s in specs:
+        out, fan_in = s["W"].shape
+        esz = s["W"].itemsize
+        w, stride = as_bytes(to_dev(np.ascontiguousarray(s["W"]))), fan_in * esz
+        if layout == ML.ColumnMajor:
+            w, stride = as_bytes(to_dev(np.ascontiguousarray(s["W"].T))), out * esz
+        elif layout != ML.RowMajor:
+            size = cv.getCooperativeVectorMatrixSize(out, fan_in, ct, layout)
+            D, dst = cv.CooperativeVectorMatrixDesc, torch.zeros(size, dtype=torch.uint8, device=DEV)
+            cv.convertCooperativeVectorMatrix(dst, [D(out, fan_in, ct, layout, size, 0, 0)], w, [D(out, fan_in, ct, ML.RowMajor, out * stride, 0, stride)])
+            w, stride = dst, 0
+        wg = torch.full((cv.getCooperativeVectorMatrixSize(out, fan_in, CT.Float32, grad_layout) // 4,), preset, device=DEV)
+        bg = torch.full((out,), preset, device=DEV)
+        layers.append(FeedForwardLayer(fan_in, out, w, as_bytes(to_dev(s["b"])) if s["b"] is not None else None, layout, stride, s["act"], s["slope"],
+                                       wg.view(torch.uint8), bg.view(torch.uint8), grad_layout, 0))
+    return layers
+
+
+def kernel_of(elem, dims):
+    """float networks whose dW fits a wave's registers (36 tiles of 16 x 16 at 1, 2 or 4 tiles per layer) run on
+    trainWaveKernel, the others on trainRoundKernel"""
+    up = lambda v: next((t for t in (1, 2, 4) if v <= 16 * t), 99)
+    ht, it, hidden = max(up(d) for d in dims[1:-1]), up(dims[0]), len(dims) - 2
+    wave = elem == "f32" and ht * it + ht * ht * (hidden - 1) + ht <= 36
+    return "train%sKernel<%s" % ("Wave" if wave else "Round", elem)
+
+
+def whole_number_network(rng, dims, dtype, act, slope, last_act):
+    specs = []
+    for i, (fi, fo) in enumerate(zip(dims, dims[1:])):
+        W = np.zeros((fo, fi))
+        for row in W:
+            row[rng.choice(fi, min(3, fi), replace=False)] = rng.integers(-1, 2, min(3, fi))
+        b = rng.integers(-1, 2, fo).astype(np.float64)
+        if i + 2 < len(dims):
+            W[::5] = 0; b[::5] = 0          # pre-activations that are always exactly 0
+        specs.append(dict(W=W.astype(dtype), b=b.astype(dtype), act=int(last_act if i == len(dims) - 2 else act), slope=slope))
+    return specs
+
+
+# (sizes at the edges of tiles, of the rows a wave takes and of the LDS; batches around a round of 64 samples)
+CASES = [
+    ("f32", [32, 64, 64, 8], 64), ("f32", [5, 17, 3], 1), ("f32", [16, 16, 16], 63), ("f32", [33, 64, 48, 33, 1], 65), ("f32", [64, 64, 16], 1000),
+    ("f32", [31, 32, 32, 32, 31, 16], 129), ("f32", [1, 1, 1], 200), ("f32", [100, 128, 4], 130), ("f32", [65, 65, 20, 3], 77), ("f32", [16, 64, 64, 64, 64, 2], 300),
+    ("f32", [64, 64, 64, 9], 4097), ("f32", [40, 32, 20, 32, 32, 16], 128), ("f32", [16, 10, 16, 16, 16, 1], 17), ("f32", [12, 50, 2], 2049), ("f32", [30, 40, 33, 64, 7], 190),
+    ("f16", [16, 128, 128, 128, 8], 64), ("f16", [16, 128, 128, 128, 8], 40001), ("f16", [33, 16, 2], 1), ("f16", [64, 64, 64, 16], 65), ("f16", [40, 20, 49, 5], 127),
+    ("f16", [127, 33, 12], 300), ("f16", [48, 96, 80, 3], 200), ("f16", [10, 65, 33, 97, 16], 63), ("f16", [20, 129 - 1, 17, 64, 30, 7], 500), ("f16", [50, 30, 30, 30, 30, 1], 70),
+]
+
+
+@pytest.mark.parametrize("elem,dims,B", CASES)
+@pytest.mark.parametrize("act,slope,last", [(Activation.ReLU, 0.0, Activation.NoActivation), (Activation.LeakyReLU, 0.5, Activation.LeakyReLU)])
+def test_whole_number_networks_are_exact(elem, dims, B, act, slope, last):
+    rng = np.random.default_rng(sum(dims) * 7 + B)
+    dtype, ct = (np.float32, CT.Float32) if elem == "f32" else (np.float16, CT.Float16)
+    if act == Activation.LeakyReLU and len(dims) > (5 if elem == "f32" else 4):
+        # Every leaky layer halves the unit the values are multiples of, forward and backward: with three hidden layers and the
+        # loss scale the gradients are multiples of 2^-7, and sums of a column's entries reach 80, more than 2048 of them (a
+        # half's 11 bits); float's 24 bits last one layer longer in the products of dW.  Slope 0 keeps the units.
+        slope = 0.0
+    specs = whole_number_network(rng, dims, dtype, act, slope, last)
+    x = rng.integers(-1, 2, (B, dims[0])).astype(dtype)
+    t = rng.integers(-2, 3, (B, dims[-1])).astype(dtype)
+    scale = 1.0 / 16
+    dW, dB, loss = reference(specs, x, t, scale)
+    layers = build(specs, ct, preset=1.0)
+    lmax = torch.zeros(1, device=DEV)
+    ws, got = cv.mlpTrainStep(layers, to_dev(x), to_dev(t), lossScale=scale, weightType=ct, lossMax=lmax)
+    assert kernel_of(elem, dims) in cv.lastKernelName(), cv.lastKernelName()
+    gW, gB = read_grads(layers, specs, CT.Float32, ML.TrainingOptimal)
+    for l in range(len(specs)):
+        assert np.array_equal(gW[l] - 1.0, dW[l]), (l, np.abs(gW[l] - 1.0 - dW[l]).max())
+        assert np.array_equal(gB[l] - 1.0, dB[l]), l
+    assert got.item() == loss
+    # the same weights in other layouts, vectors that are no aligned 16-byte pieces: the same bits
+    layouts = [ML.ColumnMajor, ML.InferencingOptimal, ML.TrainingOptimal]
+    other = build(specs, ct, layouts[B % 3], ML.RowMajor, preset=1.0)
+    xs = torch.zeros(B, dims[0] + 3, dtype=torch.float32 if elem == "f32" else torch.float16, device=DEV)
+    xs[:, 1:1 + dims[0]] = to_dev(x)
+    _, got2 = cv.mlpTrainStep(other, xs[:, 1:1 + dims[0]], to_dev(t), lossScale=scale, weightType=ct, workspace=ws)
+    oW, oB = read_grads(other, specs, CT.Float32, ML.RowMajor)
+    for l in range(len(specs)):
+        assert np.array_equal(oW[l], gW[l]) and np.array_equal(oB[l], gB[l]), l
+    assert got2.item() == got.item()
+
+
+@pytest.mark.parametrize("elem,dims,B", [("f32", [32, 64, 64, 8], 5000), ("f32", [9, 30, 12, 3], 777), ("f16", [16, 128, 128, 128, 8], 3000), ("f16", [60, 48, 20, 4], 1500)])
+@pytest.mark.parametrize("act,slope", [(Activation.ReLU, 0.0), (Activation.LeakyReLU, 0.125)])
+@pytest.mark.parametrize("targets", [True, False])
+def test_random_networks(elem, dims, B, act, slope, targets):
+    rng = np.random.default_rng(sum(dims) + B)
+    dtype, ct = (np.float32, CT.Float32) if elem == "f32" else (np.float16, CT.Float16)
+    specs = []
+    for i, (fi, fo) in enumerate(zip(dims, dims[1:])):
+        specs.append(dict(W=(rng.standard_normal((fo, fi)) * np.sqrt(2.0 / fi)).astype(dtype), b=rng.uniform(-0.1, 0.1, fo).astype(dtype) if i != 1 else None,
+                          act=int(Activation.NoActivation if i == len(dims) - 2 else act), slope=slope))
+    x = rng.uniform(-1, 1, (B, dims[0])).astype(dtype)
+    t = rng.uniform(-1, 1, (B, dims[-1])).astype(dtype) if targets else None
+    want_t = t if targets else np.repeat(np.sin(x.astype(np.float64).sum(axis=1, keepdims=True)), dims[-1], axis=1)
+    if elem == "f16":
+        rW, rB, rloss = ob.ref_mlp_train(specs, x, t, 1.0, tie_rule=True)
+        bar = 1e-3
+    else:
+        rW, rB, rloss = reference(specs, x, want_t, 1.0)
+        bar = 2e-5
+    layers, again = build(specs, ct), build(specs, ct)
+    _, loss = cv.mlpTrainStep(layers, to_dev(x), to_dev(t) if targets else None, weightType=ct)
+    assert kernel_of(elem, dims) in cv.lastKernelName(), cv.lastKernelName()
+    _, loss2 = cv.mlpTrainStep(again, to_dev(x), to_dev(t) if targets else None, weightType=ct)
+    dW, dB = read_grads(layers, specs, CT.Float32, ML.TrainingOptimal)
+    for l in range(len(specs)):
+        assert rel_err(dW[l], rW[l]) <= bar and rel_err(dB[l], rB[l]) <= bar, (l, rel_err(dW[l], rW[l]), rel_err(dB[l], rB[l]))
+        assert torch.equal(layers[l].weightsGrad, again[l].weightsGrad) and torch.equal(layers[l].biasesGrad, again[l].biasesGrad)
+    assert abs(loss.item() - rloss) <= bar * rloss and loss.item() == loss2.item()
