@@ -73,6 +73,10 @@ enum : int { kEncodeNone = 0, kEncodeXYSquares = 1 };
 hipError_t launchMlpForward(hipStream_t stream, MmaKind kind, const MlpArgs& args, int numCUs);
 // any layer sizes up to 128 (weights read from LDS); hipErrorInvalidValue beyond that
 hipError_t launchMlpGeneric(hipStream_t stream, MmaKind kind, const MlpArgs& args, int numCUs);
+// the same networks without smooth activations or a conversion of the input (cv_mlp_chain.h); hipErrorInvalidValue otherwise
+hipError_t launchMlpChainF16(hipStream_t stream, const MlpArgs& args, int numCUs);
+hipError_t launchMlpChainFp8(hipStream_t stream, MmaKind kind, const MlpArgs& args, int numCUs);
+hipError_t launchMlpChainFloat(hipStream_t stream, MmaKind kind, const MlpArgs& args, int numCUs);
 // permutohedral encoding of fp16 positions fused in front of an fp16 network (weights in LDS, every dimension <= 128);
 // hipErrorInvalidValue for encoders or networks the kernel does not take
 hipError_t launchPermutoMlp(hipStream_t stream, const CvPermutoDesc& desc, const void* positions, uint64_t positionStride,

@@ -1,0 +1,11 @@
+// cv_mlp_chain_float.hip -- mlpChainKernel for networks of float and of bfloat16.
+#include "cv_mlp_chain.h"
+
+namespace cv {
+
+hipError_t launchMlpChainFloat(hipStream_t stream, MmaKind kind, const MlpArgs& a, int numCUs)
+{
+    return kind == MmaKind::F32 ? launchChain<F32Mma>(stream, a, numCUs) : launchChain<Bf16Mma>(stream, a, numCUs);
+}
+
+} // namespace cv

@@ -207,6 +207,10 @@ hipError_t launchFloat(hipStream_t stream, const MlpArgs& a, int ct, int numCUs)
 hipError_t launchMlpFloat(hipStream_t stream, MmaKind kind, const MlpArgs& a, int numCUs)
 {
     if (a.batch == 0) return hipSuccess;
+    if (kind != MmaKind::F32 && kind != MmaKind::Bf16) return hipErrorInvalidValue;
+    // (mlpFloatKernel stays for smooth activations and rows more than 64 MB apart)
+    const hipError_t e = launchMlpChainFloat(stream, kind, a, numCUs);
+    if (e != hipErrorInvalidValue) return e;
     if (kind == MmaKind::F32) return launchFloat<F32Mma>(stream, a, kF32, numCUs);
     if (kind == MmaKind::Bf16) return launchFloat<Bf16Mma>(stream, a, kBF16, numCUs);
     return hipErrorInvalidValue;

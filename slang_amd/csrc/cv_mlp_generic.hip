@@ -127,6 +127,10 @@ hipError_t launchMlpGenericTaps(hipStream_t stream, const MlpArgs& a, uint8_t* c
 hipError_t launchMlpGeneric(hipStream_t stream, MmaKind kind, const MlpArgs& a, int numCUs)
 {
     if (a.batch == 0) return hipSuccess;
+    // (mlpGenericKernel stays for smooth activations, encoded or quantised inputs and rows more than 64 MB apart)
+    const hipError_t e = kind == MmaKind::F16 ? launchMlpChainF16(stream, a, numCUs)
+                       : kind == MmaKind::Fp8AsF16 || kind == MmaKind::Fp8Native ? launchMlpChainFp8(stream, kind, a, numCUs) : hipErrorInvalidValue;
+    if (e != hipErrorInvalidValue) return e;
     switch (kind) {
     case MmaKind::F16: return launchGeneric<F16Mma>(stream, a, numCUs);
     case MmaKind::Fp8AsF16: return launchGeneric<Fp8AsF16Mma>(stream, a, numCUs);
