@@ -14,8 +14,8 @@
 //     descriptor and a sample beyond the batch lies outside it, and both read as zero without a compare or a mask;
 //   - the loads of the next tiles are issued before the layers of the current ones;
 //   - NT = 2 tiles share every weight fragment read from LDS and give the matrix pipeline twice the independent chains.
-// Measured against the run-time-size kernels: fp32 32-64-64-8 over 2^22 samples 729 -> 554 us (108 TFLOP/s of padded
-// layers, 69 % of what v_mfma_f32_16x16x4_f32 issues at most), fp16 20-48-24-5 over 2 000 003 samples 78 -> 51 us.
+// Measured against the run-time-size kernels: fp32 32-64-64-8 over 2^22 samples 729 -> 522 us (115 TFLOP/s of padded
+// layers, 73 % of what v_mfma_f32_16x16x4_f32 issues at most), fp16 20-48-24-5 over 2 000 003 samples 78 -> 45 us.
 #pragma once
 #include <type_traits>
 
@@ -59,25 +59,26 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
 #pragma unroll
     for (int kt = 0; kt < MAXKT; ++kt) {
         if (kt == 0 || kt < KT) {
-            // groups of four row tiles: their fragments are read together, and with fp32's eight matrix instructions per
-            // fragment no instruction waits for the one before it
+            // groups of row tiles whose fragments are read together: four sums side by side, so that none of fp32's eight
+            // matrix instructions per fragment waits for the one before it, and no more registers than that takes
+            constexpr int G = F32 && NT == 2 ? 2 : 4;
 #pragma unroll
-            for (int t0 = 0; t0 < MT; t0 += 4) {
-                uint32_t w[4][FD];
+            for (int t0 = 0; t0 < MT; t0 += G) {
+                uint32_t w[G][FD];
 #pragma unroll
-                for (int t = t0; t < MT && t < t0 + 4; ++t) Mma::decode(wbase + (size_t)(t * KT + kt) * 64 * RAW, w[t - t0]);
+                for (int t = t0; t < MT && t < t0 + G; ++t) Mma::decode(wbase + (size_t)(t * KT + kt) * 64 * RAW, w[t - t0]);
                 if constexpr (F32) {
 #pragma unroll
                     for (int s = 0; s < 8; ++s)
 #pragma unroll
-                        for (int t = t0; t < MT && t < t0 + 4; ++t)
+                        for (int t = t0; t < MT && t < t0 + G; ++t)
 #pragma unroll
                             for (int nt = 0; nt < NT; ++nt)
                                 acc[nt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, w[t - t0][s]),
                                                                                   __builtin_bit_cast(float, act[nt][kt][s]), acc[nt][t], 0, 0, 0);
                 } else {
 #pragma unroll
-                    for (int t = t0; t < MT && t < t0 + 4; ++t)
+                    for (int t = t0; t < MT && t < t0 + G; ++t)
 #pragma unroll
                         for (int nt = 0; nt < NT; ++nt) acc[nt][t] = Mma::mma(w[t - t0], act[nt][kt], acc[nt][t]);
                 }
@@ -177,9 +178,10 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
 }
 
 // MAXT: the bound on a layer's row tiles; NT: 16-sample tiles per wave and round; QUAD: input vectors of whole, aligned
-// groups of four elements, which one load takes (else one load per element, any size and alignment)
+// groups of four elements, which one load takes (else one load per element, any size and alignment).
+// fp32 up to 64 wide: three waves per SIMD, four registers short of it, measure 522 us where two without a spill take 554.
 template <class Mma, int MAXT, int NT, bool QUAD>
-__global__ __launch_bounds__(256) void mlpChainKernel(const GenArgs ga)
+__global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1) void mlpChainKernel(const GenArgs ga)
 {
     constexpr int MAXKT = MAXT / 2, FD = Mma::kFD, ESZ = Mma::kEsz, RAW = Mma::kRawDW;
     constexpr int UNITS = QUAD ? 2 : 8;                    // loads per fragment
@@ -216,6 +218,7 @@ __global__ __launch_bounds__(256) void mlpChainKernel(const GenArgs ga)
         }
 
     const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + 15) / 16), step = gridDim.x * 4u * NT;
+    const int kt0 = ga.gl[0].kt;
     uint32_t raw[NT][MAXKT][UNITS * UDW];
     auto fetch = [&](uint32_t tile) {
 #pragma unroll
@@ -229,6 +232,7 @@ __global__ __launch_bounds__(256) void mlpChainKernel(const GenArgs ga)
             for (int kt = 0; kt < MAXKT; ++kt)
 #pragma unroll
                 for (int u = 0; u < UNITS; ++u) {
+                    if (kt > 0 && kt >= kt0) continue;       // (wave-uniform; empty loads of absent k-tiles cost 6 us of 51)
                     uint32_t* r = raw[nt][kt] + u * UDW;
                     if constexpr (QUAD && ESZ == 4) {
                         const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, off[kt][u], 0, 0));
