@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void permutoEncodeKernel(const PermutoArgs a)
 // system does not merge: 2.1 bytes written per byte of output), no thread loops over levels, and a feature table that
 // fits is held in LDS, where a gather of 64 scattered entries costs a few cycles instead of one cache line per lane.
 // The arithmetic per (position, level) is that of permutoEncodeKernel, instruction for instruction.
-template <typename T, int D, int F, bool LDS_TABLE>
+template <typename T, int D, int F, bool LDS_TABLE, bool PLAIN>
 __global__ __launch_bounds__(1024) void permutoEncodePairsKernel(const PermutoArgs a, uint32_t tableElems, uint32_t levelShift)
 {
     typedef typename PermutoEntry<T, F>::type Entry;
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(1024) void permutoEncodePairsKernel(const PermutoAr
         float pos[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) pos[d] = (float)((const T*)(a.pos + (size_t)s * a.posStride))[d];
-        const Entry acc = permutoEncodeEntry<T, D, F>(pos, lv, table, a.desc.maxLevel);
+        const Entry acc = permutoEncodeEntry<T, D, F, PLAIN>(pos, lv, table, a.desc.maxLevel);
         // (a streaming store: the encoded vectors are written once and read by the next kernel)
         __builtin_nontemporal_store(acc, (Entry*)((T*)(a.out + (size_t)s * a.outStride) + lv.currentLevelIndex * F));
     }
@@ -389,15 +389,18 @@ hipError_t launchEncodePairs(hipStream_t stream, const PermutoArgs& a)
     const dim3 grid((uint32_t)(want < cap ? want : cap)), block(1024);
     const uint32_t L = a.desc.maxLevels;
     const uint32_t shift = (L & (L - 1u)) == 0u ? (uint32_t)__builtin_ctz(L) : 0xffffffffu;
-    hipError_t e;
-    if (inLds) {
-        e = allowDynamicLds<permutoEncodePairsKernel<T, D, F, true>>((int)(kPairsLevelBytes + kPairsTableBytes));
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((permutoEncodePairsKernel<T, D, F, true>), grid, block, lds, stream, a, (uint32_t)tableElems, shift);
-    } else {
-        hipLaunchKernelGGL((permutoEncodePairsKernel<T, D, F, false>), grid, block, lds, stream, a, (uint32_t)tableElems, shift);
-    }
-    return hipGetLastError();
+    auto launch = [&](auto plainConst) -> hipError_t {
+        constexpr bool PLAIN = decltype(plainConst)::value;
+        if (inLds) {
+            const hipError_t e = allowDynamicLds<permutoEncodePairsKernel<T, D, F, true, PLAIN>>((int)(kPairsLevelBytes + kPairsTableBytes));
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL((permutoEncodePairsKernel<T, D, F, true, PLAIN>), grid, block, lds, stream, a, (uint32_t)tableElems, shift);
+        } else {
+            hipLaunchKernelGGL((permutoEncodePairsKernel<T, D, F, false, PLAIN>), grid, block, lds, stream, a, (uint32_t)tableElems, shift);
+        }
+        return hipGetLastError();
+    };
+    return permutoPlainLevels(a.desc) ? launch(std::true_type()) : launch(std::false_type());
 }
 
 // the kernel above takes entries of 4, 8 or 16 bytes at addresses that are multiples of their size

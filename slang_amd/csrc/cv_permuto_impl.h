@@ -82,7 +82,10 @@ __device__ __forceinline__ void barycentricWeights(const float* elevated, const 
 // (hash = sum key[d] * c^(D-d)), so the hash of vertex k is that of vertex k-1 plus the sum of the multipliers, less
 // (D+1) times the multiplier of the dimension ranked D+1-k: three integer multiplies per position instead of three per
 // vertex, same 32-bit values.
-template <int D>
+// PLAIN (permutoPlainLevels): the table of the level has 2^n entries, n <= 24.  Then no lane needs the remainder, whose
+// branch cost four divergent regions per level and kept the loads of the vertices apart, and the hash only counts modulo
+// 2^24, which the full-rate 24-bit multiplies give.
+template <int D, bool PLAIN = false>
 __device__ __forceinline__ void vertexIndices(const CvPermutoLevelInfo& lv, int F, const int* rem0, const int* rank, uint32_t* idx)
 {
     constexpr uint32_t c = 2531011u;
@@ -91,7 +94,10 @@ __device__ __forceinline__ void vertexIndices(const CvPermutoLevelInfo& lv, int 
     for (int dim = D - 1; dim >= 0; --dim) { mult[dim] = p; all += p; p *= c; }
     uint32_t hash = 0u;
 #pragma unroll
-    for (int dim = 0; dim < D; ++dim) hash += (uint32_t)rem0[dim] * mult[dim];
+    for (int dim = 0; dim < D; ++dim) {
+        if constexpr (PLAIN) hash += ((uint32_t)rem0[dim] & 0xffffffu) * (mult[dim] & 0xffffffu);
+        else hash += (uint32_t)rem0[dim] * mult[dim];
+    }
     // (a table of 2^n entries, which is what prepareLevelInfo makes, is indexed with a mask: the general remainder
     // is a division by a run-time value, some forty instructions per vertex)
     const uint32_t size = lv.featureTableSize, base = lv.offsetOfFeatureTable * (uint32_t)F;
@@ -104,9 +110,21 @@ __device__ __forceinline__ void vertexIndices(const CvPermutoLevelInfo& lv, int 
             for (int dim = 0; dim < D; ++dim) less = rank[dim] == D + 1 - k ? (uint32_t)(D + 1) * mult[dim] : less;
             hash += all - less;
         }
-        const uint32_t slot = pow2 ? (hash & (size - 1u)) : hash % size;
+        const uint32_t slot = PLAIN || pow2 ? (hash & (size - 1u)) : hash % size;
         idx[k] = base + slot * (uint32_t)F;
     }
+}
+
+// Every level has a table of 2^n entries, n <= 24, and none lies beyond maxLevel: what an encoder prepared by the library
+// and used with all its levels has.  (A table of no entries is not plain.)
+inline bool permutoPlainLevels(const CvPermutoDesc& desc)
+{
+    for (uint32_t l = 0; l < desc.maxLevels; ++l) {
+        const CvPermutoLevelInfo& lv = desc.levelInfo[l];
+        const uint32_t size = lv.featureTableSize;
+        if (size == 0u || size > (1u << 24) || (size & (size - 1u)) != 0u || (float)lv.currentLevelIndex >= desc.maxLevel + 1e-3f) return false;
+    }
+    return true;
 }
 
 // F consecutive elements of type T: one entry of the feature table, one level's share of an encoded vector
@@ -116,20 +134,21 @@ struct PermutoEntry { typedef T type __attribute__((ext_vector_type(F))); };
 // One level of encode for one position (:259-317): zeros beyond maxLevel, else the entries of the simplex vertices
 // weighted in T, vertex by vertex.  `table` may point to memory or to a copy of the table in LDS; entries are read
 // whole, so `table` and every entry offset must be multiples of the entry size.
-template <typename T, int D, int F>
+// PLAIN: a level of an encoder that permutoPlainLevels accepts.
+template <typename T, int D, int F, bool PLAIN = false>
 __device__ __forceinline__ typename PermutoEntry<T, F>::type permutoEncodeEntry(const float* pos, const CvPermutoLevelInfo& lv, const T* table, float maxLevel)
 {
     typedef typename PermutoEntry<T, F>::type Entry;
     Entry acc;
 #pragma unroll
     for (int f = 0; f < F; ++f) acc[f] = (T)0.f;
-    if (!((float)lv.currentLevelIndex >= maxLevel + 1e-3f)) {   // zero padding beyond maxLevel, :259-262
+    if (PLAIN || !((float)lv.currentLevelIndex >= maxLevel + 1e-3f)) {   // zero padding beyond maxLevel, :259-262
         float elevated[D + 1], bary[D + 2];
         int rem0[D + 1], rank[D + 1];
         latticeGeometry<D>(pos, lv, elevated, rem0, rank);
         barycentricWeights<D>(elevated, rem0, rank, bary);
         uint32_t idx[D + 1];
-        vertexIndices<D>(lv, F, rem0, rank, idx);
+        vertexIndices<D, PLAIN>(lv, F, rem0, rank, idx);
         Entry e[D + 1];
 #pragma unroll
         for (int k = 0; k <= D; ++k) e[k] = *(const Entry*)(table + idx[k]);

@@ -33,7 +33,7 @@ struct PermutoMlpArgs {
 constexpr uint32_t kLevelDwords = CV_PERMUTO_MAX_LEVELS * sizeof(CvPermutoLevelInfo) / 4;
 constexpr uint32_t kLdsLimitDwords = 160 * 1024 / 4;
 
-template <int D, int F, int MAXT, bool LDS_TABLE>
+template <int D, int F, int MAXT, bool LDS_TABLE, bool PLAIN>
 __global__ __launch_bounds__(1024) void permutoMlpKernel(const PermutoMlpArgs pa)
 {
     using Mma = F16Mma;
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(1024) void permutoMlpKernel(const PermutoMlpArgs pa
 #pragma unroll
                 for (int f = 0; f < F; ++f) v[f] = (half_t)0.f;
 #ifndef PM_NO_ENCODE
-                if (level < pa.desc.maxLevels) v = permutoEncodeEntry<half_t, D, F>(pos, levels[level], table, pa.desc.maxLevel);
+                if (level < pa.desc.maxLevels) v = permutoEncodeEntry<half_t, D, F, PLAIN>(pos, levels[level], table, pa.desc.maxLevel);
 #else
                 v[0] = (half_t)pos[0];
 #endif
@@ -131,12 +131,16 @@ hipError_t launchShape(hipStream_t stream, PermutoMlpArgs& pa, uint32_t netDword
         hipLaunchKernelGGL(kernel, dim3(need < cap ? need : cap), dim3(1024), ldsBytes, stream, pa);
         return hipGetLastError();
     };
-    if (inLds) {
-        const hipError_t e = allowDynamicLds<permutoMlpKernel<D, F, MAXT, true>>((int)(kLdsLimitDwords * 4));
-        return e != hipSuccess ? e : launch(permutoMlpKernel<D, F, MAXT, true>);
-    }
-    const hipError_t e = allowDynamicLds<permutoMlpKernel<D, F, MAXT, false>>((int)(kLdsLimitDwords * 4));
-    return e != hipSuccess ? e : launch(permutoMlpKernel<D, F, MAXT, false>);
+    auto launchLevels = [&](auto plainConst) -> hipError_t {
+        constexpr bool PLAIN = decltype(plainConst)::value;
+        if (inLds) {
+            const hipError_t e = allowDynamicLds<permutoMlpKernel<D, F, MAXT, true, PLAIN>>((int)(kLdsLimitDwords * 4));
+            return e != hipSuccess ? e : launch(permutoMlpKernel<D, F, MAXT, true, PLAIN>);
+        }
+        const hipError_t e = allowDynamicLds<permutoMlpKernel<D, F, MAXT, false, PLAIN>>((int)(kLdsLimitDwords * 4));
+        return e != hipSuccess ? e : launch(permutoMlpKernel<D, F, MAXT, false, PLAIN>);
+    };
+    return permutoPlainLevels(pa.desc) ? launchLevels(std::true_type()) : launchLevels(std::false_type());
 }
 
 } // namespace

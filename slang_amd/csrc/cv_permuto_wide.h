@@ -15,7 +15,9 @@
 namespace cv {
 namespace {
 
-template <int K0, int D, int F>
+// PLAIN (permutoPlainLevels): no branch inside a level.  3-d, 8 levels of 2^12 two-feature entries, 16-64-64-3, 2^22
+// positions: 241 -> 224 us; smaller decoders 1.13 to 1.24 times as fast.
+template <int K0, int D, int F, bool PLAIN>
 struct Wide16PermutoFront {
     struct Input { half_t pos[2][D]; };
     const uint8_t* pos; uint64_t posStride;
@@ -50,11 +52,16 @@ struct Wide16PermutoFront {
 #pragma unroll
                 for (int c = 0; c < PER; ++c) {
                     const int level = (2 * s + h) * PER + c;
-                    const auto e = permutoEncodeEntry<half_t, D, F>(p, levels[level], table, maxLevel);
+                    const auto e = permutoEncodeEntry<half_t, D, F, PLAIN>(p, levels[level], table, maxLevel);
 #pragma unroll
                     for (int f = 0; f < F; ++f) {
                         const int q = c * F + f;
                         v[q / 2] |= (uint32_t)__builtin_bit_cast(uint16_t, (half_t)e[f]) << (16 * (q & 1));
+                    }
+                    // without branches between the entries the scheduler would mix all of them and run out of registers: two
+                    // at a time (four dimensions or 32 inputs: one) cover the latency of their loads
+                    if constexpr (PLAIN) {
+                        if (D == 4 || K0 == 32 || c % 2 == 1 || c + 1 == PER) __builtin_amdgcn_sched_barrier(0);
                     }
                 }
 #pragma unroll
@@ -74,7 +81,7 @@ struct PermutoWideArgs {
 
 constexpr uint32_t kWideLevelBytes = CV_PERMUTO_MAX_LEVELS * sizeof(CvPermutoLevelInfo);
 
-template <int H, int NH, int K0, int WAVES, int D, int F>
+template <int H, int NH, int K0, int WAVES, int D, int F, bool PLAIN>
 __global__ __launch_bounds__(64 * WAVES) void permutoWide16Kernel(const PermutoWideArgs pa)
 {
     typedef typename PermutoEntry<half_t, F>::type Entry;
@@ -87,17 +94,17 @@ __global__ __launch_bounds__(64 * WAVES) void permutoWide16Kernel(const PermutoW
         for (uint32_t i = threadIdx.x; i < pa.tableElems / (uint32_t)F; i += blockDim.x) dst[i] = t[i];
     }
     // (the body synchronises the workgroup after it has staged the weights, before any wave encodes)
-    const Wide16PermutoFront<K0, D, F> front{pa.pos, pa.posStride, (const CvPermutoLevelInfo*)dyn, (const half_t*)(dyn + kWideLevelBytes), pa.desc.maxLevel};
+    const Wide16PermutoFront<K0, D, F, PLAIN> front{pa.pos, pa.posStride, (const CvPermutoLevelInfo*)dyn, (const half_t*)(dyn + kWideLevelBytes), pa.desc.maxLevel};
     mlpWide16Body<H, NH, K0, WAVES, true>(pa.mlp, front);
 }
 
-template <int H, int NH, int K0, int D, int F>
+template <int H, int NH, int K0, int D, int F, bool PLAIN>
 hipError_t launchPermutoWide16Shape(hipStream_t stream, const PermutoWideArgs& pa, int numCUs)
 {
     // waves per workgroup (= per compute unit) as the registers allow; with two or more per SIMD one encodes while another
     // is in the matrix pipeline.  The build fails if an instantiation spills.
     constexpr int WAVES = H == 1 ? 16 : (NH == 1 ? 12 : 8);
-    auto kernel = permutoWide16Kernel<H, NH, K0, WAVES, D, F>;
+    auto kernel = permutoWide16Kernel<H, NH, K0, WAVES, D, F, PLAIN>;
     // LDS the kernel declares itself (weights in operand order, biases): a property of the instantiation, asked once
     static const size_t staticLds = [&]() -> size_t {
         hipFuncAttributes attr;
@@ -105,7 +112,7 @@ hipError_t launchPermutoWide16Shape(hipStream_t stream, const PermutoWideArgs& p
     }();
     const size_t dynBytes = kWideLevelBytes + (size_t)pa.tableElems * 2;
     if (staticLds + dynBytes > 160 * 1024) return hipErrorInvalidValue;      // the table does not fit beside the weights
-    hipError_t e = allowDynamicLds<permutoWide16Kernel<H, NH, K0, WAVES, D, F>>((int)dynBytes);
+    hipError_t e = allowDynamicLds<permutoWide16Kernel<H, NH, K0, WAVES, D, F, PLAIN>>((int)dynBytes);
     if (e != hipSuccess) return e;
     const uint32_t numPairs = ((pa.mlp.batch + 31u) / 32u + 1u) / 2u;
     const uint32_t blocks = numPairs < (uint32_t)numCUs ? numPairs : (uint32_t)numCUs;
@@ -119,7 +126,9 @@ template <int K0>
 hipError_t launchPermutoWide16K(hipStream_t stream, const PermutoWideArgs& pa, int numCUs, int H, int NH)
 {
     const int D = pa.desc.dimensions, F = pa.desc.featureDimensionPerEntry;
-#define CV_PW(h_, nh_, d_, f_) if (H == h_ && NH == nh_ && D == d_ && F == f_) return launchPermutoWide16Shape<h_, nh_, K0, d_, f_>(stream, pa, numCUs);
+    const bool plain = permutoPlainLevels(pa.desc);
+#define CV_PW(h_, nh_, d_, f_) if (H == h_ && NH == nh_ && D == d_ && F == f_) \
+    return plain ? launchPermutoWide16Shape<h_, nh_, K0, d_, f_, true>(stream, pa, numCUs) : launchPermutoWide16Shape<h_, nh_, K0, d_, f_, false>(stream, pa, numCUs);
 #define CV_PW_D(h_, nh_) CV_PW(h_, nh_, 2, 2) CV_PW(h_, nh_, 3, 2) CV_PW(h_, nh_, 4, 2)
     CV_PW_D(1, 1) CV_PW_D(1, 2) CV_PW_D(2, 1) CV_PW_D(2, 2)
 #undef CV_PW_D

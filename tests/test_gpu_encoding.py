@@ -297,3 +297,38 @@ def test_encoder_and_network_argument_checks():
         enc5.encodeAndEval(to_dev(rng.uniform(0, 1, (8, 5)).astype(np.float16)),
                            to_dev(rng.standard_normal(enc5.featureTableElements).astype(np.float16)), build(make_specs(rng, [8, 16, 4])))
     assert e.value.result == cv.SLANG_E_NOT_AVAILABLE
+
+
+@pytest.mark.parametrize("D,F,levels_n,log2,dims,B", [
+    (3, 2, 8, 12, [16, 64, 64, 3], 4099),       # permutoWide16Kernel, 16 inputs
+    (2, 2, 16, 8, [32, 32, 4], 777),            # 32 inputs
+    (4, 2, 8, 10, [16, 64, 8], 65),
+    (4, 2, 16, 9, [32, 32, 32, 4], 1000),
+    (2, 4, 4, 8, [16, 32, 5], 17),              # permutoMlpKernel
+    (3, 2, 8, 15, [16, 64, 64, 3], 2500),       # a table in memory
+])
+@pytest.mark.parametrize("reach", [2.0, 3000.0])
+def test_encoder_with_all_levels_in_use(D, F, levels_n, log2, dims, B, reach):
+    # every level active and every table of 2^n entries, the kernels without branches inside a level: against the oracle, and
+    # against the general kernels, which an encoder takes as soon as one of its tables has another size.  `reach`: lattice
+    # coordinates beyond 24 bits of hash
+    rng = np.random.default_rng(D * 100 + F * 10 + len(dims))
+    enc = cv.PermutoEncoder(D, F, log2, levels_n, baseScale=2.0, log2PerLevelScale=0.9, seed=5, dtype=torch.float16)
+    pos = to_dev(rng.uniform(-reach, reach, (B, D)).astype(np.float16))
+    table = to_dev((rng.standard_normal(enc.featureTableElements) * 0.5).astype(np.float16))
+    layers = build(make_specs(rng, dims))
+    feats = enc.encode(pos, table)
+    ref = ob.permuto_encode(ob.permuto_levels(D, log2, levels_n, 2.0, 0.9, 5), F, float(np.float32(1.1) * np.float32(levels_n)),
+                            pos.cpu().numpy(), table.cpu().numpy())
+    assert np.array_equal(feats.cpu().numpy(), ref)
+    want = cv.mlpForward(layers, feats)
+    assert torch.equal(enc.encodeAndEval(pos, table, layers), want)
+    assert torch.equal(enc.encodeAndEval(pos, table, layers, flags=cv.FLAG_FORWARD_TILE16), want)
+    odd = levels_n // 2
+    enc.desc.levelInfo[odd].featureTableSize = (1 << log2) - 3
+    feats2 = enc.encode(pos, table)
+    keep = [i for i in range(levels_n * F) if i // F != odd]
+    assert torch.equal(feats2[:, keep], feats[:, keep]) and (B < 32 or not torch.equal(feats2, feats))
+    want2 = cv.mlpForward(layers, feats2)
+    assert torch.equal(enc.encodeAndEval(pos, table, layers), want2)
+    assert torch.equal(enc.encodeAndEval(pos, table, layers, flags=cv.FLAG_FORWARD_TILE16), want2)
