@@ -866,7 +866,13 @@ static CvResult trainStep(const char* who, void* stream, const CvMlpDesc* mlp, c
     const int cus = currentDeviceCUs(&rc);
     if (CV_FAILED(rc)) return rc;
     size_t need = 0;
-    const TrainStepKind kind = chooseTrainStep(t.mlp, mlp->flags, t.carrierCt, cus, &need);
+    TrainStepKind kind = chooseTrainStep(t.mlp, mlp->flags, t.carrierCt, cus, &need);
+    // The step over rounds keeps a whole set of gradients per workgroup (37 MB for 16-128-128-128-8), the step in memory the
+    // batch's vectors: a small batch of a wide network fits the built-in array only the second way.
+    if (ownScratch && kind == TrainStepKind::Rounds && workspaceBytes < need) {
+        const size_t general = cv::trainGeneralWorkspaceBytes(t.mlp, cus, t.carrierCt);
+        if (general <= workspaceBytes) { kind = TrainStepKind::General; need = general; }
+    }
     if (workspaceBytes < need) {
         if (ownScratch)
             return fail(CV_E_NOT_AVAILABLE, "%s: this network needs %zu bytes of scratch, the built-in array holds %zu; "
