@@ -490,7 +490,7 @@ def workload_c5(torch, cv, steps, warmup, flags=0, dims=None, key=None, leaky=Fa
 
 def workload_f32t(torch, cv, steps, warmup):
     """fp32 training step 32->64->64->8 (FFLayer<float> chain), ReLU, MSE against given targets, batch 2^20, fp32 TrainingOptimal
-    gradients: the layer-by-layer step on the fp32 matMul, element-wise and outer-product kernels."""
+    gradients: the step in LDS (trainWaveKernel)."""
     import numpy as np
     from slang_amd.coopvec import (Activation, CoopVecComponentType as CT, CoopVecMatrixLayout as ML,
                                    FeedForwardLayer)
@@ -543,13 +543,10 @@ def workload_f32t(torch, cv, steps, warmup):
                 "sample": "first %d samples; numpy fp32 backpropagation (for T = float the fallback's arithmetic is plain fp32 "
                           "products and sums)" % n}
 
-    # (the bytes a layer-by-layer step moves: every per-layer vector of the batch is written once and read by its consumers)
-    widths = dims[1:]
-    moved = B * 4 * (dims[0] * 2 + dims[-1] + sum(w * (2 + 3) for w in widths[:-1]) + widths[-1] * 4 + sum(w * 4 for w in widths[:-1]))
-    return dict(step=step, samples=B, alg_bytes=moved, alg_flops=B * 2 * (2 * macs + macs_dx),
-                bound="hbm", mfma="f32", dtype="f32",
+    return dict(step=step, samples=B, alg_bytes=B * 4 * (dims[0] + dims[-1]), alg_flops=B * 2 * (2 * macs + macs_dx),
+                bound="mfma", mfma="f32", dtype="f32",
                 config={"workload": "f32t: fp32 train step 32->64->64->8, ReLU, MSE against targets, batch 2^20, fp32 "
-                                    "TrainingOptimal gradients, layer-by-layer step (fp32 networks have no fused one)",
+                                    "TrainingOptimal gradients, step in LDS",
                         "batch": B, "layers": dims},
                 cpu_baseline=cpu_baseline, key="f32t")
 

@@ -106,7 +106,7 @@ typedef enum CvActivation {
  * ~2^-12 * sum|terms|.  No effect on other types. */
 #define CV_FLAG_FP8_MATRIX_PIPELINE 1u
 /* cvMlpTrainStep[WorkspaceSize]: take the layer-by-layer step (the one that serves any layer sizes)
- * also where a fused kernel exists.  Same rounding points; for cross-checking the two. */
+ * also where a fused kernel or the step in LDS would take the network.  Same rounding points; for cross-checking the two. */
 #define CV_FLAG_LAYERWISE_TRAINING 2u
 /* cvMlpForward: keep to the kernels that work on 16-sample tiles (cross-checks of the 32-sample-tile kernels) */
 #define CV_FLAG_FORWARD_TILE16 4u
@@ -412,7 +412,7 @@ typedef struct CvMlpDesc {
     int32_t  inputType;         /* element type of the input vectors in memory */
     int32_t  weightType;        /* matrix interpretation of every layer: FLOAT16 or FLOAT_E4M3; FLOAT32 or BFLOAT16 for
                                    a network of that one type (vectors, biases, results and targets too; BFLOAT16 forward
-                                   only, FLOAT32 also trains: layer by layer, FLOAT32 gradients) */
+                                   only, FLOAT32 also trains) */
     int32_t  biasType;          /* FLOAT16 (weightType for FLOAT32 / BFLOAT16 networks) */
     int32_t  outputType;        /* FLOAT16 (weightType for FLOAT32 / BFLOAT16 networks) */
     int32_t  gradType;          /* FLOAT16 or FLOAT32: element type of weightsGrad/biasesGrad */

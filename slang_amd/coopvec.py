@@ -709,7 +709,7 @@ def mlpTrainStep(layers: Sequence[FeedForwardLayer], input: torch.Tensor, target
     weight gradients accumulated into every layer's weightsGrad (coopVecOuterProductAccumulate,
     fflayer.slang:35-41) and bias gradients into biasesGrad (coopVecReduceSumAccumulate, :44),
     deterministically.  Returns (workspace, lossSum) so that both can be reused.  weightType Float32: a network
-    of float (vectors, targets, parameters), stepped layer by layer with Float32 gradients.  lossMax (one float32 on
+    of float (vectors, targets, parameters).  lossMax (one float32 on
     the device) receives the largest per-sample loss, the figure learnGradient leaves in its loss buffer
     (kernels.slang:21-26)."""
     _, inStride = _vector_info(input, weightType, "input")

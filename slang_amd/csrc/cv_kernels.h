@@ -101,7 +101,7 @@ struct TrainLaunch {
     uint8_t* bGrad[kMaxMlpLayers];
     MatrixShape gradShape[kMaxMlpLayers];
     int32_t gradCt;
-    int32_t carrierCt;           // kF16, or kF32 for a network of float (layer-by-layer step only)
+    int32_t carrierCt;           // kF16, or kF32 for a network of float (not the fused kernels)
     float* lossSum;
     float* lossMax;              // optional: max over the samples of the per-sample loss
     float* workspace;            // partials

@@ -12,7 +12,7 @@
 // partials and second stage are those of the other fused kernels (fixed order, no atomics, bitwise reproducible).
 //
 // LDS: W and W^T of 16-128-128-8 are 84 KB, the tiles of a round 36 + 32 KB: 153 KB; a third 128-wide hidden layer does not
-// fit (148 KB of weights), such networks train layer by layer.
+// fit (148 KB of weights), such networks take the step in LDS (cv_train_round.h).
 #pragma once
 #include "cv_train_pair.h"
 
@@ -60,7 +60,7 @@ struct QuadSplit {
 
 // ReLU on the hidden layers (LEAKY: each hidden layer ReLU or leaky ReLU, as the arguments say: max(z, z*slope) with the
 // product rounded to fp16, fflayer.slang:64-65), none on the last one (the launcher sends everything else to the
-// layer-by-layer step).
+// step in LDS or the layer-by-layer step).
 template <class Net, bool LEAKY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mlpTrainQuadKernel(const TrainArgs ta)
 {
