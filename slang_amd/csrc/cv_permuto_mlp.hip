@@ -93,11 +93,7 @@ __global__ __launch_bounds__(1024) void permutoMlpKernel(const PermutoMlpArgs pa
                 Entry v;
 #pragma unroll
                 for (int f = 0; f < F; ++f) v[f] = (half_t)0.f;
-#ifndef PM_NO_ENCODE
                 if (level < pa.desc.maxLevels) v = permutoEncodeEntry<half_t, D, F, PLAIN>(pos, levels[level], table, pa.desc.maxLevel);
-#else
-                v[0] = (half_t)pos[0];
-#endif
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
                     const int q = e * F + f;
@@ -106,11 +102,7 @@ __global__ __launch_bounds__(1024) void permutoMlpKernel(const PermutoMlpArgs pa
                 }
             }
         }
-#ifndef PM_NO_MLP
         genericRunLayers<Mma, MAXT, false>(ga, lds, lane, sample, act);      // plain, ReLU and leaky ReLU layers
-#else
-        if (sample < a.batch && g == 0) *(uint16_t*)(a.out + (size_t)sample * a.outStride) = (uint16_t)(act[0][0] ^ act[0][1]);
-#endif
     }
 }
 
