@@ -17,6 +17,7 @@
 #include "cv_kernels.h"
 #include "cv_launch.h"
 #include "cv_permuto_impl.h"
+#include "cv_permuto_parts.h"
 
 namespace cv {
 namespace {
@@ -324,14 +325,7 @@ __global__ __launch_bounds__(256) void permutoBackwardKernel(const PermutoArgs a
 // The table gradient, by parts of the table small enough for LDS: part p covers elements [base, base + elems), which
 // levels [first, end) add to.  Every position adds to a handful of entries per level; added in memory, where many positions
 // meet on few addresses, 2^18 positions in 3 dimensions on 8 levels of 2^12 two-feature entries took 6.6 ms (2.5 G additions
-// per second); here 40 us, of which a quarter is the start and the sums' way to memory.
-constexpr int kMaxTableParts = 144;      // with the encoder's description within 4 KB of kernel arguments
-struct TablePart { uint32_t base, elems, first, end; };
-struct TableParts {
-    TablePart part[kMaxTableParts];
-    uint32_t count, groups;          // parts, and workgroups to a part
-    uint32_t sliced;                 // some part is a slice of a level's entries
-};
+// per second); here 40 us, of which a quarter is the start and the sums' way to memory.  (cutTable: cv_permuto_parts.h)
 static_assert(sizeof(PermutoArgs) + sizeof(TableParts) <= 4096, "kernel arguments");
 
 // A workgroup owns one part and a share of the positions: it sums into LDS and adds its sums to memory once, coalesced
@@ -436,51 +430,13 @@ hipError_t launchEncode(hipStream_t stream, const PermutoArgs& a)
     return hipGetLastError();
 }
 
-// Cuts the table into parts for permutoTableGradKernel: consecutive levels as long as they fit half of a compute unit's LDS
-// together, so that two workgroups of 16 waves share it; a level beyond that by itself, up to the whole 160 KB; and a level
-// beyond those in slices of its entries, each walked by all positions of the batch.  A slice repeats the search for the
-// simplex: 2^18 positions on 8 levels of 2^16 two-feature entries, seven slices each, take 128 us, on levels of 2^17 in
-// thirteen slices 219 us, and either takes 6.3 to 6.7 ms with the additions in memory.  Sixteen slices at most, since the list of
-// parts travels with the kernel's arguments.
-// False: more parts than that, or levels that do not lie behind one another as prepareLevelInfo puts them.
-bool cutTable(const PermutoArgs& a, TableParts& t)
-{
-    constexpr uint64_t kHalf = 80 * 1024 / 8, kWhole = 160 * 1024 / 8;      // elements
-    const uint64_t F = (uint64_t)a.desc.featureDimensionPerEntry;
-    t.count = 0;
-    t.sliced = 0;
-    uint64_t next = 0;
-    for (uint32_t l = 0; l < a.desc.maxLevels; ++l) {
-        const CvPermutoLevelInfo& lv = a.desc.levelInfo[l];
-        if ((uint64_t)lv.offsetOfFeatureTable * F != next) return false;
-        const uint64_t elems = (uint64_t)lv.featureTableSize * F;
-        next += elems;
-        if (next > 0xffffffffull) return false;
-        TablePart* last = t.count ? &t.part[t.count - 1] : nullptr;
-        if (last && last->end == l && (uint64_t)last->elems + elems <= kHalf) {
-            last->elems += (uint32_t)elems;
-            last->end = l + 1;
-            continue;
-        }
-        const uint64_t slices = (elems + kWhole - 1) / kWhole;
-        if (slices > 16) return false;
-        if (slices > 1) t.sliced = 1;
-        const uint64_t perSlice = ((uint64_t)lv.featureTableSize + slices - 1) / (slices ? slices : 1) * F;
-        for (uint64_t at = 0; at < elems; at += perSlice) {
-            if (t.count == (uint32_t)kMaxTableParts) return false;
-            t.part[t.count++] = TablePart{(uint32_t)(next - elems + at), (uint32_t)(elems - at < perSlice ? elems - at : perSlice), l, l + 1};
-        }
-    }
-    return t.count > 0;
-}
-
 template <int D, int FT, bool POS, bool SLICED>
 hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, TableParts& t, int cus)
 {
     uint32_t most = 0;
     for (uint32_t p = 0; p < t.count; ++p) most = t.part[p].elems > most ? t.part[p].elems : most;
     const size_t lds = (size_t)most * 8;
-    const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED>>(160 * 1024);
+    const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED>>((int)(kPartMost * 8));
     if (e != hipSuccess) return e;
     // as many workgroups as the compute units hold, dealt evenly to the parts
     const uint32_t resident = (uint32_t)cus * (lds <= 80 * 1024 ? 2u : 1u), want = (a.batch + 1023u) / 1024u;
@@ -497,7 +453,7 @@ hipError_t launchBackwardSized(hipStream_t stream, const PermutoArgs& a)
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
     const dim3 grid((a.batch + 255) / 256), block(256);
     TableParts t;
-    const bool cut = a.dTable && cutTable(a, t);
+    const bool cut = a.dTable && cutTable(a.desc, t);
     if (cut && t.count == 1 && a.dPos) {
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
         return launchTableGrad<D, FT, true, false>(stream, a, t, cus);

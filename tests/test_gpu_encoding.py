@@ -224,6 +224,32 @@ def test_permuto_backward_table_parts(D, F, levels_n, log2, B, kernel):
     assert np.linalg.norm(alone.cpu().numpy() - r_table) <= 2.0 ** -16 * np.linalg.norm(r_table)
 
 
+@pytest.mark.parametrize("F,tables,B,kernel", [
+    # a third of the entries would be 1366 x 15 (6827 x 3) doubles, ten (one) more than the LDS holds
+    (15, [(0, 4096), (4096, 4096)], 700, "permutoTableGradKernel<D=2,8 parts> + permutoBackwardKernel<D=2,positions>"),
+    (3, [(0, 20480)], 900, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),
+])
+def test_permuto_backward_of_other_tables(F, tables, B, kernel):
+    # tables: (offset, size) in entries of every level.  The bound is that of test_permuto_backward_table_parts.
+    rng = np.random.default_rng(F * 100 + B)
+    n = len(tables)
+    enc = cv.PermutoEncoder(2, F, 12, n, baseScale=3.0, log2PerLevelScale=1.0, maxLevelRatio=1.0, seed=11)
+    levels = ob.permuto_levels(2, 12, n, 3.0, 1.0, 11)
+    for l, (offset, size) in enumerate(tables):
+        for record in (enc.desc.levelInfo[l], levels[l]):
+            record.offsetOfFeatureTable, record.featureTableSize = offset, size
+    pos = rng.uniform(-1, 1, (B, 2)).astype(np.float32)
+    table = rng.standard_normal(max(o + s for o, s in tables) * F).astype(np.float32)
+    g = rng.standard_normal((B, n * F)).astype(np.float32)
+    r_pos, r_table = ob.permuto_encode_backward(levels, F, float(n), pos, table, g)
+    d_table = torch.zeros(table.size, dtype=torch.float32, device=DEV)
+    d_pos, _ = enc.backward(to_dev(pos), to_dev(table), to_dev(g), dFeatureTable=d_table)
+    assert cv.lastKernelName() == kernel
+    assert np.linalg.norm(d_table.cpu().numpy() - r_table) <= 2.0 ** -16 * np.linalg.norm(r_table)
+    assert not d_table.cpu().numpy()[r_table == 0].any()
+    assert np.linalg.norm(d_pos.cpu().numpy() - r_pos) <= 1e-4 * np.linalg.norm(r_pos)
+
+
 def test_encoder_feeds_the_mlp():
     # encode positions, run the decoder MLP on the fp16 features: the neural-texture shape
     rng = np.random.default_rng(8)

@@ -1,0 +1,85 @@
+"""cutTable (slang_amd/csrc/cv_permuto_parts.h), the host code that cuts the permutohedral encoder's table gradient into
+parts for LDS, compiled by itself and checked for tables of every entry size: no part may exceed a compute unit's LDS,
+and the parts cover what every level adds to once."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+from slang_amd import _lib
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LDS_DOUBLES = 160 * 1024 // 8
+
+SOURCE = """
+#include "cv_permuto_parts.h"
+extern "C" int cut(const CvPermutoDesc* d, uint32_t* out, uint32_t* sliced)
+{
+    cv::TableParts t;
+    const bool ok = cv::cutTable(*d, t);
+    for (uint32_t p = 0; ok && p < t.count; ++p) {
+        const cv::TablePart& q = t.part[p];
+        out[4 * p] = q.base; out[4 * p + 1] = q.elems; out[4 * p + 2] = q.first; out[4 * p + 3] = q.end;
+    }
+    *sliced = ok ? t.sliced : 0;
+    return ok ? (int)t.count : -1;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def cut(tmp_path_factory):
+    d = tmp_path_factory.mktemp("parts")
+    (d / "parts.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(REPO, "include"),
+                    "-I", os.path.join(REPO, "slang_amd", "csrc"), "-o", str(d / "parts.so"), str(d / "parts.cpp")], check=True)
+    lib = ctypes.CDLL(str(d / "parts.so"))
+
+    def call(F, tables):
+        """tables: (offset, size) in entries per level; the parts (base, elems, first, end) and `sliced`, or None"""
+        desc = _lib.CvPermutoDesc(dimensions=3, featureDimensionPerEntry=F, maxLevels=len(tables), maxLevel=99.0)
+        for l, (offset, size) in enumerate(tables):
+            lv = desc.levelInfo[l]
+            lv.currentLevelIndex, lv.offsetOfFeatureTable, lv.featureTableSize = l, offset, size
+        out, sliced = (ctypes.c_uint32 * (4 * 144))(), ctypes.c_uint32()
+        n = lib.cut(ctypes.byref(desc), out, ctypes.byref(sliced))
+        return None if n < 0 else ([tuple(out[4 * p:4 * p + 4]) for p in range(n)], sliced.value)
+    return call
+
+
+def behind_one_another(sizes):
+    return [(sum(sizes[:l]), s) for l, s in enumerate(sizes)]
+
+
+def check(parts, sliced, F, tables):
+    """Every level's elements are covered by its parts once; slices only where `sliced` says so."""
+    for base, elems, first, end in parts:
+        assert 0 < elems <= LDS_DOUBLES and base % F == 0 and elems % F == 0 and first < end, (F, tables, base, elems)
+    for l, (offset, size) in enumerate(tables):
+        lo, hi = offset * F, (offset + size) * F
+        mine = sorted((base, base + elems) for base, elems, first, end in parts if first <= l < end)
+        if len(mine) == 1:
+            assert mine[0][0] <= lo and hi <= mine[0][1], (F, tables, l, mine)
+        else:
+            assert sliced and mine and mine[0][0] == lo and mine[-1][1] == hi, (F, tables, l, mine)
+            assert all(a[1] == b[0] for a, b in zip(mine, mine[1:])), (F, tables, l, mine)
+
+
+@pytest.mark.parametrize("F", range(1, 65))
+def test_parts_of_every_entry_size_fit_the_lds(cut, F):
+    rng = random.Random(F)
+    sizes = [[1 << n] * levels for n in range(0, 21) for levels in (1, 3, 8)]
+    sizes += [[s] * 2 for s in (13653, 20480, 20481, 40960, 3 * 4096 + 1)]
+    sizes += [[int(2 ** rng.uniform(0, 19)) for _ in range(rng.randint(1, 16))] for _ in range(200)]
+    for s in sizes:
+        got = cut(F, behind_one_another(s))
+        slices = [-(-n // (LDS_DOUBLES // F)) for n in s]
+        if max(slices) > 16:
+            assert got is None, (F, s)
+        elif sum(slices) <= 144:
+            assert got is not None, (F, s)
+        if got is not None:
+            check(*got, F, behind_one_another(s))
+            assert sum(e for _, e, _, _ in got[0]) == sum(s) * F
