@@ -19,39 +19,45 @@ struct TableParts {
 // The doubles that half and the whole of a compute unit's LDS (160 KB) hold.
 constexpr uint64_t kPartHalf = 80 * 1024 / 8, kPartMost = 160 * 1024 / 8;
 
-// Cuts the table into parts for permutoTableGradKernel: consecutive levels as long as they fit half of a compute unit's LDS
-// together, so that two workgroups of 16 waves share it; a level beyond that by itself, up to the whole 160 KB; and a level
-// beyond those in slices of its entries, each walked by all positions of the batch.  A slice repeats the search for the
-// simplex: 2^18 positions on 8 levels of 2^16 two-feature entries, seven slices each, take 128 us, on levels of 2^17 in
-// thirteen slices 219 us, and either takes 6.3 to 6.7 ms with the additions in memory.  Sixteen slices at most, since the list of
-// parts travels with the kernel's arguments.
-// False: more parts than that, or levels that do not lie behind one another as prepareLevelInfo puts them.
+// Cuts the table into parts for permutoTableGradKernel: consecutive levels as long as the range from the first to the last of
+// their entries fits half of a compute unit's LDS, so that two workgroups of 16 waves share it; a level beyond that by itself,
+// up to the whole 160 KB; and a level beyond those in slices of its entries, each walked by all positions of the batch.  A slice
+// repeats the search for the simplex: 2^18 positions on 8 levels of 2^16 two-feature entries, seven slices each, take 128 us, on
+// levels of 2^17 in thirteen slices 219 us, and either takes 6.3 to 6.7 ms with the additions in memory.  Sixteen slices at most,
+// since the list of parts travels with the kernel's arguments.
+// Levels may lie anywhere: with gaps between them (a sum that stays zero is not added to memory), in any order, on the same
+// entries (each part adds its sums to memory atomically).
+// False: more parts than that, or elements whose numbers exceed 32 bits.
 inline bool cutTable(const CvPermutoDesc& desc, TableParts& t)
 {
     const uint64_t F = (uint64_t)desc.featureDimensionPerEntry;
     t.count = 0;
     t.sliced = 0;
-    uint64_t next = 0;
+    bool whole = false;      // the part before this level is made of whole levels
     for (uint32_t l = 0; l < desc.maxLevels; ++l) {
         const CvPermutoLevelInfo& lv = desc.levelInfo[l];
-        if ((uint64_t)lv.offsetOfFeatureTable * F != next) return false;
-        const uint64_t elems = (uint64_t)lv.featureTableSize * F;
-        next += elems;
-        if (next > 0xffffffffull) return false;
-        TablePart* last = t.count ? &t.part[t.count - 1] : nullptr;
-        if (last && last->end == l && (uint64_t)last->elems + elems <= kPartHalf) {
-            last->elems += (uint32_t)elems;
-            last->end = l + 1;
-            continue;
+        const uint64_t from = (uint64_t)lv.offsetOfFeatureTable * F, elems = (uint64_t)lv.featureTableSize * F, to = from + elems;
+        if (to > 0xffffffffull) return false;
+        if (whole) {
+            TablePart& last = t.part[t.count - 1];
+            const uint64_t lastTo = (uint64_t)last.base + last.elems;
+            const uint64_t lo = from < last.base ? from : last.base, hi = to > lastTo ? to : lastTo;
+            if (hi - lo <= kPartHalf) {
+                last.base = (uint32_t)lo;
+                last.elems = (uint32_t)(hi - lo);
+                last.end = l + 1;
+                continue;
+            }
         }
         // whole entries to a slice: as many slices as their number needs, so that none comes out above kPartMost
         const uint64_t entries = lv.featureTableSize, most = kPartMost / F, slices = (entries + most - 1) / most;
         if (slices == 0 || slices > 16) return false;
         if (slices > 1) t.sliced = 1;
+        whole = slices == 1;
         const uint64_t perSlice = (entries + slices - 1) / slices * F;
         for (uint64_t at = 0; at < elems; at += perSlice) {
             if (t.count == (uint32_t)kMaxTableParts) return false;
-            t.part[t.count++] = TablePart{(uint32_t)(next - elems + at), (uint32_t)(elems - at < perSlice ? elems - at : perSlice), l, l + 1};
+            t.part[t.count++] = TablePart{(uint32_t)(from + at), (uint32_t)(elems - at < perSlice ? elems - at : perSlice), l, l + 1};
         }
     }
     return t.count > 0;

@@ -228,6 +228,13 @@ def test_permuto_backward_table_parts(D, F, levels_n, log2, B, kernel):
     # a third of the entries would be 1366 x 15 (6827 x 3) doubles, ten (one) more than the LDS holds
     (15, [(0, 4096), (4096, 4096)], 700, "permutoTableGradKernel<D=2,8 parts> + permutoBackwardKernel<D=2,positions>"),
     (3, [(0, 20480)], 900, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),
+    # small tables with gaps, in reverse order, on shared entries, all of them a single part
+    (2, [(3, 256), (267, 256), (531, 100), (700, 256)], 5000, "permutoTableGradKernel<D=2,positions>"),
+    (4, [(384, 128), (256, 128), (128, 128), (0, 128)], 4097, "permutoTableGradKernel<D=2,positions>"),
+    (2, [(0, 256), (0, 256), (128, 256)], 4500, "permutoTableGradKernel<D=2,positions>"),
+    # larger ones, a part to a level or in slices
+    (2, [(20000, 4096), (3000, 8192), (3000, 8192)], 3000, "permutoTableGradKernel<D=2,3 parts> + permutoBackwardKernel<D=2,positions>"),
+    (1, [(50, 40000), (0, 60), (45, 9000)], 2500, "permutoTableGradKernel<D=2,3 parts> + permutoBackwardKernel<D=2,positions>"),
 ])
 def test_permuto_backward_of_other_tables(F, tables, B, kernel):
     # tables: (offset, size) in entries of every level.  The bound is that of test_permuto_backward_table_parts.

@@ -83,3 +83,32 @@ def test_parts_of_every_entry_size_fit_the_lds(cut, F):
         if got is not None:
             check(*got, F, behind_one_another(s))
             assert sum(e for _, e, _, _ in got[0]) == sum(s) * F
+
+
+@pytest.mark.parametrize("F", [1, 2, 3, 4, 7, 15, 64])
+def test_parts_of_tables_in_any_layout(cut, F):
+    # levels with gaps between them, in any order, on the same entries, far apart
+    rng = random.Random(100 + F)
+    for case in range(400):
+        levels, top = rng.randint(1, 16), rng.choice([4, 8, 12, 16])
+        sizes = [max(1, int(2 ** rng.uniform(0, top))) for _ in range(levels)]
+        tables = behind_one_another(sizes)
+        kind = case % 4
+        if kind == 0: tables = [(o + 5 * l, s) for l, (o, s) in enumerate(tables)]
+        if kind == 1: tables = [(sum(sizes) - o - s, s) for o, s in tables]
+        if kind == 2: tables = [(rng.choice(tables)[0], s) for _, s in tables]
+        if kind == 3: tables = [(rng.randrange(0, (1 << 32) // F - (1 << 17)), s) for _, s in tables]
+        slices = [-(-s // (LDS_DOUBLES // F)) for s in sizes]
+        got = cut(F, tables)
+        if max(slices) <= 16 and sum(slices) <= 144:
+            assert got is not None, (F, tables)
+        if got is not None:
+            check(*got, F, tables)
+    # what fits half of the LDS is one part, which also gives the position gradients
+    small = LDS_DOUBLES // 2 // F
+    if small >= 8:
+        n = small // 4
+        for tables in ([(l * n, n - 1) for l in range(4)], [((3 - l) * n, n) for l in range(4)], [(0, n)] * 4, [(7, n), (7 + n, n), (8, 3)]):
+            assert cut(F, tables)[0] == [(min(o for o, _ in tables) * F, (max(o + s for o, s in tables) - min(o for o, _ in tables)) * F, 0, len(tables))]
+    # elements beyond 32 bits: not cut
+    assert cut(F, [(0, 4), ((1 << 32) // F - 2, 4)]) is None
