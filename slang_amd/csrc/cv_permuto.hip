@@ -312,7 +312,7 @@ __device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_
 }
 
 // Position gradients alone (TABLE false), or everything with the table's share added in memory: a table of which one level
-// alone is beyond what the LDS kernel below takes.
+// alone is beyond what the LDS kernel below takes, or a handful of positions (launchBackwardSized).
 template <int D, int FT, bool POS, bool TABLE>
 __global__ __launch_bounds__(256) void permutoBackwardKernel(const PermutoArgs a)
 {
@@ -458,7 +458,14 @@ hipError_t launchBackwardSized(hipStream_t stream, const PermutoArgs& a)
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
         return launchTableGrad<D, FT, true, false>(stream, a, t, cus);
     }
-    if (cut) {
+    // Two launches against one: a handful of positions whose few additions hardly meet is done sooner by the one kernel that adds
+    // in memory.  It takes 7.4 to 8.1 us per call back to back and the pair 11.5 to 13.5 (16 positions on 3 levels of 2^10
+    // four-feature entries, 4 of 2^12 two-feature ones, ...); its time grows with the additions and reaches the pair's at 1300 to
+    // 2000 of them (one to five and eight dimensions, 2 to 8 levels).  Where a position has more than 16 features it is the slower
+    // one from the first position (16 levels of 4 features: 34.8 against 25.3 us).
+    const uint64_t features = (uint64_t)a.desc.featureDimensionPerEntry * a.desc.maxLevels;
+    const bool few = FT > 0 && a.batch <= 64u && features <= 16u && a.batch * (uint64_t)(D + 1) * features <= 1440u;
+    if (cut && !(a.dPos && few)) {
         noteKernel(false, "permutoTableGradKernel<D=%d,%u parts>", D, t.count);
         const hipError_t e = t.sliced ? launchTableGrad<D, FT, false, true>(stream, a, t, cus) : launchTableGrad<D, FT, false, false>(stream, a, t, cus);
         if (e != hipSuccess || !a.dPos) return e;

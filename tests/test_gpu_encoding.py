@@ -257,6 +257,30 @@ def test_permuto_backward_of_other_tables(F, tables, B, kernel):
     assert np.linalg.norm(d_pos.cpu().numpy() - r_pos) <= 1e-4 * np.linalg.norm(r_pos)
 
 
+@pytest.mark.parametrize("D,F,levels_n,log2,B,in_memory", [
+    (2, 4, 3, 10, 1, True), (2, 4, 3, 10, 40, True), (2, 4, 3, 10, 41, False),       # 36 additions to a position
+    (3, 2, 8, 12, 22, True), (3, 2, 8, 12, 23, False), (1, 1, 4, 15, 64, True), (1, 1, 4, 15, 65, False),
+    (2, 2, 9, 12, 3, False), (2, 3, 3, 12, 3, False),                                # 18 features; three to an entry
+])
+def test_permuto_backward_of_a_handful_of_positions(D, F, levels_n, log2, B, in_memory):
+    # both sides of the rule that sends a few positions to the kernel that adds in memory; the bound is that of
+    # test_permuto_backward_table_parts
+    rng = np.random.default_rng(D * 1000 + F * 100 + levels_n * 10 + B)
+    enc = cv.PermutoEncoder(D, F, log2, levels_n, baseScale=3.0, log2PerLevelScale=0.5, maxLevelRatio=1.0, seed=3)
+    levels = ob.permuto_levels(D, log2, levels_n, 3.0, 0.5, 3)
+    pos = rng.uniform(-1, 1, (B, D)).astype(np.float32)
+    table = rng.standard_normal(enc.featureTableElements).astype(np.float32)
+    g = rng.standard_normal((B, levels_n * F)).astype(np.float32)
+    r_pos, r_table = ob.permuto_encode_backward(levels, F, float(levels_n), pos, table, g)
+    for want_pos in (True, False):
+        d_table = torch.zeros(table.size, dtype=torch.float32, device=DEV)
+        d_pos, _ = enc.backward(to_dev(pos), to_dev(table), to_dev(g), dFeatureTable=d_table, wantPositionGrad=want_pos)
+        assert cv.lastKernelName().startswith("permutoBackwardKernel" if want_pos and in_memory else "permutoTableGradKernel"), cv.lastKernelName()
+        assert np.linalg.norm(d_table.cpu().numpy() - r_table) <= 2.0 ** -16 * np.linalg.norm(r_table)
+        if want_pos:
+            assert np.linalg.norm(d_pos.cpu().numpy() - r_pos) <= 1e-4 * np.linalg.norm(r_pos)
+
+
 def test_encoder_feeds_the_mlp():
     # encode positions, run the decoder MLP on the fp16 features: the neural-texture shape
     rng = np.random.default_rng(8)
