@@ -12,7 +12,7 @@
 // down the columns: four 4-byte reads for float, two ds_read_b64_tr_b16 for half.  So one copy of W serves both
 // directions and no vector is stored twice: dZ_l takes the place of X_l once dW of the layer above and act'(Z_l) have used
 // it.  The sign of a stored activation carries what act' needs: positive where z > 0, +0 at z == 0 (the tie of max()),
-// negative or -0 where z < 0.
+// negative or -0 where z < 0 and, behind a ReLU, where z is NaN (which then passes no gradient).
 //
 // Work split.  Eight waves.  Forward and dX: a wave takes output tiles of 16 features x 16 samples; the epilogue (bias,
 // activation, act') is elementwise on its own tiles.  dW: a wave owns tiles of every layer's dW for the whole kernel (in
@@ -98,7 +98,7 @@ template <> struct RoundMma<float> {
     {
         if (act == kActRelu) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) z[r] = z[r] > 0.f ? z[r] : (z[r] < 0.f ? -0.f : 0.f);
+            for (int r = 0; r < 4; ++r) z[r] = z[r] > 0.f ? z[r] : (z[r] == 0.f ? 0.f : -0.f);      // (NaN: -0)
         } else if (act == kActLeakyRelu) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) { const float u = z[r] + 0.f; z[r] = fmaxf(u, u * slope); }      // (-0 + 0 = +0)
@@ -170,7 +170,7 @@ template <> struct RoundMma<half_t> {
         const halfx2 zero = {(half_t)0, (half_t)0};
         const halfx2 z0 = round2(acc[0], acc[1]) + zero, z1 = round2(acc[2], acc[3]) + zero;      // (-0 + 0 = +0)
         u32x2 x = {__builtin_bit_cast(uint32_t, z0), __builtin_bit_cast(uint32_t, z1)};
-        if (act == kActRelu) {
+        if (act == kActRelu) {      // (a NaN leaves the matrix instruction with its sign set, whatever it came from: -0)
             x.x = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(z0, zero)) | (x.x & 0x80008000u);
             x.y = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(z1, zero)) | (x.y & 0x80008000u);
         } else if (act == kActLeakyRelu) {

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
                 for (int t = 0; t < HT; ++t)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[t][r] = acc[t][r] > 0.f ? acc[t][r] : (acc[t][r] < 0.f ? -0.f : 0.f);
+                    for (int r = 0; r < 4; ++r) acc[t][r] = acc[t][r] > 0.f ? acc[t][r] : (acc[t][r] == 0.f ? 0.f : -0.f);      // (NaN: -0)
             } else if (act == kActLeakyRelu) {
 #pragma unroll
                 for (int t = 0; t < HT; ++t)

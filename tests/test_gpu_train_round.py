@@ -20,12 +20,12 @@ pytestmark = pytest.mark.gpu
 
 
 def reference(specs, x, t, scale):
-    """The step in float64 with Slang's rule for max(): (dW, db, loss)."""
+    """The step in float64 with Slang's rule for max(): (dW, db, loss).  ReLU of NaN is 0 and passes nothing."""
     hs, zs = [x.astype(np.float64)], []
     for s in specs:
         z = hs[-1] @ s["W"].astype(np.float64).T + (s["b"].astype(np.float64) if s["b"] is not None else 0.0)
         zs.append(z)
-        hs.append(np.maximum(z, 0) if s["act"] == 1 else np.maximum(z, z * s["slope"]) if s["act"] == 2 else z)
+        hs.append(np.where(z > 0, z, 0.0) if s["act"] == 1 else np.maximum(z, z * s["slope"]) if s["act"] == 2 else z)
     diff = hs[-1] - t.astype(np.float64)
     g, dW, dB = 2.0 * diff * scale, [], []
     for l in range(len(specs) - 1, -1, -1):
@@ -153,3 +153,40 @@ def test_random_networks(elem, dims, B, act, slope, targets):
         assert rel_err(dW[l], rW[l]) <= bar and rel_err(dB[l], rB[l]) <= bar, (l, rel_err(dW[l], rW[l]), rel_err(dB[l], rB[l]))
         assert torch.equal(layers[l].weightsGrad, again[l].weightsGrad) and torch.equal(layers[l].biasesGrad, again[l].biasesGrad)
     assert abs(loss.item() - rloss) <= bar * rloss and loss.item() == loss2.item()
+
+
+KERNELS = [("f32", [32, 64, 64, 8], "trainWaveKernel"), ("f32", [100, 128, 4], "trainRoundKernel"), ("f16", [64, 64, 64, 16], "trainRoundKernel"),
+           ("f16", [16, 128, 128, 128, 8], "trainRoundKernel"), ("f32", [9, 30, 12, 3], "trainWaveKernel"), ("f16", [60, 48, 20, 4], "trainRoundKernel")]
+
+
+@pytest.mark.filterwarnings("ignore:invalid value encountered in matmul")
+@pytest.mark.parametrize("flags", [0, cv.FLAG_LAYERWISE_TRAINING])
+@pytest.mark.parametrize("elem,dims,kernel", KERNELS)
+def test_nan_at_a_relu_is_no_tie(elem, dims, kernel, flags):
+    # Samples with a NaN of either sign: every hidden unit of the first layer is NaN, which ReLU turns into 0 and whose gradient
+    # is 0 (not the half of a tie), so the loss is finite and these samples add to the layers above alone.  In dW of the first
+    # layer their 0 x NaN shows in the NaN's column, nowhere else (over memory half vectors spread it to neighbouring columns).
+    # A third sample has infinities of both signs, which make the NaN, and two units are NaN for every sample, by their biases.
+    # Whole numbers: exact.  The step over memory has the same rule.
+    rng = np.random.default_rng(sum(dims))
+    dtype, ct = (np.float32, CT.Float32) if elem == "f32" else (np.float16, CT.Float16)
+    B = 150
+    specs = whole_number_network(rng, dims, dtype, Activation.ReLU, 0.0, Activation.NoActivation)
+    x = rng.integers(-1, 2, (B, dims[0])).astype(dtype)
+    t = rng.integers(-2, 3, (B, dims[-1])).astype(dtype)
+    x[77, 1], x[78, 1], x[140, 1], x[140, 2] = np.nan, -np.nan, np.inf, -np.inf
+    specs[0]["W"][:, 1:3] = 1
+    specs[0]["b"][3], specs[0]["b"][4] = np.nan, -np.nan
+    dW, dB, loss = reference(specs, x, t, 1.0 / 16)
+    assert np.isfinite(loss)
+    layers = build(specs, ct)
+    _, got = cv.mlpTrainStep(layers, to_dev(x), to_dev(t), lossScale=1.0 / 16, weightType=ct, flags=flags)
+    assert (kernel in cv.lastKernelName()) == (flags == 0), cv.lastKernelName()
+    gW, gB = read_grads(layers, specs, CT.Float32, ML.TrainingOptimal)
+    assert got.item() == loss
+    for l in range(len(specs)):
+        assert np.array_equal(gB[l], dB[l]), (l, np.abs(gB[l] - dB[l]).max())
+        keep = np.ones(dims[l], bool)
+        if l == 0: keep[slice(1, 3) if elem == "f32" or flags == 0 else slice(None)] = False
+        assert np.array_equal(gW[l][:, keep], dW[l][:, keep]), l
+    assert np.isnan(gW[0][:, 1:3]).all()
