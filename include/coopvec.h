@@ -453,8 +453,9 @@ CV_API CvResult cvPermutoMlpForward(void* stream, const CvPermutoDesc* desc, con
  * lossSum (device, optional, one float) is overwritten with sum_s loss_s; mlp->lossMax, if set, with max_s loss_s.
  * The fused kernel for 64-wide networks runs pairs of waves that wait for each other with a bounded spin; should such a
  * wait ever time out (only a defect of the kernel could cause that), the step is void: lossSum, lossMax and every
- * gradient sum the step adds are NaN, whether or not the loss outputs are requested.  A NaN loss for any other reason
- * (NaN samples) has the same effect. */
+ * gradient sum the step adds are NaN, whether or not the loss outputs are requested.  A loss that is not finite for any
+ * other reason (NaN or infinite samples, an overflow of the squares or of their sum) has the same effect, except on the step
+ * over the batch in memory, where it spreads as the arithmetic has it. */
 CV_API CvResult cvMlpTrainStepWorkspaceSize(const CvMlpDesc* mlp, uint32_t batch, size_t* outBytes);
 CV_API CvResult cvMlpTrainStep(void* stream, const CvMlpDesc* mlp,
                                const void* input, size_t inputStride,

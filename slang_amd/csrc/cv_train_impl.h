@@ -118,6 +118,9 @@ TrainReduceArgs makeTrainReduceArgs(const TrainLaunch& t, uint32_t blocks)
     return ra;
 }
 
+// a loss that voids the step
+__device__ __forceinline__ bool notFinite(float v) { return !(__builtin_fabsf(v) < __builtin_inff()); }
+
 // The largest per-sample loss of a workgroup, kept as the bits of a non-negative float (whose order is that of the
 // integers; a NaN compares above everything, so it wins).  A maximum does not depend on the order of its operands: the
 // LDS atomic keeps the result reproducible.
@@ -730,8 +733,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // ---- workgroup partial: sum the four waves in a fixed order, one tile at a time ----------
     // The only workgroup of a launch (ta.finishInKernel) does with its sums what mlpTrainReduceKernel would do with this one
     // partial: they go from its registers to the gradients.  The gradient elements they are added to are requested ahead,
-    // eight tiles at a time, so that a group of tiles costs one round trip to memory, and the loss is summed first: a NaN
-    // there makes every sum of the step NaN (see mlpTrainReduceKernel).
+    // eight tiles at a time, so that a group of tiles costs one round trip to memory, and the loss is summed first: one that is
+    // not finite makes every sum of the step NaN (see mlpTrainReduceKernel).
     float* part = ta.partials + (size_t)blockIdx.x * Net::partialFloats;
     constexpr uint32_t nValues = Net::totalGradTiles * 256 + Net::totalDbTiles * 16;
     const bool finish = ta.finishInKernel != 0;
@@ -766,7 +769,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         }
     }
     __syncthreads();
-    const bool voidStep = finish && ldsLossSum != ldsLossSum;
+    const bool voidStep = finish && notFinite(ldsLossSum);
     constexpr int kAhead = 8;
 #pragma unroll
     for (int i0 = 0; i0 < Net::totalGradTiles; i0 += kAhead) {
@@ -831,8 +834,8 @@ __global__ __launch_bounds__(64 * kReduceWaves) void mlpTrainReduceKernel(const 
     const uint32_t p = blockIdx.x * 64u + (threadIdx.x & 63u);
     constexpr uint32_t nW = Net::totalGradTiles * 256, nB = Net::totalDbTiles * 16;
     const bool inRange = p < nW + nB + 1;
-    // A workgroup whose loss partial is NaN declares its whole partial void: a wave of the paired kernel that gave up
-    // waiting for its partner has worked on stale tiles and says so there (so does a NaN that came in with the samples).
+    // A workgroup whose loss partial is not finite declares its whole partial void: a wave of the paired kernel that gave up
+    // waiting for its partner has worked on stale tiles and says so there with a NaN (so do samples whose loss is not finite).
     // Then every sum of the step is NaN, whether or not the caller reads the loss.
     __shared__ uint32_t maxBits;
     const bool ownsLoss = blockIdx.x == (nW + nB) / 64u;      // the workgroup whose values include the loss
@@ -844,7 +847,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void mlpTrainReduceKernel(const 
     if (threadIdx.x < ra.numPartials) lp0 = ra.partials[(size_t)threadIdx.x * Net::partialFloats + nW + nB];
     for (uint32_t b = threadIdx.x + 64u * kReduceWaves; b < ra.numPartials; b += 64u * kReduceWaves) {
         const float lp = ra.partials[(size_t)b * Net::partialFloats + nW + nB];
-        voidStep = voidStep || lp != lp;
+        voidStep = voidStep || notFinite(lp);
     }
     if (ra.lossMax && ownsLoss)
         for (uint32_t b = threadIdx.x; b < ra.numPartials; b += 64u * kReduceWaves)
@@ -858,7 +861,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void mlpTrainReduceKernel(const 
     }
     float s;
     const bool mine = sumPartials(ra.partials + p, Net::partialFloats, ra.numPartials, inRange, red, s);
-    voidStep = __syncthreads_or(voidStep || lp0 != lp0) != 0;
+    voidStep = __syncthreads_or(voidStep || notFinite(lp0)) != 0;
     if (ra.lossMax && ownsLoss && threadIdx.x == 0)
         *ra.lossMax = voidStep ? __builtin_nanf("") : __builtin_bit_cast(float, maxBits);
     if (!mine || !inRange) return;

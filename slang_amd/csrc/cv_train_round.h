@@ -593,7 +593,7 @@ __device__ __forceinline__ uint8_t* roundGradientSlot(const RoundArgs& a, int nu
 }
 
 // Sums the workgroups' partials in a fixed order and adds them to the gradients (mlpTrainReduceKernel for run-time sizes; a
-// NaN in the loss voids the step here, too).
+// loss that is not finite voids the step here, too).
 __global__ __launch_bounds__(64 * kReduceWaves) void trainRoundReduceKernel(const RoundArgs a)
 {
     const TrainReduceArgs& ra = a.finish;
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void trainRoundReduceKernel(cons
     bool voidStep = false;
     for (uint32_t b = threadIdx.x; b < ra.numPartials; b += 64u * kReduceWaves) {
         const float lp = ra.partials[(size_t)b * a.partialFloats + lossAt];
-        voidStep = voidStep || lp != lp;
+        voidStep = voidStep || notFinite(lp);
         if (ra.lossMax && ownsLoss) atomicMax(&maxBits, __builtin_bit_cast(uint32_t, ra.partials[(size_t)b * a.partialFloats + lossAt + 1u]));
     }
     uint8_t* slot = nullptr;

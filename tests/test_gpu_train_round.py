@@ -190,3 +190,34 @@ def test_nan_at_a_relu_is_no_tie(elem, dims, kernel, flags):
         if l == 0: keep[slice(1, 3) if elem == "f32" or flags == 0 else slice(None)] = False
         assert np.array_equal(gW[l][:, keep], dW[l][:, keep]), l
     assert np.isnan(gW[0][:, 1:3]).all()
+
+
+@pytest.mark.parametrize("value", ["nan", "inf", "infinite loss"])
+@pytest.mark.parametrize("elem,dims,kernel", KERNELS + [("f16", [8, 64, 64, 64, 64, 1], "mlpTrainPairKernel"), ("f16", [4, 16, 4], "mlpTrainKernel")])
+def test_a_loss_that_is_not_finite_voids_the_step(elem, dims, kernel, value):
+    # lossSum, lossMax and every gradient element are NaN, whatever is in the gradients before; so they are where a sample's
+    # loss is infinite and its gradients are not (float: the square of a difference of 2^66)
+    rng = np.random.default_rng(sum(dims) + 1)
+    dtype, ct = (np.float32, CT.Float32) if elem == "f32" else (np.float16, CT.Float16)
+    B = 16 if dims == [4, 16, 4] else 300
+    specs = []
+    for i, (fi, fo) in enumerate(zip(dims, dims[1:])):
+        specs.append(dict(W=(rng.standard_normal((fo, fi)) / np.sqrt(fi)).astype(dtype), b=np.zeros(fo, dtype),
+                          act=int(Activation.NoActivation if i == len(dims) - 2 else Activation.LeakyReLU), slope=0.125))
+    x = rng.uniform(-1, 1, (B, dims[0])).astype(dtype)
+    t = rng.uniform(-1, 1, (B, dims[-1])).astype(dtype)
+    at = B - 3
+    if value != "infinite loss":
+        x[at, 1] = float(value)
+    elif elem == "f32":
+        t[at, 0] = 2.0 ** 66
+    else:
+        specs[-1]["b"][0], t[:, 0], t[at, 0] = 60000, 60000, -60000       # (the difference is infinite in half)
+    layers = build(specs, ct, preset=1.0)
+    lmax = torch.zeros(1, device=DEV)
+    _, loss = cv.mlpTrainStep(layers, to_dev(x), to_dev(t), weightType=ct, lossMax=lmax)
+    assert kernel in cv.lastKernelName(), cv.lastKernelName()
+    assert np.isnan(loss.item()) and np.isnan(lmax.item()), (loss.item(), lmax.item())
+    gW, gB = read_grads(layers, specs, CT.Float32, ML.TrainingOptimal)
+    for l in range(len(specs)):
+        assert np.isnan(gW[l]).all() and np.isnan(gB[l]).all(), l
