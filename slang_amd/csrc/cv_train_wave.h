@@ -63,6 +63,15 @@ struct WaveNet {
     static constexpr bool fits = tiles <= kWaveMaxTiles && ldsBytes <= 160u * 1024u;
 };
 
+// The lanes of a wave exchange vectors through LDS, whose accesses the hardware keeps in order: what lies before this stays
+// before it for every lane.  No instruction.
+__device__ __forceinline__ void orderLanes()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <class Net>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void trainWaveKernel(const RoundArgs a)
 {
@@ -115,6 +124,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     auto oneTile = [&](const floatx4 (&xin)[IT], const float (&tgt)[4], uint32_t tile) {
         constexpr int MAXT = IT > HT ? IT : HT;
         floatx4 x[MAXT];                     // B operands: the current layer's input, later dZ
+        orderLanes();                        // (the tile before has read X and dZ)
 #pragma unroll
         for (int q = 0; q < IT; ++q) {
 #pragma unroll
@@ -124,6 +134,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         float tgtAll = 0.f;
         if (!a.targets) {
             // sin(sum of the inputs), each lane group a quarter of them, as the other steps form it
+            orderLanes();
             const int gs = (int)optGS((uint32_t)in0);
             const float* xs = (const float*)(mine + Net::xOff(0) + (uint32_t)n * Net::xStride(0));
             float part = 0.f;
@@ -201,6 +212,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             x[0] = dz;
             *(floatx4*)(mine + Net::xOff(NL) + (uint32_t)n * Net::xStride(NL) + 16 * g) = dz;
         }
+        orderLanes();
         // ---- backward -----------------------------------------------------------------------------------------------------
         staticFor<0, NL>([&](auto ic) {
             constexpr int l = NL - 1 - decltype(ic)::value, OT = Net::outTiles(l), NI = Net::inTiles(l);
@@ -241,11 +253,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
             // through the activation of the layer below, in the place of its output
             if constexpr (l > 0) {
+                orderLanes();                // (dW has read X_l)
 #pragma unroll
                 for (int t = 0; t < HT; ++t) {
                     uint8_t* p = mine + Net::xOff(l) + (uint32_t)n * Net::xStride(l) + 64 * t + 16 * g;
                     x[t] = M::storeGradient(p, gx[t], a.layers[l - 1].act, a.layers[l - 1].slope);
                 }
+                orderLanes();
             }
         });
     };
