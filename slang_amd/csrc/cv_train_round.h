@@ -262,7 +262,7 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
         }
     float lossAcc = 0.f, lossMaxAcc = 0.f;
 
-    const uint32_t numRounds = (a.batch + kRoundSamples - 1) / kRoundSamples, lastSample = a.batch - 1;
+    const uint32_t lastSample = a.batch - 1, numRounds = lastSample / kRoundSamples + 1;
 
     // ---- the network's input: eight threads to a sample, 16-byte pieces where rows are made of them, else elements.
     //      Addresses always exist; what lies past the vector is not stored.
@@ -682,7 +682,7 @@ hipError_t launchRoundSized(hipStream_t stream, const TrainLaunch& t, RoundArgs&
     constexpr int WAVES = roundWavesPerSimd(NL, RT);
     const hipError_t e = allowDynamicLds<trainRoundKernel<T, NL, RT, WAVES>>(160 * 1024);
     if (e != hipSuccess) return e;
-    const uint32_t rounds = (t.mlp.batch + kRoundSamples - 1) / kRoundSamples, resident = roundWorkgroups(a, NL, RT, numCUs);
+    const uint32_t rounds = (t.mlp.batch - 1) / kRoundSamples + 1, resident = roundWorkgroups(a, NL, RT, numCUs);
     const uint32_t blocks = rounds < resident ? rounds : resident;
     a.finish.numPartials = blocks;
     // (the tests of the step over the whole batch tell the two apart by this name: both go through the network layer by layer)

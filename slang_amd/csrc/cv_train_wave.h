@@ -99,7 +99,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     const int in0 = a.layers[0].in, topOut = a.layers[NL - 1].out, topAct = a.layers[NL - 1].act;
     const float topSlope = a.layers[NL - 1].slope;
-    const uint32_t numTiles = (a.batch + 15u) / 16u, lastSample = a.batch - 1u;
+    const uint32_t lastSample = a.batch - 1u, numTiles = lastSample / 16u + 1u;
 
     // the tile's input as B operands (lane 16g + j: features 16q + 4g .. of sample j) and its targets (rows 4g .. 4g+3)
     auto fetch = [&](floatx4 (&x)[IT], float (&t)[4], uint32_t tile) {
@@ -353,7 +353,7 @@ hipError_t launchWave(hipStream_t stream, const TrainLaunch& t, RoundArgs& a, in
     a.ldsBytes = Net::ldsBytes;
     const hipError_t e = allowDynamicLds<trainWaveKernel<Net>>(160 * 1024);
     if (e != hipSuccess) return e;
-    const uint32_t need = (t.mlp.batch + 127u) / 128u, blocks = need < (uint32_t)numCUs ? need : (uint32_t)numCUs;
+    const uint32_t need = (t.mlp.batch - 1u) / 128u + 1u, blocks = need < (uint32_t)numCUs ? need : (uint32_t)numCUs;
     a.finish.numPartials = blocks;
     noteKernel(false, "layer-by-layer training step by waves: trainWaveKernel<f32,%d layers,inputs<=%d,hidden<=%d> + trainRoundReduceKernel", Net::NL, 16 * Net::IT, 16 * Net::HT);
     hipLaunchKernelGGL((trainWaveKernel<Net>), dim3(blocks), dim3(512), Net::ldsBytes, stream, a);

@@ -221,3 +221,23 @@ def test_a_loss_that_is_not_finite_voids_the_step(elem, dims, kernel, value):
     gW, gB = read_grads(layers, specs, CT.Float32, ML.TrainingOptimal)
     for l in range(len(specs)):
         assert np.isnan(gW[l]).all() and np.isnan(gB[l]).all(), l
+
+
+def test_the_largest_batch():
+    # 2^32 - 1 samples: rounds and tiles are counted without leaving 32 bits.  All samples are 0 but the first and the last.
+    B = 0xffffffff
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 34 GB of memory")
+    x, t = torch.zeros(B, 1, device=DEV), torch.zeros(B, 1, device=DEV)
+    x[0], x[-1] = 1, 1
+    for dims, kernel in (([1, 1, 1], "trainWaveKernel"), ([1, 65, 1], "trainRoundKernel")):
+        specs = [dict(W=np.zeros((fo, fi), np.float32), b=np.zeros(fo, np.float32), act=int(a), slope=0.0)
+                 for fi, fo, a in ((1, dims[1], Activation.ReLU), (dims[1], 1, Activation.NoActivation))]
+        for s in specs:
+            s["W"][0, 0] = 1
+        layers = build(specs, CT.Float32, grad_layout=ML.RowMajor)
+        _, loss = cv.mlpTrainStep(layers, x, t, weightType=CT.Float32)
+        assert kernel in cv.lastKernelName(), cv.lastKernelName()
+        gW, gB = read_grads(layers, specs, CT.Float32, ML.RowMajor)
+        assert loss.item() == 2 and gW[1][0, 0] == 4 and gB[1][0] == 4 and gW[0][0, 0] == 4 and gB[0][0] == 4
+        assert not gW[0][1:].any() and not gB[0][1:].any() and not gW[1][0, 1:].any()
