@@ -439,7 +439,7 @@ hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, TableParts&
     const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED>>((int)(kPartMost * 8));
     if (e != hipSuccess) return e;
     // as many workgroups as the compute units hold, dealt evenly to the parts
-    const uint32_t resident = (uint32_t)cus * (lds <= 80 * 1024 ? 2u : 1u), want = (a.batch + 1023u) / 1024u;
+    const uint32_t resident = (uint32_t)cus * (lds <= 80 * 1024 ? 2u : 1u), want = (a.batch - 1u) / 1024u + 1u;
     const uint32_t each = resident / t.count ? resident / t.count : 1u;
     t.groups = want < each ? want : each;
     hipLaunchKernelGGL((permutoTableGradKernel<D, FT, POS, SLICED>), dim3(t.count * t.groups), dim3(1024), lds, stream, a, t);
@@ -451,7 +451,7 @@ hipError_t launchBackwardSized(hipStream_t stream, const PermutoArgs& a)
 {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    const dim3 grid((a.batch + 255) / 256), block(256);
+    const dim3 grid((a.batch - 1u) / 256u + 1u), block(256);
     TableParts t;
     const bool cut = a.dTable && cutTable(a.desc, t);
     if (cut && t.count == 1 && a.dPos) {

@@ -281,6 +281,24 @@ def test_permuto_backward_of_a_handful_of_positions(D, F, levels_n, log2, B, in_
             assert np.linalg.norm(d_pos.cpu().numpy() - r_pos) <= 1e-4 * np.linalg.norm(r_pos)
 
 
+def test_permuto_backward_of_the_largest_batch():
+    # 2^32 - 1 positions: workgroups are counted without leaving 32 bits.  Only the first and the last have a gradient, each
+    # position's weights sum to 1.
+    B = 0xffffffff
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 52 GB of memory")
+    enc = cv.PermutoEncoder(1, 1, 6, 1, baseScale=3.0, log2PerLevelScale=1.0, maxLevelRatio=1.0, seed=11)
+    pos, g = torch.zeros(B, 1, device=DEV), torch.zeros(B, 1, device=DEV)
+    pos[-1], g[0], g[-1] = 0.75, 1, 2
+    table = torch.randn(enc.featureTableElements, device=DEV)
+    d_table = torch.zeros_like(table)
+    d_pos, _ = enc.backward(pos, table, g, dFeatureTable=d_table)
+    assert cv.lastKernelName().startswith("permutoTableGradKernel")
+    want_pos, want_table = enc.backward(pos[[0, -1]].contiguous(), table, g[[0, -1]].contiguous())
+    assert torch.equal(d_pos[[0, -1]], want_pos) and not d_pos[1:-1].any()
+    assert torch.allclose(d_table, want_table, rtol=0, atol=2.0 ** -20) and abs(d_table.sum().item() - 3) <= 2.0 ** -20
+
+
 def test_encoder_feeds_the_mlp():
     # encode positions, run the decoder MLP on the fp16 features: the neural-texture shape
     rng = np.random.default_rng(8)
