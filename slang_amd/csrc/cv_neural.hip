@@ -262,13 +262,23 @@ CV_API CvResult cvNeuralMlpTrainStep(void* stream, const CvNeuralNetworkDesc* ne
 
 CV_API CvResult cvNeuralMlpTrainStepWorkspaceSize(const CvNeuralNetworkDesc* net, uint32_t batch, size_t* outBytes)
 {
+    if (!outBytes) return cv::failWith(CV_E_INVALID_ARG, "cvNeuralMlpTrainStepWorkspaceSize: outBytes is null");
     CvMlpLayer layers[cv::kMaxMlpLayers];
     alignas(16) static const uint8_t dummy[16] = {};      // stands for a parameter block: only its alignment is looked at
     CvResult rc = cv::layersFromBlock("cvNeuralMlpTrainStepWorkspaceSize", net, 0, dummy, nullptr, nullptr, nullptr, layers);
     if (CV_FAILED(rc)) return rc;
     const int32_t T = net->elementType;
     CvMlpDesc mlp = {layers, net->layerCount, T, T, T, T, T, 0, CV_ENCODE_NONE};
-    return cvMlpTrainStepWorkspaceSize(&mlp, batch, outBytes);
+    // The activations decide between the kernels of a step (128-wide hidden layers have a fused one with ReLU or leaky ReLU
+    // only) and are not known here: room for either.
+    size_t plain = 0;
+    rc = cvMlpTrainStepWorkspaceSize(&mlp, batch, &plain);
+    if (CV_FAILED(rc)) return rc;
+    for (int l = 0; l < net->layerCount; ++l) layers[l].activation = CV_ACT_RELU;
+    rc = cvMlpTrainStepWorkspaceSize(&mlp, batch, outBytes);
+    if (CV_FAILED(rc)) return rc;
+    if (plain > *outBytes) *outBytes = plain;
+    return CV_OK;
 }
 
 } // extern "C"

@@ -192,3 +192,38 @@ def test_training_through_a_parameter_block():
     assert g_lin.abs().sum().item() > 0
     # layer 1 has no bias: its slot in the optimal gradient block stays untouched (zero)
     assert (g_opt[nl.layer_counts(4, 16, True)[1] + 16 * 16:] == 0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [[16, 100, 70, 8], [16, 128, 128, 8], [8, 90, 4], [20, 48, 24, 5], [40, 33, 65, 2]])
+@pytest.mark.parametrize("B", [40, 5000])
+def test_workspace_of_a_parameter_block_serves_every_activation(dims, B):
+    # the size query knows the layer sizes but not the activations, which decide between the kernels of a step
+    import torch
+    from gpu_util import as_bytes, to_dev
+    from slang_amd import coopvec as cv
+    from slang_amd.coopvec import Activation, CoopVecMatrixLayout as ML, FeedForwardLayer
+    rng = np.random.default_rng(sum(dims) + B)
+    L = len(dims) - 1
+    conv = cv.NetworkParameterLayoutConverter(torch.float16, (1 << L) - 1, *dims)
+    portable = (rng.standard_normal(conv.ElementCountLogical) * 0.2).astype(np.float16)
+    pd = to_dev(portable)
+    x = to_dev(rng.uniform(-1, 1, (B, dims[0])).astype(np.float16))
+    t = to_dev(rng.uniform(-1, 1, (B, dims[-1])).astype(np.float16))
+    kernels = []
+    for hidden in (Activation.ReLU, Activation.LeakyReLU, Activation.NoActivation):
+        acts = [hidden] * (L - 1) + [Activation.NoActivation]
+        grads = torch.zeros_like(pd)
+        loss = conv.trainStep(pd, grads, x, t, optimalLayout=False, activations=acts, leakySlopes=[0.125] * L, lossScale=1.0 / B)
+        kernels.append(cv.lastKernelName())
+        layers, off = [], 0
+        for fi, fo in zip(dims, dims[1:]):
+            W, b = portable[off:off + fi * fo], portable[off + fi * fo:off + fi * fo + fo]
+            off += fi * fo + fo
+            layers.append(FeedForwardLayer(fi, fo, as_bytes(to_dev(W)), as_bytes(to_dev(b)), ML.RowMajor, fi * 2, acts[len(layers)], 0.125,
+                                           torch.zeros(fi * fo * 2, dtype=torch.uint8, device=x.device), torch.zeros(fo * 2, dtype=torch.uint8, device=x.device),
+                                           ML.RowMajor, fi * 2))
+        _, want = cv.mlpTrainStep(layers, x, t, lossScale=1.0 / B, gradType=cv.CoopVecComponentType.Float16)
+        assert cv.lastKernelName() == kernels[-1] and want.item() == loss.item()
+        assert torch.equal(torch.cat([v for y in layers for v in (y.weightsGrad, y.biasesGrad)]), grads.view(torch.uint8))
+    assert len(set(kernels)) > 1 or dims[0] > 32 or len(dims) > 4 or max(dims[1:-1]) <= 64, kernels
