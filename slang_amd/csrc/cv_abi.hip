@@ -867,8 +867,8 @@ static CvResult trainStep(const char* who, void* stream, const CvMlpDesc* mlp, c
     if (CV_FAILED(rc)) return rc;
     size_t need = 0;
     TrainStepKind kind = chooseTrainStep(t.mlp, mlp->flags, t.carrierCt, cus, &need);
-    // The step over rounds keeps a whole set of gradients per workgroup (37 MB for 16-128-128-128-8), the step in memory the
-    // batch's vectors: a small batch of a wide network fits the built-in array only the second way.
+    // The step over rounds keeps a whole set of gradients per 64 samples until the chip is full (37 MB for 16-128-128-128-8), the
+    // step in memory the batch's vectors: some batches of wide networks fit the built-in array only the second way.
     if (ownScratch && kind == TrainStepKind::Rounds && workspaceBytes < need) {
         const size_t general = cv::trainGeneralWorkspaceBytes(t.mlp, cus, t.carrierCt);
         if (general <= workspaceBytes) { kind = TrainStepKind::General; need = general; }

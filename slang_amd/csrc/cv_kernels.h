@@ -123,8 +123,9 @@ constexpr uint32_t kTrainTeamMinBatch = 16384;
 bool trainTeamTakes(const TrainLaunch& args);
 hipError_t launchMlpTrainTeam(hipStream_t stream, const TrainLaunch& args, int numCUs);
 // The step layer by layer over rounds of 64 samples inside a workgroup (cv_train_round.h), for half and float networks outside
-// the fused kernels' shapes that fit the LDS of a compute unit: bytes of workspace, 0 where it does not apply.
-size_t trainRoundWorkspaceBytes(const MlpArgs& shapes, int numCUs, int carrierCt);
+// the fused kernels' shapes that fit the LDS of a compute unit: bytes of workspace (which grow with mlp.batch until every
+// workgroup that fits the chip has work), 0 where it does not apply.
+size_t trainRoundWorkspaceBytes(const MlpArgs& shapesAndBatch, int numCUs, int carrierCt);
 hipError_t launchTrainRound(hipStream_t stream, const TrainLaunch& args, int numCUs);
 // The same step layer by layer through the batched kernels, for any layer sizes: per-layer vectors
 // of the whole batch are parked in the workspace, whose size therefore grows with mlp.batch.

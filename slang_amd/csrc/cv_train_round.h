@@ -675,6 +675,12 @@ inline uint32_t roundWorkgroups(const RoundArgs& a, int layers, int rt, int numC
     return (uint32_t)numCUs * (roundWavesPerSimd(layers, rt) == 4 && a.ldsBytes <= 80u * 1024u ? 2u : 1u);
 }
 inline int roundTiles(int maxTiles) { return maxTiles > 4 ? 4 : 2; }
+// workgroups of a launch: no more than the batch has rounds
+inline uint32_t roundBlocks(uint32_t batch, uint32_t resident)
+{
+    const uint32_t rounds = batch ? (batch - 1) / kRoundSamples + 1 : 1;
+    return rounds < resident ? rounds : resident;
+}
 
 template <typename T, int NL, int RT>
 hipError_t launchRoundSized(hipStream_t stream, const TrainLaunch& t, RoundArgs& a, int numCUs)
@@ -682,8 +688,7 @@ hipError_t launchRoundSized(hipStream_t stream, const TrainLaunch& t, RoundArgs&
     constexpr int WAVES = roundWavesPerSimd(NL, RT);
     const hipError_t e = allowDynamicLds<trainRoundKernel<T, NL, RT, WAVES>>(160 * 1024);
     if (e != hipSuccess) return e;
-    const uint32_t rounds = (t.mlp.batch - 1) / kRoundSamples + 1, resident = roundWorkgroups(a, NL, RT, numCUs);
-    const uint32_t blocks = rounds < resident ? rounds : resident;
+    const uint32_t blocks = roundBlocks(t.mlp.batch, roundWorkgroups(a, NL, RT, numCUs));
     a.finish.numPartials = blocks;
     // (the tests of the step over the whole batch tell the two apart by this name: both go through the network layer by layer)
     noteKernel(false, "layer-by-layer training step in LDS: trainRoundKernel<%s,%d layers,up to %d rows> + trainRoundReduceKernel",

@@ -223,6 +223,32 @@ def test_a_loss_that_is_not_finite_voids_the_step(elem, dims, kernel, value):
         assert np.isnan(gW[l]).all() and np.isnan(gB[l]).all(), l
 
 
+@pytest.mark.parametrize("elem,dims,kernel", KERNELS)
+def test_workspace_grows_with_the_batch_and_is_enough(elem, dims, kernel):
+    # One set of gradients for every 64 samples until the chip is full.  The step stays inside what the query says (what lies
+    # behind it keeps its bytes), and gives the same bits whatever the workspace held before.
+    rng = np.random.default_rng(sum(dims) + 5)
+    dtype, ct = (np.float32, CT.Float32) if elem == "f32" else (np.float16, CT.Float16)
+    specs = whole_number_network(rng, dims, dtype, Activation.ReLU, 0.0, Activation.NoActivation)
+    size = lambda B: cv.mlpTrainStepWorkspaceSize(build(specs, ct), B, weightType=ct)
+    one, full = size(1), size(1 << 30)
+    assert one == size(64) and size(65) == 2 * one and full % one == 0 and full >= 256 * one and size(0xffffffff) == full
+    for B in (1, 64, 65, 1000, 64 * 255 + 1, 64 * 600):
+        x = to_dev(rng.integers(-1, 2, (B, dims[0])).astype(dtype))
+        t = to_dev(rng.integers(-2, 3, (B, dims[-1])).astype(dtype))
+        need, got = size(B), []
+        assert need == min(-(-B // 64) * one, full)
+        for fill in (0xff, 0x3c):
+            layers = build(specs, ct)
+            room = torch.full((need + 4096,), fill, dtype=torch.uint8, device=DEV)
+            _, loss = cv.mlpTrainStep(layers, x, t, lossScale=1.0 / 16, weightType=ct, workspace=room[:need])
+            assert kernel in cv.lastKernelName(), cv.lastKernelName()
+            assert (room[need:] == fill).all()
+            got.append((loss.item(), [v.clone() for y in layers for v in (y.weightsGrad, y.biasesGrad)]))
+        assert got[0][0] == got[1][0] and all(torch.equal(a, b) for a, b in zip(got[0][1], got[1][1]))
+        assert np.isfinite(got[0][0])
+
+
 def test_the_largest_batch():
     # 2^32 - 1 samples: rounds and tiles are counted without leaving 32 bits.  All samples are 0 but the first and the last.
     B = 0xffffffff

@@ -57,18 +57,21 @@ def test_no_alloc_on_the_layer_by_layer_step_and_its_limit():
     assert e.value.result == cv.SLANG_E_NOT_AVAILABLE
 
 
-def test_no_alloc_takes_a_small_batch_of_a_network_whose_step_in_lds_needs_more_scratch():
-    # the step in LDS keeps a set of gradients per workgroup, more than the built-in array for this network: the step
-    # over the whole batch in memory takes the call (the same result as asking for that step)
+@pytest.mark.parametrize("dims,B,over_memory", [([16, 128, 128, 128, 8], 300, False), ([16, 128, 128, 128, 8], 7168, False),
+                                                 ([97, 118, 125, 7], 8300, True)])
+def test_no_alloc_on_the_step_in_lds_and_where_it_needs_more_scratch(dims, B, over_memory):
+    # The step in LDS keeps a set of gradients per 64 samples.  Where they exceed the built-in array and the vectors of the
+    # batch do not, the step over the batch in memory takes the call (the same result as asking for that step).
     rng = np.random.default_rng(5)
-    specs = make_specs(rng, [16, 128, 128, 128, 8])
-    x = to_dev(rng.uniform(-1, 1, (300, 16)).astype(np.float16))
+    specs = make_specs(rng, dims)
+    x = to_dev(rng.uniform(-1, 1, (B, dims[0])).astype(np.float16))
     ref_layers, layers = build(specs), build(specs)
-    assert cv.mlpTrainStepWorkspaceSize(layers, 300) > cv.NOALLOC_SCRATCH_BYTES
-    t = to_dev(rng.uniform(-1, 1, (300, 8)).astype(np.float16))
-    _, ref_loss = cv.mlpTrainStep(ref_layers, x, t, flags=cv.FLAG_LAYERWISE_TRAINING)
+    assert (cv.mlpTrainStepWorkspaceSize(layers, B) > cv.NOALLOC_SCRATCH_BYTES) == over_memory
+    t = to_dev(rng.uniform(-1, 1, (B, dims[-1])).astype(np.float16))
+    _, ref_loss = cv.mlpTrainStep(ref_layers, x, t, flags=cv.FLAG_LAYERWISE_TRAINING if over_memory else 0)
     loss = torch.zeros(1, dtype=torch.float32, device=DEV)
     cv.mlpTrainStepNoAlloc(layers, x, t, loss)
+    assert ("trainRoundKernel" in cv.lastKernelName()) == (not over_memory), cv.lastKernelName()
     for r, g in zip(ref_layers, layers):
         assert torch.equal(r.weightsGrad, g.weightsGrad) and torch.equal(r.biasesGrad, g.biasesGrad)
     assert ref_loss.item() == loss.item()
