@@ -309,9 +309,7 @@ hipError_t launchChainSized(hipStream_t stream, const GenArgs& ga, size_t ldsByt
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpChainKernel<Mma, MAXT, NT, QUAD>, 256, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
     const uint32_t numTiles = (uint32_t)(((uint64_t)ga.mlp.batch + 15) / 16), need = (numTiles + 4 * NT - 1) / (4 * NT);
     const uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU;
-    // (float and bfloat16 networks report the name of their family)
-    constexpr bool kFloatFamily = chainComponent<Mma>() != kF16;
-    noteKernel(false, "%s<%s,up to %d rows,NT=%d%s>", kFloatFamily ? "mlpFloatKernel: mlpChainKernel" : "mlpChainKernel", Mma::kName, 16 * MAXT, NT,
+    noteKernel(false, "mlpChainKernel<%s,up to %d rows,NT=%d%s>", Mma::kName, 16 * MAXT, NT,
                QUAD ? ",loads of four elements" : "");
     hipLaunchKernelGGL((mlpChainKernel<Mma, MAXT, NT, QUAD>), dim3(need < cap ? need : cap), dim3(256), ldsBytes, stream, ga);
     return hipGetLastError();

@@ -690,8 +690,7 @@ hipError_t launchRoundSized(hipStream_t stream, const TrainLaunch& t, RoundArgs&
     if (e != hipSuccess) return e;
     const uint32_t blocks = roundBlocks(t.mlp.batch, roundWorkgroups(a, NL, RT, numCUs));
     a.finish.numPartials = blocks;
-    // (the tests of the step over the whole batch tell the two apart by this name: both go through the network layer by layer)
-    noteKernel(false, "layer-by-layer training step in LDS: trainRoundKernel<%s,%d layers,up to %d rows> + trainRoundReduceKernel",
+    noteKernel(false, "trainRoundKernel<%s,%d layers,up to %d rows> + trainRoundReduceKernel",
                sizeof(T) == 4 ? "f32" : "f16", NL, 32 * RT);
     hipLaunchKernelGGL((trainRoundKernel<T, NL, RT, WAVES>), dim3(blocks), dim3(kRoundThreads), a.ldsBytes, stream, a);
     const hipError_t e1 = hipGetLastError();

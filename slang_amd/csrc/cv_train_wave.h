@@ -355,7 +355,7 @@ hipError_t launchWave(hipStream_t stream, const TrainLaunch& t, RoundArgs& a, in
     if (e != hipSuccess) return e;
     const uint32_t need = (t.mlp.batch - 1u) / 128u + 1u, blocks = need < (uint32_t)numCUs ? need : (uint32_t)numCUs;
     a.finish.numPartials = blocks;
-    noteKernel(false, "layer-by-layer training step by waves: trainWaveKernel<f32,%d layers,inputs<=%d,hidden<=%d> + trainRoundReduceKernel", Net::NL, 16 * Net::IT, 16 * Net::HT);
+    noteKernel(false, "trainWaveKernel<f32,%d layers,inputs<=%d,hidden<=%d> + trainRoundReduceKernel", Net::NL, 16 * Net::IT, 16 * Net::HT);
     hipLaunchKernelGGL((trainWaveKernel<Net>), dim3(blocks), dim3(512), Net::ldsBytes, stream, a);
     const hipError_t e1 = hipGetLastError();
     if (e1 != hipSuccess) return e1;

@@ -51,7 +51,7 @@ def test_chain_kernel_equals_single_layers(dims, ct):
             out = torch.full((B + 2, dims[-1] + pad), -7.0, dtype=want.dtype, device=DEV)
             cv.mlpForward(layers, surrounded(x, pad), weightType=ct, out=out[1:B + 1, :dims[-1]])
             name = cv.lastKernelName()
-            assert "mlpChainKernel" in name, name
+            assert name.startswith("mlpChainKernel"), name
             bits = torch.int32 if want.element_size() == 4 else torch.int16
             assert torch.equal(out[1:B + 1, :dims[-1]].contiguous().view(bits), want.contiguous().view(bits)), (dims, ct, B, pad, name)
             assert (out[0] == -7).all() and (out[B + 1] == -7).all() and (out[:, dims[-1]:] == -7).all()

@@ -75,19 +75,22 @@ def chain(params, x, ct, acts):
 
 @pytest.mark.parametrize("ct", [CT.Float32, CT.BFloat16])
 @pytest.mark.parametrize("dims", [[8, 64, 64, 4], [5, 13, 7, 19], [100, 128, 50, 3], [32, 16, 16, 16, 16, 1]])
-def test_float_networks_equal_the_chain_of_single_layer_operators(ct, dims):
+@pytest.mark.parametrize("first", [Activation.ReLU, Activation.Tanh])
+def test_float_networks_equal_the_chain_of_single_layer_operators(ct, dims, first):
+    # (smooth activations run on mlpFloatKernel, networks without them on mlpChainKernel)
     rng = np.random.default_rng(sum(dims) + int(ct))
     B = 1000
     L = len(dims) - 1
     acts = [[Activation.ReLU, Activation.NoActivation, Activation.LeakyReLU, Activation.Tanh, Activation.Sigmoid][l % 5] for l in range(L)]
-    acts[1] = Activation.NoActivation
+    acts[0], acts[1] = first, Activation.NoActivation
+    smooth = any(a in (Activation.Tanh, Activation.Sigmoid) for a in acts)
     x64 = rng.uniform(-1, 1, (B, dims[0]))
     xd = to_T(x64, ct)
     ys = []
     for layout in (ML.RowMajor, ML.InferencingOptimal, ML.TrainingOptimal):
         layers, params = build(np.random.default_rng(7), dims, ct, acts, layout)
         y = cv.mlpForward(layers, xd, weightType=ct)
-        assert cv.lastKernelName().startswith("mlpFloatKernel"), cv.lastKernelName()
+        assert cv.lastKernelName().startswith("mlpFloatKernel" if smooth else "mlpChainKernel"), cv.lastKernelName()
         assert y.dtype == TORCH[ct] and y.shape == (B, dims[-1])
         ys.append(y)
     bits = torch.int32 if ct == CT.Float32 else torch.int16
@@ -199,11 +202,16 @@ def backprop64(portable, dims, mask, acts, slope, x, t, loss_scale):
 
 
 @pytest.mark.parametrize("grad_layout", [ML.RowMajor, ML.TrainingOptimal])
-def test_fp32_training_step_against_float64(grad_layout):
-    # learnGradient for a network of float (layer by layer): loss and every gradient against float64 backpropagation
+@pytest.mark.parametrize("dims,flags,kernel", [
+    ([6, 20, 13, 3], 0, "trainWaveKernel"), ([100, 128, 13, 3], 0, "trainRoundKernel"),
+    ([6, 20, 13, 3], cv.FLAG_LAYERWISE_TRAINING, "layer-by-layer"),      # the step over memory: asked for, more than 16 outputs,
+    ([6, 20, 13, 17], 0, "layer-by-layer"), ([6, 150, 13, 3], 0, "layer-by-layer"),      # wider than 128
+])
+def test_fp32_training_step_against_float64(grad_layout, dims, flags, kernel):
+    # learnGradient for a network of float: loss and every gradient against float64 backpropagation
     # on the same fp32 parameters; "+=" into pre-filled destinations; bitwise reproducible
     rng = np.random.default_rng(17)
-    dims, mask = [6, 20, 13, 3], 0b111
+    mask = 0b111
     acts = [Activation.ReLU, Activation.LeakyReLU, Activation.NoActivation]
     n_par = sum(dims[k] * dims[k + 1] + dims[k + 1] for k in range(3))
     portable = (rng.standard_normal(n_par) * 0.5).astype(np.float32)
@@ -223,8 +231,8 @@ def test_fp32_training_step_against_float64(grad_layout):
             layers.append(FeedForwardLayer(fi, fo, as_bytes(to_dev(W)), as_bytes(to_dev(b)), ML.RowMajor, fi * 4, acts[k], 0.125,
                                            wg, as_bytes(bg), grad_layout, fi * 4 if grad_layout == ML.RowMajor else 0))
             views.append((wg, bg, gsize))
-        _, loss = cv.mlpTrainStep(layers, to_dev(x), to_dev(t), lossScale=0.5, weightType=CT.Float32)
-        assert "layer-by-layer" in cv.lastKernelName()
+        _, loss = cv.mlpTrainStep(layers, to_dev(x), to_dev(t), lossScale=0.5, weightType=CT.Float32, flags=flags)
+        assert cv.lastKernelName().startswith(kernel), cv.lastKernelName()
         out = []
         for k, (wg, bg, gsize) in enumerate(views):
             fi, fo = dims[k], dims[k + 1]
