@@ -77,3 +77,30 @@ def test_chain_kernel_keeps_non_finite_values_to_their_sample(ct):
     keep = torch.ones(B, dtype=torch.bool, device=DEV)
     keep[[37, 38, B - 1]] = False
     assert torch.equal(got[keep], clean[keep])
+
+
+@pytest.mark.parametrize("ct,other", [(CT.Float16, "mlpGenericKernel"), (CT.FloatE4M3, "mlpGenericKernel"), (CT.Float32, "mlpFloatKernel"), (CT.BFloat16, "mlpFloatKernel")])
+def test_rows_far_apart(ct, other):
+    # sixteen vectors up to 2^26 bytes apart lie within the reach of a tile's descriptor; beyond that the kernel with run-time
+    # sizes takes the network, with the same bits
+    rng = np.random.default_rng(int(ct))
+    dims, B = [20, 48, 24, 5], 33
+    floats = ct in TORCH
+    if floats:
+        acts = [Activation.ReLU, Activation.NoActivation, Activation.NoActivation]
+        layers, _ = build(rng, dims, ct, acts, ML.RowMajor)
+    else:
+        layers = gpu_layers(make_net(rng, dims, ct, act=Activation.ReLU, bias="rand", init="he" if ct == CT.Float16 else "half"), ct, ML.RowMajor)
+    x64 = rng.uniform(-1, 1, (B, dims[0]))
+    x = to_T(x64, ct) if floats else to_dev(x64.astype(np.float16))
+    if ct == CT.FloatE4M3:
+        x = x.to(torch.float8_e4m3fn)
+    want = cv.mlpForward(layers, x, weightType=ct).clone()
+    big = torch.zeros((B * ((1 << 26) + 16),), dtype=torch.uint8, device=DEV).view(x.dtype)
+    for pitch, name in (((1 << 26), "mlpChainKernel"), ((1 << 26) + 16, other)):
+        rows = big.as_strided((B, dims[0]), (pitch // x.element_size(), 1))
+        rows.copy_(x)
+        got = cv.mlpForward(layers, rows, weightType=ct)
+        assert cv.lastKernelName().startswith(name), cv.lastKernelName()
+        bits = torch.int32 if want.element_size() == 4 else torch.int16
+        assert torch.equal(got.view(bits), want.view(bits))
