@@ -3,10 +3,12 @@
 // Replaces, for a whole batch of positions, PermutoEncoder::encode and its reverse mode
 // (source/standard-modules/neural/permuto-encoder.slang:240-337, readFeatureValueBwd :222-238,
 // prepareLevelInfo :339-368) and the grid hashes it is built on
-// (source/standard-modules/neural/hash-function.slang:69-151).  One thread handles one position: it
-// walks the levels, finds the enclosing simplex of the permutohedral lattice, and gathers D+1 hashed
-// feature-table entries per level -- integer hashing plus scattered reads, bound by cache and HBM
-// latency, not by arithmetic.  The reverse pass scatters with atomic adds, as the reference does.
+// (source/standard-modules/neural/hash-function.slang:69-151).  A thread handles one position and level (or all levels of a
+// position, one after the other): it finds the enclosing simplex of the permutohedral lattice and gathers D+1 hashed
+// feature-table entries.  With the table in LDS the arithmetic binds: 160 to 230 vector instructions per position and
+// level in two and three dimensions keep the vector-ALU port full.  The reverse pass adds every position's contributions to the
+// table gradient up in LDS, by parts of the table, and only the sums to memory; tables that cannot be cut so, and a handful of
+// positions, are added in memory with atomics, as the reference does.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -325,14 +327,15 @@ __global__ __launch_bounds__(256) void permutoBackwardKernel(const PermutoArgs a
 // The table gradient, by parts of the table small enough for LDS: part p covers elements [base, base + elems), which
 // levels [first, end) add to.  Every position adds to a handful of entries per level; added in memory, where many positions
 // meet on few addresses, 2^18 positions in 3 dimensions on 8 levels of 2^12 two-feature entries took 6.6 ms (2.5 G additions
-// per second); here 40 us, of which a quarter is the start and the sums' way to memory.  (cutTable: cv_permuto_parts.h)
+// per second); here 37 us, of which a quarter is the start and the sums' way to memory.  (cutTable: cv_permuto_parts.h)
 static_assert(sizeof(PermutoArgs) + sizeof(TableParts) <= 4096, "kernel arguments");
 
 // A workgroup owns one part and a share of the positions: it sums into LDS and adds its sums to memory once, coalesced
-// (180 G additions per second).  What bounds it: the LDS's additions and the vector instructions that find the simplex
-// (170 per position and level).  The sums are kept in double: gfx950 serves a ds_add_f64 in 8.6 ns per wave and compute
-// unit, whatever the spread of the addresses, and a ds_add_f32 in 80 (measured, random addresses, 16 waves), so the wider
-// sum is also the cheaper one and needs no copies per lane to keep equal addresses apart.
+// (180 G additions per second).  What bounds it: the LDS's additions (the waves of that case wait 46 % of their time for the LDS to
+// take one) and the vector instructions, 280 per position and level, which take 36 % of the port.  The sums are kept in double:
+// at random addresses gfx950 serves a ds_add_f64 in 8.6 ns per wave and compute unit and a ds_add_f32 in 80 (16 waves), so the
+// wider sum is also the cheaper one.  Lanes that meet on one address are served one after the other: 24 ns per LDS instruction
+// in that case, 41 ns on the few entries of four coarse levels in two dimensions (2^22 positions: 256 us).
 // POS (one part that is the whole table): the position gradient in the same pass.  SLICED: some part is a slice of a level.
 template <int D, int FT, bool POS, bool SLICED>
 __global__ __launch_bounds__(1024) void permutoTableGradKernel(const PermutoArgs a, const TableParts parts)

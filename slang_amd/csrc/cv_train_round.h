@@ -21,8 +21,12 @@
 // registers allow, so that one works while the other meets.
 //
 // What bounds it: float: the matrix pipeline (v_mfma_f32_16x16x4_f32 takes 32 cycles for what two 4-byte reads supply).
-// half: LDS reads (one 16-byte read per lane and operand feeds 16 cycles of the pipeline) and the meetings.
-// 16-128-128-128-8 (half) over 200 003 samples: 187 us, 724 us over the whole batch in memory.
+// half: waiting, for operands from LDS (one 16-byte read per lane and operand feeds 16 cycles of the pipeline) and at the
+// meetings; the waves of 16-128-128-128-8 wait 57 % of their time and the pipeline is busy 10 %.  Half networks wider than 64 also
+// keep part of the prefetched input in scratch memory (32 bytes a lane, five layers 64), so that each round begins with a wait
+// for memory; five float layers up to 64 wide spill 108 bytes.
+// 16-128-128-128-8 (half) over 200 003 samples: 187 us, 724 us over the whole batch in memory.  Of these about 76 us are paid
+// once (LDS cleared, weights staged element by element, the partials written and added up) and 10 us for each further round.
 #pragma once
 #include "cv_train_impl.h"
 

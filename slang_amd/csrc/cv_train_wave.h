@@ -13,7 +13,9 @@
 // and dZ of the wave's 16 samples also go to LDS, [sample][feature], and come back by columns; dZ_l takes the place of X_l.
 // One copy of W serves both directions, by rows forward, by columns for dX.
 //
-// What bounds it: the matrix pipeline (32 cycles per instruction; 296 of them for 16 samples of 32-64-64-8).
+// What bounds it: the matrix pipeline (32 cycles per instruction; 304 of them for 16 samples of 32-64-64-8, which keep it busy
+// 65 % of the time).  Of the instantiations one spills: three layers with 33 to 64 inputs keep 136 bytes a lane in scratch memory
+// (64-64-64-9 over 2^19 samples: 245 us, 32-64-64-8: 213 us).
 #pragma once
 #include "cv_train_round.h"
 
