@@ -225,8 +225,9 @@ def test_permuto_backward_table_parts(D, F, levels_n, log2, B, kernel):
 
 
 @pytest.mark.parametrize("F,tables,B,kernel", [
-    # a third of the entries would be 1366 x 15 (6827 x 3) doubles, ten (one) more than the LDS holds
+    # a third of the entries would be 1366 x 15 (683 x 30, 6827 x 3) doubles, ten (ten, one) more than the LDS holds
     (15, [(0, 4096), (4096, 4096)], 700, "permutoTableGradKernel<D=2,8 parts> + permutoBackwardKernel<D=2,positions>"),
+    (30, [(0, 2048)], 500, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),
     (3, [(0, 20480)], 900, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),
     # small tables with gaps, in reverse order, on shared entries, all of them a single part
     (2, [(3, 256), (267, 256), (531, 100), (700, 256)], 5000, "permutoTableGradKernel<D=2,positions>"),
