@@ -6,7 +6,7 @@
 // (source/standard-modules/neural/hash-function.slang:69-151).  A thread handles one position and level (or all levels of a
 // position, one after the other): it finds the enclosing simplex of the permutohedral lattice and gathers D+1 hashed
 // feature-table entries.  With the table in LDS the arithmetic binds: 160 to 230 vector instructions per position and
-// level in two and three dimensions keep the vector-ALU port full.  The reverse pass adds every position's contributions to the
+// level in two and three dimensions kept the vector-ALU port full, some 130 in three do now (LatticeSimplex).  The reverse pass adds every position's contributions to the
 // table gradient up in LDS, by parts of the table, and only the sums to memory; tables that cannot be cut so, and a handful of
 // positions, are added in memory with atomics, as the reference does.
 #include <hip/hip_runtime.h>
@@ -109,6 +109,7 @@ struct PermutoArgs {
     uint8_t* dPos; uint64_t dPosStride;
     float* dTable;
     uint32_t batch;
+    float reach;      // latticeReach
 };
 
 template <typename T, int D>
@@ -127,17 +128,16 @@ __global__ __launch_bounds__(256) void permutoEncodeKernel(const PermutoArgs a)
         T* o = out + lv.currentLevelIndex * F;
         for (int f = 0; f < F; ++f) o[f] = (T)0.f;
         if ((float)lv.currentLevelIndex >= a.desc.maxLevel + 1e-3f) continue;   // zero padding beyond maxLevel, :259-262
-        float elevated[D + 1], bary[D + 2];
-        int rem0[D + 1], rank[D + 1];
-        latticeGeometry<D>(pos, lv, elevated, rem0, rank);
-        barycentricWeights<D>(elevated, rem0, rank, bary);
+        LatticeSimplexAny<D> simplex;
+        simplex.search(pos, latticeLevel<D>(lv));
         uint32_t idx[D + 1];
-        vertexIndices<D>(lv, F, rem0, rank, idx);
+#pragma unroll
+        for (int k = 0; k <= D; ++k) idx[k] = (lv.offsetOfFeatureTable + vertexSlot<false>(lv.featureTableSize, simplex.hash[k])) * (uint32_t)F;
         for (int f0 = 0; f0 < F; f0 += 4) {                            // four features of the entry at a time
             T acc[4] = {(T)0.f, (T)0.f, (T)0.f, (T)0.f};
 #pragma unroll
             for (int k = 0; k <= D; ++k) {
-                const T w = (T)bary[k];
+                const T w = (T)simplex.bary[k];
 #pragma unroll
                 for (int f = 0; f < 4; ++f)
                     if (f0 + f < F) acc[f] = (T)(acc[f] + (T)(w * table[idx[k] + f0 + f]));    // in T, vertex by vertex (:312-316)
@@ -153,19 +153,17 @@ __global__ __launch_bounds__(256) void permutoEncodeKernel(const PermutoArgs a)
 // consecutive in memory (one thread per position writes F elements at the pitch of a whole row, which the memory
 // system does not merge: 2.1 bytes written per byte of output), no thread loops over levels, and a feature table that
 // fits is held in LDS, where a gather of 64 scattered entries costs a few cycles instead of one cache line per lane.
-// The arithmetic per (position, level) is that of permutoEncodeKernel, instruction for instruction.
+// The arithmetic per (position, level) is that of permutoEncodeKernel, bit for bit.
 template <typename T, int D, int F, bool LDS_TABLE, bool PLAIN>
 __global__ __launch_bounds__(1024) void permutoEncodePairsKernel(const PermutoArgs a, uint32_t tableElems, uint32_t levelShift)
 {
     typedef typename PermutoEntry<T, F>::type Entry;
     extern __shared__ __align__(16) uint8_t ldsRaw[];
-    CvPermutoLevelInfo* levels = (CvPermutoLevelInfo*)ldsRaw;
+    LatticeLevel<D>* levels = (LatticeLevel<D>*)ldsRaw;
     const T* ldsTable = (const T*)(ldsRaw + kMaxLevels * sizeof(CvPermutoLevelInfo));
     const uint32_t L = a.desc.maxLevels;
     {
-        constexpr uint32_t words = sizeof(CvPermutoLevelInfo) / 4u;
-        const uint32_t* src = (const uint32_t*)a.desc.levelInfo;
-        for (uint32_t i = threadIdx.x; i < L * words; i += blockDim.x) ((uint32_t*)levels)[i] = src[i];
+        if (threadIdx.x < L) levels[threadIdx.x] = latticeLevel<D>(a.desc.levelInfo[threadIdx.x]);
         if constexpr (LDS_TABLE) {
             const Entry* t = (const Entry*)a.table;
             Entry* dst = (Entry*)(ldsRaw + kMaxLevels * sizeof(CvPermutoLevelInfo));
@@ -178,13 +176,15 @@ __global__ __launch_bounds__(1024) void permutoEncodePairsKernel(const PermutoAr
     for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < pairs; p += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t s = levelShift < 32u ? (uint32_t)(p >> levelShift) : (uint32_t)(p / L);
         const uint32_t l = (uint32_t)(p - (uint64_t)s * L);
-        const CvPermutoLevelInfo& lv = levels[l];
+        const LatticeLevel<D>& lv = levels[l];
         float pos[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) pos[d] = (float)((const T*)(a.pos + (size_t)s * a.posStride))[d];
-        const Entry acc = permutoEncodeEntry<T, D, F, PLAIN>(pos, lv, table, a.desc.maxLevel);
+        Entry acc;
+        if (!PLAIN || anyBeyondReach<D>(pos, a.reach)) acc = permutoEncodeEntry<T, D, F, PLAIN, LatticeSimplexAny<D>>(pos, lv, table, a.desc.maxLevel);
+        else if constexpr (PLAIN) acc = permutoEncodeEntry<T, D, F, PLAIN, LatticeSimplex<D>>(pos, lv, table, a.desc.maxLevel);
         // (a streaming store: the encoded vectors are written once and read by the next kernel)
-        __builtin_nontemporal_store(acc, (Entry*)((T*)(a.out + (size_t)s * a.outStride) + lv.currentLevelIndex * F));
+        __builtin_nontemporal_store(acc, (Entry*)((T*)(a.out + (size_t)s * a.outStride) + lv.index * F));
     }
 }
 
@@ -237,27 +237,29 @@ struct TableInLds {
 // gradient (of all levels: such calls take them all).
 // FT: the features per entry when they are 1, 2 or 4 (the loops over them unrolled, the loads of a level issued together:
 // with a run-time count every element was a load and a wait of its own), else 0.
-template <int D, int FT, bool POS, typename Sink>
-__device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_t s, uint32_t first, uint32_t end, const Sink& sink)
+// PLAIN, Simplex: as in permutoEncodeEntry.
+template <int D, int FT, bool POS, bool PLAIN, typename Simplex, typename Sink>
+__device__ __forceinline__ void permutoBackwardLevels(const PermutoArgs& a, const float* pos, uint32_t s, uint32_t first, uint32_t end, const Sink& sink)
 {
     const int F = FT ? FT : a.desc.featureDimensionPerEntry;
-    float pos[D], dpos[D];
+    float dpos[D];
 #pragma unroll
-    for (int d = 0; d < D; ++d) { pos[d] = ((const float*)(a.pos + (size_t)s * a.posStride))[d]; dpos[d] = 0.f; }
+    for (int d = 0; d < D; ++d) dpos[d] = 0.f;
     const float* table = (const float*)a.table;
     const float* g = (const float*)(a.dOut + (size_t)s * a.dOutStride);
     for (uint32_t l = first; l < end; ++l) {
         const CvPermutoLevelInfo& lv = a.desc.levelInfo[l];
-        if ((float)lv.currentLevelIndex >= a.desc.maxLevel + 1e-3f) continue;
-        float elevated[D + 1], bary[D + 2], dbary[D + 2];
-        int rem0[D + 1], rank[D + 1];
-        latticeGeometry<D>(pos, lv, elevated, rem0, rank);
-        barycentricWeights<D>(elevated, rem0, rank, bary);
-#pragma unroll
-        for (int i = 0; i <= D + 1; ++i) dbary[i] = 0.f;
-        const float* gl = g + lv.currentLevelIndex * F;
+        if (!PLAIN && (float)lv.currentLevelIndex >= a.desc.maxLevel + 1e-3f) continue;
+        Simplex simplex;
+        simplex.search(pos, latticeLevel<D>(lv));
+        float dbary[D + 1];
         uint32_t idx[D + 1];
-        vertexIndices<D>(lv, F, rem0, rank, idx);
+#pragma unroll
+        for (int k = 0; k <= D; ++k) {
+            dbary[k] = 0.f;
+            idx[k] = (lv.offsetOfFeatureTable + vertexSlot<PLAIN>(lv.featureTableSize, simplex.hash[k])) * (uint32_t)F;
+        }
+        const float* gl = g + lv.currentLevelIndex * F;
         if constexpr (FT > 0) {
             float gv[FT], tv[D + 1][FT];
 #pragma unroll
@@ -270,7 +272,7 @@ __device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_
             }
 #pragma unroll
             for (int k = 0; k <= D; ++k) {
-                if constexpr (Sink::kWanted) sink.template addEntry<FT>(idx[k], bary[k], gv);    // readFeatureValueBwd, :222-238
+                if constexpr (Sink::kWanted) sink.template addEntry<FT>(idx[k], simplex.bary[k], gv);    // readFeatureValueBwd, :222-238
 #pragma unroll
                 for (int f = 0; f < FT; ++f) {
                     if constexpr (POS) dbary[k] += tv[k][f] * gv[f];
@@ -280,24 +282,14 @@ __device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_
 #pragma unroll
             for (int k = 0; k <= D; ++k) {
                 for (int f = 0; f < F; ++f) {
-                    if constexpr (Sink::kWanted) sink.add(idx[k], f, bary[k] * gl[f]);    // readFeatureValueBwd, :222-238
+                    if constexpr (Sink::kWanted) sink.add(idx[k], f, simplex.bary[k] * gl[f]);    // readFeatureValueBwd, :222-238
                     if constexpr (POS) dbary[k] += table[idx[k] + f] * gl[f];
                 }
             }
         }
         if constexpr (!POS) continue;
-        dbary[D + 1] += dbary[0];                                      // the wrap-around term of barycentric[0]
         float delev[D + 1];
-#pragma unroll
-        for (int dim = 0; dim <= D; ++dim) {
-            float plus = 0.f, minus = 0.f;
-#pragma unroll
-            for (int i = 0; i <= D + 1; ++i) {
-                if (i == D - rank[dim]) plus = dbary[i];
-                if (i == D + 1 - rank[dim]) minus = dbary[i];
-            }
-            delev[dim] = (plus - minus) * (1.0f / (float)(D + 1));
-        }
+        simplex.toElevated(dbary, delev);
         // elevate: e[dim+1] = sum - (dim+1) cf, sum += cf for dim = D-1..0, e[0] = sum
         float dsum = delev[0];
 #pragma unroll
@@ -313,15 +305,30 @@ __device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_
     }
 }
 
+template <int D, int FT, bool POS, bool PLAIN, typename Sink>
+__device__ __forceinline__ void permutoBackwardOne(const PermutoArgs& a, uint32_t s, uint32_t first, uint32_t end, const Sink& sink)
+{
+    float pos[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) pos[d] = ((const float*)(a.pos + (size_t)s * a.posStride))[d];
+    if constexpr (PLAIN) {
+        if (!anyBeyondReach<D>(pos, a.reach)) {
+            permutoBackwardLevels<D, FT, POS, true, LatticeSimplex<D>>(a, pos, s, first, end, sink);
+            return;
+        }
+    }
+    permutoBackwardLevels<D, FT, POS, PLAIN, LatticeSimplexAny<D>>(a, pos, s, first, end, sink);
+}
+
 // Position gradients alone (TABLE false), or everything with the table's share added in memory: a table of which one level
 // alone is beyond what the LDS kernel below takes, or a handful of positions (launchBackwardSized).
-template <int D, int FT, bool POS, bool TABLE>
+template <int D, int FT, bool POS, bool TABLE, bool PLAIN>
 __global__ __launch_bounds__(256) void permutoBackwardKernel(const PermutoArgs a)
 {
     const uint32_t s = blockIdx.x * 256u + threadIdx.x;
     if (s >= a.batch) return;
-    if constexpr (TABLE) permutoBackwardOne<D, FT, POS>(a, s, 0u, a.desc.maxLevels, TableInMemory{a.dTable});
-    else permutoBackwardOne<D, FT, POS>(a, s, 0u, a.desc.maxLevels, NoTable{});
+    if constexpr (TABLE) permutoBackwardOne<D, FT, POS, PLAIN>(a, s, 0u, a.desc.maxLevels, TableInMemory{a.dTable});
+    else permutoBackwardOne<D, FT, POS, PLAIN>(a, s, 0u, a.desc.maxLevels, NoTable{});
 }
 
 // The table gradient, by parts of the table small enough for LDS: part p covers elements [base, base + elems), which
@@ -337,7 +344,7 @@ static_assert(sizeof(PermutoArgs) + sizeof(TableParts) <= 4096, "kernel argument
 // wider sum is also the cheaper one.  Lanes that meet on one address are served one after the other: 24 ns per LDS instruction
 // in that case, 41 ns on the few entries of four coarse levels in two dimensions (2^22 positions: 256 us).
 // POS (one part that is the whole table): the position gradient in the same pass.  SLICED: some part is a slice of a level.
-template <int D, int FT, bool POS, bool SLICED>
+template <int D, int FT, bool POS, bool SLICED, bool PLAIN>
 __global__ __launch_bounds__(1024) void permutoTableGradKernel(const PermutoArgs a, const TableParts parts)
 {
     extern __shared__ double ldsTable[];
@@ -350,7 +357,7 @@ __global__ __launch_bounds__(1024) void permutoTableGradKernel(const PermutoArgs
     __syncthreads();
     const TableInLds<FT, SLICED> sink{ldsTable, part.base, part.elems, entries, F};
     for (uint64_t s = (uint64_t)w * 1024u + threadIdx.x; s < a.batch; s += (uint64_t)parts.groups * 1024u)
-        permutoBackwardOne<D, FT, POS>(a, (uint32_t)s, part.first, part.end, sink);
+        permutoBackwardOne<D, FT, POS, PLAIN>(a, (uint32_t)s, part.first, part.end, sink);
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < part.elems; i += 1024u) {
         const uint32_t e = i / F, f = i - e * F;
@@ -433,24 +440,24 @@ hipError_t launchEncode(hipStream_t stream, const PermutoArgs& a)
     return hipGetLastError();
 }
 
-template <int D, int FT, bool POS, bool SLICED>
+template <int D, int FT, bool POS, bool SLICED, bool PLAIN>
 hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, TableParts& t, int cus)
 {
     uint32_t most = 0;
     for (uint32_t p = 0; p < t.count; ++p) most = t.part[p].elems > most ? t.part[p].elems : most;
     const size_t lds = (size_t)most * 8;
-    const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED>>((int)(kPartMost * 8));
+    const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED, PLAIN>>((int)(kPartMost * 8));
     if (e != hipSuccess) return e;
     // as many workgroups as the compute units hold, dealt evenly to the parts
     const uint32_t resident = (uint32_t)cus * (lds <= 80 * 1024 ? 2u : 1u), want = (a.batch - 1u) / 1024u + 1u;
     const uint32_t each = resident / t.count ? resident / t.count : 1u;
     t.groups = want < each ? want : each;
-    hipLaunchKernelGGL((permutoTableGradKernel<D, FT, POS, SLICED>), dim3(t.count * t.groups), dim3(1024), lds, stream, a, t);
+    hipLaunchKernelGGL((permutoTableGradKernel<D, FT, POS, SLICED, PLAIN>), dim3(t.count * t.groups), dim3(1024), lds, stream, a, t);
     return hipGetLastError();
 }
 
-template <int D, int FT>
-hipError_t launchBackwardSized(hipStream_t stream, const PermutoArgs& a)
+template <int D, int FT, bool PLAIN>
+hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
 {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
@@ -459,7 +466,7 @@ hipError_t launchBackwardSized(hipStream_t stream, const PermutoArgs& a)
     const bool cut = a.dTable && cutTable(a.desc, t);
     if (cut && t.count == 1 && a.dPos) {
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
-        return launchTableGrad<D, FT, true, false>(stream, a, t, cus);
+        return launchTableGrad<D, FT, true, false, PLAIN>(stream, a, t, cus);
     }
     // Two launches against one: a handful of positions whose few additions hardly meet is done sooner by the one kernel that adds
     // in memory.  It takes 7.4 to 8.1 us per call back to back and the pair 11.5 to 13.5 (16 positions on 3 levels of 2^10
@@ -470,17 +477,28 @@ hipError_t launchBackwardSized(hipStream_t stream, const PermutoArgs& a)
     const bool few = FT > 0 && a.batch <= 64u && features <= 16u && a.batch * (uint64_t)(D + 1) * features <= 1440u;
     if (cut && !(a.dPos && few)) {
         noteKernel(false, "permutoTableGradKernel<D=%d,%u parts>", D, t.count);
-        const hipError_t e = t.sliced ? launchTableGrad<D, FT, false, true>(stream, a, t, cus) : launchTableGrad<D, FT, false, false>(stream, a, t, cus);
+        const hipError_t e = t.sliced ? launchTableGrad<D, FT, false, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, false, false, PLAIN>(stream, a, t, cus);
         if (e != hipSuccess || !a.dPos) return e;
         noteKernel(true, "permutoBackwardKernel<D=%d,positions>", D);
-        hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false, PLAIN>), grid, block, 0, stream, a);
         return hipGetLastError();
     }
     noteKernel(false, "permutoBackwardKernel<D=%d%s%s>", D, a.dPos ? ",positions" : "", a.dTable ? ",table" : "");
-    if (a.dPos && a.dTable) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, true>), grid, block, 0, stream, a);
-    else if (a.dPos) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false>), grid, block, 0, stream, a);
-    else if (a.dTable) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, false, true>), grid, block, 0, stream, a);
+    if (a.dPos && a.dTable) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, true, PLAIN>), grid, block, 0, stream, a);
+    else if (a.dPos) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false, PLAIN>), grid, block, 0, stream, a);
+    else if (a.dTable) hipLaunchKernelGGL((permutoBackwardKernel<D, FT, false, true, PLAIN>), grid, block, 0, stream, a);
     return hipGetLastError();
+}
+
+// (kernels of their own for plain levels where vectors of few dimensions and entries of 1, 2 or 4 features make them worth
+// their code)
+template <int D, int FT>
+hipError_t launchBackwardSized(hipStream_t stream, const PermutoArgs& a)
+{
+    if constexpr (D <= 4 && FT > 0) {
+        if (permutoPlainLevels(a.desc)) return launchBackwardLevels<D, FT, true>(stream, a);
+    }
+    return launchBackwardLevels<D, FT, false>(stream, a);
 }
 
 hipError_t launchBackward(hipStream_t stream, const PermutoArgs& a)
@@ -579,7 +597,7 @@ CV_API CvResult cvPermutoEncode(void* stream, const CvPermutoDesc* desc, const v
     memset(&a, 0, sizeof(a));
     a.desc = *desc;
     a.pos = (const uint8_t*)positions; a.posStride = positionStride; a.table = (const uint8_t*)featureTable;
-    a.out = (uint8_t*)out; a.outStride = outStride; a.batch = batch;
+    a.out = (uint8_t*)out; a.outStride = outStride; a.batch = batch; a.reach = latticeReach(*desc);
     const hipError_t e = esz == 4 ? launchEncode<float>((hipStream_t)stream, a) : launchEncode<half_t>((hipStream_t)stream, a);
     if (e != hipSuccess) return failWith(CV_E_INTERNAL_FAIL, "cvPermutoEncode launch: %s", hipGetErrorString(e));
     return CV_OK;
@@ -606,7 +624,7 @@ CV_API CvResult cvPermutoEncodeBackward(void* stream, const CvPermutoDesc* desc,
     a.desc = *desc;
     a.pos = (const uint8_t*)positions; a.posStride = positionStride; a.table = (const uint8_t*)featureTable;
     a.dOut = (const uint8_t*)dOut; a.dOutStride = dOutStride;
-    a.dPos = (uint8_t*)dPositions; a.dPosStride = dPositionStride; a.dTable = (float*)dFeatureTable; a.batch = batch;
+    a.dPos = (uint8_t*)dPositions; a.dPosStride = dPositionStride; a.dTable = (float*)dFeatureTable; a.batch = batch; a.reach = latticeReach(*desc);
     const hipError_t e = launchBackward((hipStream_t)stream, a);
     if (e != hipSuccess) return failWith(CV_E_INTERNAL_FAIL, "cvPermutoEncodeBackward launch: %s", hipGetErrorString(e));
     return CV_OK;

@@ -28,6 +28,7 @@ struct PermutoMlpArgs {
     uint32_t tableElems;
     uint32_t levelDword;     // where the level records start in LDS (dwords)
     uint32_t tableDword;     // where the feature table starts in LDS (dwords); unused when it stays in memory
+    float reach;             // latticeReach
 };
 
 constexpr uint32_t kLevelDwords = CV_PERMUTO_MAX_LEVELS * sizeof(CvPermutoLevelInfo) / 4;
@@ -44,11 +45,9 @@ __global__ __launch_bounds__(1024) void permutoMlpKernel(const PermutoMlpArgs pa
     const GenArgs& ga = pa.net;
     const MlpArgs& a = ga.mlp;
     genericStage<Mma>(ga, lds);
-    CvPermutoLevelInfo* levels = (CvPermutoLevelInfo*)(lds + pa.levelDword);
+    LatticeLevel<D>* levels = (LatticeLevel<D>*)(lds + pa.levelDword);
     {
-        const uint32_t L = pa.desc.maxLevels;
-        const uint32_t* src = (const uint32_t*)pa.desc.levelInfo;
-        for (uint32_t i = threadIdx.x; i < L * (uint32_t)(sizeof(CvPermutoLevelInfo) / 4); i += blockDim.x) ((uint32_t*)levels)[i] = src[i];
+        if (threadIdx.x < pa.desc.maxLevels) levels[threadIdx.x] = latticeLevel<D>(pa.desc.levelInfo[threadIdx.x]);
         if constexpr (LDS_TABLE) {
             const Entry* t = (const Entry*)pa.table;
             Entry* dst = (Entry*)(lds + pa.tableDword);
@@ -86,22 +85,27 @@ __global__ __launch_bounds__(1024) void permutoMlpKernel(const PermutoMlpArgs pa
 #pragma unroll
             for (int d = 0; d < FD; ++d) act[kt][d] = 0u;
         // element q of the lane's share is feature (q % F) of level g * perLane + q / F; shares are whole entries
+        auto encode = [&](auto simplex) {
+            typedef decltype(simplex) Simplex;
 #pragma unroll
-        for (int e = 0; e < KT * EPL / F; ++e) {
-            if ((uint32_t)e < perLane) {                                       // uniform over the wave
-                const uint32_t level = (uint32_t)g * perLane + (uint32_t)e;
-                Entry v;
+            for (int e = 0; e < KT * EPL / F; ++e) {
+                if ((uint32_t)e < perLane) {                                       // uniform over the wave
+                    const uint32_t level = (uint32_t)g * perLane + (uint32_t)e;
+                    Entry v;
 #pragma unroll
-                for (int f = 0; f < F; ++f) v[f] = (half_t)0.f;
-                if (level < pa.desc.maxLevels) v = permutoEncodeEntry<half_t, D, F, PLAIN>(pos, levels[level], table, pa.desc.maxLevel);
+                    for (int f = 0; f < F; ++f) v[f] = (half_t)0.f;
+                    if (level < pa.desc.maxLevels) v = permutoEncodeEntry<half_t, D, F, PLAIN, Simplex>(pos, levels[level], table, pa.desc.maxLevel);
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    const int q = e * F + f;
-                    const uint32_t bits = (uint32_t)__builtin_bit_cast(uint16_t, (half_t)v[f]);
-                    act[q / EPL][(q % EPL) / 2] |= bits << (16 * (q & 1));
+                    for (int f = 0; f < F; ++f) {
+                        const int q = e * F + f;
+                        const uint32_t bits = (uint32_t)__builtin_bit_cast(uint16_t, (half_t)v[f]);
+                        act[q / EPL][(q % EPL) / 2] |= bits << (16 * (q & 1));
+                    }
                 }
             }
-        }
+        };
+        if (!PLAIN || anyBeyondReach<D>(pos, pa.reach)) encode(LatticeSimplexAny<D>());
+        else if constexpr (PLAIN) encode(LatticeSimplex<D>());
         genericRunLayers<Mma, MAXT, false>(ga, lds, lane, sample, act);      // plain, ReLU and leaky ReLU layers
     }
 }
@@ -170,6 +174,7 @@ hipError_t launchPermutoMlp(hipStream_t stream, const CvPermutoDesc& desc, const
     const uint32_t netDwords = planGeneric<F16Mma>(mlp, pa.net, kLdsLimitDwords - kLevelDwords - 4u, &widest);
     if (!netDwords) return hipErrorInvalidValue;
     pa.desc = desc;
+    pa.reach = latticeReach(desc);
     pa.pos = (const uint8_t*)positions; pa.posStride = positionStride; pa.table = (const uint8_t*)featureTable;
     uint64_t tableElems = 0;
     for (uint32_t l = 0; l < desc.maxLevels; ++l) {

@@ -8,7 +8,7 @@ hipError_t launchPermutoWide16In16(hipStream_t stream, const CvPermutoDesc& desc
 {
     PermutoWideArgs pa;
     pa.mlp = mlp; pa.desc = desc; pa.pos = (const uint8_t*)positions; pa.posStride = positionStride;
-    pa.table = (const uint8_t*)featureTable; pa.tableElems = tableElems;
+    pa.table = (const uint8_t*)featureTable; pa.tableElems = tableElems; pa.reach = latticeReach(desc);
     return launchPermutoWide16K<16>(stream, pa, numCUs, H, NH);
 }
 

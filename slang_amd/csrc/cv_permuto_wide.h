@@ -16,14 +16,14 @@ namespace cv {
 namespace {
 
 // PLAIN (permutoPlainLevels): no branch inside a level.  3-d, 8 levels of 2^12 two-feature entries, 16-64-64-3, 2^22
-// positions: 241 -> 224 us; smaller decoders 1.13 to 1.24 times as fast.
+// positions: 241 -> 224 us, smaller decoders 1.13 to 1.24 times as fast; 169 us with the simplex by exchanges (LatticeSimplex).
 template <int K0, int D, int F, bool PLAIN>
 struct Wide16PermutoFront {
     struct Input { half_t pos[2][D]; };
     const uint8_t* pos; uint64_t posStride;
-    const CvPermutoLevelInfo* levels;      // in LDS
+    const LatticeLevel<D>* levels;         // in LDS
     const half_t* table;                   // in LDS
-    float maxLevel;
+    float maxLevel, reach;
     __device__ __forceinline__ Input load(uint32_t p, int n, int, uint32_t lastSample) const
     {
         Input x;
@@ -39,6 +39,20 @@ struct Wide16PermutoFront {
     template <int NS>
     __device__ __forceinline__ void operands(const Input& x, uint32_t (&B)[2][NS][4], int, int h) const
     {
+        if constexpr (PLAIN) {
+            float p[2 * D];
+#pragma unroll
+            for (int d = 0; d < 2 * D; ++d) p[d] = (float)x.pos[d / D][d % D];
+            if (!anyBeyondReach<2 * D>(p, reach)) {
+                encode<NS, LatticeSimplex<D>>(x, B, h);
+                return;
+            }
+        }
+        encode<NS, LatticeSimplexAny<D>>(x, B, h);
+    }
+    template <int NS, typename Simplex>
+    __device__ __forceinline__ void encode(const Input& x, uint32_t (&B)[2][NS][4], int h) const
+    {
         constexpr int S0 = K0 == 8 ? 1 : 2, CE = K0 == 32 ? 8 : 4, PER = CE / F;      // k-steps; features and levels per chunk
         static_assert(CE % F == 0, "a lane's chunk holds whole table entries");
 #pragma unroll
@@ -52,7 +66,7 @@ struct Wide16PermutoFront {
 #pragma unroll
                 for (int c = 0; c < PER; ++c) {
                     const int level = (2 * s + h) * PER + c;
-                    const auto e = permutoEncodeEntry<half_t, D, F, PLAIN>(p, levels[level], table, maxLevel);
+                    const auto e = permutoEncodeEntry<half_t, D, F, PLAIN, Simplex>(p, levels[level], table, maxLevel);
 #pragma unroll
                     for (int f = 0; f < F; ++f) {
                         const int q = c * F + f;
@@ -77,6 +91,7 @@ struct PermutoWideArgs {
     const uint8_t* pos; uint64_t posStride;
     const uint8_t* table;
     uint32_t tableElems;
+    float reach;      // latticeReach
 };
 
 constexpr uint32_t kWideLevelBytes = CV_PERMUTO_MAX_LEVELS * sizeof(CvPermutoLevelInfo);
@@ -87,14 +102,13 @@ __global__ __launch_bounds__(64 * WAVES) void permutoWide16Kernel(const PermutoW
     typedef typename PermutoEntry<half_t, F>::type Entry;
     extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
     {
-        const uint32_t* src = (const uint32_t*)pa.desc.levelInfo;
-        for (uint32_t i = threadIdx.x; i < pa.desc.maxLevels * (uint32_t)(sizeof(CvPermutoLevelInfo) / 4); i += blockDim.x) ((uint32_t*)dyn)[i] = src[i];
+        if (threadIdx.x < pa.desc.maxLevels) ((LatticeLevel<D>*)dyn)[threadIdx.x] = latticeLevel<D>(pa.desc.levelInfo[threadIdx.x]);
         const Entry* t = (const Entry*)pa.table;
         Entry* dst = (Entry*)(dyn + kWideLevelBytes);
         for (uint32_t i = threadIdx.x; i < pa.tableElems / (uint32_t)F; i += blockDim.x) dst[i] = t[i];
     }
     // (the body synchronises the workgroup after it has staged the weights, before any wave encodes)
-    const Wide16PermutoFront<K0, D, F, PLAIN> front{pa.pos, pa.posStride, (const CvPermutoLevelInfo*)dyn, (const half_t*)(dyn + kWideLevelBytes), pa.desc.maxLevel};
+    const Wide16PermutoFront<K0, D, F, PLAIN> front{pa.pos, pa.posStride, (const LatticeLevel<D>*)dyn, (const half_t*)(dyn + kWideLevelBytes), pa.desc.maxLevel, pa.reach};
     mlpWide16Body<H, NH, K0, WAVES, true>(pa.mlp, front);
 }
 
