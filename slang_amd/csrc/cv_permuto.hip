@@ -343,9 +343,14 @@ static_assert(sizeof(PermutoArgs) + sizeof(TableParts) <= 4096, "kernel argument
 // at random addresses gfx950 serves a ds_add_f64 in 8.6 ns per wave and compute unit and a ds_add_f32 in 80 (16 waves), so the
 // wider sum is also the cheaper one.  Lanes that meet on one address are served one after the other: 24 ns per LDS instruction
 // in that case, 41 ns on the few entries of four coarse levels in two dimensions (2^22 positions: 256 us).
-// POS (one part that is the whole table): the position gradient in the same pass.  SLICED: some part is a slice of a level.
-template <int D, int FT, bool POS, bool SLICED, bool PLAIN>
-__global__ __launch_bounds__(1024) void permutoTableGradKernel(const PermutoArgs a, const TableParts parts)
+// POS: kPosInPass (one part that is the whole table), the position gradient in the same pass; kPosBeside (several parts), in
+// passes of its own over all levels, whose units of 64 positions are dealt to the waves of all workgroups.  The two kinds of work
+// wait for different things, additions in LDS and entries gathered from memory (64 lines each), so they go side by side: a
+// workgroup's first waves take its units of positions and the others that much more of the table's (2^18 positions in 3
+// dimensions, 8 levels of 2^12 two-feature entries: 40 us; 54.5 with the positions as a kernel of their own behind this one).  SLICED: some part is a slice of a level.
+constexpr int kPosNone = 0, kPosInPass = 1, kPosBeside = 2;
+template <int D, int FT, int POS, bool SLICED, bool PLAIN>
+__global__ __launch_bounds__(1024, D <= 4 && FT > 0 ? 8 : 4) void permutoTableGradKernel(const PermutoArgs a, const TableParts parts)
 {
     extern __shared__ double ldsTable[];
     // workgroup w: part w / groups, so that the workgroups of all parts that read the same positions (w % groups) sit on one
@@ -356,8 +361,29 @@ __global__ __launch_bounds__(1024) void permutoTableGradKernel(const PermutoArgs
     for (uint32_t i = threadIdx.x; i < part.elems; i += 1024u) ldsTable[i] = 0.0;
     __syncthreads();
     const TableInLds<FT, SLICED> sink{ldsTable, part.base, part.elems, entries, F};
-    for (uint64_t s = (uint64_t)w * 1024u + threadIdx.x; s < a.batch; s += (uint64_t)parts.groups * 1024u)
-        permutoBackwardOne<D, FT, POS, PLAIN>(a, (uint32_t)s, part.first, part.end, sink);
+    if constexpr (POS != kPosBeside) {
+        for (uint64_t s = (uint64_t)w * 1024u + threadIdx.x; s < a.batch; s += (uint64_t)parts.groups * 1024u)
+            permutoBackwardOne<D, FT, POS == kPosInPass, PLAIN>(a, (uint32_t)s, part.first, part.end, sink);
+    } else {
+        const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
+        const uint32_t units = (a.batch - 1u) / 64u + 1u;
+        for (uint64_t u = (uint64_t)wave * gridDim.x + blockIdx.x; u < units; u += 16ull * gridDim.x) {
+            const uint64_t s = u * 64u + lane;
+            if (s < a.batch) permutoBackwardOne<D, FT, true, PLAIN>(a, (uint32_t)s, 0u, a.desc.maxLevels, NoTable{});
+        }
+        // of this workgroup's units of positions (one by one to the waves) the first `more` waves have one more than the others,
+        // which for that take `worth` units of the table ahead of everyone's turns
+        const uint32_t own = blockIdx.x < units ? (units - 1u - blockIdx.x) / gridDim.x + 1u : 0u;
+        const uint32_t more = own % 16u, worth = more ? a.desc.maxLevels / (part.end - part.first) : 0u;
+        const uint32_t ahead = (16u - more) * worth;
+        const uint32_t turns = wave >= more ? worth : 0u;
+        for (uint32_t i = 0;; ++i) {
+            const uint64_t t = i < turns ? (wave - more) + (uint64_t)i * (16u - more) : ahead + wave + 16ull * (i - turns);
+            const uint64_t u = t * parts.groups + w, s = u * 64u + lane;
+            if (u >= units) break;           // (t grows with i)
+            if (s < a.batch) permutoBackwardOne<D, FT, false, PLAIN>(a, (uint32_t)s, part.first, part.end, sink);
+        }
+    }
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < part.elems; i += 1024u) {
         const uint32_t e = i / F, f = i - e * F;
@@ -440,7 +466,7 @@ hipError_t launchEncode(hipStream_t stream, const PermutoArgs& a)
     return hipGetLastError();
 }
 
-template <int D, int FT, bool POS, bool SLICED, bool PLAIN>
+template <int D, int FT, int POS, bool SLICED, bool PLAIN>
 hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, TableParts& t, int cus)
 {
     uint32_t most = 0;
@@ -466,7 +492,7 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     const bool cut = a.dTable && cutTable(a.desc, t);
     if (cut && t.count == 1 && a.dPos) {
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
-        return launchTableGrad<D, FT, true, false, PLAIN>(stream, a, t, cus);
+        return launchTableGrad<D, FT, kPosInPass, false, PLAIN>(stream, a, t, cus);
     }
     // Two launches against one: a handful of positions whose few additions hardly meet is done sooner by the one kernel that adds
     // in memory.  It takes 7.4 to 8.1 us per call back to back and the pair 11.5 to 13.5 (16 positions on 3 levels of 2^10
@@ -476,8 +502,14 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     const uint64_t features = (uint64_t)a.desc.featureDimensionPerEntry * a.desc.maxLevels;
     const bool few = FT > 0 && a.batch <= 64u && features <= 16u && a.batch * (uint64_t)(D + 1) * features <= 1440u;
     if (cut && !(a.dPos && few)) {
+        // One launch where the table's workgroups fill the chip; with fewer of them the positions, spread over all compute units by
+        // a kernel of their own, are done sooner than by the few.
+        if (a.dPos && (uint64_t)t.count * ((a.batch - 1u) / 1024u + 1u) >= (uint64_t)cus) {
+            noteKernel(false, "permutoTableGradKernel<D=%d,%u parts,positions beside>", D, t.count);
+            return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t, cus);
+        }
         noteKernel(false, "permutoTableGradKernel<D=%d,%u parts>", D, t.count);
-        const hipError_t e = t.sliced ? launchTableGrad<D, FT, false, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, false, false, PLAIN>(stream, a, t, cus);
+        const hipError_t e = t.sliced ? launchTableGrad<D, FT, kPosNone, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosNone, false, PLAIN>(stream, a, t, cus);
         if (e != hipSuccess || !a.dPos) return e;
         noteKernel(true, "permutoBackwardKernel<D=%d,positions>", D);
         hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false, PLAIN>), grid, block, 0, stream, a);

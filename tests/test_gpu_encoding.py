@@ -258,6 +258,44 @@ def test_permuto_backward_of_other_tables(F, tables, B, kernel):
     assert np.linalg.norm(d_pos.cpu().numpy() - r_pos) <= 1e-4 * np.linalg.norm(r_pos)
 
 
+@pytest.mark.parametrize("D,F,tables,B,parts", [
+    (3, 2, [(4096 * l, 4096) for l in range(8)], 31745, 8),      # the fewest positions whose table workgroups fill 256 compute units
+    (3, 2, [(4096 * l, 4096) for l in range(8)], 70001, 8),      # a last unit of 49 positions
+    (2, 1, [(4096 * l, 4096) for l in range(5)], 131073, 3),     # two levels to a part, then one
+    (4, 4, [(4096 * l, 4096) for l in range(2)], 131013, 2),     # the LDS of a compute unit to a part
+    (2, 3, [(0, 8192), (8192, 8192)], 66000, 4),                 # slices
+    (3, 2, [(0, 5000), (5000, 4096), (9096, 777)], 140000, 2),   # tables that are not 2^n entries
+    (5, 2, [(4096 * l, 4096) for l in range(4)], 65536, 4),
+    (2, 5, [(2048 * l, 2048) for l in range(4)], 65000, 4),
+])
+def test_permuto_backward_positions_beside_the_table(D, F, tables, B, parts):
+    # One launch for both gradients where the batch fills the chip: the position gradients are those of batches that do not, bit
+    # for bit, the table's the sum of theirs (in another order: bound as in test_permuto_backward_table_parts).
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the batches are those of 256 compute units")
+    rng = np.random.default_rng(D * 100 + F * 10 + len(tables))
+    n = len(tables)
+    enc = cv.PermutoEncoder(D, F, 12, n, baseScale=4.0, log2PerLevelScale=0.5, maxLevelRatio=1.0, seed=11)
+    for l, (offset, size) in enumerate(tables):
+        enc.desc.levelInfo[l].offsetOfFeatureTable, enc.desc.levelInfo[l].featureTableSize = offset, size
+    pos = rng.uniform(-1, 1, (B, D)).astype(np.float32)
+    pos[rng.integers(0, B, 20)] *= 3e6                            # beyond LatticeSimplex's reach
+    pos, g = to_dev(pos), to_dev(rng.standard_normal((B, n * F)).astype(np.float32))
+    table = to_dev(rng.standard_normal(max(o + s for o, s in tables) * F).astype(np.float32))
+    d_table = torch.zeros_like(table)
+    d_pos, _ = enc.backward(pos, table, g, dFeatureTable=d_table)
+    assert cv.lastKernelName() == "permutoTableGradKernel<D=%d,%d parts,positions beside>" % (D, parts)
+    want_table, want_pos = torch.zeros(table.numel(), dtype=torch.float64, device=DEV), []
+    for i in range(0, B, 16384):
+        part = torch.zeros_like(table)
+        d, _ = enc.backward(pos[i:i + 16384], table, g[i:i + 16384], dFeatureTable=part)
+        assert "beside" not in cv.lastKernelName()
+        want_pos.append(d)
+        want_table += part
+    assert torch.equal(d_pos, torch.cat(want_pos))
+    assert torch.linalg.norm(d_table - want_table) <= 2.0 ** -16 * torch.linalg.norm(want_table)
+
+
 @pytest.mark.parametrize("D,F,levels_n,log2,B,in_memory", [
     (2, 4, 3, 10, 1, True), (2, 4, 3, 10, 40, True), (2, 4, 3, 10, 41, False),       # 36 additions to a position
     (3, 2, 8, 12, 22, True), (3, 2, 8, 12, 23, False), (1, 1, 4, 15, 64, True), (1, 1, 4, 15, 65, False),
