@@ -109,26 +109,119 @@ struct Bf16Mma {
     }
 };
 
-// fp32 operands on v_mfma_f32_16x16x4_f32.  A fragment keeps the 8 k-slots per lane of the 16-bit
-// flavours (so the InferencingOptimal form of an fp32 matrix is the same arrangement with 4-byte
-// elements): eight instructions, the s-th multiplying slot s of every lane, i.e. the four k
-// values {g*GS + 8*kt + s : g = 0..3}.
+// fp32 operands on the bfloat16 matrix pipeline: every operand is the sum of three bfloat16 pieces (h the nearest to it, m the
+// nearest to the rest, l what is left: 24 bits, exactly), and of the nine products of pieces the six that matter are summed, the
+// h*h products by themselves (F32Sum::main, seeded with the bias) and the five small ones by themselves, added at the end.
+// Six v_mfma_f32_16x16x32_bf16 take 96 cycles of the matrix pipeline where eight v_mfma_f32_16x16x4_f32, which round every
+// product's sum to 24 bits, take 256, and the sums are closer to the exact ones (random operands, error over the norm against 64
+// bits, 32 / 64 / 128 terms: 3.9 / 5.0 / 6.5e-8 against 10.3 / 14.4 / 20.4e-8 on the fp32 instruction; the dropped products are
+// below 2^-26 of the largest term each).
+// A fragment has the 8 k-slots per lane of the 16-bit flavours, so the InferencingOptimal form of an fp32 matrix is the same
+// arrangement with 4-byte elements; decoded, four dwords each of h, m and l.
+// Infinities and values from 2^127 on: split() makes NaN of them (inf - inf), so a wave that holds one (beyond()) takes
+// splitAny(), which leaves m and l of an infinity zero; then main alone has the sum's infinity or NaN, and finish() keeps it.
+struct F32Sum { floatx4 main, small; };
 struct F32Mma {
     static constexpr const char* kName = "f32";
-    static constexpr int kEsz = 4, kEpl = 8, kRawDW = 8, kFD = 8;
+    static constexpr int kEsz = 4, kEpl = 8, kRawDW = 8, kFD = 12;
     static constexpr bool kIsFloat = true;
     typedef floatx4 Acc;
+    typedef __bf16 Pair __attribute__((ext_vector_type(2)));
+    typedef __bf16 Eight __attribute__((ext_vector_type(8)));
+    static __device__ __forceinline__ float low(uint32_t pair) { return __builtin_bit_cast(float, pair << 16); }
+    static __device__ __forceinline__ float high(uint32_t pair) { return __builtin_bit_cast(float, pair & 0xffff0000u); }
+    static __device__ __forceinline__ uint32_t pack(float a, float b)
+    {
+        const Pair p = {(__bf16)a, (__bf16)b};
+        return __builtin_bit_cast(uint32_t, p);
+    }
+    static __device__ __forceinline__ void split(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l)
+    {
+        // (11 instructions for two values; pinned, since the compiler would convert each value again to subtract it)
+        h = pack(a, b);
+        asm("" : "+v"(h));
+        const float ra = a - low(h), rb = b - high(h);
+        m = pack(ra, rb);
+        asm("" : "+v"(m));
+        l = pack(ra - low(m), rb - high(m));
+    }
+    static __device__ __forceinline__ void splitAny(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l)
+    {
+        // (the nearest bfloat16 of a large finite value may be an infinity: the one towards zero is not)
+        auto first = [](float x) { return __builtin_fabsf(x) >= 0x1p127f ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u) : x; };
+        h = pack(first(a), first(b));
+        const float ra = __builtin_isfinite(a) ? a - low(h) : 0.f, rb = __builtin_isfinite(b) ? b - high(h) : 0.f;
+        m = pack(ra, rb);
+        l = pack(ra - low(m), rb - high(m));
+    }
+    template <bool ANY = false>
     static __device__ __forceinline__ void decode(const uint32_t* raw, uint32_t* frag)
     {
 #pragma unroll
-        for (int d = 0; d < 8; ++d) frag[d] = raw[d];
+        for (int d = 0; d < 4; ++d) {
+            float a = __builtin_bit_cast(float, raw[2 * d]), b = __builtin_bit_cast(float, raw[2 * d + 1]);
+            if constexpr (ANY) {
+                // (stays in its branch: the compiler would rather compute it on every path)
+                asm volatile("" : "+v"(a), "+v"(b));
+                splitAny(a, b, frag[d], frag[4 + d], frag[8 + d]);
+            } else {
+                split(a, b, frag[d], frag[4 + d], frag[8 + d]);
+            }
+        }
     }
-    static __device__ __forceinline__ Acc mma(const uint32_t* a, const uint32_t* b, Acc c)
+    // the largest magnitude of n (an even number of) values and `most` (NaN does not count: its pieces need no care).  One
+    // instruction for two values; of fmaxf the compiler makes two for each.  (As relu.)
+    static __device__ __forceinline__ float largest(const uint32_t* raw, int n, float most)
     {
 #pragma unroll
-        for (int s = 0; s < 8; ++s)
-            c = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s]), __builtin_bit_cast(float, b[s]), c, 0, 0, 0);
+        for (int d = 0; d < n; d += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(raw[d]), "v"(raw[d + 1]));
+        return most;
+    }
+    // x > 0 ? x : 0 (NaN: 0) in one instruction.  Not for results of matrix instructions: the compiler does not see that it reads them.
+    static __device__ __forceinline__ float relu(float x)
+    {
+        float r;
+        asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(x));
+        return r;
+    }
+    static __device__ __forceinline__ bool beyond(float largest) { return __any(largest >= 0x1p127f); }
+    // the p-th product of pieces (0..4 small ones, 5: h*h)
+    template <int P>
+    static __device__ __forceinline__ void product(const uint32_t* a, const uint32_t* b, F32Sum& c)
+    {
+        constexpr int kA[6] = {4, 8, 0, 4, 0, 0}, kB[6] = {4, 0, 8, 0, 4, 0};
+        const u32x4 av = {a[kA[P]], a[kA[P] + 1], a[kA[P] + 2], a[kA[P] + 3]}, bv = {b[kB[P]], b[kB[P] + 1], b[kB[P] + 2], b[kB[P] + 3]};
+        floatx4& sum = P < 5 ? c.small : c.main;
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(Eight, av), __builtin_bit_cast(Eight, bv), sum, 0, 0, 0);
+    }
+    static __device__ __forceinline__ F32Sum mma(const uint32_t* a, const uint32_t* b, F32Sum c)
+    {
+        product<0>(a, b, c); product<1>(a, b, c); product<2>(a, b, c); product<3>(a, b, c); product<4>(a, b, c); product<5>(a, b, c);
         return c;
+    }
+};
+
+// The sums of a flavour on their way: its accumulators, or F32Sum.
+template <class Mma, bool F32 = Mma::kEsz == 4>
+struct SumOf {
+    typedef typename Mma::Acc T;
+    static __device__ __forceinline__ T start(typename Mma::Acc seed) { return seed; }
+    static __device__ __forceinline__ typename Mma::Acc finish(T s) { return s; }
+    static __device__ __forceinline__ typename Mma::Acc finishAny(T s) { return s; }
+};
+template <class Mma>
+struct SumOf<Mma, true> {
+    typedef F32Sum T;
+    static __device__ __forceinline__ T start(floatx4 seed) { return F32Sum{seed, floatx4{0.f, 0.f, 0.f, 0.f}}; }
+    static __device__ __forceinline__ floatx4 finish(T s) { return s.main + s.small; }
+    // ... where some operand was beyond(): an infinity or NaN of the sum stands in `main` alone
+    static __device__ __forceinline__ floatx4 finishAny(T s)
+    {
+        asm volatile("" : "+v"(s.main));      // (as in decode)
+        floatx4 r = s.main + s.small;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = __builtin_isfinite(s.main[i]) ? r[i] : s.main[i];
+        return r;
     }
 };
 

@@ -292,7 +292,9 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
     constexpr int OUT_DW = ROWS * (int)sizeof(OutT) / 4;
     typedef typename Fl::Acc Acc;
 
-    __shared__ __attribute__((aligned(16))) uint32_t ldsW[MT * KT * 64 * RAW];
+    constexpr bool F32 = Fl::kEsz == 4;       // fragments as F32Mma's pieces
+    constexpr int LANE_DW = F32 ? FD : RAW;
+    __shared__ __attribute__((aligned(16))) uint32_t ldsW[MT * KT * 64 * LANE_DW];
     // Output rows of 128 bytes or more leave through a per-wave LDS transpose so that every
     // store instruction writes whole 128-byte lines (lane l -> 16 consecutive bytes of the
     // tile's output block) instead of 16-byte pieces of many lines.  Rows are padded by 16
@@ -369,16 +371,29 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
     uint32_t bufA[NT][SLOT_DW], bufB[NT][SLOT_DW];
     if (haveTile) loadTile(bufA, tile);
 
-    stageFragments<ESZ, EPL>(ldsW, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k,
-                             a.rowOff, (Fl::kAnySign && a.matUnsigned) ? 0x80u : 0u);
-    __syncthreads();
+    bool matBeyond = false;                   // F32Mma::beyond of the matrix
+    if constexpr (F32) {
+        const float most = stageFragmentPieces(ldsW, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff, 0.f);
+        matBeyond = __syncthreads_or(most >= 0x1p127f);
+    } else {
+        stageFragments<ESZ, EPL>(ldsW, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k,
+                                 a.rowOff, (Fl::kAnySign && a.matUnsigned) ? 0x80u : 0u);
+        __syncthreads();
+    }
 
     uint32_t afrag[MT][KT][FD];
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-            Fl::decode(&ldsW[((t * KT + kt) * 64 + lane) * RAW], afrag[t][kt]);
+        for (int kt = 0; kt < KT; ++kt) {
+            const uint32_t* raw = &ldsW[((t * KT + kt) * 64 + lane) * LANE_DW];
+            if constexpr (F32) {
+#pragma unroll
+                for (int d = 0; d < FD; ++d) afrag[t][kt][d] = raw[d];
+            } else {
+                Fl::decode(raw, afrag[t][kt]);
+            }
+        }
 
     if constexpr (Fl::kAnySign) {
         if (a.inUnsigned) {
@@ -412,9 +427,11 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
                 }
             }
             const uint32_t (&buf)[SLOT_DW] = slot;
-            Acc acc[MT];
+            bool any = false;
+            if constexpr (F32) any = matBeyond | Fl::beyond(Fl::largest(buf, SLOT_DW, 0.f));
+            typename SumOf<Fl>::T sum[MT];
 #pragma unroll
-            for (int t = 0; t < MT; ++t) acc[t] = lo.bias[t];
+            for (int t = 0; t < MT; ++t) sum[t] = SumOf<Fl>::start(lo.bias[t]);
             int xSum = 0;       // unsigned matrix: sum of this lane's signed input bytes
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt) {
@@ -428,11 +445,23 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
                         if (a.matUnsigned) xSum += sumSignedBytes(x[d]);
                     }
                     Fl::decodeIn(x, bfrag);
+                } else if constexpr (F32) {
+                    Fl::decode(&buf[kt * IRAW], bfrag);
+                    if (any) Fl::template decode<true>(&buf[kt * IRAW], bfrag);
                 } else {
                     Fl::decodeIn(&buf[kt * IRAW], bfrag);
                 }
 #pragma unroll
-                for (int t = 0; t < MT; ++t) acc[t] = Fl::mma(afrag[t][kt], bfrag, acc[t]);
+                for (int t = 0; t < MT; ++t) sum[t] = Fl::mma(afrag[t][kt], bfrag, sum[t]);
+            }
+            Acc acc[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finish(sum[t]);
+            if constexpr (F32) {
+                if (any) {
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finishAny(sum[t]);
+                }
             }
             if constexpr (Fl::kAnySign) {
                 if (a.matUnsigned) {
@@ -518,19 +547,48 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
 constexpr int kLargeKC = 4;
 constexpr int kLargeLdsBytes = 128 * 1024;
 
-template <class Fl, int MT, typename OutT>
-__global__ __launch_bounds__(256) void matmulLargeKernel(const MatMulArgs a, const int KT)
+// fp32: fragments as F32Mma's pieces (PIECES), or, where they would not fit (k beyond 1600), as they are in memory and split at
+// every use; twelve waves share the block of the matrix, and the bias, which four waves keep in registers, lies in LDS.  128x128 over
+// 2^18 samples: 107 us on v_mfma_f32_16x16x4_f32 (four waves, blocks of 128 rows up to k = 256), 123 us splitting at every use, 80 us
+// here; 256x256 over 2^16: 154, 197, 113 us.
+template <class Fl>
+struct LargeShape {
+    static constexpr bool kF32 = Fl::kEsz == 4;
+    static constexpr int kWaves = kF32 ? 12 : 4, kSteps = kF32 ? 2 : kLargeKC;
+};
+constexpr int kLargePieceBytes = 158 * 1024;
+
+template <class Fl, int MT, typename OutT, bool PIECES>
+__global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel(const MatMulArgs a, const int KT)
 {
-    constexpr int EPL = Fl::kEpl, FD = Fl::kFD, ESZ = Fl::kEsz, RAW = Fl::kRawDW;
+    constexpr int EPL = Fl::kEpl, FD = Fl::kFD, ESZ = Fl::kEsz, RAW = Fl::kRawDW, LANE_DW = PIECES ? FD : RAW;
     constexpr int IESZ = Fl::kInEsz, IRAW = Fl::kInRawDW;
-    constexpr int KC = kLargeKC, STEP_DW = KC * IRAW, ROWS = 4 * MT;
+    constexpr int WAVES = LargeShape<Fl>::kWaves;
+    constexpr int KC = LargeShape<Fl>::kSteps, STEP_DW = KC * IRAW, ROWS = 4 * MT;
+    constexpr bool F32 = LargeShape<Fl>::kF32;
     typedef typename Fl::Acc Acc;
     extern __shared__ __attribute__((aligned(16))) uint32_t ldsDyn[];
+    __shared__ __attribute__((aligned(16))) float ldsBias[F32 ? 16 * MT : 1];
 
     const uint32_t gs = optGS((uint32_t)a.k);
-    stageFragments<ESZ, EPL>(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k,
-                             a.rowOff, (Fl::kAnySign && a.matUnsigned) ? 0x80u : 0u);
-    __syncthreads();
+    bool matBeyond = false;                    // F32Mma::beyond of the matrix
+    if constexpr (F32) {
+        float most = 0.f;
+        if constexpr (PIECES) {
+            most = stageFragmentPieces(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff, most);
+        } else {
+            stageFragments<ESZ, EPL>(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff);
+            __syncthreads();
+            for (int i = threadIdx.x; i < MT * KT * 64; i += 64 * WAVES) most = Fl::largest(ldsDyn + (size_t)i * RAW, RAW, most);
+        }
+        for (int row = threadIdx.x; row < 16 * MT; row += 64 * WAVES)
+            ldsBias[row] = (a.bias && row < a.m) ? loadAsFloat(a.bias + (size_t)row * elemSize(a.biasCt), a.biasCt) : 0.f;
+        matBeyond = __syncthreads_or(most >= 0x1p127f);
+    } else {
+        stageFragments<ESZ, EPL>(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k,
+                                 a.rowOff, (Fl::kAnySign && a.matUnsigned) ? 0x80u : 0u);
+        __syncthreads();
+    }
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, n = lane & 15;
@@ -539,7 +597,8 @@ __global__ __launch_bounds__(256) void matmulLargeKernel(const MatMulArgs a, con
     const int validBytes = min((int)gs, max(a.k - colBase, 0)) * IESZ;
 
     LaneOut<Fl, MT> lo;
-    loadBias<Fl, MT>(lo, a, rowBase);
+    if constexpr (F32) lo.validRows = min(max(a.m - rowBase, 0), ROWS);
+    else loadBias<Fl, MT>(lo, a, rowBase);
     if constexpr (Fl::kAnySign) {
         if (a.inUnsigned) {
             int rowSum[MT];
@@ -556,14 +615,18 @@ __global__ __launch_bounds__(256) void matmulLargeKernel(const MatMulArgs a, con
 
     const uint8_t* inLane = a.in + (size_t)colBase * IESZ;
     uint8_t* outLane = a.out + (size_t)rowBase * sizeof(OutT);
-    const uint32_t numTiles = (a.batch + 15) / 16;
-    for (uint32_t tile = blockIdx.x * 4 + wave; tile < numTiles; tile += gridDim.x * 4) {
-        const uint32_t sample = tile * 16 + n;
-        const uint8_t* p = inLane + (size_t)min(sample, a.batch - 1) * a.inStride;
-        Acc acc[MT];
+    const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + 15) / 16);
+    for (uint64_t tile = blockIdx.x * WAVES + wave; tile < numTiles; tile += (uint64_t)gridDim.x * WAVES) {
+        const uint64_t sample = tile * 16 + n;
+        const uint8_t* p = inLane + (size_t)(sample < a.batch ? sample : a.batch - 1) * a.inStride;
+        typename SumOf<Fl>::T sum[MT];
 #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[t] = lo.bias[t];
+        for (int t = 0; t < MT; ++t) {
+            if constexpr (F32) sum[t] = SumOf<Fl>::start(*(const floatx4*)(ldsBias + rowBase + 4 * t));
+            else sum[t] = SumOf<Fl>::start(lo.bias[t]);
+        }
         int xSum = 0;
+        bool any = matBeyond;
         for (int kc = 0; kc < KT; kc += KC) {
             const int off = kc * IRAW * 4;                         // byte offset of this step in the lane's slice
             const int vb = min(max(validBytes - off, 0), STEP_DW * 4);
@@ -577,16 +640,58 @@ __global__ __launch_bounds__(256) void matmulLargeKernel(const MatMulArgs a, con
                     if (a.matUnsigned) xSum += sumSignedBytes(x[d]);
                 }
             }
+            if constexpr (F32) any = any | Fl::beyond(Fl::largest(x, STEP_DW, 0.f));
 #pragma unroll
             for (int j = 0; j < KC; ++j) {
                 uint32_t bfrag[FD];
                 Fl::decodeIn(&x[j * IRAW], bfrag);
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    uint32_t af[FD];
-                    Fl::decode(&ldsDyn[((t * KT + kc + j) * 64 + lane) * RAW], af);
-                    acc[t] = Fl::mma(af, bfrag, acc[t]);
+                if constexpr (F32) {
+                    if (any) Fl::template decode<true>(&x[j * IRAW], bfrag);
                 }
+                // (fp32: two row tiles together, product by product, so that no matrix instruction waits for the one before it)
+                constexpr int G = F32 && MT > 1 ? 2 : 1;
+#pragma unroll
+                for (int t0 = 0; t0 < MT; t0 += G) {
+                    uint32_t af[G][FD];
+#pragma unroll
+                    for (int t = t0; t < t0 + G; ++t) {
+                        const uint32_t* raw = &ldsDyn[((t * KT + kc + j) * 64 + lane) * LANE_DW];
+                        if constexpr (PIECES) {
+#pragma unroll
+                            for (int d = 0; d < FD; ++d) af[t - t0][d] = raw[d];
+                        } else {
+                            Fl::decode(raw, af[t - t0]);
+                            if constexpr (F32) {
+                                if (matBeyond) Fl::template decode<true>(raw, af[t - t0]);
+                            }
+                        }
+                    }
+                    if constexpr (F32) {
+#pragma unroll
+                        for (int t = t0; t < t0 + G; ++t) Fl::template product<0>(af[t - t0], bfrag, sum[t]);
+#pragma unroll
+                        for (int t = t0; t < t0 + G; ++t) Fl::template product<1>(af[t - t0], bfrag, sum[t]);
+#pragma unroll
+                        for (int t = t0; t < t0 + G; ++t) Fl::template product<2>(af[t - t0], bfrag, sum[t]);
+#pragma unroll
+                        for (int t = t0; t < t0 + G; ++t) Fl::template product<3>(af[t - t0], bfrag, sum[t]);
+#pragma unroll
+                        for (int t = t0; t < t0 + G; ++t) Fl::template product<4>(af[t - t0], bfrag, sum[t]);
+#pragma unroll
+                        for (int t = t0; t < t0 + G; ++t) Fl::template product<5>(af[t - t0], bfrag, sum[t]);
+                    } else {
+                        sum[t0] = Fl::mma(af[0], bfrag, sum[t0]);
+                    }
+                }
+            }
+        }
+        Acc acc[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finish(sum[t]);
+        if constexpr (F32) {
+            if (any) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finishAny(sum[t]);
             }
         }
         if constexpr (Fl::kAnySign) {
@@ -671,35 +776,40 @@ hipError_t launchShape(hipStream_t stream, const MatMulArgs& a, int numCUs, bool
     }
 }
 
-template <class Fl, int MT, typename OutT>
+template <class Fl, int MT, typename OutT, bool PIECES>
 hipError_t launchLarge(hipStream_t stream, const MatMulArgs& a, int KT, int numCUs, bool append)
 {
-    const size_t ldsBytes = (size_t)MT * KT * 64 * Fl::kRawDW * 4;
-    const hipError_t ea = allowDynamicLds<matmulLargeKernel<Fl, MT, OutT>>(kLargeLdsBytes);
+    const size_t ldsBytes = (size_t)MT * KT * 64 * (PIECES ? Fl::kFD : Fl::kRawDW) * 4;
+    const hipError_t ea = allowDynamicLds<matmulLargeKernel<Fl, MT, OutT, PIECES>>(PIECES ? kLargePieceBytes : kLargeLdsBytes);
     if (ea != hipSuccess) return ea;
+    constexpr uint32_t kWaves = LargeShape<Fl>::kWaves;
     int perCU = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, matmulLargeKernel<Fl, MT, OutT>, 256, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
-    const uint32_t numTiles = (a.batch + 15) / 16, need = (numTiles + 3) / 4;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, matmulLargeKernel<Fl, MT, OutT, PIECES>, 64 * kWaves, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
+    const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + 15) / 16), need = (numTiles + kWaves - 1) / kWaves;
     const uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU;
     noteKernel(append, "matmulLargeKernel<%s,MT=%d,KT=%d,out=%dB>", Fl::kName, MT, KT, (int)sizeof(OutT));
-    hipLaunchKernelGGL((matmulLargeKernel<Fl, MT, OutT>), dim3(need < cap ? need : cap), dim3(256), ldsBytes, stream, a, KT);
+    hipLaunchKernelGGL((matmulLargeKernel<Fl, MT, OutT, PIECES>), dim3(need < cap ? need : cap), dim3(64 * kWaves), ldsBytes, stream, a, KT);
     return hipGetLastError();
 }
 
 // One block of at most 16*MTs rows at row a.rowOff (a.m = rows of the block; out and bias already
 // point at the block's first row).
 template <class Fl, typename OutT>
-hipError_t dispatchBlock(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append, int largeKT)
+hipError_t dispatchBlock(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append, int largeKT, bool largePieces)
 {
     const uint32_t mt = optMT((uint32_t)a.m), kt = optKT((uint32_t)a.k, Fl::kEpl);
     const int MTs = mt <= 1 ? 1 : mt <= 2 ? 2 : mt <= 4 ? 4 : mt <= 8 ? 8 : 0;
     if (!MTs) return hipErrorInvalidValue;
     if (largeKT) {
+        constexpr bool PIECES = LargeShape<Fl>::kF32;
+        if constexpr (PIECES) {
+            if (!largePieces) return launchLarge<Fl, 1, OutT, false>(stream, a, largeKT, numCUs, append);
+        }
         switch (MTs) {
-        case 1: return launchLarge<Fl, 1, OutT>(stream, a, largeKT, numCUs, append);
-        case 2: return launchLarge<Fl, 2, OutT>(stream, a, largeKT, numCUs, append);
-        case 4: return launchLarge<Fl, 4, OutT>(stream, a, largeKT, numCUs, append);
-        default: return launchLarge<Fl, 8, OutT>(stream, a, largeKT, numCUs, append);
+        case 1: return launchLarge<Fl, 1, OutT, PIECES>(stream, a, largeKT, numCUs, append);
+        case 2: return launchLarge<Fl, 2, OutT, PIECES>(stream, a, largeKT, numCUs, append);
+        case 4: return launchLarge<Fl, 4, OutT, PIECES>(stream, a, largeKT, numCUs, append);
+        default: return launchLarge<Fl, 8, OutT, PIECES>(stream, a, largeKT, numCUs, append);
         }
     }
     const int KTs = kt <= 1 ? 1 : kt <= 2 ? 2 : kt <= 4 ? 4 : 0;
@@ -725,13 +835,18 @@ hipError_t dispatchShape(hipStream_t stream, const MatMulArgs& a, int numCUs)
 {
     const uint32_t kt = optKT((uint32_t)a.k, Fl::kEpl);
     int blockTiles = 8, largeKT = 0;
+    bool largePieces = false;
     const bool inRegisters = Fl::kWideFragments ? (kt <= 2 && a.m <= 64) : kt <= 4;
     if (Fl::kWideFragments && inRegisters) blockTiles = 4;
     if (!inRegisters) {
-        largeKT = (int)((kt + kLargeKC - 1) / kLargeKC * kLargeKC);
-        const size_t tileBytes = (size_t)largeKT * 64 * Fl::kRawDW * 4;
-        while (blockTiles > 1 && blockTiles * tileBytes > (size_t)kLargeLdsBytes) blockTiles /= 2;
-        if (blockTiles * tileBytes > (size_t)kLargeLdsBytes) return hipErrorInvalidValue;
+        constexpr uint32_t kSteps = LargeShape<Fl>::kSteps;
+        largeKT = (int)((kt + kSteps - 1) / kSteps * kSteps);
+        const size_t pieceBytes = (size_t)largeKT * 64 * Fl::kFD * 4;
+        largePieces = LargeShape<Fl>::kF32 && pieceBytes <= (size_t)kLargePieceBytes;
+        const size_t tileBytes = largePieces ? pieceBytes : (size_t)largeKT * 64 * Fl::kRawDW * 4, most = largePieces ? kLargePieceBytes : kLargeLdsBytes;
+        if (LargeShape<Fl>::kF32 && !largePieces) blockTiles = 1;
+        while (blockTiles > 1 && blockTiles * tileBytes > most) blockTiles /= 2;
+        if (blockTiles * tileBytes > most) return hipErrorInvalidValue;
     }
     const int blockRows = 16 * blockTiles;
     const uint32_t biasEsz = a.bias ? elemSize(a.biasCt) : 0;
@@ -745,7 +860,7 @@ hipError_t dispatchShape(hipStream_t stream, const MatMulArgs& a, int numCUs)
         uint32_t al = a.outAlign;
         while (al > 1 && ((size_t)r0 * sizeof(OutT)) % al) al >>= 1;
         b.outAlign = al;
-        const hipError_t e = dispatchBlock<Fl, OutT>(stream, b, numCUs, r0 != 0, largeKT);
+        const hipError_t e = dispatchBlock<Fl, OutT>(stream, b, numCUs, r0 != 0, largeKT, largePieces);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

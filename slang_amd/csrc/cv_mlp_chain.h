@@ -3,8 +3,7 @@
 // rows and columns without smooth activations, element type fp16, e4m3, fp32 or bfloat16.  Values and rounding points
 // are those of mlpGenericKernel / mlpFloatKernel, bit for bit (same order of sums per accumulator).
 //
-// What bounds it: vector-ALU issue for 16- and 8-bit elements (conversion between layers), the fp32 matrix
-// instructions for T = float.  The run-time-size kernels spent most of their issue slots elsewhere: they computed tiles
+// What bounds it: vector-ALU issue (conversion between layers; for T = float the split into F32Mma's pieces).  The run-time-size kernels spent most of their issue slots elsewhere: they computed tiles
 // a layer does not have, formed an address and a mask for every input element of every tile, and waited for the inputs
 // of a tile after asking for them.  Here
 //   - a layer is a wave-uniform switch over its number of 16-row tiles MT; each arm is straight-line code for exactly
@@ -13,9 +12,10 @@
 //     are the same for every tile and are computed once, a slot beyond the vector has an offset outside the
 //     descriptor and a sample beyond the batch lies outside it, and both read as zero without a compare or a mask;
 //   - the loads of the next tiles are issued before the layers of the current ones;
-//   - NT = 2 tiles share every weight fragment read from LDS and give the matrix pipeline twice the independent chains.
-// Measured against the run-time-size kernels: fp32 32-64-64-8 over 2^22 samples 729 -> 522 us (115 TFLOP/s of padded
-// layers, 73 % of what v_mfma_f32_16x16x4_f32 issues at most), fp16 20-48-24-5 over 2 000 003 samples 78 -> 45 us.
+//   - NT = 2 tiles share every weight fragment read from LDS and give the matrix pipeline twice the independent chains
+//     (T = float: one, for the registers of the pieces).
+// Measured against the run-time-size kernels: fp16 20-48-24-5 over 2 000 003 samples 78 -> 45 us; T = float, 20-48-24-5 over 2^20
+// samples 91 us with v_mfma_f32_16x16x4_f32, 74 us with the pieces.  (Equal hidden layers: cv_mlp_equal_f32.h.)
 #pragma once
 #include <type_traits>
 
@@ -27,6 +27,8 @@ namespace {
 
 constexpr uint32_t kChainOutside = 0x80000000u;      // an offset no descriptor of a tile reaches
 
+constexpr uint32_t kChainPieceDwords = (160 * 1024 - 512) / 4;      // a compute unit's LDS, less what the kernel declares itself
+
 template <class Mma>
 constexpr int chainComponent()
 {
@@ -36,18 +38,21 @@ constexpr int chainComponent()
 template <int ACT>
 __device__ __forceinline__ float chainActivateF32(float x, float slope)
 {
-    if constexpr (ACT == kActRelu) return x > 0.f ? x : 0.f;
+    if constexpr (ACT == kActRelu) return F32Mma::relu(x);
     if constexpr (ACT == kActLeakyRelu) return fmaxf(x, x * slope);
     return x;
 }
 
 // One layer of MT row tiles for NT sample tiles: `act` holds its B operands and receives the next layer's, or, for the
 // last layer, the results are stored.
-template <class Mma, int MAXT, int MT, int NT>
+// PIECES (T = float): fragments lie in LDS as F32Mma's pieces; else as they lie in memory, split at every use.
+// matBeyond, any (T = float): F32Mma::beyond of some layer's matrix, and of it or the vectors in `act`.
+template <class Mma, int MAXT, int MT, int NT, bool PIECES>
 __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs& ly, const uint32_t* wbase, const float* bbase, int KT,
-                                           bool last, bool quads, int g, uint32_t sample, uint32_t (&act)[NT][MAXT / 2][Mma::kFD])
+                                           bool last, bool quads, int g, uint32_t sample, uint32_t (&act)[NT][MAXT / 2][Mma::kFD],
+                                           bool matBeyond, bool& any)
 {
-    constexpr int FD = Mma::kFD, RAW = Mma::kRawDW, MAXKT = MAXT / 2, OKT = (MT + 1) / 2;
+    constexpr int FD = Mma::kFD, RAW = PIECES ? FD : Mma::kRawDW, MAXKT = MAXT / 2, OKT = (MT + 1) / 2;
     constexpr bool F32 = std::is_same<Mma, F32Mma>::value, BF16 = std::is_same<Mma, Bf16Mma>::value;
     floatx4 acc[NT][MT];
 #pragma unroll
@@ -56,32 +61,59 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[nt][t] = b;
     }
+    if constexpr (F32) {
+        // Fragments of G row tiles together and product by product, so that no matrix instruction waits for the one before it.
+        // Operands beyond() are put right in branches that hardly ever run, so that the rest is straight-line code.
+        static_assert(NT == 1, "one tile: two leave a SIMD fewer than two waves for their registers");
+        constexpr int G = MT < 2 ? 1 : 2;
+#pragma unroll
+        for (int t0 = 0; t0 < MT; t0 += G) {
+            F32Sum sum[G];
+#pragma unroll
+            for (int t = t0; t < MT && t < t0 + G; ++t) sum[t - t0] = SumOf<Mma>::start(acc[0][t]);
+#pragma unroll
+            for (int kt = 0; kt < MAXKT; ++kt) {
+                if (kt == 0 || kt < KT) {
+                    uint32_t w[G][FD];
+#pragma unroll
+                    for (int t = t0; t < MT && t < t0 + G; ++t) {
+                        const uint32_t* raw = wbase + (size_t)(t * KT + kt) * 64 * RAW;
+                        if constexpr (PIECES) {
+#pragma unroll
+                            for (int d = 0; d < FD; ++d) w[t - t0][d] = raw[d];
+                        } else {
+                            Mma::decode(raw, w[t - t0]);
+                            if (matBeyond) Mma::template decode<true>(raw, w[t - t0]);
+                        }
+                    }
+                    staticFor<0, 6>([&](auto pc) {
+#pragma unroll
+                        for (int t = t0; t < MT && t < t0 + G; ++t) Mma::template product<decltype(pc)::value>(w[t - t0], act[0][kt], sum[t - t0]);
+                    });
+                }
+            }
+#pragma unroll
+            for (int t = t0; t < MT && t < t0 + G; ++t) acc[0][t] = SumOf<Mma>::finish(sum[t - t0]);
+            if (any) {
+#pragma unroll
+                for (int t = t0; t < MT && t < t0 + G; ++t) acc[0][t] = SumOf<Mma>::finishAny(sum[t - t0]);
+            }
+        }
+    } else
 #pragma unroll
     for (int kt = 0; kt < MAXKT; ++kt) {
         if (kt == 0 || kt < KT) {
-            // groups of row tiles whose fragments are read together: four sums side by side, so that none of fp32's eight
-            // matrix instructions per fragment waits for the one before it, and no more registers than that takes
-            constexpr int G = F32 && NT == 2 ? 2 : 4;
+            // groups of row tiles whose fragments are read together, and no more registers than that takes
+            constexpr int G = 4;
 #pragma unroll
             for (int t0 = 0; t0 < MT; t0 += G) {
                 uint32_t w[G][FD];
 #pragma unroll
                 for (int t = t0; t < MT && t < t0 + G; ++t) Mma::decode(wbase + (size_t)(t * KT + kt) * 64 * RAW, w[t - t0]);
-                if constexpr (F32) {
 #pragma unroll
-                    for (int s = 0; s < 8; ++s)
+                for (int t = t0; t < MT && t < t0 + G; ++t)
 #pragma unroll
-                        for (int t = t0; t < MT && t < t0 + G; ++t)
-#pragma unroll
-                            for (int nt = 0; nt < NT; ++nt)
-                                acc[nt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, w[t - t0][s]),
-                                                                                  __builtin_bit_cast(float, act[nt][kt][s]), acc[nt][t], 0, 0, 0);
-                } else {
-#pragma unroll
-                    for (int t = t0; t < MT && t < t0 + G; ++t)
-#pragma unroll
-                        for (int nt = 0; nt < NT; ++nt) acc[nt][t] = Mma::mma(w[t - t0], act[nt][kt], acc[nt][t]);
-                }
+                    for (int nt = 0; nt < NT; ++nt) acc[nt][t] = Mma::mma(w[t - t0], act[nt][kt], acc[nt][t]);
             }
         }
     }
@@ -98,6 +130,40 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
                 cc.floor2 = halfx2{lo, lo};
             }
         }
+        if constexpr (F32) {
+            if (!last) {
+                float most = 0.f;
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[nt][t][r] = chainActivateF32<ACT>(acc[nt][t][r], ly.slope);
+                        const u32x4 bits = __builtin_bit_cast(u32x4, acc[nt][t]);
+                        const uint32_t raw[4] = {bits.x, bits.y, bits.z, bits.w};
+                        most = Mma::largest(raw, 4, most);
+                    }
+                any = Mma::beyond(most);
+                auto split = [&](auto anyConst) {
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                        for (int kt = 0; kt < OKT; ++kt) {
+                            uint32_t raw[8];
+#pragma unroll
+                            for (int t = 0; t < 2; ++t) {    // (an odd number of tiles: the upper half of the last fragment is zero)
+                                const u32x4 v = 2 * kt + t < MT ? __builtin_bit_cast(u32x4, acc[nt][2 * kt + t < MT ? 2 * kt + t : 0]) : u32x4{0u, 0u, 0u, 0u};
+                                raw[4 * t] = v.x; raw[4 * t + 1] = v.y; raw[4 * t + 2] = v.z; raw[4 * t + 3] = v.w;
+                            }
+                            Mma::template decode<decltype(anyConst)::value>(raw, act[nt][kt]);
+                        }
+                };
+                split(std::false_type());
+                if (any) split(std::true_type());
+                any = any | matBeyond;
+                return;
+            }
+        }
         if (!last) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
@@ -105,13 +171,7 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
                 for (int kt = 0; kt < OKT; ++kt) {
                     const bool two = 2 * kt + 1 < MT;        // an odd number of tiles: the upper half of the last fragment is zero
                     const floatx4 x0 = acc[nt][2 * kt], x1 = two ? acc[nt][two ? 2 * kt + 1 : 2 * kt] : floatx4{0.f, 0.f, 0.f, 0.f};
-                    if constexpr (F32) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            act[nt][kt][r] = __builtin_bit_cast(uint32_t, chainActivateF32<ACT>(x0[r], ly.slope));
-                            act[nt][kt][4 + r] = two ? __builtin_bit_cast(uint32_t, chainActivateF32<ACT>(x1[r], ly.slope)) : 0u;
-                        }
-                    } else if constexpr (BF16) {
+                    if constexpr (BF16) {
                         float z[8];
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
@@ -124,7 +184,7 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
                         halfx2 lo01, lo23, hi01 = {(half_t)0, (half_t)0}, hi23 = hi01;
                         carrierFromAcc<false>(x0, cc, lo01, lo23);
                         if (two) carrierFromAcc<false>(x1, cc, hi01, hi23);
-                        fragFromCarrier<Mma>(lo01, lo23, hi01, hi23, cc, act[nt][kt]);
+                        if constexpr (!F32) fragFromCarrier<Mma>(lo01, lo23, hi01, hi23, cc, act[nt][kt]);
                     }
                 }
             return;
@@ -179,9 +239,9 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
 
 // MAXT: the bound on a layer's row tiles; NT: 16-sample tiles per wave and round; QUAD: input vectors of whole, aligned
 // groups of four elements, which one load takes (else one load per element, any size and alignment).
-// fp32 up to 64 wide: three waves per SIMD, four registers short of it, measure 522 us where two without a spill take 554.
-template <class Mma, int MAXT, int NT, bool QUAD>
-__global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1) void mlpChainKernel(const GenArgs ga)
+// INKT: the bound on the input's k-tiles.
+template <class Mma, int MAXT, int NT, bool QUAD, bool PIECES, int INKT>
+__global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void mlpChainKernel(const GenArgs ga)
 {
     constexpr int MAXKT = MAXT / 2, FD = Mma::kFD, ESZ = Mma::kEsz, RAW = Mma::kRawDW;
     constexpr int UNITS = QUAD ? 2 : 8;                    // loads per fragment
@@ -190,17 +250,27 @@ __global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1)
     const MlpArgs& a = ga.mlp;
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     float* ldsB = (float*)(lds + ga.biasDwordBase);
+    constexpr bool F32 = std::is_same<Mma, F32Mma>::value;
+    constexpr int LANE_DW = PIECES ? FD : RAW;             // dwords per lane of a fragment in LDS
+    float most = 0.f;
     for (int l = 0; l < a.numLayers; ++l) {
         const MlpLayerArgs& ly = a.layers[l];
         const int MT = ga.gl[l].mt, KT = ga.gl[l].kt;
-        stageFragments<ESZ, 8>(lds + ga.gl[l].fragBase * 64 * RAW, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in),
-                               (uint32_t)ly.out, (uint32_t)ly.in);
+        uint32_t* dst = lds + ga.gl[l].fragBase * 64 * LANE_DW;
+        if constexpr (PIECES) most = stageFragmentPieces(dst, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in), (uint32_t)ly.out, (uint32_t)ly.in, 0, most);
+        else stageFragments<ESZ, 8>(dst, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in), (uint32_t)ly.out, (uint32_t)ly.in);
         for (int e = threadIdx.x; e < MT * 16; e += 256) {
             const int t = e >> 4, gg = (e >> 2) & 3, r = e & 3, row = gg * 4 * MT + 4 * t + r;
             ldsB[ga.gl[l].biasBase + e] = (ly.bias && row < ly.out) ? loadAsFloat(ly.bias + (size_t)row * (chainComponent<Mma>() == kF32 ? 4 : 2), chainComponent<Mma>()) : 0.f;
         }
     }
     __syncthreads();
+    bool matBeyond = false;
+    if constexpr (F32) {
+        if constexpr (!PIECES)
+            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += 256) most = Mma::largest(lds + (size_t)i * RAW, RAW, most);
+        matBeyond = __syncthreads_or(most >= 0x1p127f);
+    }
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, n = lane & 15;
@@ -208,9 +278,9 @@ __global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1)
     const uint32_t in0 = (uint32_t)a.layers[0].in, gs0 = optGS(in0), rowBytes = in0 * ESZ;
     const bool quads = a.layers[L - 1].out % 4 == 0 && a.outAlign >= (std::is_same<Mma, F32Mma>::value ? 16u : 8u);
 
-    uint32_t off[MAXKT][UNITS];
+    uint32_t off[INKT][UNITS];
 #pragma unroll
-    for (int kt = 0; kt < MAXKT; ++kt)
+    for (int kt = 0; kt < INKT; ++kt)
 #pragma unroll
         for (int u = 0; u < UNITS; ++u) {
             const uint32_t q = kt * 8 + u * (8 / UNITS), col = g * gs0 + q;
@@ -219,7 +289,7 @@ __global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1)
 
     const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + 15) / 16), step = gridDim.x * 4u * NT;
     const int kt0 = ga.gl[0].kt;
-    uint32_t raw[NT][MAXKT][UNITS * UDW];
+    uint32_t raw[NT][INKT][UNITS * UDW];
     auto fetch = [&](uint32_t tile) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
@@ -229,7 +299,7 @@ __global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1)
             const uint32_t bytes = rows ? (rows - 1) * (uint32_t)a.inStride + rowBytes : 0u;
             const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc((void*)(a.in + (size_t)first * a.inStride), 0, bytes, 0x00027000);
 #pragma unroll
-            for (int kt = 0; kt < MAXKT; ++kt)
+            for (int kt = 0; kt < INKT; ++kt)
 #pragma unroll
                 for (int u = 0; u < UNITS; ++u) {
                     if (kt > 0 && kt >= kt0) continue;       // (wave-uniform; empty loads of absent k-tiles cost 6 us of 51)
@@ -256,11 +326,25 @@ __global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1)
     fetch(tile);
     for (;;) {
         uint32_t act[NT][MAXKT][FD];
+        bool any = matBeyond;
+        if constexpr (F32) {
+            float most = 0.f;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int kt = 0; kt < INKT; ++kt)
+                    if (kt == 0 || kt < kt0) most = Mma::largest(raw[nt][kt], RAW, most);
+            any = any | Mma::beyond(most);
+        }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int kt = 0; kt < MAXKT; ++kt) {
-                if constexpr (QUAD || ESZ == 4) {
+            for (int kt = 0; kt < INKT; ++kt) {
+                if constexpr (F32) {
+                    if (kt > 0 && kt >= kt0) continue;
+                    Mma::decode(raw[nt][kt], act[nt][kt]);
+                    if (any) Mma::template decode<true>(raw[nt][kt], act[nt][kt]);
+                } else if constexpr (QUAD) {
                     Mma::decode(raw[nt][kt], act[nt][kt]);
                 } else {
                     uint32_t packed[RAW];
@@ -280,11 +364,11 @@ __global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1)
         const uint32_t sample = tile * 16u + n;
         for (int l = 0; l < L; ++l) {
             const MlpLayerArgs& ly = a.layers[l];
-            const uint32_t* wbase = lds + ((size_t)ga.gl[l].fragBase * 64 + lane) * RAW;
+            const uint32_t* wbase = lds + ((size_t)ga.gl[l].fragBase * 64 + lane) * LANE_DW;
             const float* bbase = ldsB + ga.gl[l].biasBase + 4 * g;
             const int KT = ga.gl[l].kt;
             const bool last = l + 1 == L;
-#define CV_CHAIN_ARM(mt_) case mt_: chainLayer<Mma, MAXT, mt_, NT>(a, ly, wbase, bbase, KT, last, quads, g, sample, act); break;
+#define CV_CHAIN_ARM(mt_) case mt_: chainLayer<Mma, MAXT, mt_, NT, PIECES>(a, ly, wbase, bbase, KT, last, quads, g, sample, act, matBeyond, any); break;
             if constexpr (MAXT == 4) {
                 switch (ga.gl[l].mt) { CV_CHAIN_ARM(1) CV_CHAIN_ARM(2) CV_CHAIN_ARM(3) CV_CHAIN_ARM(4) }
             } else {
@@ -300,39 +384,44 @@ __global__ __launch_bounds__(256, (Mma::kEsz == 4 && MAXT == 4 && QUAD) ? 3 : 1)
     }
 }
 
-template <class Mma, int MAXT, int NT, bool QUAD>
+template <class Mma, int MAXT, int NT, bool QUAD, bool PIECES, int INKT = MAXT / 2>
 hipError_t launchChainSized(hipStream_t stream, const GenArgs& ga, size_t ldsBytes, int numCUs)
 {
-    const hipError_t ea = allowDynamicLds<mlpChainKernel<Mma, MAXT, NT, QUAD>>((int)(kGenLdsDwords * 4));
+    const hipError_t ea = allowDynamicLds<mlpChainKernel<Mma, MAXT, NT, QUAD, PIECES, INKT>>((int)((PIECES ? kChainPieceDwords : kGenLdsDwords) * 4));
     if (ea != hipSuccess) return ea;
     int perCU = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpChainKernel<Mma, MAXT, NT, QUAD>, 256, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpChainKernel<Mma, MAXT, NT, QUAD, PIECES, INKT>, 256, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
     const uint32_t numTiles = (uint32_t)(((uint64_t)ga.mlp.batch + 15) / 16), need = (numTiles + 4 * NT - 1) / (4 * NT);
     const uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU;
     noteKernel(false, "mlpChainKernel<%s,up to %d rows,NT=%d%s>", Mma::kName, 16 * MAXT, NT,
                QUAD ? ",loads of four elements" : "");
-    hipLaunchKernelGGL((mlpChainKernel<Mma, MAXT, NT, QUAD>), dim3(need < cap ? need : cap), dim3(256), ldsBytes, stream, ga);
+    hipLaunchKernelGGL((mlpChainKernel<Mma, MAXT, NT, QUAD, PIECES, INKT>), dim3(need < cap ? need : cap), dim3(256), ldsBytes, stream, ga);
     return hipGetLastError();
 }
 
-template <class Mma, int MAXT>
+template <class Mma, int MAXT, bool PIECES>
 hipError_t launchChainRows(hipStream_t stream, const GenArgs& ga, size_t ldsBytes, int numCUs)
 {
     constexpr uint32_t ESZ = Mma::kEsz;
     const MlpArgs& a = ga.mlp;
     const bool quad = a.layers[0].in % 4 == 0 && a.inAlign >= 4 * ESZ;
     // Two tiles per wave as soon as every SIMD has two waves of them; below that the tiles are spread over the chip.
-    // (One where two would leave a SIMD one wave for their registers: fp32 layers wider than 64, and layers wider than 64
-    // whose input comes element by element)
-    if ((uint64_t)a.batch > (uint64_t)numCUs * 8 * 16) {
-        if constexpr (MAXT == 4) {
-            if (!quad) return launchChainSized<Mma, MAXT, 2, false>(stream, ga, ldsBytes, numCUs);
-        }
-        if constexpr (MAXT == 4 || ESZ < 4) {
-            if (quad) return launchChainSized<Mma, MAXT, 2, true>(stream, ga, ldsBytes, numCUs);
+    // (One where two would leave a SIMD one wave for their registers: fp32, and layers wider than 64 whose input comes element
+    // by element)
+    if constexpr (ESZ < 4) {
+        if ((uint64_t)a.batch > (uint64_t)numCUs * 8 * 16) {
+            if constexpr (MAXT == 4) {
+                if (!quad) return launchChainSized<Mma, MAXT, 2, false, PIECES>(stream, ga, ldsBytes, numCUs);
+            }
+            if (quad) return launchChainSized<Mma, MAXT, 2, true, PIECES>(stream, ga, ldsBytes, numCUs);
         }
     }
-    return quad ? launchChainSized<Mma, MAXT, 1, true>(stream, ga, ldsBytes, numCUs) : launchChainSized<Mma, MAXT, 1, false>(stream, ga, ldsBytes, numCUs);
+    // (up to 64 inputs before wide layers of float: the registers of the other k-tiles would be spilled ones)
+    if constexpr (ESZ == 4 && MAXT == 8) {
+        if (ga.gl[0].kt <= 2)
+            return quad ? launchChainSized<Mma, MAXT, 1, true, PIECES, 2>(stream, ga, ldsBytes, numCUs) : launchChainSized<Mma, MAXT, 1, false, PIECES, 2>(stream, ga, ldsBytes, numCUs);
+    }
+    return quad ? launchChainSized<Mma, MAXT, 1, true, PIECES>(stream, ga, ldsBytes, numCUs) : launchChainSized<Mma, MAXT, 1, false, PIECES>(stream, ga, ldsBytes, numCUs);
 }
 
 // hipErrorInvalidValue for calls this kernel does not take: smooth activations, inputs that are encoded or quantised on
@@ -343,9 +432,15 @@ hipError_t launchChain(hipStream_t stream, const MlpArgs& a, int numCUs)
     if (hasSmoothActivation(a) || a.inEncoding != kEncodeNone || a.inHalfAsE4M3 || a.inStride > (1u << 26)) return hipErrorInvalidValue;
     GenArgs ga{};
     uint32_t widest = 0;
+    // (the pieces of a network of float take half as much again: where they do not fit, fragments stay as they are in memory)
+    if constexpr (Mma::kEsz == 4) {
+        const uint32_t dwords = planGeneric<Mma>(a, ga, kChainPieceDwords, &widest, Mma::kFD);
+        if (dwords)
+            return widest <= 4 ? launchChainRows<Mma, 4, true>(stream, ga, (size_t)dwords * 4, numCUs) : launchChainRows<Mma, 8, true>(stream, ga, (size_t)dwords * 4, numCUs);
+    }
     const uint32_t dwords = planGeneric<Mma>(a, ga, kGenLdsDwords, &widest);
     if (!dwords) return hipErrorInvalidValue;
-    return widest <= 4 ? launchChainRows<Mma, 4>(stream, ga, (size_t)dwords * 4, numCUs) : launchChainRows<Mma, 8>(stream, ga, (size_t)dwords * 4, numCUs);
+    return widest <= 4 ? launchChainRows<Mma, 4, false>(stream, ga, (size_t)dwords * 4, numCUs) : launchChainRows<Mma, 8, false>(stream, ga, (size_t)dwords * 4, numCUs);
 }
 
 } // namespace

@@ -41,11 +41,12 @@ __device__ __forceinline__ float activateFloat(float x, int act, float slope)
 
 // MAXT: the unrolled bound on a layer's 16-row tiles (4 for networks up to 64 wide, which then need half the
 // registers and run more waves per SIMD; 8 up to 128)
-template <class Mma, int MAXT>
+// PIECES (T = float): fragments lie in LDS as F32Mma's pieces; else as they lie in memory, split at every use.
+template <class Mma, int MAXT, bool PIECES>
 __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
 {
     constexpr int kFltMaxTiles = MAXT, kFltMaxKT = MAXT / 2;
-    constexpr int EPL = Mma::kEpl, FD = Mma::kFD, ESZ = Mma::kEsz, RAW = Mma::kRawDW;
+    constexpr int EPL = Mma::kEpl, FD = Mma::kFD, ESZ = Mma::kEsz, RAW = Mma::kRawDW, LANE_DW = PIECES ? FD : RAW;
     constexpr bool F32 = ESZ == 4;
     static_assert(EPL == 8, "the layer chain needs 8 k-slots per lane per fragment");
     const MlpArgs& a = ga.mlp;
@@ -53,11 +54,13 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     float* ldsB = (float*)(lds + ga.biasDwordBase);
 
+    float most = 0.f;
     for (int l = 0; l < L; ++l) {
         const MlpLayerArgs& ly = a.layers[l];
         const int MT = ga.gl[l].mt, KT = ga.gl[l].kt, ROWS = 4 * MT;
-        stageFragments<ESZ, EPL>(lds + ga.gl[l].fragBase * 64 * RAW, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in),
-                                 (uint32_t)ly.out, (uint32_t)ly.in);
+        uint32_t* dst = lds + ga.gl[l].fragBase * 64 * LANE_DW;
+        if constexpr (PIECES) most = stageFragmentPieces(dst, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in), (uint32_t)ly.out, (uint32_t)ly.in, 0, most);
+        else stageFragments<ESZ, EPL>(dst, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in), (uint32_t)ly.out, (uint32_t)ly.in);
         for (int e = threadIdx.x; e < MT * 16; e += 256) {
             const int t = e >> 4, g = (e >> 2) & 3, r = e & 3;
             const int row = g * ROWS + 4 * t + r;
@@ -65,6 +68,12 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
         }
     }
     __syncthreads();
+    bool matBeyond = false;                  // F32Mma::beyond of some layer's matrix
+    if constexpr (F32) {
+        if constexpr (!PIECES)
+            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += 256) most = Mma::largest(lds + (size_t)i * RAW, RAW, most);
+        matBeyond = __syncthreads_or(most >= 0x1p127f);
+    }
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, n = lane & 15;
@@ -78,13 +87,13 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
     for (uint32_t tile = blockIdx.x * 4 + wave; tile < numTiles; tile += gridDim.x * 4) {
         const uint32_t sample = tile * 16 + n;
         const uint32_t sc = min(sample, a.batch - 1);
-        uint32_t act[kFltMaxKT][FD];
+        uint32_t act[kFltMaxKT][RAW];          // the layer's input as it lies in memory
         {
             const uint8_t* p = a.in + (size_t)sc * a.inStride;
 #pragma unroll
             for (int kt = 0; kt < kFltMaxKT; ++kt) {
 #pragma unroll
-                for (int d = 0; d < FD; ++d) act[kt][d] = 0u;
+                for (int d = 0; d < RAW; ++d) act[kt][d] = 0u;
                 if (kt < kt0) {
 #pragma unroll
                     for (int s = 0; s < EPL; ++s) {
@@ -101,25 +110,50 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
 
         for (int l = 0; l < L; ++l) {
             const int MT = ga.gl[l].mt, KT = ga.gl[l].kt;
-            const uint32_t* wbase = lds + ((size_t)ga.gl[l].fragBase * 64 + lane) * RAW;
+            const uint32_t* wbase = lds + ((size_t)ga.gl[l].fragBase * 64 + lane) * LANE_DW;
             const float* bbase = ldsB + ga.gl[l].biasBase + 4 * g;
             const int actKind = a.layers[l].act;
             const float slope = a.layers[l].slope;
-            floatx4 acc[kFltMaxTiles];
+            bool any = matBeyond;
+            if constexpr (F32) {
+                float most = 0.f;
 #pragma unroll
-            for (int t = 0; t < kFltMaxTiles; ++t)
-                if (t < MT) acc[t] = *(const floatx4*)(bbase + 16 * t);
+                for (int kt = 0; kt < kFltMaxKT; ++kt) most = Mma::largest(act[kt], RAW, most);
+                any = any | Mma::beyond(most);
+            }
+            uint32_t x[kFltMaxKT][FD];
 #pragma unroll
             for (int kt = 0; kt < kFltMaxKT; ++kt) {
-                if (kt < KT) {
+                Mma::decode(act[kt], x[kt]);
+                if constexpr (F32) {
+                    if (any) Mma::template decode<true>(act[kt], x[kt]);
+                }
+            }
+            floatx4 acc[kFltMaxTiles];
 #pragma unroll
-                    for (int t = 0; t < kFltMaxTiles; ++t) {
-                        if (t < MT) {
+            for (int t = 0; t < kFltMaxTiles; ++t) {
+                acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+                if (t < MT) {
+                    typename SumOf<Mma>::T sum = SumOf<Mma>::start(*(const floatx4*)(bbase + 16 * t));
+#pragma unroll
+                    for (int kt = 0; kt < kFltMaxKT; ++kt) {
+                        if (kt < KT) {
                             uint32_t w[FD];
-                            Mma::decode(wbase + (size_t)(t * KT + kt) * 64 * RAW, w);
-                            acc[t] = Mma::mma(w, act[kt], acc[t]);
+                            const uint32_t* raw = wbase + (size_t)(t * KT + kt) * 64 * LANE_DW;
+                            if constexpr (PIECES) {
+#pragma unroll
+                                for (int d = 0; d < FD; ++d) w[d] = raw[d];
+                            } else {
+                                Mma::decode(raw, w);
+                                if constexpr (F32) {
+                                    if (matBeyond) Mma::template decode<true>(raw, w);
+                                }
+                            }
+                            sum = Mma::mma(w, x[kt], sum);
                         }
                     }
+                    acc[t] = SumOf<Mma>::finish(sum);
+                    if (F32 && any) acc[t] = SumOf<Mma>::finishAny(sum);
                 }
             }
             // the layer's result in T, activated: what coopVecMatMulAdd + activation returns
@@ -163,17 +197,17 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
     }
 }
 
-template <class Mma, int MAXT>
+template <class Mma, int MAXT, bool PIECES>
 hipError_t launchFloatSized(hipStream_t stream, const FltArgs& ga, size_t ldsBytes, int numCUs)
 {
-    const hipError_t ea = allowDynamicLds<mlpFloatKernel<Mma, MAXT>>((int)(kFltLdsDwords * 4));
+    const hipError_t ea = allowDynamicLds<mlpFloatKernel<Mma, MAXT, PIECES>>((int)(kFltLdsDwords * 4));
     if (ea != hipSuccess) return ea;
     int perCU = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpFloatKernel<Mma, MAXT>, 256, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpFloatKernel<Mma, MAXT, PIECES>, 256, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
     const uint32_t numTiles = (ga.mlp.batch + 15) / 16, need = (numTiles + 3) / 4;
     const uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU;
     noteKernel(false, "mlpFloatKernel<%s,up to %d rows>", Mma::kName, 16 * MAXT);
-    hipLaunchKernelGGL((mlpFloatKernel<Mma, MAXT>), dim3(need < cap ? need : cap), dim3(256), ldsBytes, stream, ga);
+    hipLaunchKernelGGL((mlpFloatKernel<Mma, MAXT, PIECES>), dim3(need < cap ? need : cap), dim3(256), ldsBytes, stream, ga);
     return hipGetLastError();
 }
 
@@ -193,11 +227,18 @@ hipError_t launchFloat(hipStream_t stream, const MlpArgs& a, int ct, int numCUs)
         if (mt > widest) widest = mt;
         if (2 * kt > widest) widest = 2 * kt;
     }
+    if constexpr (Mma::kEsz == 4) {
+        ga.biasDwordBase = frag * 64 * Mma::kFD;
+        if (ga.biasDwordBase + bias <= kFltLdsDwords) {
+            const size_t ldsBytes = (size_t)(ga.biasDwordBase + bias) * 4;
+            return widest <= 4 ? launchFloatSized<Mma, 4, true>(stream, ga, ldsBytes, numCUs) : launchFloatSized<Mma, 8, true>(stream, ga, ldsBytes, numCUs);
+        }
+    }
     ga.biasDwordBase = frag * 64 * Mma::kRawDW;
     const uint32_t dwords = ga.biasDwordBase + bias;
     if (dwords > kFltLdsDwords) return hipErrorInvalidValue;
     const size_t ldsBytes = (size_t)dwords * 4;
-    return widest <= 4 ? launchFloatSized<Mma, 4>(stream, ga, ldsBytes, numCUs) : launchFloatSized<Mma, 8>(stream, ga, ldsBytes, numCUs);
+    return widest <= 4 ? launchFloatSized<Mma, 4, false>(stream, ga, ldsBytes, numCUs) : launchFloatSized<Mma, 8, false>(stream, ga, ldsBytes, numCUs);
 }
 
 } // namespace

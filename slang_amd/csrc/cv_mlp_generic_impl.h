@@ -29,7 +29,7 @@ struct GenArgs {
 // Tile counts and LDS placement of every layer; the dwords of LDS taken (fragments, then biases), or 0 when a layer is
 // wider than 128 or the network does not fit `limitDwords`.  `widest` receives the largest tile count of any layer.
 template <class Mma>
-inline uint32_t planGeneric(const MlpArgs& a, GenArgs& ga, uint32_t limitDwords, uint32_t* widest)
+inline uint32_t planGeneric(const MlpArgs& a, GenArgs& ga, uint32_t limitDwords, uint32_t* widest, uint32_t laneDwords = Mma::kRawDW)
 {
     ga.mlp = a;
     uint32_t frag = 0, bias = 0, w = 0;
@@ -42,7 +42,7 @@ inline uint32_t planGeneric(const MlpArgs& a, GenArgs& ga, uint32_t limitDwords,
         if (mt > w) w = mt;
         if (2 * kt > w) w = 2 * kt;
     }
-    ga.biasDwordBase = frag * 64 * Mma::kRawDW;
+    ga.biasDwordBase = frag * 64 * laneDwords;
     const uint32_t dwords = ga.biasDwordBase + bias;
     if (dwords > limitDwords) return 0;
     *widest = w;

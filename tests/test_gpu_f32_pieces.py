@@ -1,0 +1,115 @@
+"""fp32 matrix products as sums of bfloat16 pieces (F32Mma, slang_amd/csrc/cv_device.h): accuracy against 64 bits, infinities,
+NaN, the largest and the smallest values, and the kernel for equal hidden layers against the chain of single-layer operators.
+
+Bound of a sum of K terms: an operand is three pieces exactly; of the nine products the three dropped ones are below 2^-26 of the
+term each, the others are exact; of the sums, one rounding to 24 bits per matrix instruction (K/32 of them on the h*h products,
+of which one begins with the bias; the five small ones count below 2^-7 of it) and one at the end."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import DEV, as_bytes, to_dev
+from slang_amd import coopvec as cv
+from slang_amd.coopvec import Activation, CoopVecComponentType as CT, CoopVecMatrixLayout as ML, FeedForwardLayer
+
+pytestmark = pytest.mark.gpu
+
+
+def matmul(x, W, b):
+    M, K = W.shape
+    return cv.coopVecMatMulAdd(to_dev(x), CT.Float32, as_bytes(to_dev(W)), 0, CT.Float32, as_bytes(to_dev(b)), 0, CT.Float32,
+                               ML.RowMajor, False, 4 * K, M=M, resultType=CT.Float32).cpu().numpy()
+
+
+def bound(x, W, b):
+    K = W.shape[1]
+    mag = np.abs(x.astype(np.float64)) @ np.abs(W.astype(np.float64)).T + np.abs(b.astype(np.float64))
+    return (K / 32 + 4) * 2.0 ** -24 * mag
+
+
+# registers up to 64 x 64, then LDS: remainders of tiles, the last k whose pieces fit (1664), the first whose do not, 2048
+@pytest.mark.parametrize("M,K,B", [(1, 1, 1), (16, 32, 64), (17, 33, 100), (64, 64, 1027), (65, 64, 500), (128, 192, 400), (130, 200, 300),
+                                   (20, 1664, 60), (20, 1680, 60), (33, 2048, 50)])
+def test_products_against_64_bits(M, K, B):
+    rng = np.random.default_rng(M * 3000 + K)
+    x = (rng.standard_normal((B, K)) * np.exp2(rng.integers(-12, 13, (B, K)))).astype(np.float32)
+    W = (rng.standard_normal((M, K)) * np.exp2(rng.integers(-6, 7, (M, K)))).astype(np.float32)
+    b = rng.standard_normal(M).astype(np.float32)
+    ref = x.astype(np.float64) @ W.astype(np.float64).T + b
+    assert (np.abs(matmul(x, W, b) - ref) <= bound(x, W, b)).all()
+
+
+# (63 x 64: the kernel in registers; its streaming form for 64 x 64 takes NaN through a maximum)
+@pytest.mark.parametrize("M,K", [(24, 40), (63, 64), (100, 96), (8, 1700)])
+def test_values_at_the_ends_of_the_range(M, K):
+    rng = np.random.default_rng(M + K)
+    B = 200
+    x, W, b = (rng.standard_normal(s).astype(np.float32) for s in ((B, K), (M, K), (M,)))
+    plain = matmul(x, W, b)
+    big = np.float32(3.4e38)                             # its nearest bfloat16 is infinite
+    y = x.copy()
+    y[3, 5], y[20, 0], y[40, K - 1], y[60, 7] = np.inf, -np.inf, np.nan, big
+    y[80] = np.where(np.arange(K) % 3 == 0, np.inf, y[80])
+    y[100] = x[100] * np.float32(1e-38)                  # down into the subnormal numbers
+    V = W.copy()
+    V[2, 5], V[5, 7], V[6, 9] = 0.0, 1e-3, np.inf
+    def want(xs, ws):
+        with np.errstate(all="ignore"):
+            return (xs.astype(np.float64) @ ws.astype(np.float64).T + b).astype(np.float32)
+    got = matmul(y, W, b)
+    special = [3, 20, 40, 60, 80]
+    others = np.setdiff1d(np.arange(B), special + [100])
+    assert np.array_equal(got[others].view(np.uint32), plain[others].view(np.uint32))
+    for rows in ([3], [20], [40], [80]):
+        ref = want(y[rows], W)
+        assert np.array_equal(np.isnan(got[rows]), np.isnan(ref)) and np.array_equal(got[rows][~np.isnan(ref)], ref[~np.isnan(ref)])
+    ref = y[[60, 100]].astype(np.float64) @ W.astype(np.float64).T + b
+    fits = np.abs(ref) < 1e38
+    assert (np.abs(got[[60, 100]] - ref)[fits] <= bound(y[[60, 100]], W, b)[fits]).all() and fits[1].all()
+    # an infinite element of the matrix: its row alone
+    got = matmul(x, V, b)
+    ref = want(x, V)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(got[:, 6][~np.isnan(ref[:, 6])], ref[:, 6][~np.isnan(ref[:, 6])])
+    same = np.setdiff1d(np.arange(M), [2, 5, 6])
+    assert np.array_equal(got[:, same].view(np.uint32), plain[:, same].view(np.uint32))
+    got = matmul(y, V, b)                                # ... and infinite vectors before it: 0 x inf is NaN
+    ref = want(y[special], V)
+    ok = np.isfinite(ref) & (np.abs(ref) < 1e38)
+    assert np.array_equal(np.isnan(got[special]), np.isnan(ref)) and np.array_equal(np.isinf(got[special]) & ~ok, np.isinf(ref) & ~ok)
+
+
+def network(rng, dims, acts):
+    layers, params = [], []
+    for fi, fo, act in zip(dims, dims[1:], acts):
+        W = (rng.standard_normal((fo, fi)) * np.sqrt(2.0 / fi)).astype(np.float32)
+        b = (rng.standard_normal(fo) * 0.1).astype(np.float32)
+        wd, bd = as_bytes(to_dev(W)), as_bytes(to_dev(b))
+        layers.append(FeedForwardLayer(fi, fo, wd, bd, ML.RowMajor, fi * 4, act, 0.125))
+        params.append((fi, fo, wd, bd, act))
+    return layers, params
+
+
+def chain(params, x):
+    for fi, fo, wd, bd, act in params:
+        x = cv.coopVecMatMulAdd(x, CT.Float32, wd, 0, CT.Float32, bd, 0, CT.Float32, ML.RowMajor, False, fi * 4, M=fo, resultType=CT.Float32,
+                                activation=act, leakySlope=0.125)
+    return x
+
+
+@pytest.mark.parametrize("dims", [[4, 16, 1], [3, 16, 16, 16], [32, 32, 5], [20, 20, 24, 31, 8], [8, 64, 64, 64, 3], [33, 50, 64, 16], [64, 60, 60, 9],
+                                  [7, 128, 4], [64, 120, 113, 16], [40, 16, 16, 16, 16, 16, 2], [36, 30, 7]])
+def test_equal_hidden_layers_equal_the_chain_of_single_layer_operators(dims):
+    rng = np.random.default_rng(sum(dims))
+    acts = [[Activation.ReLU, Activation.NoActivation, Activation.LeakyReLU][l % 3] for l in range(len(dims) - 1)]
+    layers, params = network(rng, dims, acts)
+    for B, pad in ((1, 0), (15, 0), (65, 3), (20000, 0), (5001, 4)):      # `pad`: rows at a pitch, of which 3 leaves them unaligned
+        wide = torch.zeros((B, dims[0] + pad), dtype=torch.float32, device=DEV)
+        wide[:, :dims[0]] = to_dev(rng.uniform(-1, 1, (B, dims[0])).astype(np.float32))
+        if B > 100:
+            wide[7, 0], wide[B - 1, dims[0] - 1], wide[50, 1] = float("inf"), float("-inf"), 3.4e38
+        x = wide[:, :dims[0]]
+        y = cv.mlpForward(layers, x, weightType=CT.Float32)
+        assert cv.lastKernelName().startswith("mlpChainKernelEqualF32"), cv.lastKernelName()
+        ref = chain(params, x)
+        assert torch.equal(torch.isnan(y), torch.isnan(ref))
+        assert torch.equal(y[~torch.isnan(y)].view(torch.int32), ref[~torch.isnan(ref)].view(torch.int32)), (B, pad)
