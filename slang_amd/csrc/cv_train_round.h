@@ -22,11 +22,10 @@
 //
 // What bounds it: float: the matrix pipeline (v_mfma_f32_16x16x4_f32 takes 32 cycles for what two 4-byte reads supply).
 // half: waiting, for operands from LDS (one 16-byte read per lane and operand feeds 16 cycles of the pipeline) and at the
-// meetings; the waves of 16-128-128-128-8 wait 57 % of their time and the pipeline is busy 10 %.  Half networks wider than 64 also
-// keep part of the prefetched input in scratch memory (32 bytes a lane, five layers 64), so that each round begins with a wait
-// for memory; five float layers up to 64 wide spill 108 bytes.
-// 16-128-128-128-8 (half) over 200 003 samples: 187 us, 724 us over the whole batch in memory.  Of these about 76 us are paid
-// once (LDS cleared, weights staged element by element, the partials written and added up) and 10 us for each further round.
+// meetings.  Five float layers up to 64 wide and five layers beyond 64 spill.
+// 16-128-128-128-8 (half) over 200 003 samples: 151 us, 724 us over the whole batch in memory.  187 us while the weights were staged
+// element by element (now in 16-byte pieces, all layers requested together) and half networks wider than 64 kept part of the
+// prefetched input in scratch memory, so that each round began with a wait for memory.
 #pragma once
 #include "cv_train_impl.h"
 
@@ -213,16 +212,65 @@ template <> struct RoundMma<half_t> {
 // every wave of the workgroup has finished its LDS accesses; loads from memory stay in flight
 __device__ __forceinline__ void meetInLds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Weights and biases of all layers to LDS.  A row-major matrix of whole aligned 16-byte pieces (what a program's own matrices
+// mostly are) goes in pieces, and the first kAhead pieces of a thread of every layer are requested before the first is stored: one
+// round trip to memory for all of them instead of one for every four elements.  16-128-128-128-8 (half), 64 samples to a
+// workgroup, see the head of this file.
 template <typename T>
-__device__ __forceinline__ void stageRoundWeights(const RoundLayer& ly, uint8_t* lds)
+__device__ __forceinline__ size_t roundWeightLine(const RoundLayer& ly) { return ly.shape.stride ? ly.shape.stride : (size_t)ly.shape.cols * sizeof(T); }
+template <typename T>
+__device__ __forceinline__ bool roundWeightPieces(const RoundLayer& ly)
 {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int col = lane; col < ly.in; col += 64) {
-#pragma unroll 4
-        for (int row = wave; row < ly.out; row += kRoundThreads / 64)
-            *(T*)(lds + ly.wOff + (uint32_t)row * ly.wStride + (uint32_t)col * sizeof(T)) = *(const T*)(ly.w + elemOffset(ly.shape, (uint32_t)row, (uint32_t)col));
+    return ly.shape.layout == kRowMajor && ((size_t)ly.in * sizeof(T)) % 16u == 0 && (((uintptr_t)ly.w | roundWeightLine<T>(ly)) & 15u) == 0;
+}
+template <typename T, int NL, int MAXT>
+__device__ __forceinline__ void stageRoundWeights(const RoundLayer (&layers)[kRoundMaxLayers], uint8_t* lds)
+{
+    constexpr int kMost = MAXT * 16 * MAXT * 16 * (int)sizeof(T) / 16 / kRoundThreads, kUpTo = NL < 5 ? 4 : 2, kAhead = kMost < 1 ? 1 : kMost < kUpTo ? kMost : kUpTo;
+    u32x4 v[NL][kAhead];
+    auto piece = [&](const RoundLayer& ly, uint32_t c, uint32_t& row, uint32_t& at) {
+        const uint32_t perRow = (uint32_t)ly.in * sizeof(T) / 16u;
+        row = c / perRow;
+        at = c - row * perRow;
+        return row < (uint32_t)ly.out;
+    };
+    auto load = [&](const RoundLayer& ly, uint32_t row, uint32_t at) {
+        return *(const u32x4*)(ly.w + row * roundWeightLine<T>(ly) + 16u * at);
+    };
+    auto store = [&](const RoundLayer& ly, uint32_t row, uint32_t at, u32x4 x) { *(u32x4*)(lds + ly.wOff + row * ly.wStride + 16u * at) = x; };
+    float bias[NL];
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+        const RoundLayer& ly = layers[l];
+        const int e = threadIdx.x;
+        bias[l] = ly.bias && e < ly.out ? (float)((const T*)ly.bias)[e] : 0.f;      // (no layer has more rows than the workgroup threads)
+        if (!roundWeightPieces<T>(ly)) continue;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            uint32_t row, at;
+            const bool on = piece(ly, threadIdx.x + (uint32_t)(i * kRoundThreads), row, at);
+            v[l][i] = load(ly, on ? row : 0u, on ? at : 0u);
+        }
     }
-    for (int e = threadIdx.x; e < ly.out; e += kRoundThreads) *(float*)(lds + ly.biasOff + 4 * e) = ly.bias ? (float)((const T*)ly.bias)[e] : 0.f;
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+        const RoundLayer& ly = layers[l];
+        if ((int)threadIdx.x < ly.out) *(float*)(lds + ly.biasOff + 4 * threadIdx.x) = bias[l];
+        uint32_t row, at;
+        if (roundWeightPieces<T>(ly)) {
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i)
+                if (piece(ly, threadIdx.x + (uint32_t)(i * kRoundThreads), row, at)) store(ly, row, at, v[l][i]);
+            for (uint32_t c = threadIdx.x + (uint32_t)(kAhead * kRoundThreads); piece(ly, c, row, at); c += kRoundThreads) store(ly, row, at, load(ly, row, at));
+        } else {
+            const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+            for (int col = lane; col < ly.in; col += 64) {
+#pragma unroll 4
+                for (int r = wave; r < ly.out; r += kRoundThreads / 64)
+                    *(T*)(lds + ly.wOff + (uint32_t)r * ly.wStride + (uint32_t)col * sizeof(T)) = *(const T*)(ly.w + elemOffset(ly.shape, (uint32_t)r, (uint32_t)col));
+            }
+        }
+    }
 }
 
 // WAVES: per SIMD; 4 where two workgroups share a compute unit (128 registers a wave), else 2
@@ -238,7 +286,7 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
 
     for (uint32_t i = threadIdx.x; i < a.ldsBytes / 16; i += kRoundThreads) ((u32x4*)lds)[i] = u32x4{0u, 0u, 0u, 0u};
     __syncthreads();
-    for (int l = 0; l < NL; ++l) stageRoundWeights<T>(a.layers[l], lds);
+    stageRoundWeights<T, NL, 2 * RT>(a.layers, lds);
     __syncthreads();
 
     // The layers' sizes and places in LDS are read from the kernel's arguments where they are used (scalar loads): hoisted out
@@ -284,6 +332,8 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
                 const u32x4 p = *(const u32x4*)(row + 16 * min(inCol + 8 * c, a.inPieces - 1));
                 v[4 * c] = p.x; v[4 * c + 1] = p.y; v[4 * c + 2] = p.z; v[4 * c + 3] = p.w;
             }
+            asm volatile("");               // (the ends of the two branches differ: else their stores become one, to an address
+                                            // chosen between registers, and the array moves to scratch memory)
         } else {
 #pragma unroll
             for (int c = 0; c < ELEMS; ++c) {
@@ -413,8 +463,10 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
             LayerInArgs& top = layer(NL - 1);
             floatx4 acc[NS][NT];
             product(std::integral_constant<int, 1>{}, top, acc);
-#pragma unroll
-            for (int s = 0; s < NS; ++s) {
+            // (the sample tile a constant from the start: an array indexed by a loop that is unrolled too late lies in scratch
+            // memory, and its loads wait for the prefetched input as well)
+            staticFor<0, NS>([&](auto sc) {
+                constexpr int s = decltype(sc)::value;
                 const int row = 16 * (NS * sg + s) + n;
                 const bool live = r * kRoundSamples + row < a.batch;
                 float tgtAll = 0.f;
@@ -456,7 +508,7 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
                 T* out = (T*)(lds + a.zOff + (uint32_t)row * a.zStride + 4 * g * ESZ);
                 typedef T TVec __attribute__((ext_vector_type(4)));
                 *(TVec*)out = TVec{dz[0], dz[1], dz[2], dz[3]};
-            }
+            });
         }
         meetInLds();
 

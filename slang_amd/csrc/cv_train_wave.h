@@ -84,7 +84,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     for (uint32_t i = threadIdx.x; i < Net::ldsBytes / 16u; i += 512u) ((u32x4*)lds)[i] = u32x4{0u, 0u, 0u, 0u};
     __syncthreads();
-    for (int l = 0; l < NL; ++l) stageRoundWeights<float>(a.layers[l], lds);
+    stageRoundWeights<float, NL, (IT > HT ? IT : HT)>(a.layers, lds);
     __syncthreads();
 
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
