@@ -111,11 +111,14 @@ struct Bf16Mma {
 
 // fp32 operands on the bfloat16 matrix pipeline: every operand is the sum of three bfloat16 pieces (h the nearest to it, m the
 // nearest to the rest, l what is left: 24 bits, exactly), and of the nine products of pieces the six that matter are summed, the
-// h*h products by themselves (F32Sum::main, seeded with the bias) and the five small ones by themselves, added at the end.
+// h*h products by themselves (F32Sum::main) and the five small ones by themselves, added at the end with the bias.
 // Six v_mfma_f32_16x16x32_bf16 take 96 cycles of the matrix pipeline where eight v_mfma_f32_16x16x4_f32, which round every
 // product's sum to 24 bits, take 256, and the sums are closer to the exact ones (random operands, error over the norm against 64
 // bits, 32 / 64 / 128 terms: 3.9 / 5.0 / 6.5e-8 against 10.3 / 14.4 / 20.4e-8 on the fp32 instruction; the dropped products are
-// below 2^-26 of the largest term each).
+// below 2^-26 of the largest term each).  What the instruction drops, the low bits of products far below its largest one, it drops in
+// one direction: where inputs of one sign meet many sizes, the mean error of a row over all samples is 1e-8 to 1e-7 of the row's
+// mean (fp32 instruction: 1e-10), though each element is nearer.  The training kernels, which sum over samples, therefore
+// stay on the fp32 instruction: 32-64-64-8 over 2^20 samples would take 350 us for 394, with gradients up to 3.5 times as far off.
 // A fragment has the 8 k-slots per lane of the 16-bit flavours, so the InferencingOptimal form of an fp32 matrix is the same
 // arrangement with 4-byte elements; decoded, four dwords each of h, m and l.
 // Infinities and values from 2^127 on: split() makes NaN of them (inf - inf), so a wave that holds one (beyond()) takes
@@ -206,21 +209,23 @@ template <class Mma, bool F32 = Mma::kEsz == 4>
 struct SumOf {
     typedef typename Mma::Acc T;
     static __device__ __forceinline__ T start(typename Mma::Acc seed) { return seed; }
-    static __device__ __forceinline__ typename Mma::Acc finish(T s) { return s; }
-    static __device__ __forceinline__ typename Mma::Acc finishAny(T s) { return s; }
+    static __device__ __forceinline__ typename Mma::Acc finish(T s, typename Mma::Acc) { return s; }
+    static __device__ __forceinline__ typename Mma::Acc finishAny(T s, typename Mma::Acc) { return s; }
 };
 template <class Mma>
 struct SumOf<Mma, true> {
     typedef F32Sum T;
-    static __device__ __forceinline__ T start(floatx4 seed) { return F32Sum{seed, floatx4{0.f, 0.f, 0.f, 0.f}}; }
-    static __device__ __forceinline__ floatx4 finish(T s) { return s.main + s.small; }
+    // The seed (the bias) joins at the end: a matrix instruction drops the bits of its C operand that lie below what it keeps of the
+    // products, and of a bias that is the same for every sample it would drop the same ones every time.
+    static __device__ __forceinline__ T start(floatx4) { return F32Sum{floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}}; }
+    static __device__ __forceinline__ floatx4 finish(T s, floatx4 seed) { return s.main + (s.small + seed); }
     // ... where some operand was beyond(): an infinity or NaN of the sum stands in `main` alone
-    static __device__ __forceinline__ floatx4 finishAny(T s)
+    static __device__ __forceinline__ floatx4 finishAny(T s, floatx4 seed)
     {
         asm volatile("" : "+v"(s.main));      // (as in decode)
-        floatx4 r = s.main + s.small;
+        floatx4 r = s.main + (s.small + seed);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = __builtin_isfinite(s.main[i]) ? r[i] : s.main[i];
+        for (int i = 0; i < 4; ++i) r[i] = __builtin_isfinite(s.main[i]) ? r[i] : s.main[i] + seed[i];
         return r;
     }
 };

@@ -456,11 +456,11 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
             }
             Acc acc[MT];
 #pragma unroll
-            for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finish(sum[t]);
+            for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finish(sum[t], lo.bias[t]);
             if constexpr (F32) {
                 if (any) {
 #pragma unroll
-                    for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finishAny(sum[t]);
+                    for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finishAny(sum[t], lo.bias[t]);
                 }
             }
             if constexpr (Fl::kAnySign) {
@@ -547,9 +547,9 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
 constexpr int kLargeKC = 4;
 constexpr int kLargeLdsBytes = 128 * 1024;
 
-// fp32: fragments as F32Mma's pieces (PIECES), or, where they would not fit (k beyond 1600), as they are in memory and split at
+// fp32: fragments as F32Mma's pieces (PIECES), or, where they would not fit (k beyond 1664), as they are in memory and split at
 // every use; twelve waves share the block of the matrix, and the bias, which four waves keep in registers, lies in LDS.  128x128 over
-// 2^18 samples: 107 us on v_mfma_f32_16x16x4_f32 (four waves, blocks of 128 rows up to k = 256), 123 us splitting at every use, 80 us
+// 2^18 samples: 107 us on v_mfma_f32_16x16x4_f32 (four waves, blocks of 128 rows up to k = 256), 123 us splitting at every use, 77 us
 // here; 256x256 over 2^16: 154, 197, 113 us.
 template <class Fl>
 struct LargeShape {
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
         typename SumOf<Fl>::T sum[MT];
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            if constexpr (F32) sum[t] = SumOf<Fl>::start(*(const floatx4*)(ldsBias + rowBase + 4 * t));
+            if constexpr (F32) sum[t] = SumOf<Fl>::start(Acc{});
             else sum[t] = SumOf<Fl>::start(lo.bias[t]);
         }
         int xSum = 0;
@@ -687,11 +687,13 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
         }
         Acc acc[MT];
 #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finish(sum[t]);
-        if constexpr (F32) {
-            if (any) {
-#pragma unroll
-                for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finishAny(sum[t]);
+        for (int t = 0; t < MT; ++t) {
+            if constexpr (F32) {
+                const floatx4 bias = *(const floatx4*)(ldsBias + rowBase + 4 * t);
+                acc[t] = SumOf<Fl>::finish(sum[t], bias);
+                if (any) acc[t] = SumOf<Fl>::finishAny(sum[t], bias);
+            } else {
+                acc[t] = SumOf<Fl>::finish(sum[t], lo.bias[t]);
             }
         }
         if constexpr (Fl::kAnySign) {

@@ -93,10 +93,10 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
                 }
             }
 #pragma unroll
-            for (int t = t0; t < MT && t < t0 + G; ++t) acc[0][t] = SumOf<Mma>::finish(sum[t - t0]);
-            if (any) {
-#pragma unroll
-                for (int t = t0; t < MT && t < t0 + G; ++t) acc[0][t] = SumOf<Mma>::finishAny(sum[t - t0]);
+            for (int t = t0; t < MT && t < t0 + G; ++t) {
+                const floatx4 bias = acc[0][t];
+                acc[0][t] = SumOf<Mma>::finish(sum[t - t0], bias);
+                if (any) acc[0][t] = SumOf<Mma>::finishAny(sum[t - t0], bias);
             }
         }
     } else

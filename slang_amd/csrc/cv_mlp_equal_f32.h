@@ -7,7 +7,7 @@
 // arm of a switch, whose results meet behind it.  Here the hidden layers are one straight-line body, run once per layer, 16
 // samples to a wave and four waves per SIMD (128 registers), so that one wave's matrix instructions run beside
 // another's conversions.  32-64-64-8 over 2^22 samples: 523 us on v_mfma_f32_16x16x4_f32 in the any-shape kernel, 402 us there with the
-// pieces, 350 us here; 8-64-64-64-64-3 over 2^20: 276, 276, 160 us.
+// pieces, 367 us here; 8-64-64-64-64-3 over 2^20: 276, 276, 161 us.
 #pragma once
 #include "cv_mlp_chain.h"
 
@@ -23,7 +23,7 @@ __device__ __forceinline__ void equalProduct(const uint32_t* wbase, const float*
     for (int t0 = 0; t0 < MT; t0 += G) {
         F32Sum sum[G];
 #pragma unroll
-        for (int t = t0; t < t0 + G; ++t) sum[t - t0] = SumOf<F32Mma>::start(*(const floatx4*)(bbase + 16 * t));
+        for (int t = t0; t < t0 + G; ++t) sum[t - t0] = SumOf<F32Mma>::start(floatx4{});
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
             uint32_t w[G][FD];
@@ -37,10 +37,10 @@ __device__ __forceinline__ void equalProduct(const uint32_t* wbase, const float*
             });
         }
 #pragma unroll
-        for (int t = t0; t < t0 + G; ++t) acc[t] = SumOf<F32Mma>::finish(sum[t - t0]);
-        if (any) {
-#pragma unroll
-            for (int t = t0; t < t0 + G; ++t) acc[t] = SumOf<F32Mma>::finishAny(sum[t - t0]);
+        for (int t = t0; t < t0 + G; ++t) {
+            const floatx4 bias = *(const floatx4*)(bbase + 16 * t);
+            acc[t] = SumOf<F32Mma>::finish(sum[t - t0], bias);
+            if (any) acc[t] = SumOf<F32Mma>::finishAny(sum[t - t0], bias);
         }
     }
 }

@@ -3,9 +3,9 @@
 // (source/standard-modules/neural/layers.slang:34-110) and this library's bfloat16 extension.
 //
 // Every layer is coopVecMatMulAdd + activation in T, exactly as the single-layer kernels of
-// cv_matmul_impl.h evaluate it (fp32 accumulation seeded with the bias, k ascending; T = bfloat16 rounds
-// the sum to bfloat16 before the activation, T = float applies the activation to the sum itself), so the
-// fused network equals the chain of single-layer operators bit for bit.  Layer sizes are run-time values up
+// cv_matmul_impl.h evaluate it (fp32 accumulation, k ascending, seeded with the bias for
+// T = bfloat16, joined by it at the end for T = float; T = bfloat16 rounds the sum to bfloat16 before the
+// activation, T = float applies the activation to the sum itself), so the fused network equals the chain of single-layer operators bit for bit.  Layer sizes are run-time values up
 // to 128; the A fragments of all layers live in LDS.  Activations stay in registers between layers: a
 // layer's accumulators (lane%16 = sample, rows 4t..4t+3 of lane group g) are the next layer's B operand.
 #include <type_traits>
@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
             for (int t = 0; t < kFltMaxTiles; ++t) {
                 acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
                 if (t < MT) {
-                    typename SumOf<Mma>::T sum = SumOf<Mma>::start(*(const floatx4*)(bbase + 16 * t));
+                    const floatx4 bias = *(const floatx4*)(bbase + 16 * t);
+                    typename SumOf<Mma>::T sum = SumOf<Mma>::start(bias);
 #pragma unroll
                     for (int kt = 0; kt < kFltMaxKT; ++kt) {
                         if (kt < KT) {
@@ -152,8 +153,8 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
                             sum = Mma::mma(w, x[kt], sum);
                         }
                     }
-                    acc[t] = SumOf<Mma>::finish(sum);
-                    if (F32 && any) acc[t] = SumOf<Mma>::finishAny(sum);
+                    acc[t] = SumOf<Mma>::finish(sum, bias);
+                    if (F32 && any) acc[t] = SumOf<Mma>::finishAny(sum, bias);
                 }
             }
             // the layer's result in T, activated: what coopVecMatMulAdd + activation returns

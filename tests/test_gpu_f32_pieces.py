@@ -2,8 +2,8 @@
 NaN, the largest and the smallest values, and the kernel for equal hidden layers against the chain of single-layer operators.
 
 Bound of a sum of K terms: an operand is three pieces exactly; of the nine products the three dropped ones are below 2^-26 of the
-term each, the others are exact; of the sums, one rounding to 24 bits per matrix instruction (K/32 of them on the h*h products,
-of which one begins with the bias; the five small ones count below 2^-7 of it) and one at the end."""
+term each, the others are exact; of the sums, one rounding to 24 bits per matrix instruction (K/32 of them on the h*h products;
+the five small ones count below 2^-7 of it) and two at the end, where the bias and the small products join."""
 import numpy as np
 import pytest
 import torch
