@@ -425,7 +425,7 @@ def workload_f32(torch, cv, steps, warmup):
 
     return dict(step=step, samples=B, alg_bytes=B * (dims[0] + dims[-1]) * 4, alg_flops=B * 2 * macs, bound="hbm", mfma="f32",
                 dtype="f32", config={"workload": "f32: fp32 MLP 32->64->64->8, ReLU, fp32 in and out, batch 2^22, fused forward "
-                                                 "(v_mfma_f32_16x16x4_f32)", "batch": B, "layers": dims},
+                                                 "(bfloat16 pieces, v_mfma_f32_16x16x32_bf16)", "batch": B, "layers": dims},
                 cpu_baseline=cpu_baseline, key="f32")
 
 

@@ -1,5 +1,5 @@
 // cv_matmul_f32.hip -- fp32 instantiations of the batched matMul kernel
-// (v_mfma_f32_16x16x4_f32; fp32 vectors, matrix, bias and results).
+// (bfloat16 pieces on v_mfma_f32_16x16x32_bf16, F32Mma; fp32 vectors, matrix, bias and results).
 #include "cv_matmul_impl.h"
 
 namespace cv {
