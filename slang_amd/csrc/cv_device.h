@@ -121,8 +121,10 @@ struct Bf16Mma {
 // stay on the fp32 instruction: 32-64-64-8 over 2^20 samples would take 350 us for 394, with gradients up to 3.5 times as far off.
 // A fragment has the 8 k-slots per lane of the 16-bit flavours, so the InferencingOptimal form of an fp32 matrix is the same
 // arrangement with 4-byte elements; decoded, four dwords each of h, m and l.
-// Infinities and values from 2^127 on: split() makes NaN of them (inf - inf), so a wave that holds one (beyond()) takes
-// splitAny(), which leaves m and l of an infinity zero; then main alone has the sum's infinity or NaN, and finish() keeps it.
+// Operands from 2^32 on, infinities and NaN are not for the pieces: an h rounded up may be infinite, and products that overflow leave
+// main and the small sum infinite with signs of their own.  A wave that holds such an operand (beyond()) evaluates its tiles by
+// F32Careful: rows and samples with such an operand on v_mfma_f32_16x16x4_f32, the others on the pieces as ever, so that no result depends
+// on what its neighbours hold.
 struct F32Sum { floatx4 main, small; };
 struct F32Mma {
     static constexpr const char* kName = "f32";
@@ -148,36 +150,57 @@ struct F32Mma {
         asm("" : "+v"(m));
         l = pack(ra - low(m), rb - high(m));
     }
-    static __device__ __forceinline__ void splitAny(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l)
-    {
-        // (the nearest bfloat16 of a large finite value may be an infinity: the one towards zero is not)
-        auto first = [](float x) { return __builtin_fabsf(x) >= 0x1p127f ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u) : x; };
-        h = pack(first(a), first(b));
-        const float ra = __builtin_isfinite(a) ? a - low(h) : 0.f, rb = __builtin_isfinite(b) ? b - high(h) : 0.f;
-        m = pack(ra, rb);
-        l = pack(ra - low(m), rb - high(m));
-    }
-    template <bool ANY = false>
+    // MARK: values whose pieces do not add up to them are kept as they are, the upper half in h, the lower in m, and all ones in l
+    // (which no conversion gives), for join()
+    template <bool MARK = false>
     static __device__ __forceinline__ void decode(const uint32_t* raw, uint32_t* frag)
     {
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            float a = __builtin_bit_cast(float, raw[2 * d]), b = __builtin_bit_cast(float, raw[2 * d + 1]);
-            if constexpr (ANY) {
-                // (stays in its branch: the compiler would rather compute it on every path)
-                asm volatile("" : "+v"(a), "+v"(b));
-                splitAny(a, b, frag[d], frag[4 + d], frag[8 + d]);
-            } else {
-                split(a, b, frag[d], frag[4 + d], frag[8 + d]);
+            uint32_t pair[2] = {raw[2 * d], raw[2 * d + 1]};
+            // (stays in its branch: the compiler would rather compute it on every path)
+            if constexpr (MARK) asm volatile("" : "+v"(pair[0]), "+v"(pair[1]));
+            split(__builtin_bit_cast(float, pair[0]), __builtin_bit_cast(float, pair[1]), frag[d], frag[4 + d], frag[8 + d]);
+            if constexpr (MARK) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const uint32_t bits = pair[i], keep = i ? 0xffffu : 0xffff0000u;
+                    if (magnitude(bits) < kExactBits) continue;
+                    frag[d] = (frag[d] & keep) | (bits >> 16) << 16 * i;
+                    frag[4 + d] = (frag[4 + d] & keep) | (bits & 0xffffu) << 16 * i;
+                    frag[8 + d] |= ~keep;
+                }
             }
         }
     }
-    // the largest magnitude of n (an even number of) values and `most` (NaN does not count: its pieces need no care).  One
-    // instruction for two values; of fmaxf the compiler makes two for each.  (As relu.)
+    // the eight values of pieces made by decode<true>
+    static __device__ __forceinline__ void join(const uint32_t* frag, uint32_t* raw)
+    {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int d = e / 2;
+            const uint32_t h = e & 1 ? frag[d] >> 16 : frag[d] & 0xffffu, m = e & 1 ? frag[4 + d] >> 16 : frag[4 + d] & 0xffffu,
+                           l = e & 1 ? frag[8 + d] >> 16 : frag[8 + d] & 0xffffu;
+            const float sum = low(h) + low(m) + low(l);
+            raw[e] = l == 0xffffu ? h << 16 | m : __builtin_bit_cast(uint32_t, sum);
+        }
+    }
+    static __device__ __forceinline__ uint32_t magnitude(uint32_t bits) { return bits & 0x7fffffffu; }
+    static constexpr uint32_t kBeyondBits = 0x4f800000u;      // 2^32: beyond()
+    static constexpr uint32_t kExactBits = 0x7f000000u;       // 2^127: below it h is finite, and the pieces add up to the value
+    // the largest magnitude of n (an even number of) values and `most` (NaN does not count: with one, every sum of the sample is NaN).
+    // One instruction for two values; of fmaxf the compiler makes two for each.  (As relu.)
     static __device__ __forceinline__ float largest(const uint32_t* raw, int n, float most)
     {
 #pragma unroll
         for (int d = 0; d < n; d += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(raw[d]), "v"(raw[d + 1]));
+        return most;
+    }
+    // ... of the matrix, as bits.  (A signalling NaN would make v_max3_f32 forget what it had; there other rows may need it.)
+    static __device__ __forceinline__ uint32_t largestBits(const uint32_t* raw, int n, uint32_t most)
+    {
+#pragma unroll
+        for (int d = 0; d < n; ++d) most = max(most, magnitude(raw[d]));
         return most;
     }
     // x > 0 ? x : 0 (NaN: 0) in one instruction.  Not for results of matrix instructions: the compiler does not see that it reads them.
@@ -187,7 +210,7 @@ struct F32Mma {
         asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(x));
         return r;
     }
-    static __device__ __forceinline__ bool beyond(float largest) { return __any(largest >= 0x1p127f); }
+    static __device__ __forceinline__ bool beyond(float largest) { return __any(largest >= 0x1p32f); }
     // the p-th product of pieces (0..4 small ones, 5: h*h)
     template <int P>
     static __device__ __forceinline__ void product(const uint32_t* a, const uint32_t* b, F32Sum& c)
@@ -210,7 +233,6 @@ struct SumOf {
     typedef typename Mma::Acc T;
     static __device__ __forceinline__ T start(typename Mma::Acc seed) { return seed; }
     static __device__ __forceinline__ typename Mma::Acc finish(T s, typename Mma::Acc) { return s; }
-    static __device__ __forceinline__ typename Mma::Acc finishAny(T s, typename Mma::Acc) { return s; }
 };
 template <class Mma>
 struct SumOf<Mma, true> {
@@ -219,13 +241,82 @@ struct SumOf<Mma, true> {
     // products, and of a bias that is the same for every sample it would drop the same ones every time.
     static __device__ __forceinline__ T start(floatx4) { return F32Sum{floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}}; }
     static __device__ __forceinline__ floatx4 finish(T s, floatx4 seed) { return s.main + (s.small + seed); }
-    // ... where some operand was beyond(): an infinity or NaN of the sum stands in `main` alone
-    static __device__ __forceinline__ floatx4 finishAny(T s, floatx4 seed)
+};
+
+// 16 rows times 16 samples where some operand is beyond(): both kinds of sums, and of each result the one that its row and its
+// sample ask for.  Rare, so that it is written for few registers and little code and not for speed.
+struct F32Careful {
+    F32Sum pieces;
+    floatx4 whole;                // seeded with the bias, k ascending
+    uint32_t row, sample;         // largest magnitude (bits) in this lane's share of its row of the matrix, of its vector
+    __device__ __forceinline__ void start(floatx4 seed)
     {
-        asm volatile("" : "+v"(s.main));      // (as in decode)
-        floatx4 r = s.main + (s.small + seed);
+        pieces = SumOf<F32Mma>::start(seed);
+        whole = seed;
+        row = sample = 0u;
+    }
+    // w, x: eight values of the matrix and of the vector each, or (W_PIECES, X_PIECES) their pieces from decode<true>.
+    template <bool W_PIECES, bool X_PIECES>
+    __device__ __forceinline__ void step(const uint32_t* w, const uint32_t* x)
+    {
+        // (the two sums one after the other and the operands made where they are used, not ahead of a loop over tiles: registers)
+        {
+            uint32_t wv[8], xv[8];
+            values<W_PIECES>(w, wv);
+            values<X_PIECES>(x, xv);
+            row = F32Mma::largestBits(wv, 8, row);
+            sample = F32Mma::largestBits(xv, 8, sample);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = __builtin_isfinite(s.main[i]) ? r[i] : s.main[i] + seed[i];
+            for (int s = 0; s < 8; ++s)
+                whole = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, wv[s]), __builtin_bit_cast(float, xv[s]), whole, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        {
+            uint32_t wp[F32Mma::kFD], xp[F32Mma::kFD];
+            piecesOf<W_PIECES>(w, wp);
+            piecesOf<X_PIECES>(x, xp);
+            pieces = F32Mma::mma(wp, xp, pieces);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    template <int N>
+    static __device__ __forceinline__ void here(const uint32_t* from, uint32_t (&to)[N])
+    {
+#pragma unroll
+        for (int d = 0; d < N; ++d) { to[d] = from[d]; asm volatile("" : "+v"(to[d])); }
+    }
+    template <bool PIECES>
+    static __device__ __forceinline__ void values(const uint32_t* from, uint32_t (&v)[8])
+    {
+        if constexpr (PIECES) {
+            uint32_t p[F32Mma::kFD];
+            here(from, p);
+            F32Mma::join(p, v);
+        } else {
+            here(from, v);
+        }
+    }
+    template <bool PIECES>
+    static __device__ __forceinline__ void piecesOf(const uint32_t* from, uint32_t (&p)[F32Mma::kFD])
+    {
+        if constexpr (PIECES) {
+#pragma unroll
+            for (int d = 0; d < F32Mma::kFD; ++d) p[d] = from[d];
+        } else {
+            uint32_t v[8];
+            here(from, v);
+            F32Mma::decode(v, p);
+        }
+    }
+    __device__ __forceinline__ floatx4 finish(floatx4 seed) const
+    {
+        // bit i: row i of the tile, sample i of the tile (lanes i, i + 16, i + 32 and i + 48 hold a share each)
+        auto fold = [](uint64_t b) { const uint32_t v = (uint32_t)b | (uint32_t)(b >> 32); return v | v >> 16; };
+        const uint32_t rows = fold(__ballot(row >= F32Mma::kBeyondBits)), samples = fold(__ballot(sample >= F32Mma::kBeyondBits));
+        const uint32_t lane = __lane_id(), g = lane >> 4, n = lane & 15u;
+        floatx4 r = SumOf<F32Mma>::finish(pieces, seed);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = ((rows >> (4 * g + i) | samples >> n) & 1u) ? whole[i] : r[i];
         return r;
     }
 };

@@ -282,8 +282,9 @@ __device__ __forceinline__ void addUnsignedRowTerm(LaneOut<Fl, MT>& lo, int (&ro
 
 // LINES (streaming kernel only): the vectors on both sides are whole, aligned 128-byte lines, which the
 // kernel then reads and writes with non-temporal accesses.
+// (fp32: two waves per SIMD, of which F32Careful would take one)
 template <class Fl, int MT, int KT, int NT, typename OutT, bool FAST, bool LINES = false>
-__global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
+__global__ __launch_bounds__(256, Fl::kEsz == 4 ? 2 : 1) void matmulKernel(const MatMulArgs a)
 {
     constexpr int EPL = Fl::kEpl, FD = Fl::kFD, ESZ = Fl::kEsz, RAW = Fl::kRawDW;
     constexpr int IESZ = Fl::kInEsz, IRAW = Fl::kInRawDW;
@@ -373,8 +374,8 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
 
     bool matBeyond = false;                   // F32Mma::beyond of the matrix
     if constexpr (F32) {
-        const float most = stageFragmentPieces(ldsW, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff, 0.f);
-        matBeyond = __syncthreads_or(most >= 0x1p127f);
+        const uint32_t most = stageFragmentPieces(ldsW, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff, 0u);
+        matBeyond = __syncthreads_or(most >= Fl::kBeyondBits);
     } else {
         stageFragments<ESZ, EPL>(ldsW, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k,
                                  a.rowOff, (Fl::kAnySign && a.matUnsigned) ? 0x80u : 0u);
@@ -382,18 +383,21 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
     }
 
     uint32_t afrag[MT][KT][FD];
+    auto readMatrix = [&]() {
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+        for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-            const uint32_t* raw = &ldsW[((t * KT + kt) * 64 + lane) * LANE_DW];
-            if constexpr (F32) {
+            for (int kt = 0; kt < KT; ++kt) {
+                const uint32_t* raw = &ldsW[((t * KT + kt) * 64 + lane) * LANE_DW];
+                if constexpr (F32) {
 #pragma unroll
-                for (int d = 0; d < FD; ++d) afrag[t][kt][d] = raw[d];
-            } else {
-                Fl::decode(raw, afrag[t][kt]);
+                    for (int d = 0; d < FD; ++d) afrag[t][kt][d] = raw[d];
+                } else {
+                    Fl::decode(raw, afrag[t][kt]);
+                }
             }
-        }
+    };
+    readMatrix();
 
     if constexpr (Fl::kAnySign) {
         if (a.inUnsigned) {
@@ -445,9 +449,6 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
                         if (a.matUnsigned) xSum += sumSignedBytes(x[d]);
                     }
                     Fl::decodeIn(x, bfrag);
-                } else if constexpr (F32) {
-                    Fl::decode(&buf[kt * IRAW], bfrag);
-                    if (any) Fl::template decode<true>(&buf[kt * IRAW], bfrag);
                 } else {
                     Fl::decodeIn(&buf[kt * IRAW], bfrag);
                 }
@@ -459,8 +460,24 @@ __global__ __launch_bounds__(256) void matmulKernel(const MatMulArgs a)
             for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finish(sum[t], lo.bias[t]);
             if constexpr (F32) {
                 if (any) {
+                    // (registers: the general kernel reads the vectors again, both the matrix afterwards)
+                    uint32_t x[SLOT_DW];
+                    if constexpr (!FAST) {
+                        loadSlots<SLOT_DW>(x, inLane + (size_t)min(t0 * TILE + 16 * j + n, lastSample) * a.inStride, validBytes, loadMode);
+                    } else {
 #pragma unroll
-                    for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finishAny(sum[t], lo.bias[t]);
+                        for (int d = 0; d < SLOT_DW; ++d) x[d] = buf[d];
+                    }
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) {
+                        F32Careful c;
+                        c.start(lo.bias[t]);
+#pragma unroll
+                        for (int kt = 0; kt < KT; ++kt) c.template step<true, false>(&ldsW[((t * KT + kt) * 64 + lane) * LANE_DW], &x[kt * IRAW]);
+                        acc[t] = c.finish(lo.bias[t]);
+                    }
+                    asm volatile("" ::: "memory");
+                    readMatrix();
                 }
             }
             if constexpr (Fl::kAnySign) {
@@ -573,17 +590,17 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
     const uint32_t gs = optGS((uint32_t)a.k);
     bool matBeyond = false;                    // F32Mma::beyond of the matrix
     if constexpr (F32) {
-        float most = 0.f;
+        uint32_t most = 0u;
         if constexpr (PIECES) {
             most = stageFragmentPieces(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff, most);
         } else {
             stageFragments<ESZ, EPL>(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff);
             __syncthreads();
-            for (int i = threadIdx.x; i < MT * KT * 64; i += 64 * WAVES) most = Fl::largest(ldsDyn + (size_t)i * RAW, RAW, most);
+            for (int i = threadIdx.x; i < MT * KT * 64; i += 64 * WAVES) most = Fl::largestBits(ldsDyn + (size_t)i * RAW, RAW, most);
         }
         for (int row = threadIdx.x; row < 16 * MT; row += 64 * WAVES)
             ldsBias[row] = (a.bias && row < a.m) ? loadAsFloat(a.bias + (size_t)row * elemSize(a.biasCt), a.biasCt) : 0.f;
-        matBeyond = __syncthreads_or(most >= 0x1p127f);
+        matBeyond = __syncthreads_or(most >= Fl::kBeyondBits);
     } else {
         stageFragments<ESZ, EPL>(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k,
                                  a.rowOff, (Fl::kAnySign && a.matUnsigned) ? 0x80u : 0u);
@@ -626,13 +643,17 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
             else sum[t] = SumOf<Fl>::start(lo.bias[t]);
         }
         int xSum = 0;
-        bool any = matBeyond;
-        for (int kc = 0; kc < KT; kc += KC) {
+        float most = 0.f;
+        auto load = [&](int kc, uint32_t (&x)[STEP_DW], int& vb) {
             const int off = kc * IRAW * 4;                         // byte offset of this step in the lane's slice
-            const int vb = min(max(validBytes - off, 0), STEP_DW * 4);
+            vb = min(max(validBytes - off, 0), STEP_DW * 4);
             const int mode = (vb == STEP_DW * 4 && a.inAlign >= 16u && ((colBase * IESZ) & 15) == 0) ? 0 : ((vb & 3) == 0 && a.inAlign >= 4u) ? 1 : 2;
-            uint32_t x[STEP_DW];
             loadSlots<STEP_DW>(x, p + off, vb, mode);
+        };
+        for (int kc = 0; kc < KT; kc += KC) {
+            int vb;
+            uint32_t x[STEP_DW];
+            load(kc, x, vb);
             if constexpr (Fl::kAnySign) {
 #pragma unroll
                 for (int d = 0; d < STEP_DW; ++d) {
@@ -640,14 +661,11 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
                     if (a.matUnsigned) xSum += sumSignedBytes(x[d]);
                 }
             }
-            if constexpr (F32) any = any | Fl::beyond(Fl::largest(x, STEP_DW, 0.f));
+            if constexpr (F32) most = Fl::largest(x, STEP_DW, most);
 #pragma unroll
             for (int j = 0; j < KC; ++j) {
                 uint32_t bfrag[FD];
                 Fl::decodeIn(&x[j * IRAW], bfrag);
-                if constexpr (F32) {
-                    if (any) Fl::template decode<true>(&x[j * IRAW], bfrag);
-                }
                 // (fp32: two row tiles together, product by product, so that no matrix instruction waits for the one before it)
                 constexpr int G = F32 && MT > 1 ? 2 : 1;
 #pragma unroll
@@ -661,9 +679,6 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
                             for (int d = 0; d < FD; ++d) af[t - t0][d] = raw[d];
                         } else {
                             Fl::decode(raw, af[t - t0]);
-                            if constexpr (F32) {
-                                if (matBeyond) Fl::template decode<true>(raw, af[t - t0]);
-                            }
                         }
                     }
                     if constexpr (F32) {
@@ -691,9 +706,29 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
             if constexpr (F32) {
                 const floatx4 bias = *(const floatx4*)(ldsBias + rowBase + 4 * t);
                 acc[t] = SumOf<Fl>::finish(sum[t], bias);
-                if (any) acc[t] = SumOf<Fl>::finishAny(sum[t], bias);
             } else {
                 acc[t] = SumOf<Fl>::finish(sum[t], lo.bias[t]);
+            }
+        }
+        if constexpr (F32) {
+            if (matBeyond | Fl::beyond(most)) {
+#pragma unroll 1
+                for (int t = 0; t < MT; ++t) {
+                    const floatx4 bias = *(const floatx4*)(ldsBias + rowBase + 4 * t);
+                    F32Careful c;
+                    c.start(bias);
+#pragma unroll 1
+                    for (int kc = 0; kc < KT; kc += KC) {
+                        int vb;
+                        uint32_t x[STEP_DW];
+                        load(kc, x, vb);
+#pragma unroll
+                        for (int j = 0; j < KC; ++j) c.template step<PIECES, false>(&ldsDyn[((t * KT + kc + j) * 64 + lane) * LANE_DW], &x[j * IRAW]);
+                    }
+                    const floatx4 r = c.finish(bias);
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) acc[i] = t == i ? r : acc[i];
+                }
             }
         }
         if constexpr (Fl::kAnySign) {

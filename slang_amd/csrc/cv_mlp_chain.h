@@ -43,6 +43,26 @@ __device__ __forceinline__ float chainActivateF32(float x, float slope)
     return x;
 }
 
+// One layer of float where some operand is beyond() (F32Careful); `act` holds pieces from decode<true>.
+template <int MT, int KTS, bool PIECES>
+__device__ __forceinline__ void carefulProduct(const uint32_t* wbase, const float* bbase, int KT, const uint32_t (&act)[KTS][F32Mma::kFD], floatx4 (&acc)[MT])
+{
+    constexpr int LANE_DW = PIECES ? F32Mma::kFD : F32Mma::kRawDW;
+#pragma unroll 1
+    for (int t = 0; t < MT; ++t) {
+        const floatx4 bias = *(const floatx4*)(bbase + 16 * t);
+        F32Careful c;
+        c.start(bias);
+#pragma unroll
+        for (int kt = 0; kt < KTS; ++kt) {
+            if (kt == 0 || kt < KT) c.template step<PIECES, true>(wbase + (size_t)(t * KT + kt) * 64 * LANE_DW, act[kt]);
+        }
+        const floatx4 r = c.finish(bias);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i] = t == i ? r : acc[i];
+    }
+}
+
 // One layer of MT row tiles for NT sample tiles: `act` holds its B operands and receives the next layer's, or, for the
 // last layer, the results are stored.
 // PIECES (T = float): fragments lie in LDS as F32Mma's pieces; else as they lie in memory, split at every use.
@@ -63,7 +83,6 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
     }
     if constexpr (F32) {
         // Fragments of G row tiles together and product by product, so that no matrix instruction waits for the one before it.
-        // Operands beyond() are put right in branches that hardly ever run, so that the rest is straight-line code.
         static_assert(NT == 1, "one tile: two leave a SIMD fewer than two waves for their registers");
         constexpr int G = MT < 2 ? 1 : 2;
 #pragma unroll
@@ -83,7 +102,6 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
                             for (int d = 0; d < FD; ++d) w[t - t0][d] = raw[d];
                         } else {
                             Mma::decode(raw, w[t - t0]);
-                            if (matBeyond) Mma::template decode<true>(raw, w[t - t0]);
                         }
                     }
                     staticFor<0, 6>([&](auto pc) {
@@ -93,12 +111,9 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
                 }
             }
 #pragma unroll
-            for (int t = t0; t < MT && t < t0 + G; ++t) {
-                const floatx4 bias = acc[0][t];
-                acc[0][t] = SumOf<Mma>::finish(sum[t - t0], bias);
-                if (any) acc[0][t] = SumOf<Mma>::finishAny(sum[t - t0], bias);
-            }
+            for (int t = t0; t < MT && t < t0 + G; ++t) acc[0][t] = SumOf<Mma>::finish(sum[t - t0], acc[0][t]);
         }
+        if (any) carefulProduct<MT, MAXKT, PIECES>(wbase, bbase, KT, act[0], acc[0]);      // (hardly ever: the rest stays straight-line code)
     } else
 #pragma unroll
     for (int kt = 0; kt < MAXKT; ++kt) {
@@ -252,7 +267,7 @@ __global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void
     float* ldsB = (float*)(lds + ga.biasDwordBase);
     constexpr bool F32 = std::is_same<Mma, F32Mma>::value;
     constexpr int LANE_DW = PIECES ? FD : RAW;             // dwords per lane of a fragment in LDS
-    float most = 0.f;
+    uint32_t most = 0u;
     for (int l = 0; l < a.numLayers; ++l) {
         const MlpLayerArgs& ly = a.layers[l];
         const int MT = ga.gl[l].mt, KT = ga.gl[l].kt;
@@ -268,8 +283,8 @@ __global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void
     bool matBeyond = false;
     if constexpr (F32) {
         if constexpr (!PIECES)
-            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += 256) most = Mma::largest(lds + (size_t)i * RAW, RAW, most);
-        matBeyond = __syncthreads_or(most >= 0x1p127f);
+            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += 256) most = Mma::largestBits(lds + (size_t)i * RAW, RAW, most);
+        matBeyond = __syncthreads_or(most >= Mma::kBeyondBits);
     }
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

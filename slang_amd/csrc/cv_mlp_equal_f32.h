@@ -40,9 +40,9 @@ __device__ __forceinline__ void equalProduct(const uint32_t* wbase, const float*
         for (int t = t0; t < t0 + G; ++t) {
             const floatx4 bias = *(const floatx4*)(bbase + 16 * t);
             acc[t] = SumOf<F32Mma>::finish(sum[t - t0], bias);
-            if (any) acc[t] = SumOf<F32Mma>::finishAny(sum[t - t0], bias);
         }
     }
+    if (any) carefulProduct<MT, KT, true>(wbase, bbase, KT, act, acc);      // (hardly ever: the rest stays straight-line code)
 }
 
 template <int MT>
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256 * equalWaves(HT), equalWaves(HT)) void mlpChain
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     float* ldsB = (float*)(lds + ga.biasDwordBase);
     const int L = a.numLayers;
-    float most = 0.f;
+    uint32_t most = 0u;
     for (int l = 0; l < L; ++l) {
         const MlpLayerArgs& ly = a.layers[l];
         const int MT = ga.gl[l].mt, KT = ga.gl[l].kt;
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256 * equalWaves(HT), equalWaves(HT)) void mlpChain
             ldsB[ga.gl[l].biasBase + e] = (ly.bias && row < ly.out) ? ((const float*)ly.bias)[row] : 0.f;
         }
     }
-    const bool matBeyond = __syncthreads_or(most >= 0x1p127f);
+    const bool matBeyond = __syncthreads_or(most >= F32Mma::kBeyondBits);
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int g = lane >> 4, n = lane & 15;

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     float* ldsB = (float*)(lds + ga.biasDwordBase);
 
-    float most = 0.f;
+    uint32_t most = 0u;
     for (int l = 0; l < L; ++l) {
         const MlpLayerArgs& ly = a.layers[l];
         const int MT = ga.gl[l].mt, KT = ga.gl[l].kt, ROWS = 4 * MT;
@@ -71,8 +71,8 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
     bool matBeyond = false;                  // F32Mma::beyond of some layer's matrix
     if constexpr (F32) {
         if constexpr (!PIECES)
-            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += 256) most = Mma::largest(lds + (size_t)i * RAW, RAW, most);
-        matBeyond = __syncthreads_or(most >= 0x1p127f);
+            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += 256) most = Mma::largestBits(lds + (size_t)i * RAW, RAW, most);
+        matBeyond = __syncthreads_or(most >= Mma::kBeyondBits);
     }
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -125,9 +125,6 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
 #pragma unroll
             for (int kt = 0; kt < kFltMaxKT; ++kt) {
                 Mma::decode(act[kt], x[kt]);
-                if constexpr (F32) {
-                    if (any) Mma::template decode<true>(act[kt], x[kt]);
-                }
             }
             floatx4 acc[kFltMaxTiles];
 #pragma unroll
@@ -146,15 +143,27 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
                                 for (int d = 0; d < FD; ++d) w[d] = raw[d];
                             } else {
                                 Mma::decode(raw, w);
-                                if constexpr (F32) {
-                                    if (matBeyond) Mma::template decode<true>(raw, w);
-                                }
                             }
                             sum = Mma::mma(w, x[kt], sum);
                         }
                     }
                     acc[t] = SumOf<Mma>::finish(sum, bias);
-                    if (F32 && any) acc[t] = SumOf<Mma>::finishAny(sum, bias);
+                }
+            }
+            if constexpr (F32) {
+                if (any) {
+#pragma unroll 1
+                    for (int t = 0; t < MT; ++t) {
+                        const floatx4 bias = *(const floatx4*)(bbase + 16 * t);
+                        F32Careful c;
+                        c.start(bias);
+#pragma unroll
+                        for (int kt = 0; kt < kFltMaxKT; ++kt)
+                            if (kt < KT) c.template step<PIECES, false>(wbase + (size_t)(t * KT + kt) * 64 * LANE_DW, act[kt]);
+                        const floatx4 r = c.finish(bias);
+#pragma unroll
+                        for (int i = 0; i < kFltMaxTiles; ++i) acc[i] = t == i ? r : acc[i];
+                    }
                 }
             }
             // the layer's result in T, activated: what coopVecMatMulAdd + activation returns

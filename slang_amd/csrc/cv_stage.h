@@ -150,19 +150,21 @@ __device__ __forceinline__ void stageFragments(uint32_t* ldsDst, const uint8_t* 
     }
 }
 
-// An fp32 matrix as the three bfloat16 pieces of F32Mma: 12 dwords per lane and fragment.  Returns the largest magnitude of
+// An fp32 matrix as the three bfloat16 pieces of F32Mma: 12 dwords per lane and fragment.  Returns the largest magnitude (bits) of
 // `most` and what the thread met.
-__device__ __forceinline__ float stageFragmentPieces(uint32_t* ldsDst, const uint8_t* w, const MatrixShape& shape, bool transposed, int MT, int KT,
-                                                     uint32_t gs, uint32_t rows, uint32_t cols, uint32_t rowOff, float most)
+__device__ __forceinline__ uint32_t stageFragmentPieces(uint32_t* ldsDst, const uint8_t* w, const MatrixShape& shape, bool transposed, int MT, int KT,
+                                                        uint32_t gs, uint32_t rows, uint32_t cols, uint32_t rowOff, uint32_t most)
 {
     const int chunks = MT * KT * 64;
     const bool direct = fragmentSourceIsDirect<4, 8>(shape, transposed, MT, KT, gs, rows, cols, rowOff, 0);
     for (int c = (int)threadIdx.x; c < chunks; c += blockDim.x) {
         uint32_t v[8], p[F32Mma::kFD];
         fetchFragmentChunk<4, 8>(v, w, shape, transposed, direct, MT, KT, gs, rows, cols, rowOff, 0, c);
-        most = F32Mma::largest(v, 8, most);
-        F32Mma::decode<true>(v, p);
+        const uint32_t own = F32Mma::largestBits(v, 8, 0u);
+        F32Mma::decode(v, p);
+        if (own >= F32Mma::kExactBits) F32Mma::decode<true>(v, p);
         storeFragmentChunk<F32Mma::kFD>(ldsDst + (size_t)c * F32Mma::kFD, p);
+        most = max(most, own);
     }
     return most;
 }

@@ -15,10 +15,10 @@ from slang_amd.coopvec import Activation, CoopVecComponentType as CT, CoopVecMat
 pytestmark = pytest.mark.gpu
 
 
-def matmul(x, W, b):
+def matmul(x, W, b, act=Activation.NoActivation):
     M, K = W.shape
     return cv.coopVecMatMulAdd(to_dev(x), CT.Float32, as_bytes(to_dev(W)), 0, CT.Float32, as_bytes(to_dev(b)), 0, CT.Float32,
-                               ML.RowMajor, False, 4 * K, M=M, resultType=CT.Float32).cpu().numpy()
+                               ML.RowMajor, False, 4 * K, M=M, resultType=CT.Float32, activation=act).cpu().numpy()
 
 
 def bound(x, W, b):
@@ -76,6 +76,72 @@ def test_values_at_the_ends_of_the_range(M, K):
     ref = want(y[special], V)
     ok = np.isfinite(ref) & (np.abs(ref) < 1e38)
     assert np.array_equal(np.isnan(got[special]), np.isnan(ref)) and np.array_equal(np.isinf(got[special]) & ~ok, np.isinf(ref) & ~ok)
+
+
+def large(rng, *shape):
+    return (10.0 ** rng.uniform(22, 30, shape) * rng.choice([-1.0, 1.0], shape)).astype(np.float32)
+
+
+# (64 x 64: the streaming kernel, 37 samples beyond its whole tiles on the general one; then LDS, as pieces and split at each use)
+@pytest.mark.parametrize("M,K", [(64, 64), (24, 40), (100, 96), (8, 1700)])
+def test_products_of_finite_operands_that_overflow(M, K):
+    rng = np.random.default_rng(M * 7 + K)
+    B = 293
+    x, W, b = rng.standard_normal((B, K)).astype(np.float32), rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal(M).astype(np.float32)
+    rows, samples = rng.permutation(M)[: M // 2], rng.permutation(B)[:40]
+    V = W.copy()
+    V[rows, 3] = large(rng, len(rows))
+    plain = matmul(x, V, b)
+    y = x.copy()
+    y[samples, 3] = large(rng, 40)
+    ref = y.astype(np.float64) @ V.astype(np.float64).T + b
+    over = np.abs(ref) > 3.5e38
+    assert over[np.ix_(samples, rows)].all()
+    got = matmul(y, V, b)
+    assert np.array_equal(got[over], np.where(ref[over] > 0, np.inf, -np.inf).astype(np.float32))
+    assert (np.abs(got - ref)[~over] <= bound(y, V, b)[~over]).all()
+    others = np.setdiff1d(np.arange(B), samples)
+    assert np.array_equal(got[others].view(np.uint32), plain[others].view(np.uint32))
+    # what other samples hold, infinities too, changes nothing
+    z = y.copy()
+    z[others[::5], 1] = np.inf
+    keep = np.setdiff1d(np.arange(B), others[::5])
+    assert np.array_equal(matmul(z, V, b)[keep].view(np.uint32), got[keep].view(np.uint32))
+    # every element of a vector and of a row
+    y[samples], V[rows] = np.abs(large(rng, 40, K)), np.abs(large(rng, len(rows), K))
+    got = matmul(y, V, b, Activation.ReLU)
+    assert (got[np.ix_(samples, rows)] == np.inf).all()
+    assert np.array_equal(matmul(y, -V, b, Activation.ReLU)[np.ix_(samples, rows)], np.zeros((40, len(rows)), np.float32))
+
+
+# the kernels for equal hidden layers, for any, and with a smooth activation
+@pytest.mark.parametrize("dims,last", [([32, 64, 64, 8], Activation.ReLU), ([8, 128, 128, 3], Activation.NoActivation), ([20, 48, 24, 5], Activation.ReLU),
+                                       ([64, 112, 96, 12], Activation.NoActivation), ([16, 112, 112, 112, 8], Activation.ReLU), ([20, 48, 24, 5], Activation.Sigmoid)])
+def test_networks_whose_hidden_layers_overflow(dims, last):
+    rng = np.random.default_rng(sum(dims))
+    acts = [Activation.ReLU] * (len(dims) - 2) + [last]
+    layers, params = network(rng, dims, acts)
+    for fi, fo, wd, bd, act in params:
+        wd.view(torch.float32).abs_()
+    B = 20000
+    x = rng.uniform(0.1, 1, (B, dims[0])).astype(np.float32)
+    x[::33] *= np.float32(1e30)
+    x[5::66] *= np.float32(1e20)
+    params[1][2].view(torch.float32)[:dims[1]] *= 1e25                 # the first unit of the second layer
+    x = to_dev(x)
+    y = cv.mlpForward(layers, x, weightType=CT.Float32)
+    ref = chain(params, x)
+    assert torch.equal(y.view(torch.int32), ref.view(torch.int32)), cv.lastKernelName()
+    want = x.double()
+    for fi, fo, wd, bd, act in params[:-1]:
+        want = torch.relu(want @ wd.view(torch.float32).view(fo, fi).double().T + bd.view(torch.float32).double()).float().double()
+    fi, fo, wd, bd, act = params[-1]
+    want = (want @ wd.view(torch.float32).view(fo, fi).double().T + bd.view(torch.float32).double()).float()
+    want = torch.sigmoid(want) if last == Activation.Sigmoid else torch.relu(want) if last == Activation.ReLU else want
+    assert not torch.isnan(y).any()
+    if last != Activation.Sigmoid:
+        assert torch.equal(torch.isinf(y), torch.isinf(want)) and torch.isinf(y).any(dim=1).sum() >= B // 33
+    assert torch.allclose(y.nan_to_num(posinf=0.0), want.nan_to_num(posinf=0.0), rtol=1e-5, atol=1e-5)
 
 
 def network(rng, dims, acts):
