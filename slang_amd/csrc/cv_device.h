@@ -109,9 +109,11 @@ struct Bf16Mma {
     }
 };
 
-// fp32 operands on the bfloat16 matrix pipeline: every operand is the sum of three bfloat16 pieces (h the nearest to it, m the
-// nearest to the rest, l what is left: 24 bits, exactly), and of the nine products of pieces the six that matter are summed, the
-// h*h products by themselves (F32Sum::main) and the five small ones by themselves, added at the end with the bias.
+// fp32 operands on the bfloat16 matrix pipeline: every operand, times 2^24, is the sum of three bfloat16 pieces (h the nearest to it, m
+// the nearest to the rest, l what is left: 24 bits, exactly), and of the nine products of pieces the six that matter are summed, the
+// h*h products by themselves (F32Sum::main) and the five small ones by themselves, added at the end with the bias.  The scale keeps
+// the last bit of every fp32 number, subnormal ones included, above bfloat16's smallest normal one: unscaled, l would lose bits from 2^-110
+// on downwards (at 2^-124 a thousandth of the value).
 // Six v_mfma_f32_16x16x32_bf16 take 96 cycles of the matrix pipeline where eight v_mfma_f32_16x16x4_f32, which round every
 // product's sum to 24 bits, take 256, and the sums are closer to the exact ones (random operands, error over the norm against 64
 // bits, 32 / 64 / 128 terms: 3.9 / 5.0 / 6.5e-8 against 10.3 / 14.4 / 20.4e-8 on the fp32 instruction; the dropped products are
@@ -122,7 +124,7 @@ struct Bf16Mma {
 // A fragment has the 8 k-slots per lane of the 16-bit flavours, so the InferencingOptimal form of an fp32 matrix is the same
 // arrangement with 4-byte elements; decoded, four dwords each of h, m and l.
 // Operands from 2^32 on, infinities and NaN are not for the pieces: an h rounded up may be infinite, and products that overflow leave
-// main and the small sum infinite with signs of their own.  A wave that holds such an operand (beyond()) evaluates its tiles by
+// main and the small sum infinite with signs of their own.  (Below 2^32, sums of up to 2048 scaled products stay below 2^123.)  A wave that holds such an operand (beyond()) evaluates its tiles by
 // F32Careful: rows and samples with such an operand on v_mfma_f32_16x16x4_f32, the others on the pieces as ever, so that no result depends
 // on what its neighbours hold.
 struct F32Sum { floatx4 main, small; };
@@ -142,7 +144,7 @@ struct F32Mma {
     }
     static __device__ __forceinline__ void split(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l)
     {
-        // (11 instructions for two values; pinned, since the compiler would convert each value again to subtract it)
+        // (11 instructions for two values and two to scale them; pinned, since the compiler would convert each value again to subtract it)
         h = pack(a, b);
         asm("" : "+v"(h));
         const float ra = a - low(h), rb = b - high(h);
@@ -160,7 +162,7 @@ struct F32Mma {
             uint32_t pair[2] = {raw[2 * d], raw[2 * d + 1]};
             // (stays in its branch: the compiler would rather compute it on every path)
             if constexpr (MARK) asm volatile("" : "+v"(pair[0]), "+v"(pair[1]));
-            split(__builtin_bit_cast(float, pair[0]), __builtin_bit_cast(float, pair[1]), frag[d], frag[4 + d], frag[8 + d]);
+            split(__builtin_bit_cast(float, pair[0]) * kUp, __builtin_bit_cast(float, pair[1]) * kUp, frag[d], frag[4 + d], frag[8 + d]);
             if constexpr (MARK) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
@@ -181,13 +183,14 @@ struct F32Mma {
             const int d = e / 2;
             const uint32_t h = e & 1 ? frag[d] >> 16 : frag[d] & 0xffffu, m = e & 1 ? frag[4 + d] >> 16 : frag[4 + d] & 0xffffu,
                            l = e & 1 ? frag[8 + d] >> 16 : frag[8 + d] & 0xffffu;
-            const float sum = low(h) + low(m) + low(l);
+            const float sum = (low(h) + low(m) + low(l)) * (1.f / kUp);
             raw[e] = l == 0xffffu ? h << 16 | m : __builtin_bit_cast(uint32_t, sum);
         }
     }
     static __device__ __forceinline__ uint32_t magnitude(uint32_t bits) { return bits & 0x7fffffffu; }
+    static constexpr float kUp = 0x1p24f, kDown = 0x1p-48f;   // scale of the operands; back, of sums of products
     static constexpr uint32_t kBeyondBits = 0x4f800000u;      // 2^32: beyond()
-    static constexpr uint32_t kExactBits = 0x7f000000u;       // 2^127: below it h is finite, and the pieces add up to the value
+    static constexpr uint32_t kExactBits = 0x73000000u;       // 2^103: below it h is finite, and the pieces add up to the value
     // the largest magnitude of n (an even number of) values and `most` (NaN does not count: with one, every sum of the sample is NaN).
     // One instruction for two values; of fmaxf the compiler makes two for each.  (As relu.)
     static __device__ __forceinline__ float largest(const uint32_t* raw, int n, float most)
@@ -240,7 +243,13 @@ struct SumOf<Mma, true> {
     // The seed (the bias) joins at the end: a matrix instruction drops the bits of its C operand that lie below what it keeps of the
     // products, and of a bias that is the same for every sample it would drop the same ones every time.
     static __device__ __forceinline__ T start(floatx4) { return F32Sum{floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}}; }
-    static __device__ __forceinline__ floatx4 finish(T s, floatx4 seed) { return s.main + (s.small + seed); }
+    static __device__ __forceinline__ floatx4 finish(T s, floatx4 seed)
+    {
+        floatx4 r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = __builtin_fmaf(s.main[i], F32Mma::kDown, __builtin_fmaf(s.small[i], F32Mma::kDown, seed[i]));
+        return r;
+    }
 };
 
 // 16 rows times 16 samples where some operand is beyond(): both kinds of sums, and of each result the one that its row and its

@@ -1,7 +1,7 @@
 """fp32 matrix products as sums of bfloat16 pieces (F32Mma, slang_amd/csrc/cv_device.h): accuracy against 64 bits, infinities,
 NaN, the largest and the smallest values, and the kernel for equal hidden layers against the chain of single-layer operators.
 
-Bound of a sum of K terms: an operand is three pieces exactly; of the nine products the three dropped ones are below 2^-26 of the
+Bound of a sum of K terms: an operand (times 2^24) is three pieces exactly; of the nine products the three dropped ones are below 2^-26 of the
 term each, the others are exact; of the sums, one rounding to 24 bits per matrix instruction (K/32 of them on the h*h products;
 the five small ones count below 2^-7 of it) and two at the end, where the bias and the small products join."""
 import numpy as np
@@ -66,6 +66,8 @@ def test_values_at_the_ends_of_the_range(M, K):
     ref = y[[60, 100]].astype(np.float64) @ W.astype(np.float64).T + b
     fits = np.abs(ref) < 1e38
     assert (np.abs(got[[60, 100]] - ref)[fits] <= bound(y[[60, 100]], W, b)[fits]).all() and fits[1].all()
+    ref = y[[100]].astype(np.float64) @ W.astype(np.float64).T      # ... of which the bias hides everything
+    assert (np.abs(matmul(y[[100]], W, 0 * b) - ref) <= bound(y[[100]], W, 0 * b) + 2.0 ** -149).all()
     # an infinite element of the matrix: its row alone
     got = matmul(x, V, b)
     ref = want(x, V)
@@ -112,6 +114,59 @@ def test_products_of_finite_operands_that_overflow(M, K):
     got = matmul(y, V, b, Activation.ReLU)
     assert (got[np.ix_(samples, rows)] == np.inf).all()
     assert np.array_equal(matmul(y, -V, b, Activation.ReLU)[np.ix_(samples, rows)], np.zeros((40, len(rows)), np.float32))
+
+
+def same_as(got, ref):
+    # bit for bit; a subnormal result, which is the sum of two values rounded to multiples of 2^-149, within one of these
+    return (np.abs(got - ref) <= np.where(np.abs(ref) < 2.0 ** -126, 2.0 ** -149, 0.0)).all()
+
+
+@pytest.mark.parametrize("M,K", [(64, 64), (24, 40), (100, 96), (8, 1700)])
+def test_small_operands(M, K):
+    # one element of every row: the products are exact
+    rng = np.random.default_rng(M * 11 + K)
+    B = 160
+    zero = np.zeros(M, np.float32)
+    pick = rng.integers(0, K, M)
+    for e in (-60, -100, -110, -118, -124, -126, -135, -147):
+        x = np.ldexp(rng.uniform(1, 2, (B, K)), e).astype(np.float32)
+        for s in (0, 31, -20, 100):
+            W = np.zeros((M, K), np.float32)
+            W[np.arange(M), pick] = 2.0 ** s
+            assert same_as(matmul(x, W, zero).astype(np.float64), x[:, pick].astype(np.float64) * 2.0 ** s), (e, s)
+            y = np.zeros((B, K), np.float32)                          # ... the small ones in the matrix
+            y[np.arange(B), np.arange(B) % K] = 2.0 ** s
+            assert same_as(matmul(y, x[:M], zero).astype(np.float64), x[:M, np.arange(B) % K].T.astype(np.float64) * 2.0 ** s), (e, s)
+    # full rows, of every size within 2^24: the bound of the products alone
+    for s in (0, 20, 100):
+        x = (rng.standard_normal((B, K)) * np.exp2(rng.integers(-136, -111, (B, K)))).astype(np.float32)
+        W = (rng.standard_normal((M, K)) * np.exp2(rng.integers(-6, 7, (M, K)) + s)).astype(np.float32)
+        ref = x.astype(np.float64) @ W.astype(np.float64).T
+        # (from 2^32 on, the fp32 instruction: a rounding for every term)
+        b = bound(x, W, zero) if s < 32 else K * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(W.astype(np.float64)).T)
+        assert (np.abs(matmul(x, W, zero) - ref) <= b + 2.0 ** -149).all(), s
+
+
+# hidden values of 2^-127 to 2^-107, brought back by the last layer
+@pytest.mark.parametrize("dims,last", [([32, 64, 64, 8], Activation.NoActivation), ([20, 48, 24, 5], Activation.NoActivation), ([20, 48, 24, 5], Activation.Sigmoid)])
+def test_networks_with_small_hidden_values(dims, last):
+    rng = np.random.default_rng(sum(dims))
+    layers, params = network(rng, dims, [Activation.ReLU, Activation.NoActivation, last])
+    for fi, fo, wd, bd, act in params:
+        bd.zero_()
+    params[0][2].view(torch.float32).mul_(2.0 ** -60)
+    params[1][2].view(torch.float32).mul_(2.0 ** -57)
+    params[2][2].view(torch.float32).mul_(2.0 ** 117)
+    x = to_dev(rng.uniform(-1, 1, (3000, dims[0])).astype(np.float32))
+    y = cv.mlpForward(layers, x, weightType=CT.Float32)
+    assert torch.equal(y.view(torch.int32), chain(params, x).view(torch.int32))
+    h, mag = x.double(), x.double().abs()
+    for l, (fi, fo, wd, bd, act) in enumerate(params):
+        w = wd.view(torch.float32).view(fo, fi).double()
+        h, mag = h @ w.T, mag @ w.abs().T
+        h = torch.relu(h) if l == 0 else h
+    h = torch.sigmoid(h) if last == Activation.Sigmoid else h
+    assert ((y - h).abs() <= 2.0 ** -18 * mag).all()
 
 
 # the kernels for equal hidden layers, for any, and with a smooth activation
