@@ -11,6 +11,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "cv_layout.h"
 
@@ -119,8 +120,9 @@ struct Bf16Mma {
 // bits, 32 / 64 / 128 terms: 3.9 / 5.0 / 6.5e-8 against 10.3 / 14.4 / 20.4e-8 on the fp32 instruction; the dropped products are
 // below 2^-26 of the largest term each).  What the instruction drops, the low bits of products far below its largest one, it drops in
 // one direction: where inputs of one sign meet many sizes, the mean error of a row over all samples is 1e-8 to 1e-7 of the row's
-// mean (fp32 instruction: 1e-10), though each element is nearer.  The training kernels, which sum over samples, therefore
-// stay on the fp32 instruction: 32-64-64-8 over 2^20 samples would take 350 us for 394, with gradients up to 3.5 times as far off.
+// mean (fp32 instruction: 1e-10), though each element is nearer.  Training steps, which sum over samples, therefore
+// stay on the fp32 instruction, in LDS (32-64-64-8 over 2^20 samples would take 350 us for 394, with gradients up to 3.5 times as far
+// off) and layer by layer over memory (F32WholeMma).
 // A fragment has the 8 k-slots per lane of the 16-bit flavours, so the InferencingOptimal form of an fp32 matrix is the same
 // arrangement with 4-byte elements; decoded, four dwords each of h, m and l.
 // Operands from 2^32 on, infinities and NaN are not for the pieces: an h rounded up may be infinite, and products that overflow leave
@@ -230,8 +232,32 @@ struct F32Mma {
     }
 };
 
+template <class Mma>
+constexpr bool kInPieces = std::is_base_of<F32Mma, Mma>::value;
+
+// fp32 operands on v_mfma_f32_16x16x4_f32: eight instructions a fragment, the s-th multiplying slot s of every lane, each of which
+// rounds its sum to nearest, k ascending from the bias.
+struct F32WholeMma {
+    static constexpr const char* kName = "f32-whole";
+    static constexpr int kEsz = 4, kEpl = 8, kRawDW = 8, kFD = 8;
+    static constexpr bool kIsFloat = true;
+    typedef floatx4 Acc;
+    static __device__ __forceinline__ void decode(const uint32_t* raw, uint32_t* frag)
+    {
+#pragma unroll
+        for (int d = 0; d < 8; ++d) frag[d] = raw[d];
+    }
+    static __device__ __forceinline__ Acc mma(const uint32_t* a, const uint32_t* b, Acc c)
+    {
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s]), __builtin_bit_cast(float, b[s]), c, 0, 0, 0);
+        return c;
+    }
+};
+
 // The sums of a flavour on their way: its accumulators, or F32Sum.
-template <class Mma, bool F32 = Mma::kEsz == 4>
+template <class Mma, bool PIECES = kInPieces<Mma>>
 struct SumOf {
     typedef typename Mma::Acc T;
     static __device__ __forceinline__ T start(typename Mma::Acc seed) { return seed; }

@@ -37,7 +37,8 @@ enum class MmaKind : int {
     F16VecAsE4M3 = 6,    // fp16 vectors quantised to e4m3 on load, e4m3 matrix (matMul only)
     I8AnySign = 7,       // signed/unsigned bytes on either side (matMul only)
     F32 = 8,             // fp32 vectors and matrix (matMul only)
-    Scalar = 9           // combinations without a matrix instruction (16/32-bit integers, mixed forms): cv_matmul_scalar.hip
+    Scalar = 9,          // combinations without a matrix instruction (16/32-bit integers, mixed forms): cv_matmul_scalar.hip
+    F32Whole = 10        // F32 on the fp32 matrix instruction: the products of the training step over memory
 };
 
 // Returns hipSuccess, or hipErrorInvalidValue when no kernel covers (m,k): k beyond what one

@@ -48,7 +48,7 @@ struct VecAsMatrix : Mma {
     static constexpr bool kStreaming = !std::is_same<Mma, Bf8AsF16Mma>::value;
     // kWideFragments: fp32 fragments are twice as wide; a block of the matrix stays in registers up to 64 rows and two
     // k-tiles (64 columns), everything larger runs on matmulLargeKernel
-    static constexpr bool kWideFragments = std::is_same<Mma, F32Mma>::value;
+    static constexpr bool kWideFragments = Mma::kEsz == 4;
     static __device__ __forceinline__ void decodeIn(const uint32_t* raw, uint32_t* frag) { Mma::decode(raw, frag); }
 };
 
@@ -282,9 +282,9 @@ __device__ __forceinline__ void addUnsignedRowTerm(LaneOut<Fl, MT>& lo, int (&ro
 
 // LINES (streaming kernel only): the vectors on both sides are whole, aligned 128-byte lines, which the
 // kernel then reads and writes with non-temporal accesses.
-// (fp32: two waves per SIMD, of which F32Careful would take one)
+// (fp32 in pieces: two waves per SIMD, of which F32Careful would take one)
 template <class Fl, int MT, int KT, int NT, typename OutT, bool FAST, bool LINES = false>
-__global__ __launch_bounds__(256, Fl::kEsz == 4 ? 2 : 1) void matmulKernel(const MatMulArgs a)
+__global__ __launch_bounds__(256, kInPieces<Fl> ? 2 : 1) void matmulKernel(const MatMulArgs a)
 {
     constexpr int EPL = Fl::kEpl, FD = Fl::kFD, ESZ = Fl::kEsz, RAW = Fl::kRawDW;
     constexpr int IESZ = Fl::kInEsz, IRAW = Fl::kInRawDW;
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256, Fl::kEsz == 4 ? 2 : 1) void matmulKernel(const
     constexpr int OUT_DW = ROWS * (int)sizeof(OutT) / 4;
     typedef typename Fl::Acc Acc;
 
-    constexpr bool F32 = Fl::kEsz == 4;       // fragments as F32Mma's pieces
+    constexpr bool F32 = kInPieces<Fl>;       // fragments as F32Mma's pieces
     constexpr int LANE_DW = F32 ? FD : RAW;
     __shared__ __attribute__((aligned(16))) uint32_t ldsW[MT * KT * 64 * LANE_DW];
     // Output rows of 128 bytes or more leave through a per-wave LDS transpose so that every
@@ -570,7 +570,7 @@ constexpr int kLargeLdsBytes = 128 * 1024;
 // here; 256x256 over 2^16: 154, 197, 113 us.
 template <class Fl>
 struct LargeShape {
-    static constexpr bool kF32 = Fl::kEsz == 4;
+    static constexpr bool kF32 = kInPieces<Fl>;
     static constexpr int kWaves = kF32 ? 12 : 4, kSteps = kF32 ? 2 : kLargeKC;
 };
 constexpr int kLargePieceBytes = 158 * 1024;

@@ -317,7 +317,8 @@ hipError_t launchMlpTrainGeneral(hipStream_t stream, const TrainLaunch& t, int n
     const int ct = t.carrierCt;                 // kF16 or kF32: vectors, weights, biases
     const bool f32 = ct == kF32;
     const uint64_t esz = elemSize(ct);
-    const MmaKind mma = f32 ? MmaKind::F32 : MmaKind::F16;
+    // (fp32: sums over samples follow, which take up what the bfloat16 pieces drop in one direction, F32Mma)
+    const MmaKind mma = f32 ? MmaKind::F32Whole : MmaKind::F16;
     const GeneralPlan p = makePlan(a, numCUs, ct);
     uint8_t* ws = (uint8_t*)t.workspace;
     hipError_t e;

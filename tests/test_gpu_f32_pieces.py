@@ -234,3 +234,26 @@ def test_equal_hidden_layers_equal_the_chain_of_single_layer_operators(dims):
         ref = chain(params, x)
         assert torch.equal(torch.isnan(y), torch.isnan(ref))
         assert torch.equal(y[~torch.isnan(y)].view(torch.int32), ref[~torch.isnan(ref)].view(torch.int32)), (B, pad)
+
+
+# A training step over memory stays on the fp32 instruction, whose roundings, to nearest, cancel over samples; what the bfloat16 instruction
+# drops it drops in one direction (means off by 1.3e-8 of the products there, by 6e-10 here).  Targets are the results in 64 bits,
+# so that the bias gradient is the sum of the errors alone: each at most K roundings of 2^-24 of the sum so far, with signs as they
+# come, hence over B samples a mean within 6 * sqrt(K / 12) * 2^-23 / sqrt(B) of the products' magnitudes, and a rounding of the targets.
+# (The first layer is the identity.)
+@pytest.mark.parametrize("dims", [[64, 24], [40, 130], [100, 48]])
+def test_training_over_memory_keeps_the_means_of_rows(dims):
+    rng = np.random.default_rng(sum(dims))
+    B, (K, M) = 1 << 17, dims
+    x = (rng.uniform(0, 1, (B, K)) * np.exp2(-rng.integers(0, 12, (B, K)))).astype(np.float32)
+    W = (rng.uniform(0, 1, (M, K)) * np.exp2(-rng.integers(0, 6, (M, K)))).astype(np.float32)
+    ref = x.astype(np.float64) @ W.astype(np.float64).T
+    layers = [FeedForwardLayer(K, w.shape[0], as_bytes(to_dev(w)), None, ML.RowMajor, K * 4, Activation.NoActivation, 0.0,
+                               as_bytes(torch.zeros(w.shape, device=DEV)), as_bytes(torch.zeros(w.shape[0], device=DEV)), ML.RowMajor, K * 4)
+              for w in (np.eye(K, dtype=np.float32), W)]
+    t = ref.astype(np.float32)
+    cv.mlpTrainStep(layers, to_dev(x), to_dev(t), lossScale=0.5, weightType=CT.Float32)
+    assert "layer-by-layer" in cv.lastKernelName(), cv.lastKernelName()
+    mean = (layers[1].biasesGrad.view(torch.float32).cpu().numpy() + (t - ref).sum(axis=0)) / ref.sum(axis=0)
+    print("mean errors of rows:", np.abs(mean).max(), np.abs(mean).mean())
+    assert (np.abs(mean) <= 6 * np.sqrt(K / 12) * 2.0 ** -23 / np.sqrt(B)).all(), np.abs(mean).max()
