@@ -562,27 +562,26 @@ __global__ __launch_bounds__(256, kInPieces<Fl> ? 2 : 1) void matmulKernel(const
 // walks the k-tiles of a 16-sample tile KC at a time, reading its vector slice from memory and the
 // matrix fragments from LDS.  KT is a multiple of KC (fragments past the matrix hold zeros).
 constexpr int kLargeKC = 4;
-constexpr int kLargeLdsBytes = 128 * 1024;
 
-// fp32: fragments as F32Mma's pieces (PIECES), or, where they would not fit (k beyond 1664), as they are in memory and split at
-// every use; twelve waves share the block of the matrix, and the bias, which four waves keep in registers, lies in LDS.  128x128 over
-// 2^18 samples: 107 us on v_mfma_f32_16x16x4_f32 (four waves, blocks of 128 rows up to k = 256), 123 us splitting at every use, 77 us
-// here; 256x256 over 2^16: 154, 197, 113 us.
+// F32Mma: fragments as its pieces; twelve waves share the block of the matrix, and the bias, which four waves keep in registers, lies
+// in LDS.  128x128 over 2^18 samples: 106 us on v_mfma_f32_16x16x4_f32 (F32WholeMma: four waves, blocks of 128 rows up to k = 256), 78 us
+// here; 256x256 over 2^16: 156, 114 us.  Which of the two a product takes: cv_matmul_f32.hip.
 template <class Fl>
 struct LargeShape {
     static constexpr bool kF32 = kInPieces<Fl>;
     static constexpr int kWaves = kF32 ? 12 : 4, kSteps = kF32 ? 2 : kLargeKC;
+    static constexpr int kTileBytes = 64 * (kF32 ? Fl::kFD : Fl::kRawDW) * 4, kLdsBytes = (kF32 ? 158 : 128) * 1024;
 };
-constexpr int kLargePieceBytes = 158 * 1024;
 
-template <class Fl, int MT, typename OutT, bool PIECES>
+template <class Fl, int MT, typename OutT>
 __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel(const MatMulArgs a, const int KT)
 {
-    constexpr int EPL = Fl::kEpl, FD = Fl::kFD, ESZ = Fl::kEsz, RAW = Fl::kRawDW, LANE_DW = PIECES ? FD : RAW;
+    constexpr int EPL = Fl::kEpl, FD = Fl::kFD, ESZ = Fl::kEsz, RAW = Fl::kRawDW;
+    constexpr bool F32 = LargeShape<Fl>::kF32;
+    constexpr int LANE_DW = F32 ? FD : RAW;
     constexpr int IESZ = Fl::kInEsz, IRAW = Fl::kInRawDW;
     constexpr int WAVES = LargeShape<Fl>::kWaves;
     constexpr int KC = LargeShape<Fl>::kSteps, STEP_DW = KC * IRAW, ROWS = 4 * MT;
-    constexpr bool F32 = LargeShape<Fl>::kF32;
     typedef typename Fl::Acc Acc;
     extern __shared__ __attribute__((aligned(16))) uint32_t ldsDyn[];
     __shared__ __attribute__((aligned(16))) float ldsBias[F32 ? 16 * MT : 1];
@@ -590,14 +589,7 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
     const uint32_t gs = optGS((uint32_t)a.k);
     bool matBeyond = false;                    // F32Mma::beyond of the matrix
     if constexpr (F32) {
-        uint32_t most = 0u;
-        if constexpr (PIECES) {
-            most = stageFragmentPieces(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff, most);
-        } else {
-            stageFragments<ESZ, EPL>(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff);
-            __syncthreads();
-            for (int i = threadIdx.x; i < MT * KT * 64; i += 64 * WAVES) most = Fl::largestBits(ldsDyn + (size_t)i * RAW, RAW, most);
-        }
+        const uint32_t most = stageFragmentPieces(ldsDyn, a.mat, a.shape, a.transpose != 0, MT, KT, gs, (uint32_t)a.m, (uint32_t)a.k, a.rowOff, 0u);
         for (int row = threadIdx.x; row < 16 * MT; row += 64 * WAVES)
             ldsBias[row] = (a.bias && row < a.m) ? loadAsFloat(a.bias + (size_t)row * elemSize(a.biasCt), a.biasCt) : 0.f;
         matBeyond = __syncthreads_or(most >= Fl::kBeyondBits);
@@ -674,7 +666,7 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
 #pragma unroll
                     for (int t = t0; t < t0 + G; ++t) {
                         const uint32_t* raw = &ldsDyn[((t * KT + kc + j) * 64 + lane) * LANE_DW];
-                        if constexpr (PIECES) {
+                        if constexpr (F32) {
 #pragma unroll
                             for (int d = 0; d < FD; ++d) af[t - t0][d] = raw[d];
                         } else {
@@ -723,7 +715,7 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
                         uint32_t x[STEP_DW];
                         load(kc, x, vb);
 #pragma unroll
-                        for (int j = 0; j < KC; ++j) c.template step<PIECES, false>(&ldsDyn[((t * KT + kc + j) * 64 + lane) * LANE_DW], &x[j * IRAW]);
+                        for (int j = 0; j < KC; ++j) c.template step<true, false>(&ldsDyn[((t * KT + kc + j) * 64 + lane) * LANE_DW], &x[j * IRAW]);
                     }
                     const floatx4 r = c.finish(bias);
 #pragma unroll
@@ -813,40 +805,36 @@ hipError_t launchShape(hipStream_t stream, const MatMulArgs& a, int numCUs, bool
     }
 }
 
-template <class Fl, int MT, typename OutT, bool PIECES>
+template <class Fl, int MT, typename OutT>
 hipError_t launchLarge(hipStream_t stream, const MatMulArgs& a, int KT, int numCUs, bool append)
 {
-    const size_t ldsBytes = (size_t)MT * KT * 64 * (PIECES ? Fl::kFD : Fl::kRawDW) * 4;
-    const hipError_t ea = allowDynamicLds<matmulLargeKernel<Fl, MT, OutT, PIECES>>(PIECES ? kLargePieceBytes : kLargeLdsBytes);
+    const size_t ldsBytes = (size_t)KT * MT * LargeShape<Fl>::kTileBytes;
+    const hipError_t ea = allowDynamicLds<matmulLargeKernel<Fl, MT, OutT>>(LargeShape<Fl>::kLdsBytes);
     if (ea != hipSuccess) return ea;
     constexpr uint32_t kWaves = LargeShape<Fl>::kWaves;
     int perCU = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, matmulLargeKernel<Fl, MT, OutT, PIECES>, 64 * kWaves, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, matmulLargeKernel<Fl, MT, OutT>, 64 * kWaves, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
     const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + 15) / 16), need = (numTiles + kWaves - 1) / kWaves;
     const uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU;
     noteKernel(append, "matmulLargeKernel<%s,MT=%d,KT=%d,out=%dB>", Fl::kName, MT, KT, (int)sizeof(OutT));
-    hipLaunchKernelGGL((matmulLargeKernel<Fl, MT, OutT, PIECES>), dim3(need < cap ? need : cap), dim3(64 * kWaves), ldsBytes, stream, a, KT);
+    hipLaunchKernelGGL((matmulLargeKernel<Fl, MT, OutT>), dim3(need < cap ? need : cap), dim3(64 * kWaves), ldsBytes, stream, a, KT);
     return hipGetLastError();
 }
 
 // One block of at most 16*MTs rows at row a.rowOff (a.m = rows of the block; out and bias already
 // point at the block's first row).
 template <class Fl, typename OutT>
-hipError_t dispatchBlock(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append, int largeKT, bool largePieces)
+hipError_t dispatchBlock(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append, int largeKT)
 {
     const uint32_t mt = optMT((uint32_t)a.m), kt = optKT((uint32_t)a.k, Fl::kEpl);
     const int MTs = mt <= 1 ? 1 : mt <= 2 ? 2 : mt <= 4 ? 4 : mt <= 8 ? 8 : 0;
     if (!MTs) return hipErrorInvalidValue;
     if (largeKT) {
-        constexpr bool PIECES = LargeShape<Fl>::kF32;
-        if constexpr (PIECES) {
-            if (!largePieces) return launchLarge<Fl, 1, OutT, false>(stream, a, largeKT, numCUs, append);
-        }
         switch (MTs) {
-        case 1: return launchLarge<Fl, 1, OutT, PIECES>(stream, a, largeKT, numCUs, append);
-        case 2: return launchLarge<Fl, 2, OutT, PIECES>(stream, a, largeKT, numCUs, append);
-        case 4: return launchLarge<Fl, 4, OutT, PIECES>(stream, a, largeKT, numCUs, append);
-        default: return launchLarge<Fl, 8, OutT, PIECES>(stream, a, largeKT, numCUs, append);
+        case 1: return launchLarge<Fl, 1, OutT>(stream, a, largeKT, numCUs, append);
+        case 2: return launchLarge<Fl, 2, OutT>(stream, a, largeKT, numCUs, append);
+        case 4: return launchLarge<Fl, 4, OutT>(stream, a, largeKT, numCUs, append);
+        default: return launchLarge<Fl, 8, OutT>(stream, a, largeKT, numCUs, append);
         }
     }
     const int KTs = kt <= 1 ? 1 : kt <= 2 ? 2 : kt <= 4 ? 4 : 0;
@@ -872,16 +860,12 @@ hipError_t dispatchShape(hipStream_t stream, const MatMulArgs& a, int numCUs)
 {
     const uint32_t kt = optKT((uint32_t)a.k, Fl::kEpl);
     int blockTiles = 8, largeKT = 0;
-    bool largePieces = false;
     const bool inRegisters = Fl::kWideFragments ? (kt <= 2 && a.m <= 64) : kt <= 4;
     if (Fl::kWideFragments && inRegisters) blockTiles = 4;
     if (!inRegisters) {
         constexpr uint32_t kSteps = LargeShape<Fl>::kSteps;
         largeKT = (int)((kt + kSteps - 1) / kSteps * kSteps);
-        const size_t pieceBytes = (size_t)largeKT * 64 * Fl::kFD * 4;
-        largePieces = LargeShape<Fl>::kF32 && pieceBytes <= (size_t)kLargePieceBytes;
-        const size_t tileBytes = largePieces ? pieceBytes : (size_t)largeKT * 64 * Fl::kRawDW * 4, most = largePieces ? kLargePieceBytes : kLargeLdsBytes;
-        if (LargeShape<Fl>::kF32 && !largePieces) blockTiles = 1;
+        const size_t tileBytes = (size_t)largeKT * LargeShape<Fl>::kTileBytes, most = LargeShape<Fl>::kLdsBytes;
         while (blockTiles > 1 && blockTiles * tileBytes > most) blockTiles /= 2;
         if (blockTiles * tileBytes > most) return hipErrorInvalidValue;
     }
@@ -897,7 +881,7 @@ hipError_t dispatchShape(hipStream_t stream, const MatMulArgs& a, int numCUs)
         uint32_t al = a.outAlign;
         while (al > 1 && ((size_t)r0 * sizeof(OutT)) % al) al >>= 1;
         b.outAlign = al;
-        const hipError_t e = dispatchBlock<Fl, OutT>(stream, b, numCUs, r0 != 0, largeKT, largePieces);
+        const hipError_t e = dispatchBlock<Fl, OutT>(stream, b, numCUs, r0 != 0, largeKT);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
