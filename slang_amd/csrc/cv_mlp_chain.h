@@ -16,6 +16,10 @@
 //     (T = float: one, for the registers of the pieces).
 // Measured against the run-time-size kernels: fp16 20-48-24-5 over 2 000 003 samples 78 -> 45 us; T = float, 20-48-24-5 over 2^20
 // samples 91 us with v_mfma_f32_16x16x4_f32, 74 us with the pieces.  (Equal hidden layers: cv_mlp_equal_f32.h.)
+// Networks of float whose pieces exceed the LDS (more than 52 fragments) split a fragment at every use, 52 vector instructions
+// beside six matrix instructions, and are no faster than the fp32 instruction was: 64-128-128-64 over 2^18 samples 173 us (161),
+// 128-128-128 183 (161), over 2^12 28.9 (20.1) and 29.5 us (20.3).  They stay on the pieces all the same, for the bits of the
+// single-layer operators.
 #pragma once
 #include <type_traits>
 
@@ -34,6 +38,12 @@ constexpr int chainComponent()
 {
     return std::is_same<Mma, F32Mma>::value ? (int)kF32 : std::is_same<Mma, Bf16Mma>::value ? (int)kBF16 : (int)kF16;
 }
+
+// Four waves to a workgroup; eight for networks of float whose weights leave room for one workgroup in a compute unit's LDS, so that a
+// SIMD still has two waves, one converting and splitting beside the other's matrix instructions (four waves / eight, 2^18 samples:
+// 64-112-96-12 104 / 66 us, 96-80-72-16 106 / 63, split at use 64-128-128-64 282 / 173).
+template <class Mma>
+constexpr int chainThreads() { return Mma::kEsz == 4 ? 512 : 256; }
 
 template <int ACT>
 __device__ __forceinline__ float chainActivateF32(float x, float slope)
@@ -256,7 +266,7 @@ __device__ __forceinline__ void chainLayer(const MlpArgs& a, const MlpLayerArgs&
 // groups of four elements, which one load takes (else one load per element, any size and alignment).
 // INKT: the bound on the input's k-tiles.
 template <class Mma, int MAXT, int NT, bool QUAD, bool PIECES, int INKT>
-__global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void mlpChainKernel(const GenArgs ga)
+__global__ __launch_bounds__(chainThreads<Mma>(), Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void mlpChainKernel(const GenArgs ga)
 {
     constexpr int MAXKT = MAXT / 2, FD = Mma::kFD, ESZ = Mma::kEsz, RAW = Mma::kRawDW;
     constexpr int UNITS = QUAD ? 2 : 8;                    // loads per fragment
@@ -267,6 +277,7 @@ __global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void
     float* ldsB = (float*)(lds + ga.biasDwordBase);
     constexpr bool F32 = std::is_same<Mma, F32Mma>::value;
     constexpr int LANE_DW = PIECES ? FD : RAW;             // dwords per lane of a fragment in LDS
+    const uint32_t threads = F32 ? blockDim.x : 256u;
     uint32_t most = 0u;
     for (int l = 0; l < a.numLayers; ++l) {
         const MlpLayerArgs& ly = a.layers[l];
@@ -274,7 +285,7 @@ __global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void
         uint32_t* dst = lds + ga.gl[l].fragBase * 64 * LANE_DW;
         if constexpr (PIECES) most = stageFragmentPieces(dst, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in), (uint32_t)ly.out, (uint32_t)ly.in, 0, most);
         else stageFragments<ESZ, 8>(dst, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in), (uint32_t)ly.out, (uint32_t)ly.in);
-        for (int e = threadIdx.x; e < MT * 16; e += 256) {
+        for (int e = threadIdx.x; e < MT * 16; e += (int)threads) {
             const int t = e >> 4, gg = (e >> 2) & 3, r = e & 3, row = gg * 4 * MT + 4 * t + r;
             ldsB[ga.gl[l].biasBase + e] = (ly.bias && row < ly.out) ? loadAsFloat(ly.bias + (size_t)row * (chainComponent<Mma>() == kF32 ? 4 : 2), chainComponent<Mma>()) : 0.f;
         }
@@ -283,7 +294,7 @@ __global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void
     bool matBeyond = false;
     if constexpr (F32) {
         if constexpr (!PIECES)
-            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += 256) most = Mma::largestBits(lds + (size_t)i * RAW, RAW, most);
+            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += threads) most = Mma::largestBits(lds + (size_t)i * RAW, RAW, most);
         matBeyond = __syncthreads_or(most >= Mma::kBeyondBits);
     }
 
@@ -293,19 +304,25 @@ __global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void
     const uint32_t in0 = (uint32_t)a.layers[0].in, gs0 = optGS(in0), rowBytes = in0 * ESZ;
     const bool quads = a.layers[L - 1].out % 4 == 0 && a.outAlign >= (std::is_same<Mma, F32Mma>::value ? 16u : 8u);
 
-    uint32_t off[INKT][UNITS];
+    // offsets of a lane's elements, the same for every tile; of float, where registers are scarce, only the first and how many there are
+    uint32_t off[F32 ? 1 : INKT][F32 ? 1 : UNITS];
+    const uint32_t col0 = g * gs0, have = col0 < in0 ? min(gs0, in0 - col0) : 0u, off0 = (uint32_t)n * (uint32_t)a.inStride + col0 * ESZ;
+    if constexpr (!F32) {
 #pragma unroll
-    for (int kt = 0; kt < INKT; ++kt)
+        for (int kt = 0; kt < INKT; ++kt)
 #pragma unroll
-        for (int u = 0; u < UNITS; ++u) {
-            const uint32_t q = kt * 8 + u * (8 / UNITS), col = g * gs0 + q;
-            off[kt][u] = q < gs0 && col < in0 ? (uint32_t)n * (uint32_t)a.inStride + col * ESZ : kChainOutside;
-        }
+            for (int u = 0; u < UNITS; ++u) {
+                const uint32_t q = kt * 8 + u * (8 / UNITS);
+                off[kt][u] = q < have ? off0 + q * ESZ : kChainOutside;
+            }
+    }
 
-    const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + 15) / 16), step = gridDim.x * 4u * NT;
+    const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + 15) / 16), waves = threads / 64u, step = gridDim.x * waves * NT;
     const int kt0 = ga.gl[0].kt;
     uint32_t raw[NT][INKT][UNITS * UDW];
     auto fetch = [&](uint32_t tile) {
+        uint32_t first0 = off0;
+        if constexpr (F32) asm volatile("" : "+v"(first0));      // (else the compiler keeps every offset over the tiles)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             // the vectors of this tile that exist: none for a tile beyond the batch
@@ -319,27 +336,33 @@ __global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void
                 for (int u = 0; u < UNITS; ++u) {
                     if (kt > 0 && kt >= kt0) continue;       // (wave-uniform; empty loads of absent k-tiles cost 6 us of 51)
                     uint32_t* r = raw[nt][kt] + u * UDW;
+                    constexpr uint32_t kPerUnit = 8 / UNITS;
+                    const uint32_t q = kt * 8 + u * kPerUnit;
+                    const uint32_t at = F32 ? (q < have ? first0 + q * ESZ : kChainOutside) : off[F32 ? 0 : kt][F32 ? 0 : u];
                     if constexpr (QUAD && ESZ == 4) {
-                        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, off[kt][u], 0, 0));
+                        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, at, 0, 0));
                         r[0] = v.x; r[1] = v.y; r[2] = v.z; r[3] = v.w;
                     } else if constexpr (QUAD && ESZ == 2) {
-                        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(src, off[kt][u], 0, 0));
+                        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(src, at, 0, 0));
                         r[0] = v.x; r[1] = v.y;
                     } else if constexpr (QUAD || ESZ == 4) {
-                        r[0] = __builtin_amdgcn_raw_buffer_load_b32(src, off[kt][u], 0, 0);
+                        r[0] = __builtin_amdgcn_raw_buffer_load_b32(src, at, 0, 0);
                     } else if constexpr (ESZ == 2) {
-                        r[0] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(src, off[kt][u], 0, 0);
+                        r[0] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(src, at, 0, 0);
                     } else {
-                        r[0] = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(src, off[kt][u], 0, 0);
+                        r[0] = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(src, at, 0, 0);
                     }
                 }
         }
     };
 
-    uint32_t tile = (blockIdx.x * 4u + wave) * NT;
+    uint32_t tile = (blockIdx.x * waves + wave) * NT;
     if (tile >= numTiles) return;
-    fetch(tile);
+    // (not ahead for more than 64 inputs of float: the registers would be spilled ones, and the other wave's work covers the wait)
+    constexpr bool AHEAD = !F32 || INKT <= 2;
+    if constexpr (AHEAD) fetch(tile);
     for (;;) {
+        if constexpr (!AHEAD) fetch(tile);
         uint32_t act[NT][MAXKT][FD];
         bool any = matBeyond;
         if constexpr (F32) {
@@ -374,7 +397,7 @@ __global__ __launch_bounds__(256, Mma::kEsz == 4 ? (MAXT == 4 ? 3 : 2) : 1) void
             }
         const uint64_t following = (uint64_t)tile + step;
         const uint32_t next = following < numTiles ? (uint32_t)following : numTiles;
-        fetch(next);                     // (beyond the batch: an empty descriptor, nothing is read)
+        if constexpr (AHEAD) fetch(next);                     // (beyond the batch: an empty descriptor, nothing is read)
 
         const uint32_t sample = tile * 16u + n;
         for (int l = 0; l < L; ++l) {
@@ -404,13 +427,14 @@ hipError_t launchChainSized(hipStream_t stream, const GenArgs& ga, size_t ldsByt
 {
     const hipError_t ea = allowDynamicLds<mlpChainKernel<Mma, MAXT, NT, QUAD, PIECES, INKT>>((int)((PIECES ? kChainPieceDwords : kGenLdsDwords) * 4));
     if (ea != hipSuccess) return ea;
+    const uint32_t numTiles = (uint32_t)(((uint64_t)ga.mlp.batch + 15) / 16);
+    const uint32_t waves = chainThreads<Mma>() == 512 && ldsBytes > 80 * 1024 ? 8u : 4u;
     int perCU = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpChainKernel<Mma, MAXT, NT, QUAD, PIECES, INKT>, 256, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
-    const uint32_t numTiles = (uint32_t)(((uint64_t)ga.mlp.batch + 15) / 16), need = (numTiles + 4 * NT - 1) / (4 * NT);
-    const uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU;
-    noteKernel(false, "mlpChainKernel<%s,up to %d rows,NT=%d%s>", Mma::kName, 16 * MAXT, NT,
-               QUAD ? ",loads of four elements" : "");
-    hipLaunchKernelGGL((mlpChainKernel<Mma, MAXT, NT, QUAD, PIECES, INKT>), dim3(need < cap ? need : cap), dim3(256), ldsBytes, stream, ga);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpChainKernel<Mma, MAXT, NT, QUAD, PIECES, INKT>, (int)(64 * waves), ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
+    const uint32_t need = (numTiles + waves * NT - 1) / (waves * NT), cap = (uint32_t)numCUs * (uint32_t)perCU;
+    noteKernel(false, "mlpChainKernel<%s,up to %d rows,NT=%d%s%s>", Mma::kName, 16 * MAXT, NT,
+               QUAD ? ",loads of four elements" : "", PIECES || Mma::kEsz < 4 ? "" : ",split at use");
+    hipLaunchKernelGGL((mlpChainKernel<Mma, MAXT, NT, QUAD, PIECES, INKT>), dim3(need < cap ? need : cap), dim3(64 * waves), ldsBytes, stream, ga);
     return hipGetLastError();
 }
 

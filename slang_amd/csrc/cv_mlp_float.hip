@@ -43,7 +43,7 @@ __device__ __forceinline__ float activateFloat(float x, int act, float slope)
 // registers and run more waves per SIMD; 8 up to 128)
 // PIECES (T = float): fragments lie in LDS as F32Mma's pieces; else as they lie in memory, split at every use.
 template <class Mma, int MAXT, bool PIECES>
-__global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
+__global__ __launch_bounds__(Mma::kEsz == 4 ? 512 : 256) void mlpFloatKernel(const FltArgs ga)
 {
     constexpr int kFltMaxTiles = MAXT, kFltMaxKT = MAXT / 2;
     constexpr int EPL = Mma::kEpl, FD = Mma::kFD, ESZ = Mma::kEsz, RAW = Mma::kRawDW, LANE_DW = PIECES ? FD : RAW;
@@ -54,6 +54,7 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     float* ldsB = (float*)(lds + ga.biasDwordBase);
 
+    const uint32_t threads = F32 ? blockDim.x : 256u, waves = threads / 64u;
     uint32_t most = 0u;
     for (int l = 0; l < L; ++l) {
         const MlpLayerArgs& ly = a.layers[l];
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
         uint32_t* dst = lds + ga.gl[l].fragBase * 64 * LANE_DW;
         if constexpr (PIECES) most = stageFragmentPieces(dst, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in), (uint32_t)ly.out, (uint32_t)ly.in, 0, most);
         else stageFragments<ESZ, EPL>(dst, ly.w, ly.shape, false, MT, KT, optGS((uint32_t)ly.in), (uint32_t)ly.out, (uint32_t)ly.in);
-        for (int e = threadIdx.x; e < MT * 16; e += 256) {
+        for (int e = threadIdx.x; e < MT * 16; e += (int)threads) {
             const int t = e >> 4, g = (e >> 2) & 3, r = e & 3;
             const int row = g * ROWS + 4 * t + r;
             ldsB[ga.gl[l].biasBase + e] = (ly.bias && row < ly.out) ? loadAsFloat(ly.bias + (size_t)row * ESZ, ga.ct) : 0.f;
@@ -71,7 +72,7 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
     bool matBeyond = false;                  // F32Mma::beyond of some layer's matrix
     if constexpr (F32) {
         if constexpr (!PIECES)
-            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += 256) most = Mma::largestBits(lds + (size_t)i * RAW, RAW, most);
+            for (uint32_t i = threadIdx.x; i < ga.biasDwordBase / RAW; i += threads) most = Mma::largestBits(lds + (size_t)i * RAW, RAW, most);
         matBeyond = __syncthreads_or(most >= Mma::kBeyondBits);
     }
 
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(256) void mlpFloatKernel(const FltArgs ga)
     const int orows = 4 * ga.gl[L - 1].mt;
 
     const uint32_t numTiles = (a.batch + 15) / 16;
-    for (uint32_t tile = blockIdx.x * 4 + wave; tile < numTiles; tile += gridDim.x * 4) {
+    for (uint32_t tile = blockIdx.x * waves + wave; tile < numTiles; tile += gridDim.x * waves) {
         const uint32_t sample = tile * 16 + n;
         const uint32_t sc = min(sample, a.batch - 1);
         uint32_t act[kFltMaxKT][RAW];          // the layer's input as it lies in memory
@@ -212,12 +213,14 @@ hipError_t launchFloatSized(hipStream_t stream, const FltArgs& ga, size_t ldsByt
 {
     const hipError_t ea = allowDynamicLds<mlpFloatKernel<Mma, MAXT, PIECES>>((int)(kFltLdsDwords * 4));
     if (ea != hipSuccess) return ea;
+    // (eight waves to a workgroup where one fills the LDS, as mlpChainKernel: 16-112-112-112-8 with a sigmoid over 2^18 samples 487 -> 243 us)
+    const uint32_t waves = Mma::kEsz == 4 && ldsBytes > 80 * 1024 ? 8u : 4u;
     int perCU = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpFloatKernel<Mma, MAXT, PIECES>, 256, ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
-    const uint32_t numTiles = (ga.mlp.batch + 15) / 16, need = (numTiles + 3) / 4;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, mlpFloatKernel<Mma, MAXT, PIECES>, (int)(64 * waves), ldsBytes) != hipSuccess || perCU < 1) perCU = 1;
+    const uint32_t numTiles = (ga.mlp.batch + 15) / 16, need = (numTiles + waves - 1) / waves;
     const uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU;
-    noteKernel(false, "mlpFloatKernel<%s,up to %d rows>", Mma::kName, 16 * MAXT);
-    hipLaunchKernelGGL((mlpFloatKernel<Mma, MAXT, PIECES>), dim3(need < cap ? need : cap), dim3(256), ldsBytes, stream, ga);
+    noteKernel(false, "mlpFloatKernel<%s,up to %d rows%s>", Mma::kName, 16 * MAXT, PIECES || Mma::kEsz < 4 ? "" : ",split at use");
+    hipLaunchKernelGGL((mlpFloatKernel<Mma, MAXT, PIECES>), dim3(need < cap ? need : cap), dim3(64 * waves), ldsBytes, stream, ga);
     return hipGetLastError();
 }
 

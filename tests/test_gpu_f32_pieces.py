@@ -251,6 +251,25 @@ def test_equal_hidden_layers_equal_the_chain_of_single_layer_operators(dims):
         assert torch.equal(y[~torch.isnan(y)].view(torch.int32), ref[~torch.isnan(ref)].view(torch.int32)), (B, pad)
 
 
+# the last and the first network whose pieces fit the LDS and do not, on either kernel; workgroups of eight waves, the last partly filled
+@pytest.mark.parametrize("dims,last,split", [([128, 128, 80], Activation.NoActivation, False), ([128, 128, 96], Activation.NoActivation, True),
+                                             ([101, 128, 67], Activation.NoActivation, False), ([101, 113, 85], Activation.NoActivation, True),
+                                             ([128, 128, 48], Activation.Tanh, False), ([128, 128, 64], Activation.Tanh, True)])
+def test_networks_that_fill_the_lds_equal_the_chain_of_single_layer_operators(dims, last, split):
+    rng = np.random.default_rng(sum(dims))
+    layers, params = network(rng, dims, [Activation.LeakyReLU, last])
+    for B in (1, 113, 70001):
+        x = to_dev(rng.uniform(-1, 1, (B, dims[0])).astype(np.float32))
+        if B > 100:
+            x[7, 0], x[B - 1, dims[0] - 1], x[50, 1], x[9, 2] = float("inf"), float("-inf"), 3.4e38, float("nan")
+        y = cv.mlpForward(layers, x, weightType=CT.Float32)
+        name = cv.lastKernelName()
+        assert name.startswith("mlpChainKernel<" if last == Activation.NoActivation else "mlpFloatKernel<") and ("split at use" in name) == split, name
+        ref = chain(params, x)
+        assert torch.equal(torch.isnan(y), torch.isnan(ref))
+        assert torch.equal(y[~torch.isnan(y)].view(torch.int32), ref[~torch.isnan(ref)].view(torch.int32)), B
+
+
 # A training step over memory stays on the fp32 instruction, whose roundings, to nearest, cancel over samples; what the bfloat16 instruction
 # drops it drops in one direction (means off by 1.3e-8 of the products there, by 6e-10 here).  Targets are the results in 64 bits,
 # so that the bias gradient is the sum of the errors alone: each at most K roundings of 2^-24 of the sum so far, with signs as they
