@@ -369,7 +369,8 @@ CV_API CvResult cvPermutoPrepareLevels(CvPermutoDesc* desc, float baseScale, flo
 CV_API CvResult cvPermutoEncode(void* stream, const CvPermutoDesc* desc, const void* positions, size_t positionStride,
                                 const void* featureTable, void* out, size_t outStride, uint32_t batch);
 /* bwd_diff of encode for FLOAT32 data: dPositions[s] (overwritten; may be NULL) and dFeatureTable
- * (+=, atomic adds like readFeatureValueBwd :222-238; may be NULL). */
+ * (+=, atomic adds like readFeatureValueBwd :222-238; may be NULL).  dPositions may lie on positions or on dOut, row s on
+ * row s; it lies apart from the tables, and dFeatureTable apart from everything else. */
 CV_API CvResult cvPermutoEncodeBackward(void* stream, const CvPermutoDesc* desc, const void* positions, size_t positionStride,
                                         const void* featureTable, const void* dOut, size_t dOutStride,
                                         void* dPositions, size_t dPositionStride, void* dFeatureTable, uint32_t batch);

@@ -503,8 +503,12 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     const bool few = FT > 0 && a.batch <= 64u && features <= 16u && a.batch * (uint64_t)(D + 1) * features <= 1440u;
     if (cut && !(a.dPos && few)) {
         // One launch where the table's workgroups fill the chip; with fewer of them the positions, spread over all compute units by
-        // a kernel of their own, are done sooner than by the few.
-        if (a.dPos && (uint64_t)t.count * ((a.batch - 1u) / 1024u + 1u) >= (uint64_t)cus) {
+        // a kernel of their own, are done sooner than by the few.  Where position gradients are written on top of what is read (rows
+        // on rows), other workgroups of the one launch would still read it.
+        const Rows dPos{(uint64_t)(uintptr_t)a.dPos, a.dPosStride, D * 4ull}, pos{(uint64_t)(uintptr_t)a.pos, a.posStride, D * 4ull},
+            dOut{(uint64_t)(uintptr_t)a.dOut, a.dOutStride, features * 4ull};
+        const bool apart = a.dPos && !rowsMeet(dPos, pos, a.batch) && !rowsMeet(dPos, dOut, a.batch);
+        if (apart && (uint64_t)t.count * ((a.batch - 1u) / 1024u + 1u) >= (uint64_t)cus) {
             noteKernel(false, "permutoTableGradKernel<D=%d,%u parts,positions beside>", D, t.count);
             return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t, cus);
         }

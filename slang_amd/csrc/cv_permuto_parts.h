@@ -63,5 +63,14 @@ inline bool cutTable(const CvPermutoDesc& desc, TableParts& t)
     return t.count > 0;
 }
 
+// Whether two regions of `rows` rows each, `stride` bytes apart and `width` bytes wide, may have a byte in common (between their first
+// and their last byte: rows of one in the gaps of the other count as well).
+struct Rows { uint64_t at, stride, width; };
+inline bool rowsMeet(const Rows& a, const Rows& b, uint32_t rows)
+{
+    const uint64_t aEnd = a.at + (rows - 1ull) * a.stride + a.width, bEnd = b.at + (rows - 1ull) * b.stride + b.width;
+    return a.at < bEnd && b.at < aEnd;
+}
+
 } // namespace
 } // namespace cv

@@ -296,6 +296,29 @@ def test_permuto_backward_positions_beside_the_table(D, F, tables, B, parts):
     assert torch.linalg.norm(d_table - want_table) <= 2.0 ** -16 * torch.linalg.norm(want_table)
 
 
+@pytest.mark.parametrize("D,F,tables,B,kernel", [(3, 2, [1 << 12] * 8, 1 << 16, "permutoTableGradKernel<D=3,8 parts>"), (2, 4, [1 << 8] * 4, 4099, "permutoTableGradKernel<D=2,positions>"),
+                                                  (3, 1, [1 << 15] * 3, 70001, "permutoTableGradKernel<D=3,6 parts>")])
+@pytest.mark.parametrize("where", ["positions", "dOut"])
+def test_permuto_backward_positions_on_top_of_inputs(D, F, tables, B, kernel, where):
+    # dPositions row on row of positions, or of the gradients that come in: as into a buffer of its own
+    rng = np.random.default_rng(B)
+    enc = cv.PermutoEncoder(D, F, 4, len(tables), baseScale=2.0, log2PerLevelScale=0.5, seed=5)
+    for l, n in enumerate(tables):
+        enc.desc.levelInfo[l].featureTableSize, enc.desc.levelInfo[l].offsetOfFeatureTable = n, sum(tables[:l])
+    pos = to_dev(rng.uniform(-1, 1, (B, D)).astype(np.float32))
+    table = to_dev(rng.standard_normal(sum(tables) * F).astype(np.float32))
+    g = to_dev(rng.integers(-4, 5, (B, len(tables) * F)).astype(np.float32))
+    want_pos, want_table = enc.backward(pos, table, g)
+    assert cv.lastKernelName() == (kernel if "positions" in kernel else kernel[:-1] + ",positions beside>"), cv.lastKernelName()
+    d_table, into = torch.zeros_like(table), pos if where == "positions" else g
+    lib = cv._lib.load()
+    rc = lib.cvPermutoEncodeBackward(torch.cuda.current_stream().cuda_stream, cv.ctypes.byref(enc.desc), pos.data_ptr(), 4 * D, table.data_ptr(), g.data_ptr(),
+                                     4 * g.shape[1], into.data_ptr(), 4 * into.shape[1], d_table.data_ptr(), B)
+    assert rc == 0 and cv.lastKernelName().startswith(kernel), cv.lastKernelName()
+    assert torch.equal(into[:, :D], want_pos)
+    assert torch.allclose(d_table, want_table, rtol=1e-6, atol=1e-4)
+
+
 @pytest.mark.parametrize("D,F,levels_n,log2,B,in_memory", [
     (2, 4, 3, 10, 1, True), (2, 4, 3, 10, 40, True), (2, 4, 3, 10, 41, False),       # 36 additions to a position
     (3, 2, 8, 12, 22, True), (3, 2, 8, 12, 23, False), (1, 1, 4, 15, 64, True), (1, 1, 4, 15, 65, False),

@@ -26,16 +26,22 @@ extern "C" int cut(const CvPermutoDesc* d, uint32_t* out, uint32_t* sliced)
     *sliced = ok ? t.sliced : 0;
     return ok ? (int)t.count : -1;
 }
+extern "C" int meet(const uint64_t* a, const uint64_t* b, uint32_t rows) { return cv::rowsMeet({a[0], a[1], a[2]}, {b[0], b[1], b[2]}, rows); }
 """
 
 
 @pytest.fixture(scope="module")
-def cut(tmp_path_factory):
+def built(tmp_path_factory):
     d = tmp_path_factory.mktemp("parts")
     (d / "parts.cpp").write_text(SOURCE)
     subprocess.run(["g++", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(REPO, "include"),
                     "-I", os.path.join(REPO, "slang_amd", "csrc"), "-o", str(d / "parts.so"), str(d / "parts.cpp")], check=True)
-    lib = ctypes.CDLL(str(d / "parts.so"))
+    return ctypes.CDLL(str(d / "parts.so"))
+
+
+@pytest.fixture(scope="module")
+def cut(built):
+    lib = built
 
     def call(F, tables):
         """tables: (offset, size) in entries per level; the parts (base, elems, first, end) and `sliced`, or None"""
@@ -112,3 +118,17 @@ def test_parts_of_tables_in_any_layout(cut, F):
             assert cut(F, tables)[0] == [(min(o for o, _ in tables) * F, (max(o + s for o, s in tables) - min(o for o, _ in tables)) * F, 0, len(tables))]
     # elements beyond 32 bits: not cut
     assert cut(F, [(0, 4), ((1 << 32) // F - 2, 4)]) is None
+
+
+def test_rows_that_meet(built):
+    def meet(a, b, rows):
+        got = {bool(built.meet((ctypes.c_uint64 * 3)(*x), (ctypes.c_uint64 * 3)(*y), rows)) for x, y in ((a, b), (b, a))}
+        assert len(got) == 1
+        return got.pop()
+    for at in (0x1000, (1 << 48) - 4):
+        assert meet((at, 12, 12), (at, 64, 64), 5) and meet((at, 12, 12), (at, 12, 12), 1)
+        assert not meet((at, 12, 12), (at + 60, 12, 12), 5) and meet((at, 12, 12), (at + 59, 12, 12), 5)
+        assert meet((at, 64, 12), (at + 12, 64, 52), 2)                     # columns of one buffer
+        assert not meet((at, 64, 12), (at + 12, 64, 52), 1)
+        assert not meet((at, 1 << 33, 12), (at + 12, 0, 12), 1)             # one row: its stride says nothing
+        assert meet((at, 1 << 33, 12), (at + (1 << 40), 4, 4), 200)
