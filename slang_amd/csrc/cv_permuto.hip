@@ -467,17 +467,11 @@ hipError_t launchEncode(hipStream_t stream, const PermutoArgs& a)
 }
 
 template <int D, int FT, int POS, bool SLICED, bool PLAIN>
-hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, TableParts& t, int cus)
+hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, const TableParts& t)
 {
-    uint32_t most = 0;
-    for (uint32_t p = 0; p < t.count; ++p) most = t.part[p].elems > most ? t.part[p].elems : most;
-    const size_t lds = (size_t)most * 8;
+    const size_t lds = (size_t)largestPart(t) * 8;
     const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED, PLAIN>>((int)(kPartMost * 8));
     if (e != hipSuccess) return e;
-    // as many workgroups as the compute units hold, dealt evenly to the parts
-    const uint32_t resident = (uint32_t)cus * (lds <= 80 * 1024 ? 2u : 1u), want = (a.batch - 1u) / 1024u + 1u;
-    const uint32_t each = resident / t.count ? resident / t.count : 1u;
-    t.groups = want < each ? want : each;
     hipLaunchKernelGGL((permutoTableGradKernel<D, FT, POS, SLICED, PLAIN>), dim3(t.count * t.groups), dim3(1024), lds, stream, a, t);
     return hipGetLastError();
 }
@@ -490,9 +484,10 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     const dim3 grid((a.batch - 1u) / 256u + 1u), block(256);
     TableParts t;
     const bool cut = a.dTable && cutTable(a.desc, t);
+    if (cut) dealGroups(t, a.batch, (uint32_t)cus);
     if (cut && t.count == 1 && a.dPos) {
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
-        return launchTableGrad<D, FT, kPosInPass, false, PLAIN>(stream, a, t, cus);
+        return launchTableGrad<D, FT, kPosInPass, false, PLAIN>(stream, a, t);
     }
     // Two launches against one: a handful of positions whose few additions hardly meet is done sooner by the one kernel that adds
     // in memory.  It takes 7.4 to 8.1 us per call back to back and the pair 11.5 to 13.5 (16 positions on 3 levels of 2^10
@@ -502,18 +497,17 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     const uint64_t features = (uint64_t)a.desc.featureDimensionPerEntry * a.desc.maxLevels;
     const bool few = FT > 0 && a.batch <= 64u && features <= 16u && a.batch * (uint64_t)(D + 1) * features <= 1440u;
     if (cut && !(a.dPos && few)) {
-        // One launch where the table's workgroups fill the chip; with fewer of them the positions, spread over all compute units by
-        // a kernel of their own, are done sooner than by the few.  Where position gradients are written on top of what is read (rows
+        // One launch where that is sooner (positionsBeside).  Where position gradients are written on top of what is read (rows
         // on rows), other workgroups of the one launch would still read it.
         const Rows dPos{(uint64_t)(uintptr_t)a.dPos, a.dPosStride, D * 4ull}, pos{(uint64_t)(uintptr_t)a.pos, a.posStride, D * 4ull},
             dOut{(uint64_t)(uintptr_t)a.dOut, a.dOutStride, features * 4ull};
         const bool apart = a.dPos && !rowsMeet(dPos, pos, a.batch) && !rowsMeet(dPos, dOut, a.batch);
-        if (apart && (uint64_t)t.count * ((a.batch - 1u) / 1024u + 1u) >= (uint64_t)cus) {
+        if (apart && positionsBeside(t, a.batch, (uint32_t)cus)) {
             noteKernel(false, "permutoTableGradKernel<D=%d,%u parts,positions beside>", D, t.count);
-            return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t, cus);
+            return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t);
         }
         noteKernel(false, "permutoTableGradKernel<D=%d,%u parts>", D, t.count);
-        const hipError_t e = t.sliced ? launchTableGrad<D, FT, kPosNone, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosNone, false, PLAIN>(stream, a, t, cus);
+        const hipError_t e = t.sliced ? launchTableGrad<D, FT, kPosNone, true, PLAIN>(stream, a, t) : launchTableGrad<D, FT, kPosNone, false, PLAIN>(stream, a, t);
         if (e != hipSuccess || !a.dPos) return e;
         noteKernel(true, "permutoBackwardKernel<D=%d,positions>", D);
         hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false, PLAIN>), grid, block, 0, stream, a);

@@ -63,6 +63,31 @@ inline bool cutTable(const CvPermutoDesc& desc, TableParts& t)
     return t.count > 0;
 }
 
+// As many workgroups (of 1024 threads) as the compute units hold, dealt evenly to the parts, and none without positions.
+inline uint32_t largestPart(const TableParts& t)
+{
+    uint32_t most = 0;
+    for (uint32_t p = 0; p < t.count; ++p) most = t.part[p].elems > most ? t.part[p].elems : most;
+    return most;
+}
+inline void dealGroups(TableParts& t, uint32_t batch, uint32_t cus)
+{
+    const uint32_t resident = cus * (largestPart(t) <= kPartHalf ? 2u : 1u), want = (batch - 1u) / 1024u + 1u;
+    const uint32_t each = resident / t.count ? resident / t.count : 1u;
+    t.groups = want < each ? want : each;
+}
+
+// Whether position gradients go into the table's launch (of several parts; after dealGroups).  Not with too few positions for
+// workgroups on every compute unit: spread by a kernel of their own they are done sooner.  And not where a part has but one or two
+// workgroups and many positions: a table of 91 parts or more, whose grid leaves compute units without one or deals some of them twice the
+// work.  One launch against two, 3 dimensions, 9 or 7 levels of two-feature entries, 2^14 / 2^16 / 2^18 positions: 144 parts (144
+// workgroups) 41.7, 149, 606 us against 53.9, 150, 542; 126 parts (252) 24.0, 79.2, 304 against 36.6, 86.5, 288; 105 parts (210) 23.7,
+// 77.2, 297 against 33.2, 81.7, 276; 64 parts (256) 62.5 and 258 against 84.6 and 273 over 2^16 and 2^18, and still 1063 against 1108 over 2^20.
+inline bool positionsBeside(const TableParts& t, uint32_t batch, uint32_t cus)
+{
+    return (uint64_t)t.count * ((batch - 1u) / 1024u + 1u) >= cus && !(t.groups <= 2u && batch > 65536u * t.groups);
+}
+
 // Whether two regions of `rows` rows each, `stride` bytes apart and `width` bytes wide, may have a byte in common (between their first
 // and their last byte: rows of one in the gaps of the other count as well).
 struct Rows { uint64_t at, stride, width; };

@@ -296,6 +296,25 @@ def test_permuto_backward_positions_beside_the_table(D, F, tables, B, parts):
     assert torch.linalg.norm(d_table - want_table) <= 2.0 ** -16 * torch.linalg.norm(want_table)
 
 
+def test_permuto_backward_of_many_parts():
+    # 144 parts, one workgroup each: the positions beside them up to 2^16, by a kernel of their own beyond
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the batches are those of 256 compute units")
+    D, F, n, L, B = 2, 2, 16 * 10240, 9, (1 << 16) + 1
+    enc = cv.PermutoEncoder(D, F, 4, L, baseScale=4.0, log2PerLevelScale=0.5, seed=3)
+    for l in range(L):
+        enc.desc.levelInfo[l].featureTableSize, enc.desc.levelInfo[l].offsetOfFeatureTable = n, n * l
+    rng = np.random.default_rng(9)
+    pos, table, g = (to_dev(rng.standard_normal(s).astype(np.float32)) for s in ((B, D), n * L * F, (B, L * F)))
+    d_pos, d_table = enc.backward(pos, table, g)
+    assert cv.lastKernelName() == "permutoTableGradKernel<D=2,144 parts> + permutoBackwardKernel<D=2,positions>", cv.lastKernelName()
+    d_pos2, d_table2 = enc.backward(pos[:-1], table, g[:-1])
+    assert cv.lastKernelName() == "permutoTableGradKernel<D=2,144 parts,positions beside>", cv.lastKernelName()
+    enc.backward(pos[-1:], table, g[-1:], dFeatureTable=d_table2)
+    assert torch.equal(d_pos[:-1], d_pos2)
+    assert torch.linalg.norm((d_table - d_table2).double()) <= 2.0 ** -16 * torch.linalg.norm(d_table.double())
+
+
 @pytest.mark.parametrize("D,F,tables,B,kernel", [(3, 2, [1 << 12] * 8, 1 << 16, "permutoTableGradKernel<D=3,8 parts>"), (2, 4, [1 << 8] * 4, 4099, "permutoTableGradKernel<D=2,positions>"),
                                                   (3, 1, [1 << 15] * 3, 70001, "permutoTableGradKernel<D=3,6 parts>")])
 @pytest.mark.parametrize("where", ["positions", "dOut"])

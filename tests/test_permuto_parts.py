@@ -26,6 +26,15 @@ extern "C" int cut(const CvPermutoDesc* d, uint32_t* out, uint32_t* sliced)
     *sliced = ok ? t.sliced : 0;
     return ok ? (int)t.count : -1;
 }
+extern "C" int beside(uint32_t count, uint32_t elems, uint32_t batch, uint32_t cus, uint32_t* groups)
+{
+    cv::TableParts t{};
+    t.count = count;
+    for (uint32_t p = 0; p < count; ++p) t.part[p].elems = p + 1 < count ? 1u : elems;
+    cv::dealGroups(t, batch, cus);
+    *groups = t.groups;
+    return cv::positionsBeside(t, batch, cus);
+}
 extern "C" int meet(const uint64_t* a, const uint64_t* b, uint32_t rows) { return cv::rowsMeet({a[0], a[1], a[2]}, {b[0], b[1], b[2]}, rows); }
 """
 
@@ -132,3 +141,14 @@ def test_rows_that_meet(built):
         assert not meet((at, 64, 12), (at + 12, 64, 52), 1)
         assert not meet((at, 1 << 33, 12), (at + 12, 0, 12), 1)             # one row: its stride says nothing
         assert meet((at, 1 << 33, 12), (at + (1 << 40), 4, 4), 200)
+
+
+@pytest.mark.parametrize("count,elems,batch,groups,one", [
+    (8, 8192, 31 * 1024, 31, False), (8, 8192, 31 * 1024 + 1, 32, True), (8, 8192, 1 << 18, 64, True),       # fewer positions than workgroups
+    (3, 16384, 1 << 18, 85, True), (2, 10240, 1 << 18, 256, True), (2, 10241, 1 << 18, 128, True),           # half of the LDS
+    (144, 20480, 1 << 16, 1, True), (144, 20480, (1 << 16) + 1, 1, False), (144, 20480, 1 << 18, 1, False),  # more than 128 parts: not every compute unit
+    (129, 10241, 1 << 18, 1, False), (128, 20480, 1 << 17, 2, True), (128, 20480, (1 << 17) + 1, 2, False), (64, 20480, 1 << 20, 4, True),
+    (144, 20480, 1, 1, False), (144, 20480, (1 << 32) - 1, 1, False), (85, 20480, (1 << 32) - 1, 3, True)])
+def test_one_launch_for_table_and_positions(built, count, elems, batch, groups, one):
+    got = ctypes.c_uint32()
+    assert (bool(built.beside(count, elems, batch, 256, ctypes.byref(got))), got.value) == (one, groups)
