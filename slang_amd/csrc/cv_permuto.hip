@@ -349,8 +349,10 @@ static_assert(sizeof(PermutoArgs) + sizeof(TableParts) <= 4096, "kernel argument
 // workgroup's first waves take its units of positions and the others that much more of the table's (2^18 positions in 3
 // dimensions, 8 levels of 2^12 two-feature entries: 40 us; 54.5 with the positions as a kernel of their own behind this one).  SLICED: some part is a slice of a level.
 constexpr int kPosNone = 0, kPosInPass = 1, kPosBeside = 2;
-template <int D, int FT, int POS, bool SLICED, bool PLAIN>
-__global__ __launch_bounds__(1024, D <= 4 && FT > 0 ? 8 : 4) void permutoTableGradKernel(const PermutoArgs a, const TableParts parts)
+// WAVES: on a SIMD; eight where two workgroups share a compute unit (64 registers a wave, two to thirteen of which spill in four
+// dimensions or with four features and positions in the same pass), else four.
+template <int D, int FT, int POS, bool SLICED, bool PLAIN, int WAVES>
+__global__ __launch_bounds__(1024, WAVES) void permutoTableGradKernel(const PermutoArgs a, const TableParts parts)
 {
     extern __shared__ double ldsTable[];
     // workgroup w: part w / groups, so that the workgroups of all parts that read the same positions (w % groups) sit on one
@@ -466,14 +468,24 @@ hipError_t launchEncode(hipStream_t stream, const PermutoArgs& a)
     return hipGetLastError();
 }
 
-template <int D, int FT, int POS, bool SLICED, bool PLAIN>
-hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, const TableParts& t)
+template <int D, int FT, int POS, bool SLICED, bool PLAIN, int WAVES>
+hipError_t launchTableGradWaves(hipStream_t stream, const PermutoArgs& a, const TableParts& t)
 {
-    const size_t lds = (size_t)largestPart(t) * 8;
-    const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED, PLAIN>>((int)(kPartMost * 8));
+    const hipError_t e = allowDynamicLds<permutoTableGradKernel<D, FT, POS, SLICED, PLAIN, WAVES>>((int)(kPartMost * 8));
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((permutoTableGradKernel<D, FT, POS, SLICED, PLAIN>), dim3(t.count * t.groups), dim3(1024), lds, stream, a, t);
+    hipLaunchKernelGGL((permutoTableGradKernel<D, FT, POS, SLICED, PLAIN, WAVES>), dim3(t.count * t.groups), dim3(1024), (size_t)largestPart(t) * 8, stream, a, t);
     return hipGetLastError();
+}
+template <int D, int FT, int POS, bool SLICED, bool PLAIN>
+hipError_t launchTableGrad(hipStream_t stream, const PermutoArgs& a, const TableParts& t, int cus)
+{
+    constexpr bool kSmall = D <= 4 && FT > 0;
+    // (one part, table and positions in a pass: 64 registers are too few for some, so a table or a batch that puts one workgroup on a
+    // compute unit has twice as many; 4 dimensions, one level of 2^12 four-feature entries, 2^18 positions: 22.4 -> 20.9 us)
+    if constexpr (kSmall && POS == kPosInPass) {
+        if (largestPart(t) > kPartHalf || t.count * t.groups <= (uint32_t)cus) return launchTableGradWaves<D, FT, POS, SLICED, PLAIN, 4>(stream, a, t);
+    }
+    return launchTableGradWaves<D, FT, POS, SLICED, PLAIN, kSmall ? 8 : 4>(stream, a, t);
 }
 
 template <int D, int FT, bool PLAIN>
@@ -487,7 +499,7 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     if (cut) dealGroups(t, a.batch, (uint32_t)cus);
     if (cut && t.count == 1 && a.dPos) {
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
-        return launchTableGrad<D, FT, kPosInPass, false, PLAIN>(stream, a, t);
+        return launchTableGrad<D, FT, kPosInPass, false, PLAIN>(stream, a, t, cus);
     }
     // Two launches against one: a handful of positions whose few additions hardly meet is done sooner by the one kernel that adds
     // in memory.  It takes 7.4 to 8.1 us per call back to back and the pair 11.5 to 13.5 (16 positions on 3 levels of 2^10
@@ -504,10 +516,10 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
         const bool apart = a.dPos && !rowsMeet(dPos, pos, a.batch) && !rowsMeet(dPos, dOut, a.batch);
         if (apart && positionsBeside(t, a.batch, (uint32_t)cus)) {
             noteKernel(false, "permutoTableGradKernel<D=%d,%u parts,positions beside>", D, t.count);
-            return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t);
+            return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t, cus);
         }
         noteKernel(false, "permutoTableGradKernel<D=%d,%u parts>", D, t.count);
-        const hipError_t e = t.sliced ? launchTableGrad<D, FT, kPosNone, true, PLAIN>(stream, a, t) : launchTableGrad<D, FT, kPosNone, false, PLAIN>(stream, a, t);
+        const hipError_t e = t.sliced ? launchTableGrad<D, FT, kPosNone, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosNone, false, PLAIN>(stream, a, t, cus);
         if (e != hipSuccess || !a.dPos) return e;
         noteKernel(true, "permutoBackwardKernel<D=%d,positions>", D);
         hipLaunchKernelGGL((permutoBackwardKernel<D, FT, true, false, PLAIN>), grid, block, 0, stream, a);

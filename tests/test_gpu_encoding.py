@@ -296,6 +296,27 @@ def test_permuto_backward_positions_beside_the_table(D, F, tables, B, parts):
     assert torch.linalg.norm(d_table - want_table) <= 2.0 ** -16 * torch.linalg.norm(want_table)
 
 
+@pytest.mark.parametrize("D,F,size", [(4, 4, 256), (4, 4, 255), (3, 4, 256), (4, 1, 1024)])
+def test_permuto_backward_in_one_pass_of_one_and_two_workgroups(D, F, size):
+    # one part of half the LDS or less, table and positions in a pass: up to 256 x 1024 positions one workgroup on a compute unit,
+    # beyond that two, whose waves have half the registers.  Position gradients are the same, bit for bit.
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the batches are those of 256 compute units")
+    L, B, part = 4, 256 * 1024 + 77, 256 * 1024
+    enc = cv.PermutoEncoder(D, F, 4, L, baseScale=4.0, log2PerLevelScale=0.5, seed=3)
+    for l in range(L):
+        enc.desc.levelInfo[l].featureTableSize, enc.desc.levelInfo[l].offsetOfFeatureTable = size, size * l
+    rng = np.random.default_rng(D * F + size)
+    pos, table, g = (to_dev(rng.standard_normal(s).astype(np.float32)) for s in ((B, D), size * L * F, (B, L * F)))
+    pos[torch.randint(0, B, (20,), device=DEV)] *= 3e6                # beyond LatticeSimplex's reach
+    d_pos, d_table = enc.backward(pos, table, g)
+    assert cv.lastKernelName() == "permutoTableGradKernel<D=%d,positions>" % D
+    a_pos, want = enc.backward(pos[:part], table, g[:part])
+    b_pos, _ = enc.backward(pos[part:], table, g[part:], dFeatureTable=want)
+    assert torch.equal(d_pos, torch.cat((a_pos, b_pos)))
+    assert torch.linalg.norm((d_table - want).double()) <= 2.0 ** -16 * torch.linalg.norm(want.double())
+
+
 def test_permuto_backward_of_many_parts():
     # 144 parts, one workgroup each: the positions beside them up to 2^16, by a kernel of their own beyond
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
