@@ -159,6 +159,7 @@ __global__ __launch_bounds__(1024) void permutoEncodePairsKernel(const PermutoAr
 {
     typedef typename PermutoEntry<T, F>::type Entry;
     extern __shared__ __align__(16) uint8_t ldsRaw[];
+    static_assert(sizeof(LatticeLevel<D>) <= sizeof(CvPermutoLevelInfo), "the records' room in LDS is that of the description's");
     LatticeLevel<D>* levels = (LatticeLevel<D>*)ldsRaw;
     const T* ldsTable = (const T*)(ldsRaw + kMaxLevels * sizeof(CvPermutoLevelInfo));
     const uint32_t L = a.desc.maxLevels;

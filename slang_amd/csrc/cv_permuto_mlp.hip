@@ -45,6 +45,7 @@ __global__ __launch_bounds__(1024) void permutoMlpKernel(const PermutoMlpArgs pa
     const GenArgs& ga = pa.net;
     const MlpArgs& a = ga.mlp;
     genericStage<Mma>(ga, lds);
+    static_assert(sizeof(LatticeLevel<D>) <= sizeof(CvPermutoLevelInfo), "the records' room in LDS is that of the description's");
     LatticeLevel<D>* levels = (LatticeLevel<D>*)(lds + pa.levelDword);
     {
         if (threadIdx.x < pa.desc.maxLevels) levels[threadIdx.x] = latticeLevel<D>(pa.desc.levelInfo[threadIdx.x]);

@@ -102,6 +102,7 @@ __global__ __launch_bounds__(64 * WAVES) void permutoWide16Kernel(const PermutoW
     typedef typename PermutoEntry<half_t, F>::type Entry;
     extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
     {
+        static_assert(sizeof(LatticeLevel<D>) <= sizeof(CvPermutoLevelInfo), "the records' room in LDS is that of the description's");
         if (threadIdx.x < pa.desc.maxLevels) ((LatticeLevel<D>*)dyn)[threadIdx.x] = latticeLevel<D>(pa.desc.levelInfo[threadIdx.x]);
         const Entry* t = (const Entry*)pa.table;
         Entry* dst = (Entry*)(dyn + kWideLevelBytes);

@@ -509,3 +509,33 @@ def test_encoder_with_all_levels_in_use(D, F, levels_n, log2, dims, B, reach):
     want2 = cv.mlpForward(layers, feats2)
     assert torch.equal(enc.encodeAndEval(pos, table, layers), want2)
     assert torch.equal(enc.encodeAndEval(pos, table, layers, flags=cv.FLAG_FORWARD_TILE16), want2)
+
+
+@pytest.mark.parametrize("D", [1, 2, 3, 4])
+def test_encoder_at_half_way_values(D):
+    # The rounding to the nearest lattice point on the GPU (one instruction where D + 1 is a power of two) against the steps as the
+    # reference has them, which a wave takes when one of its positions is out of reach: values in the middle between two lattice
+    # points, their neighbours among the floats, and any others, up to the reach.
+    L, F, log2, B = 1, 4, 12, 1 << 21
+    enc = cv.PermutoEncoder(D, F, log2, L, baseScale=1.0, log2PerLevelScale=0.0, seed=1)
+    lv = enc.desc.levelInfo[0]
+    for d in range(D):
+        lv.scalesPerDim[d], lv.shiftsPerDim[d] = 1.0, 0.0
+    reach = 4194304.0 / sum(d + 2 for d in range(D))
+    rng = np.random.default_rng(D)
+    pos = (rng.integers(-1 << 22, 1 << 22, (B, D)) * 0.5 * np.exp2(-rng.integers(0, 21, (B, 1)))).astype(np.float32)
+    pos = np.where(rng.random((B, D)) < 0.7, np.rint(2 * pos) / 2, pos).astype(np.float32)          # whole and half numbers
+    if D == 1:
+        pos[: 1 << 20, 0] = np.arange(1 << 20) * 2.0 + 1 - (1 << 20)                                # every middle to 2^20
+    step = np.where(pos == 0, 0, rng.integers(-1, 2, (B, D)))     # (values below 2^-147 count as zero)
+    pos = np.where(step == 0, pos, np.nextafter(pos, np.where(step > 0, np.inf, -np.inf).astype(np.float32))).clip(-reach, reach)
+    table = to_dev(rng.standard_normal(enc.featureTableElements).astype(np.float32))
+    pos = to_dev(pos.astype(np.float32))
+    far = pos.clone()
+    far[::64] = 1e30
+    got, want = enc.encode(pos, table), enc.encode(far, table)
+    keep = torch.arange(B, device=DEV) % 64 != 0
+    assert torch.equal(got[keep].view(torch.int32), want[keep].view(torch.int32))
+    g = to_dev(rng.standard_normal((B, F)).astype(np.float32))
+    got, want = enc.backward(pos, table, g)[0], enc.backward(far, table, g)[0]
+    assert torch.equal(got[keep], want[keep]), pos[keep][(got != want)[keep].any(dim=1)][:8]
