@@ -196,6 +196,11 @@ CV_API CvResult cvConvertMatrices(void* stream, void* dstBuffer, const CvMatrixD
  *
  * W is M x k unless `transpose`, in which case memory holds k x M and is used transposed.
  * Float types accumulate in fp32, integer types in int32 (exact).
+ * FLOAT32 throughout: up to 192 terms (m <= 16), 320 (m <= 32) or 384 (more rows) an operand is multiplied as three exact bfloat16
+ * pieces and a result is nearer to the exact sum than a chain of fp32 roundings, beyond that it is such a chain.  Products of pieces
+ * lose their lowest bits in one direction: where inputs of one sign meet many sizes, the mean of a row's errors over all samples is 1e-8
+ * to 2e-8 of the row's mean (1e-10 to 1e-9 in the chain), which a program that sums results over the batch, as gradients are, may
+ * want to know.  Training steps (cvMlpTrainStep) use the chain.
  * Type combinations: those with a matrix instruction (cvQuerySupportedCombinations lists all), and, for
  * the rest of the fallback's switch (hlsl.meta.slang:32866-32907), every mix of SINT8/16/32/64, UINT8/16/32/64,
  * FLOAT16, FLOAT32 and FLOAT64 for vector, matrix, bias and result (FLOAT16/32/64, SINT32/64 or UINT32/64):

@@ -22,7 +22,8 @@
 //
 // What bounds it: float: the matrix pipeline (v_mfma_f32_16x16x4_f32 takes 32 cycles for what two 4-byte reads supply).
 // half: waiting, for operands from LDS (one 16-byte read per lane and operand feeds 16 cycles of the pipeline) and at the
-// meetings.  Five float layers up to 64 wide and five layers beyond 64 spill.
+// meetings.  Five float layers up to 64 wide spill 100 registers (196 bytes a lane; 16-64-64-64-64-2 over 2^17 samples 159 us, and
+// 169 us with 38 of them while the weights were staged element by element), five half layers beyond 64 wide 13 (44 bytes).
 // 16-128-128-128-8 (half) over 200 003 samples: 151 us, 724 us over the whole batch in memory.  187 us while the weights were staged
 // element by element (now in 16-byte pieces, all layers requested together) and half networks wider than 64 kept part of the
 // prefetched input in scratch memory, so that each round began with a wait for memory.
