@@ -92,17 +92,12 @@ __global__ __launch_bounds__(256 * equalWaves(HT), equalWaves(HT)) void mlpChain
     const bool quads = out % 4 == 0 && a.outAlign >= 16u;
 
     // the input as mlpChainKernel loads it: a descriptor of exactly the tile's vectors, what lies beyond reads as zero
-    uint32_t off[KT0][UNITS];
-#pragma unroll
-    for (int kt = 0; kt < KT0; ++kt)
-#pragma unroll
-        for (int u = 0; u < UNITS; ++u) {
-            const uint32_t q = kt * 8 + u * UDW, col = g * gs0 + q;
-            off[kt][u] = q < gs0 && col < in0 ? (uint32_t)n * (uint32_t)a.inStride + col * 4u : kChainOutside;
-        }
+    const uint32_t col0 = g * gs0, have = col0 < in0 ? min(gs0, in0 - col0) : 0u, off0 = (uint32_t)n * (uint32_t)a.inStride + col0 * 4u;
     const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + 15) / 16), step = gridDim.x * waves;
     uint32_t raw[KT0][8];
     auto fetch = [&](uint32_t tile) {
+        uint32_t first0 = off0;
+        asm volatile("" : "+v"(first0));                 // (else the compiler keeps every offset over the tiles, and spills: 61-64-64-16 over 2^18 samples 41.7 -> 36.8 us)
         const uint32_t first = min(tile, numTiles - 1) * 16u, rows = tile < numTiles ? min(16u, a.batch - first) : 0u;
         const uint32_t bytes = rows ? (rows - 1) * (uint32_t)a.inStride + rowBytes : 0u;
         const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc((void*)(a.in + (size_t)first * a.inStride), 0, bytes, 0x00027000);
@@ -110,11 +105,12 @@ __global__ __launch_bounds__(256 * equalWaves(HT), equalWaves(HT)) void mlpChain
         for (int kt = 0; kt < KT0; ++kt)
 #pragma unroll
             for (int u = 0; u < UNITS; ++u) {
+                const uint32_t q = kt * 8 + u * UDW, at = q < have ? first0 + q * 4u : kChainOutside;
                 if constexpr (QUAD) {
-                    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, off[kt][u], 0, 0));
+                    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, at, 0, 0));
                     raw[kt][4 * u] = v.x; raw[kt][4 * u + 1] = v.y; raw[kt][4 * u + 2] = v.z; raw[kt][4 * u + 3] = v.w;
                 } else {
-                    raw[kt][u] = __builtin_amdgcn_raw_buffer_load_b32(src, off[kt][u], 0, 0);
+                    raw[kt][u] = __builtin_amdgcn_raw_buffer_load_b32(src, at, 0, 0);
                 }
             }
     };
