@@ -335,12 +335,13 @@ __global__ __launch_bounds__(256) void permutoBackwardKernel(const PermutoArgs a
 // The table gradient, by parts of the table small enough for LDS: part p covers elements [base, base + elems), which
 // levels [first, end) add to.  Every position adds to a handful of entries per level; added in memory, where many positions
 // meet on few addresses, 2^18 positions in 3 dimensions on 8 levels of 2^12 two-feature entries took 6.6 ms (2.5 G additions
-// per second); here 37 us, of which a quarter is the start and the sums' way to memory.  (cutTable: cv_permuto_parts.h)
+// per second); here 36 us, of which a quarter is the start and the sums' way to memory.  (cutTable: cv_permuto_parts.h)
 static_assert(sizeof(PermutoArgs) + sizeof(TableParts) <= 4096, "kernel arguments");
 
 // A workgroup owns one part and a share of the positions: it sums into LDS and adds its sums to memory once, coalesced
-// (180 G additions per second).  What bounds it: the LDS's additions (the waves of that case wait 46 % of their time for the LDS to
-// take one) and the vector instructions, 280 per position and level, which take 36 % of the port.  The sums are kept in double:
+// (180 G additions per second).  What bounds it: the LDS's additions and entries gathered from
+// memory (with the position gradients beside it, 40 us, the waves of that case wait 48 % of their time for operands and 15 % for the LDS
+// to take an instruction; the 351 vector instructions per position and level of both walks take 44 % of the port).  The sums are kept in double:
 // at random addresses gfx950 serves a ds_add_f64 in 8.6 ns per wave and compute unit and a ds_add_f32 in 80 (16 waves), so the
 // wider sum is also the cheaper one.  Lanes that meet on one address are served one after the other: 24 ns per LDS instruction
 // in that case, 41 ns on the few entries of four coarse levels in two dimensions (2^22 positions: 256 us).

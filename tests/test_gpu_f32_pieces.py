@@ -1,4 +1,4 @@
-"""fp32 matrix products as sums of bfloat16 pieces (F32Mma, slang_amd/csrc/cv_device.h): accuracy against 64 bits, infinities,
+"""fp32 matrix products as sums of bfloat16 pieces (F32Mma, slang_amd/csrc/cv_device.h), and where the fp32 instruction stays: accuracy against 64 bits, infinities,
 NaN, the largest and the smallest values, and the kernel for equal hidden layers against the chain of single-layer operators.
 
 Bound of a sum of K terms: an operand (times 2^24) is three pieces exactly; of the nine products the three dropped ones are below 2^-26 of the
