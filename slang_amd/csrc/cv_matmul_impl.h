@@ -17,13 +17,13 @@
 //    of 128 B is read by four lanes with two 16-byte loads each and written the same way;
 //  - bias seeds the accumulators; activation and the cast to the result type are fused.
 //
-// Two instantiations per shape: FAST (full-width aligned vectors, m a multiple of 16, no
-// leaky ReLU, no accumulate form: a branch-free streaming loop) and the general one (ragged
-// shapes, unaligned vectors, `this += ...`, every activation).
-//
-// Shapes beyond the register-resident ones: more than 128 rows are served in blocks of rows
-// (one launch per block, MatMulArgs::rowOff), more than four k-tiles by matmulLargeKernel, which
-// keeps its block of the matrix in LDS and walks the k-tiles in a loop.
+// This kernel serves the shapes it streams best (FAST: full-width aligned vectors, at most 128
+// rows and four k-tiles, both powers of two, no leaky ReLU, no accumulate form: a branch-free loop).
+// Everything else up to eight k-tiles (ragged shapes, unaligned vectors, `this += ...`, every
+// activation, more rows) runs on cv_matmul_packed.h, and what has more k-tiles on
+// matmulLargeKernel, which keeps a block of rows in LDS and walks the k-tiles in a loop (one launch
+// per block, MatMulArgs::rowOff).  The less common flavours (kPackedRows) have a general
+// instantiation of this kernel instead.
 #pragma once
 #include <type_traits>
 
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(256, kInPieces<Fl> ? 2 : 1) void matmulKernel(const
 #pragma unroll
                     for (int d = 0; d < IRAW; ++d) {
                         x[d] = buf[kt * IRAW + d];
-                        if (a.inUnsigned) x[d] ^= FAST ? 0x80808080u : signFlipMask(kt * IRAW + d, validBytes);
+                        if (a.inUnsigned) x[d] ^= 0x80808080u;
                         if (a.matUnsigned) xSum += sumSignedBytes(x[d]);
                     }
                     Fl::decodeIn(x, bfrag);
@@ -460,14 +460,10 @@ __global__ __launch_bounds__(256, kInPieces<Fl> ? 2 : 1) void matmulKernel(const
             for (int t = 0; t < MT; ++t) acc[t] = SumOf<Fl>::finish(sum[t], lo.bias[t]);
             if constexpr (F32) {
                 if (any) {
-                    // (registers: the general kernel reads the vectors again, both the matrix afterwards)
+                    // (registers: the matrix is read again afterwards)
                     uint32_t x[SLOT_DW];
-                    if constexpr (!FAST) {
-                        loadSlots<SLOT_DW>(x, inLane + (size_t)min(t0 * TILE + 16 * j + n, lastSample) * a.inStride, validBytes, loadMode);
-                    } else {
 #pragma unroll
-                        for (int d = 0; d < SLOT_DW; ++d) x[d] = buf[d];
-                    }
+                    for (int d = 0; d < SLOT_DW; ++d) x[d] = buf[d];
 #pragma unroll
                     for (int t = 0; t < MT; ++t) {
                         F32Careful c;
@@ -737,6 +733,19 @@ __global__ __launch_bounds__(64 * LargeShape<Fl>::kWaves) void matmulLargeKernel
     }
 }
 
+} // namespace
+} // namespace cv
+#include "cv_matmul_packed.h"
+namespace cv {
+namespace {
+
+// kPackedRows: everything but the streaming form and k-tiles beyond the registers runs on cv_matmul_packed.h (the less common
+// flavours keep to the kernels above)
+template <class Fl>
+constexpr bool kPackedRows = std::is_same<Fl, VecAsMatrix<F16Mma>>::value || std::is_same<Fl, VecAsMatrix<Bf16Mma>>::value || std::is_same<Fl, VecAsMatrix<Fp8AsF16Mma>>::value ||
+                             std::is_same<Fl, VecAsMatrix<F32Mma>>::value || std::is_same<Fl, VecAsMatrix<F32WholeMma>>::value || std::is_same<Fl, VecAsMatrix<I8Mma>>::value ||
+                             std::is_same<Fl, I8AnySign>::value;
+
 #ifndef CV_MATMUL_NT_SMALL
 #define CV_MATMUL_NT_SMALL 2
 #endif
@@ -766,20 +775,40 @@ hipError_t launchOne(hipStream_t stream, const MatMulArgs& a, int numCUs, bool a
     return hipGetLastError();
 }
 
+// whole, aligned vectors on both sides, of the sizes the streaming instantiations are made for
+template <class Fl, typename OutT>
+bool streamingApplies(const MatMulArgs& a)
+{
+    if (!Fl::kStreaming || a.accumulate || a.act > kActRelu) return false;
+    const uint32_t kt = (uint32_t)a.k / (4u * Fl::kEpl), mt = (uint32_t)a.m / 16u, slotBytes = (uint32_t)Fl::kInRawDW * 4u * kt;
+    const uint32_t most = Fl::kWideFragments ? 2u : 4u, mostRows = Fl::kWideFragments ? 4u : 8u;
+    if ((uint32_t)a.k != 4u * Fl::kEpl * kt || (uint32_t)a.m != 16u * mt) return false;
+    if (kt == 0 || kt > most || (kt & (kt - 1u)) || mt == 0 || mt > mostRows || (mt & (mt - 1u))) return false;
+    return a.inAlign >= (slotBytes % 16u == 0 ? 16u : 8u) && a.outAlign >= (4u * mt * sizeof(OutT) % 16u == 0 ? 16u : 8u);
+}
+
+// samples that the streaming instantiations leave, or do not take
+template <class Fl, int MT, int KT, typename OutT>
+hipError_t launchRest(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append)
+{
+    if constexpr (kPackedRows<Fl>) {
+        // (a block of a larger matrix does not come here: its rows would begin inside the matrix)
+        hipError_t e = hipErrorInvalidValue;
+        return a.rowOff == 0 && launchPacked<Fl, OutT>(stream, a, numCUs, append, e) ? e : hipErrorInvalidValue;
+    } else {
+        return launchOne<Fl, MT, KT, OutT, false>(stream, a, numCUs, append);
+    }
+}
+
 template <class Fl, int MT, int KT, typename OutT>
 hipError_t launchShape(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append)
 {
-    constexpr uint32_t slotBytes = Fl::kInRawDW * 4 * KT;
     constexpr uint32_t tile = 16 * TileShape<MT, KT>::NT;
-    const bool fast = (uint32_t)a.k == 4u * Fl::kEpl * KT && a.m == 16 * MT &&
-                      a.inAlign >= (slotBytes % 16 == 0 ? 16u : 8u) &&
-                      a.outAlign >= ((4 * MT * sizeof(OutT)) % 16 == 0 ? 16u : 8u) &&
-                      !a.accumulate && a.act <= kActRelu;
     if constexpr (!Fl::kStreaming) {
-        return launchOne<Fl, MT, KT, OutT, false>(stream, a, numCUs, append);
+        return launchRest<Fl, MT, KT, OutT>(stream, a, numCUs, append);
     } else {
-        if (!fast) return launchOne<Fl, MT, KT, OutT, false>(stream, a, numCUs, append);
-        // whole tiles on the streaming kernel, the ragged tail (< one tile) on the general one
+        if (!streamingApplies<Fl, OutT>(a)) return launchRest<Fl, MT, KT, OutT>(stream, a, numCUs, append);
+        // whole tiles on the streaming kernel, the ragged tail (< one tile) by launchRest
         const uint32_t whole = a.batch / tile * tile;
         if (whole) {
             MatMulArgs b = a;
@@ -801,7 +830,7 @@ hipError_t launchShape(hipStream_t stream, const MatMulArgs& a, int numCUs, bool
         t.in += (size_t)whole * a.inStride;
         t.out += (size_t)whole * a.outStride;
         t.batch = a.batch - whole;
-        return launchOne<Fl, MT, KT, OutT, false>(stream, t, numCUs, append || whole != 0);
+        return launchRest<Fl, MT, KT, OutT>(stream, t, numCUs, append || whole != 0);
     }
 }
 
@@ -858,6 +887,15 @@ hipError_t dispatchBlock(hipStream_t stream, const MatMulArgs& a, int numCUs, bo
 template <class Fl, typename OutT>
 hipError_t dispatchShape(hipStream_t stream, const MatMulArgs& a, int numCUs)
 {
+    if constexpr (kPackedRows<Fl>) {
+        hipError_t packed;
+        // fp32 vectors of many aligned elements: six and more k-tiles of pieces leave no registers to read ahead with, and matmulLargeKernel reads
+        // aligned vectors as well.  Packed against large: 27 x 256 over 34 000 samples 21.8, 14.5 us, 64 x 256 over 200 000 94, 64 us; 8 x 188
+        // over 3 000 10.3, 8.2 us, 27 x 188 over 34 000 12.6, 11.2 us; but 100 x 256 over 3 000 16.5, 27.9 us and 27 x 188 over 200 000 39, 50 us.
+        const bool many = Fl::kWideFragments && a.inAlign >= 16u &&
+                          (a.k > 224 ? a.m <= 64 || a.batch >= 16384u : a.k > 160 && a.batch < 65536u && (a.m <= 32 || (a.m <= 64 && a.batch >= 16384u)));
+        if (!many && !(a.m <= 128 && streamingApplies<Fl, OutT>(a)) && launchPacked<Fl, OutT>(stream, a, numCUs, false, packed)) return packed;
+    }
     const uint32_t kt = optKT((uint32_t)a.k, Fl::kEpl);
     int blockTiles = 8, largeKT = 0;
     const bool inRegisters = Fl::kWideFragments ? (kt <= 2 && a.m <= 64) : kt <= 4;

@@ -1,0 +1,602 @@
+// cv_matmul_packed.h -- the batched matMul for vectors of any length and alignment.
+//
+// Vectors.  A wave takes 16 * NT samples at a time and a lane its k-slots of a sample in reads of 16 bytes at whatever element
+// they begin, a tile ahead; what lies behind the end of a vector (of the next one) is cleared in registers.  The samples whose reads
+// would leave the buffer, the last few of a batch, are read element by element.
+// Results.  A tile's results meet in the wave's own part of the LDS, whole rows or segments of them, exactly as they lie in
+// memory, and leave in pieces of 16 bytes at whatever element these begin; packed vectors of any length are one block, 16 of which
+// are a whole number of pieces.
+// Matrix.  The whole of it lies in LDS in fragment order, one copy to a workgroup of eight waves; the row tiles are a loop, so
+// that one kernel serves every number of rows (tile t: rows 16t .. 16t+15).  A matrix beyond the LDS is split by row tiles
+// (blockIdx.y).
+// Sums are formed as in matmulKernel and matmulLargeKernel on MatMulArgs alone (the same k-slots in the same instructions): the same bits.
+//
+// What it replaced: loads and stores of single elements wherever k, m or an address was no multiple of 16 bytes, one launch for every 128
+// rows, and a matrix gathered element by element for every such launch (before, now; us): half 79 x 29 over 221 953 samples 110, 18.8;
+// bfloat16 18 x 221 over 129 870 245, 26.7; int8 221 x 9 over 292 087 306, 60 (5.1 TB/s; floor 52); fp32 18 x 238 over 60 333 74, 16.9;
+// bfloat16 156 x 211 over 16 447 144, 15; half 256 x 256 over 400 000 213, 141.  200 sizes between 8 and 256 over 2^10 to 2^22 samples: 2.26
+// times as fast (geometric mean).  The largest are bound by HBM, small batches by launching and two trips to memory (matrix and
+// vectors are requested together), those between by the trip of a tile while few waves find registers or LDS.
+// Vectors staged through LDS in whole pieces took as long as read directly, 1.2 to 1.6 times for fp32 of many terms, and need the LDS.
+#pragma once
+
+namespace cv {
+namespace {
+
+struct PackedPlan {
+    int32_t mt, tb;                  // row tiles of the matrix, of a workgroup's block (blockIdx.y)
+    int32_t segment;                 // row tiles whose results wait in LDS together
+    uint32_t outRow;                 // bytes from one sample's results to the next in LDS
+    uint32_t stageBytes;             // a wave's part of the LDS
+    uint32_t outPieces, outMagic;    // 16-byte pieces of a row of results (a segment) and 2^20 / outPieces, rounded up; 0: one block
+    int32_t outElements;             // the results leave element by element
+    int32_t outLines;                // rows and segments of results are whole 128-byte lines: they pass by the caches (storeStream16)
+    uint64_t matBytes;               // RowMajor matrices at least a lane-chunk long: their bytes, else 0
+};
+
+// f(integral_constant<int, B>) ... f(integral_constant<int, E - 1>)
+template <int B, int E, class F>
+void forEach(F&& f)
+{
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        forEach<B + 1, E>(f);
+    }
+}
+
+// 16-byte (8-byte) accesses of LDS and memory at the alignment of an element
+template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose16 { u32x4 v; };
+template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose8 { u32x2 v; };
+
+template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose4 { uint32_t v; };
+
+template <int ALIGN, int DW>
+__device__ __forceinline__ void loadLoose(const uint8_t* q, uint32_t (&x)[DW])
+{
+    if constexpr (DW % 4 == 0) {
+#pragma unroll
+        for (int d = 0; d < DW; d += 4) {
+            const u32x4 v = ((const Loose16<ALIGN>*)(q + 4 * d))->v;
+            x[d] = v.x; x[d + 1] = v.y; x[d + 2] = v.z; x[d + 3] = v.w;
+        }
+    } else {
+        const u32x2 v = ((const Loose8<ALIGN>*)q)->v;
+        x[0] = v.x; x[1] = v.y;
+    }
+}
+
+// The same where what is read may end beyond `end`, behind which nothing is read and zeros stand (at least 16 bytes lie before it).
+template <int ALIGN, int DW>
+__device__ __forceinline__ void loadUpTo(const uint8_t* q, const uint8_t* end, uint32_t (&x)[DW])
+{
+    constexpr int P = DW % 4 == 0 ? 4 : 2;      // dwords of a read
+#pragma unroll
+    for (int d0 = 0; d0 < DW; d0 += P) {
+        const uint8_t* at = q + 4 * d0;
+        const int64_t over = (at + 4 * P) - end;
+        const int shift = (int)(over < 0 ? 0 : over > 4 * P ? 4 * P : over), words = shift >> 2;
+        uint32_t v[2 * P + 1];
+        uint32_t part[P];
+        loadLoose<ALIGN>(over > 0 ? end - 4 * P : at, part);
+#pragma unroll
+        for (int i = 0; i < 2 * P + 1; ++i) v[i] = i < P ? part[i < P ? i : 0] : 0u;
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+            for (int w = 0; w <= P; ++w) {
+                lo = words == w ? v[i + w] : lo;
+                hi = words == w ? v[i + w + 1 <= 2 * P ? i + w + 1 : 2 * P] : hi;
+            }
+            x[d0 + i] = __builtin_amdgcn_alignbyte(hi, lo, shift & 3);
+        }
+    }
+}
+
+// clears all but the first `bytes` bytes (none if that is negative)
+template <int ESZ, int DW>
+__device__ __forceinline__ void clearBehind(uint32_t (&x)[DW], int bytes)
+{
+#pragma unroll
+    for (int d = 0; d < DW; ++d) {
+        const int left = bytes - 4 * d;
+        if constexpr (ESZ == 4) x[d] = left > 0 ? x[d] : 0u;
+        else x[d] = left > 0 ? x[d] & (0xffffffffu >> max(32 - 8 * left, 0)) : 0u;
+    }
+}
+
+__device__ __forceinline__ void meetInWave()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Lane-chunks of row tiles t0 .. t0+tb-1 to LDS, row i of tile t being row 16 t + i.  The loads of several chunks of a thread are in
+// flight together: a RowMajor chunk is one read at whatever element it begins, one of a ColumnMajor matrix EPL elements.
+template <class Fl, int KT, int TOGETHER, class Store>
+__device__ __forceinline__ void stageRowTiles(const MatMulArgs& a, const PackedPlan& p, int t0, int tb, uint32_t gs, uint32_t xorByte, Store&& store)
+{
+    constexpr int EPL = Fl::kEpl, ESZ = Fl::kEsz, DW = Fl::kRawDW;
+    const int chunks = tb * KT * 64, rowsLane = 4 * p.mt;
+    const bool direct = fragmentSourceIsDirect<ESZ, EPL>(a.shape, a.transpose != 0, p.mt, KT, gs, (uint32_t)a.m, (uint32_t)a.k, 0, xorByte);
+    const bool columns = a.shape.layout == kColumnMajor && !a.transpose;
+    const size_t line = a.shape.stride ? a.shape.stride : (size_t)(columns ? a.shape.rows : a.shape.cols) * ESZ;
+    for (int c0 = threadIdx.x; c0 < chunks; c0 += TOGETHER * blockDim.x) {
+        uint32_t v[TOGETHER][DW];
+        if (p.matBytes || columns) {
+            int valid[TOGETHER];
+            const uint8_t* at[TOGETHER];
+#pragma unroll
+            for (int u = 0; u < TOGETHER; ++u) {
+                const int c = c0 + u * (int)blockDim.x, ln = c & 63, f = c >> 6;
+                const uint32_t row = (uint32_t)(16 * (t0 + f / KT) + (ln & 15)), q0 = (uint32_t)(f % KT * EPL), col = (uint32_t)(ln >> 4) * gs + q0;
+                valid[u] = 0;
+                if (c < chunks && row < (uint32_t)a.m && q0 < gs && col < (uint32_t)a.k) valid[u] = min(min((int)(gs - q0), a.k - (int)col), EPL);
+                at[u] = a.mat + (valid[u] ? columns ? (size_t)col * line + (size_t)row * ESZ : (size_t)row * line + (size_t)col * ESZ : 0);
+            }
+            if (columns) {
+                uint32_t e[TOGETHER][EPL];
+#pragma unroll
+                for (int u = 0; u < TOGETHER; ++u)
+#pragma unroll
+                    for (int s = 0; s < EPL; ++s) {
+                        const uint8_t* q = s < valid[u] ? at[u] + (size_t)s * line : a.mat;
+                        if constexpr (ESZ == 4) e[u][s] = *(const uint32_t*)q;
+                        else if constexpr (ESZ == 2) e[u][s] = *(const uint16_t*)q;
+                        else e[u][s] = *q;
+                    }
+#pragma unroll
+                for (int u = 0; u < TOGETHER; ++u)
+#pragma unroll
+                    for (int d = 0; d < DW; ++d) {
+                        if constexpr (ESZ == 4) v[u][d] = e[u][d];
+                        else if constexpr (ESZ == 2) v[u][d] = e[u][2 * d] | e[u][2 * d + 1] << 16;
+                        else v[u][d] = e[u][4 * d] | e[u][4 * d + 1] << 8 | e[u][4 * d + 2] << 16 | e[u][4 * d + 3] << 24;
+                    }
+            } else {
+                bool inside[TOGETHER];
+#pragma unroll
+                for (int u = 0; u < TOGETHER; ++u) {
+                    inside[u] = (size_t)(at[u] - a.mat) + EPL * ESZ <= p.matBytes;
+                    loadLoose<ESZ>(inside[u] ? at[u] : a.mat, v[u]);
+                }
+#pragma unroll
+                for (int u = 0; u < TOGETHER; ++u)
+                    if (!inside[u]) loadSlots<DW>(v[u], at[u], valid[u] * ESZ, 2);      // (the end of the last row)
+            }
+#pragma unroll
+            for (int u = 0; u < TOGETHER; ++u) {
+                if constexpr (ESZ == 1) {
+#pragma unroll
+                    for (int d = 0; d < DW; ++d) v[u][d] ^= xorByte * 0x01010101u;
+                }
+                clearBehind<ESZ>(v[u], valid[u] * ESZ);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < TOGETHER; ++u) {
+                // (beyond the end: chunk 0 once more, which is not stored)
+                const int c = c0 + u * (int)blockDim.x < chunks ? c0 + u * (int)blockDim.x : 0, ln = c & 63, f = c >> 6, kt = f % KT, row = 16 * (t0 + f / KT) + (ln & 15);
+                // the place of (row, kt) in the fragment order of cv_layout.h
+                const int src = (((row % rowsLane) / 4) * KT + kt) * 64 + (ln & 48) + 4 * (row / rowsLane) + (row & 3);
+                fetchFragmentChunk<ESZ, EPL>(v[u], a.mat, a.shape, a.transpose != 0, direct, p.mt, KT, gs, (uint32_t)a.m, (uint32_t)a.k, 0, xorByte, src);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < TOGETHER; ++u)
+            if (c0 + u * (int)blockDim.x < chunks) store(c0 + u * (int)blockDim.x, v[u]);
+    }
+}
+
+template <class Fl, int KT, int NT, typename OutT>
+__device__ __forceinline__ void packedRows(const MatMulArgs& a, const PackedPlan& p, uint8_t* lds)
+{
+    constexpr int EPL = Fl::kEpl, FD = Fl::kFD, IESZ = Fl::kInEsz, IRAW = Fl::kInRawDW;
+    constexpr bool F32 = kInPieces<Fl>;
+    constexpr int LANE_DW = F32 ? FD : Fl::kRawDW, OESZ = sizeof(OutT);
+    constexpr uint32_t S = 16 * NT;
+    typedef typename Fl::Acc Acc;
+    typedef typename std::conditional<Fl::kIsFloat, float, int>::type BiasT;
+
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int t0 = (int)blockIdx.y * p.tb, tb = min(p.tb, p.mt - t0);
+    uint32_t* const ldsW = (uint32_t*)lds;
+    BiasT* const ldsBias = (BiasT*)(lds + (size_t)p.tb * KT * 64 * LANE_DW * 4);
+    uint8_t* const stage = (uint8_t*)(ldsBias + 16 * p.tb) + wave * p.stageBytes;
+
+    const uint32_t gs = optGS((uint32_t)a.k);
+    const uint32_t numTiles = (uint32_t)(((uint64_t)a.batch + S - 1) / S), tileStride = gridDim.x * waves;
+    uint32_t tile = blockIdx.x * waves + wave;
+
+    // which of a lane's k-slots exist: in every lane all of the first wholeFragments fragments' ones
+    const int colBase = (int)(g * gs), validBytes = min((int)gs, max(a.k - colBase, 0)) * IESZ;
+    const int wholeFragments = min((int)gs, max(a.k - 3 * (int)gs, 0)) / EPL;
+    constexpr bool MASK = Fl::kIsFloat || Fl::kAnySign;      // (signed bytes: what has no weight adds nothing)
+
+    // a tile whose lanes' reads, up to the last k-slot of the last lane group, end inside the buffer
+    const uint64_t inEnd = (uint64_t)(a.batch - 1) * a.inStride + (uint64_t)a.k * IESZ;
+    auto inside = [&](uint32_t t) { return ((uint64_t)t * S + S - 1) * a.inStride + (3 * gs + KT * EPL) * IESZ <= inEnd; };
+    const int tailSlots = (int)gs - (KT - 1) * EPL, tailDwords = tailSlots * IESZ == 12 ? 4 : tailSlots * IESZ / 4;
+    uint32_t raw[NT][KT][IRAW] = {};
+    auto request = [&](uint32_t t) {
+        const uint8_t* q = a.in + ((uint64_t)t * S + n) * a.inStride + colBase * IESZ;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                const uint8_t* at = q + (uint64_t)(16 * j) * a.inStride + kt * EPL * IESZ;
+                if (kt + 1 == KT && tailDwords < IRAW) {
+                    // no more of the last fragment than some lane needs (what is not read has no weight, and is cleared)
+                    if (tailDwords == 1) raw[j][kt][0] = ((const Loose4<IESZ>*)at)->v;
+                    if (IRAW > 2 && tailDwords == 2) { const u32x2 v = ((const Loose8<IESZ>*)at)->v; raw[j][kt][0] = v.x; raw[j][kt][IRAW > 2 ? 1 : 0] = v.y; }
+                    if (IRAW > 4 && tailDwords == 4) { const u32x4 v = ((const Loose16<IESZ>*)at)->v; raw[j][kt][0] = v.x; raw[j][kt][1] = v.y; raw[j][kt][IRAW > 4 ? 2 : 0] = v.z; raw[j][kt][IRAW > 4 ? 3 : 0] = v.w; }
+                    continue;
+                }
+                loadLoose<IESZ>(at, raw[j][kt]);
+            }
+    };
+    constexpr bool AHEAD = !F32 || KT <= 4;      // the next tile is requested before this one's products (registers)
+
+    if (AHEAD && tile < numTiles && inside(tile)) request(tile);
+
+    // ---- the block of the matrix and of the bias (whose loads overlap)
+    auto biasOf = [&](int i) {
+        const int row = 16 * t0 + i;
+        if constexpr (Fl::kIsFloat) return (a.bias && row < a.m) ? loadAsFloat(a.bias + (size_t)row * elemSize(a.biasCt), a.biasCt) : 0.f;
+        else return (a.bias && row < a.m) ? ((const int32_t*)a.bias)[row] : 0;
+    };
+    const BiasT firstBias = (int)threadIdx.x < 16 * tb ? biasOf(threadIdx.x) : (BiasT)0;
+    bool matBeyond = false;                   // F32Mma::beyond of the matrix
+    {
+        uint32_t most = 0u;
+        auto store = [&](int c, uint32_t (&v)[Fl::kRawDW]) {
+            if constexpr (F32) {
+                uint32_t pieces[FD];
+                const uint32_t own = Fl::largestBits(v, 8, 0u);
+                Fl::decode(v, pieces);
+                if (own >= Fl::kExactBits) Fl::template decode<true>(v, pieces);
+                storeFragmentChunk<FD>(ldsW + (size_t)c * FD, pieces);
+                most = max(most, own);
+            } else {
+                storeFragmentChunk<LANE_DW>(ldsW + (size_t)c * LANE_DW, v);
+            }
+        };
+        const uint32_t xorByte = (Fl::kAnySign && a.matUnsigned) ? 0x80u : 0u;
+        if (tb * KT * 64 <= (int)blockDim.x) stageRowTiles<Fl, KT, 1>(a, p, t0, tb, gs, xorByte, store);
+        else stageRowTiles<Fl, KT, Fl::kEsz == 4 ? 2 : 4>(a, p, t0, tb, gs, xorByte, store);
+        if ((int)threadIdx.x < 16 * tb) ldsBias[threadIdx.x] = firstBias;
+        for (int i = threadIdx.x + blockDim.x; i < 16 * tb; i += blockDim.x) ldsBias[i] = biasOf(i);
+        if constexpr (F32) matBeyond = __syncthreads_or(most >= Fl::kBeyondBits);
+        else __syncthreads();
+        if constexpr (Fl::kAnySign) {
+            if (a.inUnsigned) {               // see addUnsignedRowTerm
+                for (int i = threadIdx.x; i < 16 * tb; i += blockDim.x) {
+                    int sum = 0;
+                    for (int f = 0; f < 4 * KT; ++f)
+#pragma unroll
+                        for (int d = 0; d < Fl::kRawDW; ++d) sum += sumSignedBytes(ldsW[(((i >> 4) * KT + (f >> 2)) * 64 + 16 * (f & 3) + (i & 15)) * Fl::kRawDW + d]);
+                    ldsBias[i] += 128 * sum + (a.matUnsigned ? 16384 * a.k : 0);
+                }
+                __syncthreads();
+            }
+        }
+    }
+
+    while (tile < numTiles) {
+        if (inside(tile)) {
+            if (!AHEAD) request(tile);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const uint8_t* q = a.in + min((uint64_t)tile * S + 16 * j + n, (uint64_t)(a.batch - 1)) * a.inStride + colBase * IESZ;
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt) {
+                    if (inEnd >= 16) loadUpTo<IESZ>(q + kt * EPL * IESZ, a.in + inEnd, raw[j][kt]);
+                    else loadSlots<IRAW>(raw[j][kt], q + kt * EPL * IESZ, validBytes - kt * EPL * IESZ, 2);
+                }
+            }
+        }
+        int valid = validBytes;
+        pinHere(valid);      // (the comparisons with it stay in the loop: hoisted, they take more scalar registers than there are)
+        uint32_t b[NT][KT][FD];
+        bool any[NT];
+        int xSum[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            float most = 0.f;
+            xSum[j] = 0;
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                uint32_t x[IRAW];
+#pragma unroll
+                for (int d = 0; d < IRAW; ++d) x[d] = raw[j][kt][d];
+                if constexpr (Fl::kAnySign) {
+#pragma unroll
+                    for (int d = 0; d < IRAW; ++d) x[d] ^= a.inUnsigned ? 0x80808080u : 0u;
+                }
+                if (MASK && kt >= wholeFragments) clearBehind<IESZ>(x, valid - kt * EPL * IESZ);
+                if constexpr (Fl::kAnySign) {
+                    if (a.matUnsigned) {
+#pragma unroll
+                        for (int d = 0; d < IRAW; ++d) xSum[j] += sumSignedBytes(x[d]);
+                    }
+                }
+                if constexpr (F32) most = Fl::largest(x, IRAW, most);
+                Fl::decodeIn(x, b[j][kt]);
+            }
+            if constexpr (F32) any[j] = matBeyond | Fl::beyond(most);
+            if constexpr (Fl::kAnySign) {
+                if (a.matUnsigned) xSum[j] = 128 * sumOverGroups(xSum[j]);
+            }
+        }
+        const uint32_t next = tile + tileStride;
+        if (AHEAD && next < numTiles && inside(next)) request(next);
+
+        for (int ts = 0; ts < tb; ts += p.segment) {
+            const int te = min(ts + p.segment, tb);
+            for (int t = ts; t < te; ++t) {
+                const Acc bias = *(const Acc*)(ldsBias + 16 * t + 4 * g);
+                typename SumOf<Fl>::T sum[NT];
+#pragma unroll
+                for (int j = 0; j < NT; ++j) sum[j] = SumOf<Fl>::start(bias);
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt) {
+                    const uint32_t* rawW = &ldsW[((t * KT + kt) * 64 + lane) * LANE_DW];
+                    uint32_t w[FD];
+                    if constexpr (F32) {
+#pragma unroll
+                        for (int d = 0; d < FD; ++d) w[d] = rawW[d];
+                    } else {
+                        Fl::decode(rawW, w);
+                    }
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) sum[j] = Fl::mma(w, b[j][kt], sum[j]);
+                }
+                const int left = a.m - (16 * (t0 + t) + 4 * g);
+                uint8_t* const o0 = stage + (uint32_t)n * p.outRow + (16 * (t - ts) + 4 * g) * OESZ;
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    Acc acc = SumOf<Fl>::finish(sum[j], bias);
+                    if constexpr (F32) {
+                        if (any[j]) {
+                            const uint8_t* row = a.in + min((uint64_t)tile * S + 16 * j + n, (uint64_t)(a.batch - 1)) * a.inStride + (size_t)colBase * IESZ;
+                            F32Careful c;
+                            c.start(bias);
+#pragma unroll 1
+                            for (int kt = 0; kt < KT; ++kt) {
+                                uint32_t x[IRAW];
+                                loadSlots<IRAW>(x, row + kt * EPL * IESZ, validBytes - kt * EPL * IESZ, 1);
+                                c.template step<true, false>(&ldsW[((t * KT + kt) * 64 + lane) * LANE_DW], x);
+                            }
+                            acc = c.finish(bias);
+                        }
+                    }
+                    if constexpr (Fl::kAnySign) {
+                        if (a.matUnsigned) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[r] += xSum[j];
+                        }
+                    }
+                    if constexpr (Fl::kIsFloat) {
+                        if (a.act == kActRelu) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[r] = acc[r] > 0.f ? acc[r] : 0.f;
+                        } else if (a.act == kActLeakyRelu) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                if constexpr (OESZ == 2) acc[r] = activate16<OutT>(acc[r], kActLeakyRelu, a.slope);
+                                else acc[r] = fmaxf(acc[r], acc[r] * a.slope);
+                            }
+                        } else if (a.act >= kActSigmoid) {
+#pragma unroll 1
+                            for (int r = 0; r < 4; ++r) {      // (one copy of their code)
+                                const float x = r == 0 ? acc[0] : r == 1 ? acc[1] : r == 2 ? acc[2] : acc[3];
+                                const float y = OESZ == 2 ? activate16<OutT>(x, a.act, 0.f) : smoothActivation(x, a.act);
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) acc[i] = r == i ? y : acc[i];
+                            }
+                        }
+                    } else {
+                        if (a.act == kActRelu) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[r] = max(acc[r], 0);
+                        }
+                    }
+                    uint8_t* const o = o0 + (uint32_t)(16 * j) * p.outRow;
+                    if constexpr (OESZ == 2) {
+                        const u32x2 v = {pack16<OutT>(acc[0], acc[1]), pack16<OutT>(acc[2], acc[3])};
+                        if (left >= 4) {
+                            ((Loose8<2>*)o)->v = v;
+                        } else {
+                            if (left > 0) ((uint16_t*)o)[0] = (uint16_t)v.x;
+                            if (left > 1) ((uint16_t*)o)[1] = (uint16_t)(v.x >> 16);
+                            if (left > 2) ((uint16_t*)o)[2] = (uint16_t)v.y;
+                        }
+                    } else {
+                        const u32x4 v = __builtin_bit_cast(u32x4, acc);
+                        if (left >= 4) {
+                            ((Loose16<4>*)o)->v = v;
+                        } else {
+                            if (left > 0) ((uint32_t*)o)[0] = v.x;
+                            if (left > 1) ((uint32_t*)o)[1] = v.y;
+                            if (left > 2) ((uint32_t*)o)[2] = v.z;
+                        }
+                    }
+                }
+            }
+            meetInWave();
+
+            // ---- these rows' results
+            const int row0 = 16 * (t0 + ts), rowsHere = min(a.m - row0, 16 * (te - ts));
+            const uint32_t bytes = (uint32_t)rowsHere * OESZ;
+            if (((uint64_t)tile + 1) * S <= a.batch && !p.outElements && (bytes >= 16u || !p.outPieces)) {
+                uint8_t* const base = a.out + (uint64_t)tile * S * a.outStride + (size_t)row0 * OESZ;
+                const uint32_t pieces = p.outPieces;
+                const uint32_t last = (pieces ? S * pieces : S * bytes / 16u) - 1u;
+#pragma unroll 4
+                for (uint32_t c0 = 0; c0 <= last; c0 += 64) {
+                    // (beyond the last piece that one again; a row's last pieces end where the row does)
+                    const uint32_t c = min(c0 + lane, last), row = pieces ? (c * p.outMagic) >> 20 : 0u;
+                    uint32_t at = 16u * (c - row * pieces);
+                    if (pieces) at = min(at, bytes - 16u);
+                    const u32x4 v = ((const Loose16<OESZ>*)(stage + row * p.outRow + at))->v;
+                    uint8_t* const to = base + row * (uint32_t)a.outStride + at;
+                    if (p.outLines) storeStream16(to, v);
+                    else ((Loose16<OESZ>*)to)->v = v;
+                }
+            } else {
+                // element by element: neighbouring lanes neighbouring elements of a vector
+                const uint32_t first = tile * S, rows = min(S, a.batch - first);
+                for (uint32_t row = 0; row < rows; ++row) {
+                    OutT* dst = (OutT*)(a.out + (uint64_t)(first + row) * a.outStride) + row0;
+                    for (int e = lane; e < rowsHere; e += 64) {
+                        OutT v = *(const OutT*)(stage + row * p.outRow + e * OESZ);
+                        if (a.accumulate) {
+                            if constexpr (OESZ == 2) v = (OutT)((float)dst[e] + (float)v);
+                            else v = dst[e] + v;
+                        }
+                        dst[e] = v;
+                    }
+                }
+            }
+            meetInWave();
+        }
+        tile = next;
+    }
+}
+
+constexpr uint32_t kPackedLds = 159u * 1024u;      // (__syncthreads_or has some of its own)
+// waves of a workgroup: eight, of which two workgroups find the registers on a compute unit; twelve of one where fp32 operands take more
+template <class Fl, int KT>
+constexpr int kPackedWaves = kInPieces<Fl> && KT > 2 ? 12 : 8;
+template <class Fl, int KT>
+constexpr int kPackedResident = kInPieces<Fl> ? 2 : Fl::kEsz == 4 && KT > 4 ? 2 : 4;      // waves of a SIMD at least
+// fp32 blocks beyond 64 rows or two k-tiles keep the name of the kernel that serves such blocks otherwise
+template <class Fl, int KT, int NT, typename OutT>
+__global__ __launch_bounds__((64 * kPackedWaves<Fl, KT>), (kPackedResident<Fl, KT>)) void matmulKernel(const MatMulArgs a, const PackedPlan p)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t ldsPacked[];
+    packedRows<Fl, KT, NT, OutT>(a, p, ldsPacked);
+}
+template <class Fl, int KT, int NT, typename OutT>
+__global__ __launch_bounds__((64 * kPackedWaves<Fl, KT>), (kPackedResident<Fl, KT>)) void matmulLargeKernel(const MatMulArgs a, const PackedPlan p)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t ldsPacked[];
+    packedRows<Fl, KT, NT, OutT>(a, p, ldsPacked);
+}
+
+template <class Fl, int KT, int NT, typename OutT, bool LARGE>
+hipError_t launchPackedSized(hipStream_t stream, const MatMulArgs& a, const PackedPlan& p, uint32_t ldsBytes, int waves, int numCUs, bool append)
+{
+    constexpr auto kernel = [] {
+        typedef void (*Kernel)(const MatMulArgs, const PackedPlan);
+        if constexpr (LARGE) return (Kernel)matmulLargeKernel<Fl, KT, NT, OutT>;
+        else return (Kernel)matmulKernel<Fl, KT, NT, OutT>;
+    }();
+    const hipError_t e = allowDynamicLds<kernel>((int)kPackedLds);
+    if (e != hipSuccess) return e;
+    int perCU = residentBlocksPerCU<kernel>(64 * kPackedWaves<Fl, KT>) * kPackedWaves<Fl, KT> / waves;
+    const int byLds = (int)(kPackedLds / ldsBytes);
+    if (perCU > byLds) perCU = byLds;
+    const uint32_t blocksY = (uint32_t)((p.mt + p.tb - 1) / p.tb);
+    const uint32_t tiles = (uint32_t)(((uint64_t)a.batch + 16 * NT - 1) / (16 * NT)), need = (tiles + waves - 1) / waves;
+    uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU / blocksY;
+    if (cap < 1) cap = 1;
+    noteKernel(append, "matmul%sKernel<%s,KT=%d,NT=%d,out=%dB,packed>", LARGE ? "Large" : "", Fl::kName, KT, NT, (int)sizeof(OutT));
+    hipLaunchKernelGGL(kernel, dim3(need < cap ? need : cap, blocksY), dim3(64 * waves), ldsBytes, stream, a, p);
+    return hipGetLastError();
+}
+
+// How rows of `bytes` bytes leave: as one block (pieces = 0) where they lie one behind the other, or in pieces of every row.  False: rows
+// shorter than a piece that are not packed.
+inline bool rowsInPieces(const void* base, uint64_t stride, uint32_t bytes, PackedPlan& p)
+{
+    p.outPieces = p.outMagic = 0u;
+    p.outRow = bytes % 16u ? bytes : bytes + 16u;      // (so that the 16 rows of a tile lie on different banks)
+    if (((uintptr_t)base & 15u) == 0 && stride == bytes && bytes % 16u) return true;
+    if (bytes < 16u || stride >= (1u << 26)) return false;
+    p.outPieces = (bytes + 15u) / 16u;
+    p.outMagic = ((1u << 20) + p.outPieces - 1u) / p.outPieces;
+    return true;
+}
+
+// false where the k-tiles are beyond the registers
+template <class Fl, typename OutT>
+bool launchPacked(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append, hipError_t& result)
+{
+    const uint32_t kt = optKT((uint32_t)a.k, Fl::kEpl), mt = optMT((uint32_t)a.m);
+    constexpr int kMostKT = Fl::kEpl == 16 ? 4 : 8;
+    if (kt > kMostKT) return false;
+    PackedPlan p = {};
+    p.mt = (int32_t)mt;
+    if (a.shape.layout == kRowMajor && !a.transpose) {
+        p.matBytes = matrixSize(a.shape);
+        if (p.matBytes < Fl::kEpl * Fl::kEsz) p.matBytes = 0;
+    }
+    const uint32_t fragment = 64u * 4u * (uint32_t)(kInPieces<Fl> ? Fl::kFD : Fl::kRawDW);
+    constexpr int kMostPairs = Fl::kEsz == 4 ? 2 : 4;      // k-tiles up to which a wave takes two tiles (registers)
+    const int mostWaves = kt > 2 ? kPackedWaves<Fl, 3> : kPackedWaves<Fl, 1>;
+    int nt = kt <= kMostPairs && a.batch / 32u >= (uint32_t)(numCUs * 8) ? 2 : 1;
+    uint32_t ldsBytes = 0;
+    int waves = mostWaves;
+    bool fits = false;
+    const uint32_t rowBytes = (uint32_t)a.m * (uint32_t)sizeof(OutT);
+    auto plan = [&](uint32_t blocks, uint32_t mostStage) {
+        p.tb = (int32_t)((mt + blocks - 1) / blocks);
+        const uint32_t tileBytes = 16u * nt * 16u * (uint32_t)sizeof(OutT);
+        p.outElements = a.accumulate;
+        p.segment = p.tb;
+        if (blocks == 1 && mt * tileBytes <= mostStage) {
+            if (!rowsInPieces(a.out, a.outStride, rowBytes, p)) p.outElements = 1;
+        } else {
+            const int most = (int)(mostStage / tileBytes);
+            if (most < p.tb) p.segment = most;
+            p.outPieces = (uint32_t)p.segment * (uint32_t)sizeof(OutT);
+            p.outRow = 16u * p.outPieces + 16u;
+            p.outMagic = ((1u << 20) + p.outPieces - 1u) / p.outPieces;
+            if (a.outStride >= (1u << 26)) p.outElements = 1;
+        }
+        p.stageBytes = (16u * nt * p.outRow + 15u) / 16u * 16u;
+        ldsBytes = (uint32_t)p.tb * (kt * fragment + 64u) + (uint32_t)waves * p.stageBytes;
+        fits = ldsBytes <= kPackedLds;
+        const uint32_t segmentBytes = p.segment == (int32_t)mt ? rowBytes : (uint32_t)p.segment * 16u * (uint32_t)sizeof(OutT);
+        p.outLines = (((uintptr_t)a.out | a.outStride | rowBytes | segmentBytes) & 127u) == 0;
+    };
+    // a batch that leaves compute units idle: the rows are split between them, down to a lane-chunk of the matrix a thread
+    const uint32_t groups = (uint32_t)(((uint64_t)a.batch + 16 * nt * mostWaves - 1) / (16 * nt * mostWaves));
+    uint32_t blocks = 1;
+    while (blocks < mt && groups * (blocks + 1) <= (uint32_t)numCUs && (mt + blocks - 1) / blocks * kt > 8u) ++blocks;
+    // where the LDS is short, fewer results wait, then a wave takes one tile, then the rows are split
+    const int wanted = nt;
+    for (; !fits && blocks <= mt; ++blocks)
+        for (int n = wanted; !fits && n >= 1; --n) {
+            nt = n;
+            for (uint32_t stage = 8192u; !fits && stage >= 2048u; stage /= 2u) plan(blocks, stage);
+        }
+    if (!fits) return false;
+    bool done = false;
+    forEach<1, kMostKT + 1>([&](auto kc) {
+        constexpr int K = decltype(kc)::value;
+        if ((int)kt != K) return;
+        auto launch = [&](auto nc, auto large) {
+            result = launchPackedSized<Fl, K, decltype(nc)::value, OutT, decltype(large)::value>(stream, a, p, ldsBytes, waves, numCUs, append);
+            done = true;
+        };
+        auto sized = [&](auto nc) {
+            if constexpr (Fl::kWideFragments) {
+                if (K > 2 || a.m > 64) return launch(nc, std::true_type{});
+            }
+            if constexpr (!Fl::kWideFragments || K <= 2) launch(nc, std::false_type{});
+        };
+        if constexpr (K <= kMostPairs) {
+            if (nt == 2) return sized(std::integral_constant<int, 2>{});
+        }
+        sized(std::integral_constant<int, 1>{});
+    });
+    return done;
+}
+
+} // namespace
+} // namespace cv
