@@ -75,9 +75,13 @@ hipError_t launchNet(hipStream_t stream, const TrainLaunch& t, int numCUs)
     const bool xy = t.mlp.inEncoding == kEncodeXYSquares;
     const bool dwords = !xy && t.mlp.layers[0].in % 2 == 0 && t.mlp.inAlign >= 4u;
     const int variant = !plain || !(xy || dwords) ? 0 : xy ? 2 : 1;
-    const bool pairLeaky = kPairShape && leaky && (dwords || xy);
+    // Vectors of an odd number of halves (three or more: a dword is read), which lie at any half.  One-wave kernel against paired one: 23-64x4-1 over
+    // 697 samples 58.8 against 17 us, 27-32x3-6 over 14 110 31 against 16, 13-32-2 over 2^20 97 against 57, 21-64-4 148 against 78; a few hundred
+    // samples of one hidden layer the same.
+    const bool halves = kPairShape && t.mlp.inEncoding == kEncodeNone && t.mlp.layers[0].in % 2 == 1 && t.mlp.layers[0].in >= 3;
+    const bool pairLeaky = kPairShape && leaky && (dwords || xy || halves), pairPlain = kPairShape && plain && halves;
     // a launch of one workgroup of the one-wave-per-SIMD kernel finishes the step itself
-    ta.finishInKernel = (blocks == 1 && !(kPairShape && (variant != 0 || pairLeaky))) ? 1 : 0;
+    ta.finishInKernel = (blocks == 1 && !(kPairShape && (variant != 0 || pairLeaky || pairPlain))) ? 1 : 0;
     ta.finish = ra;
     noteKernel(false, "mlpTrainKernel<IT0=%d,KT0=%d,HT=%d,hidden=%d,MTL=%d,%s> + mlpTrainReduceKernel", Net::IT0, Net::KT0,
                Net::HT, Net::L - 1, Net::MTL,
@@ -85,10 +89,12 @@ hipError_t launchNet(hipStream_t stream, const TrainLaunch& t, int numCUs)
     // 64- and 32-wide networks with these activations run on the two-waves-per-SIMD kernel
     constexpr bool kPair = kPairShape;
     if constexpr (kPair) {
-        if (variant != 0 || pairLeaky)
+        if (variant != 0 || pairLeaky || pairPlain)
             noteKernel(false, "mlpTrainPairKernel<IT0=%d,KT0=%d,HT=%d,hidden=%d,MTL=%d,%s,%s> + mlpTrainReduceKernel", Net::IT0,
-                       Net::KT0, Net::HT, Net::L - 1, Net::MTL, pairLeaky ? "leaky-or-relu" : "relu/none", xy ? "xy-input" : "dword-input");
+                       Net::KT0, Net::HT, Net::L - 1, Net::MTL, pairLeaky ? "leaky-or-relu" : "relu/none", xy ? "xy-input" : halves ? "half-input" : "dword-input");
         if (pairLeaky && xy)   hipLaunchKernelGGL((mlpTrainPairKernel<Net, kLoadXY, true>), dim3(blocks), dim3(512), 0, stream, ta);
+        else if (pairLeaky && halves) hipLaunchKernelGGL((mlpTrainPairKernel<Net, kLoadHalves, true>), dim3(blocks), dim3(512), 0, stream, ta);
+        else if (pairPlain)    hipLaunchKernelGGL((mlpTrainPairKernel<Net, kLoadHalves>), dim3(blocks), dim3(512), 0, stream, ta);
         else if (pairLeaky)    hipLaunchKernelGGL((mlpTrainPairKernel<Net, kLoadDwords, true>), dim3(blocks), dim3(512), 0, stream, ta);
         else if (variant == 1) hipLaunchKernelGGL((mlpTrainPairKernel<Net, kLoadDwords>), dim3(blocks), dim3(512), 0, stream, ta);
         else if (variant == 2) hipLaunchKernelGGL((mlpTrainPairKernel<Net, kLoadXY>), dim3(blocks), dim3(512), 0, stream, ta);
@@ -96,7 +102,7 @@ hipError_t launchNet(hipStream_t stream, const TrainLaunch& t, int numCUs)
         if (variant == 1)      hipLaunchKernelGGL((mlpTrainKernel<Net, kActRelu, kActNone, kLoadDwords>), dim3(blocks), dim3(256), 0, stream, ta);
         else if (variant == 2) hipLaunchKernelGGL((mlpTrainKernel<Net, kActRelu, kActNone, kLoadXY>), dim3(blocks), dim3(256), 0, stream, ta);
     }
-    if (variant == 0 && !pairLeaky) hipLaunchKernelGGL((mlpTrainKernel<Net, -1, -1, kLoadAny>), dim3(blocks), dim3(256), 0, stream, ta);
+    if (variant == 0 && !pairLeaky && !pairPlain) hipLaunchKernelGGL((mlpTrainKernel<Net, -1, -1, kLoadAny>), dim3(blocks), dim3(256), 0, stream, ta);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (ta.finishInKernel) return hipSuccess;

@@ -295,9 +295,10 @@ __device__ __forceinline__ void stageTrainingWeights(const MlpArgs& a, uint32_t*
 // LOADS selects how the network input is fetched.  kLoadDwords (every lane's slice is whole, 4-byte
 // aligned dwords) and kLoadXY (float2 samples of the example's encoding) are straight-line code: every
 // lane loads from an address that is always valid and masks afterwards, so the requests of the next
-// round stay in flight during the whole current round.  kLoadAny covers everything else with
-// predicated loads, which the round has to wait for.
-enum : int { kLoadDwords = 0, kLoadAny = 1, kLoadXY = 2 };
+// round stay in flight during the whole current round.  So is kLoadHalves (the paired kernel: vectors of at least two
+// elements at any element): dwords read at whatever half they begin, the last one of a slice of odd length ending where the
+// slice does.  kLoadAny covers everything else with predicated loads, which the round has to wait for.
+enum : int { kLoadDwords = 0, kLoadAny = 1, kLoadXY = 2, kLoadHalves = 3 };
 
 // HACT / LACT fix the activation of the hidden layers / the last layer at compile time (the round
 // then is straight-line code the scheduler can interleave); -1 reads them from the arguments and

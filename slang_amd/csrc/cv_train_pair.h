@@ -213,6 +213,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if constexpr (LOADS == kLoadXY) {
 #pragma unroll
             for (int i = 0; i < IN_DW; ++i) raw[i] = i < 2 ? ((const uint32_t*)row)[i] : 0u;
+        } else if constexpr (LOADS == kLoadHalves) {
+#pragma unroll
+            for (int i = 0; i < IN_DW; ++i)
+                __builtin_memcpy(&raw[i], 4 * i + 4 <= validBytes ? p + 4 * i : 4 * i + 2 == validBytes ? p + 4 * i - 2 : row, 4);
         } else {
 #pragma unroll
             for (int i = 0; i < IN_DW; ++i) raw[i] = *(const uint32_t*)(4 * i < validBytes ? p + 4 * i : row);
@@ -232,6 +236,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int d = 0; d < IN_DW; ++d) {
             if constexpr (LOADS == kLoadDwords) buf[d] = 4 * d < validBytes ? raw[d] : 0u;
+            else if constexpr (LOADS == kLoadHalves) buf[d] = 4 * d + 4 <= validBytes ? raw[d] : 4 * d + 2 == validBytes ? raw[d] >> 16 : 0u;
             else buf[d] = 0u;
         }
         if constexpr (LOADS == kLoadXY) {

@@ -697,3 +697,35 @@ def test_activation_behind_the_last_layer_on_the_four_wave_kernel(last):
     gW, gB = read_grads(general, specs, CT.Float32, ML.RowMajor)
     for l in range(len(specs)):
         assert rel_err(gW[l], dW[l]) <= 1e-3 and rel_err(gB[l], dB[l]) <= 1e-3
+
+
+@pytest.mark.parametrize("dims,B,pad", [([3, 32, 32, 2], 1, 0), ([5, 64, 64, 64, 64, 1], 4099, 0), ([15, 32, 4], 700, 0), ([17, 64, 64, 7], 1001, 2),
+                                        ([31, 16, 16, 16, 16, 3], 65, 0), ([7, 48, 24, 3], 640, 4), ([23, 64, 64, 64, 1], 333, 1)])
+@pytest.mark.parametrize("act", [Activation.ReLU, Activation.LeakyReLU])
+def test_vectors_of_an_odd_number_of_halves_on_the_paired_kernel(dims, B, pad, act):
+    # rows one behind the other (every second one begins at an odd half) and inside wider rows, beside which NaN stands: against the
+    # oracle, and bit for bit against the same vectors with a zero behind them (an even number, read in aligned dwords)
+    rng = np.random.default_rng(sum(dims) + B)
+    slope = float(np.float16(0.01)) if act == Activation.LeakyReLU else 0.0
+    specs = make_specs(rng, dims, act=act, slope=slope)
+    x = rng.uniform(-1, 1, (B, dims[0])).astype(np.float16)
+    t = rng.uniform(-1, 1, (B, dims[-1])).astype(np.float16)
+    wide = torch.full((B, dims[0] + pad), float("nan"), dtype=torch.float16, device=DEV); wide[:, :dims[0]] = to_dev(x)
+    layers = build(specs)
+    _, loss = cv.mlpTrainStep(layers, wide[:, :dims[0]], to_dev(t), lossScale=0.25)
+    assert cv.lastKernelName().startswith("mlpTrainPairKernel") and "half-input" in cv.lastKernelName(), cv.lastKernelName()
+    dW, dB = read_grads(layers, specs, CT.Float32, ML.RowMajor)
+    rW, rB, rloss = ob.ref_mlp_train(specs, x, t, 0.25, tie_rule=True)
+    for l in range(len(specs)):
+        assert rel_err(dW[l], rW[l]) <= 1e-3, (l, rel_err(dW[l], rW[l]))
+        assert rel_err(dB[l], rB[l]) <= 1e-3, (l, rel_err(dB[l], rB[l]))
+    assert abs(loss.item() - rloss) <= 1e-3 * rloss
+    even = [dict(s) for s in specs]
+    even[0]["W"] = np.concatenate([specs[0]["W"], np.zeros((dims[1], 1), np.float16)], axis=1)
+    even[0]["in"] = dims[0] + 1
+    other = build(even)
+    _, loss1 = cv.mlpTrainStep(other, to_dev(np.concatenate([x, np.zeros((B, 1), np.float16)], axis=1)), to_dev(t), lossScale=0.25)
+    assert cv.lastKernelName().startswith("mlpTrainPairKernel") and "dword-input" in cv.lastKernelName(), cv.lastKernelName()
+    eW, eB = read_grads(other, even, CT.Float32, ML.RowMajor)
+    assert np.array_equal(dW[0], eW[0][:, :dims[0]]) and loss.item() == loss1.item()
+    assert all(np.array_equal(a, b) for a, b in zip(dW[1:] + dB, eW[1:] + eB))
