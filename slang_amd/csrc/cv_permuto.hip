@@ -366,7 +366,8 @@ __global__ __launch_bounds__(1024, WAVES) void permutoTableGradKernel(const Perm
     __syncthreads();
     const TableInLds<FT, SLICED> sink{ldsTable, part.base, part.elems, entries, F};
     if constexpr (POS != kPosBeside) {
-        for (uint64_t s = (uint64_t)w * 1024u + threadIdx.x; s < a.batch; s += (uint64_t)parts.groups * 1024u)
+        // units of 64 positions, dealt to the part's workgroups in turn
+        for (uint64_t s = ((uint64_t)(threadIdx.x >> 6) * parts.groups + w) * 64u + (threadIdx.x & 63u); s < a.batch; s += (uint64_t)parts.groups * 1024u)
             permutoBackwardOne<D, FT, POS == kPosInPass, PLAIN>(a, (uint32_t)s, part.first, part.end, sink);
     } else {
         const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
@@ -498,7 +499,17 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     const dim3 grid((a.batch - 1u) / 256u + 1u), block(256);
     TableParts t;
     const bool cut = a.dTable && cutTable(a.desc, t);
-    if (cut) dealGroups(t, a.batch, (uint32_t)cus);
+    const uint64_t features = (uint64_t)a.desc.featureDimensionPerEntry * a.desc.maxLevels;
+    // Where position gradients are written on top of what is read (rows on rows), other workgroups of one launch would still read it.
+    const Rows dPos{(uint64_t)(uintptr_t)a.dPos, a.dPosStride, D * 4ull}, pos{(uint64_t)(uintptr_t)a.pos, a.posStride, D * 4ull},
+        dOut{(uint64_t)(uintptr_t)a.dOut, a.dOutStride, features * 4ull};
+    const bool apart = a.dPos && !rowsMeet(dPos, pos, a.batch) && !rowsMeet(dPos, dOut, a.batch);
+    const uint32_t natural = cut ? t.count : 0u;
+    const bool byLevel = cut && FT > 0 && (apart || !a.dPos) && cutByLevel(a.desc, a.batch, (uint32_t)cus, t);
+    if (cut) {
+        if (FT > 0 && !t.sliced && a.batch >= kFewPositions) dealGroups(t, a.batch, (uint32_t)cus, positionsShare(t, a.batch, (uint32_t)(FT * (D + 1)), (uint32_t)cus));
+        else dealGroups(t, a.batch, (uint32_t)cus);
+    }
     if (cut && t.count == 1 && a.dPos) {
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
         return launchTableGrad<D, FT, kPosInPass, false, PLAIN>(stream, a, t, cus);
@@ -508,16 +519,15 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     // four-feature entries, 4 of 2^12 two-feature ones, ...); its time grows with the additions and reaches the pair's at 1300 to
     // 2000 of them (one to five and eight dimensions, 2 to 8 levels).  Where a position has more than 16 features it is the slower
     // one from the first position (16 levels of 4 features: 34.8 against 25.3 us).
-    const uint64_t features = (uint64_t)a.desc.featureDimensionPerEntry * a.desc.maxLevels;
     const bool few = FT > 0 && a.batch <= 64u && features <= 16u && a.batch * (uint64_t)(D + 1) * features <= 1440u;
     if (cut && !(a.dPos && few)) {
-        // One launch where that is sooner (positionsBeside).  Where position gradients are written on top of what is read (rows
-        // on rows), other workgroups of the one launch would still read it.
-        const Rows dPos{(uint64_t)(uintptr_t)a.dPos, a.dPosStride, D * 4ull}, pos{(uint64_t)(uintptr_t)a.pos, a.posStride, D * 4ull},
-            dOut{(uint64_t)(uintptr_t)a.dOut, a.dOutStride, features * 4ull};
-        const bool apart = a.dPos && !rowsMeet(dPos, pos, a.batch) && !rowsMeet(dPos, dOut, a.batch);
-        if (apart && positionsBeside(t, a.batch, (uint32_t)cus)) {
-            noteKernel(false, "permutoTableGradKernel<D=%d,%u parts,positions beside>", D, t.count);
+        // One launch where that is sooner: always behind cutByLevel; else for workgroups on every compute unit (positionsBeside), or on a quarter of
+        // them where levels are no slices and entries of 1, 2 or 4 features (8 levels of 2^12 two-feature entries, 3 dimensions, 2^14 positions:
+        // 11.9 us, in two launches 19.4, and 11.9 against 16.0 over 4096, where calls keep the two launches they had).
+        const bool many = positionsBeside(t, a.batch, (uint32_t)cus), quarter = FT > 0 && !t.sliced && (uint64_t)t.count * ((a.batch - 1u) / 1024u + 1u) >= (uint32_t)cus / 4u;
+        if (apart && (byLevel || many || quarter)) {
+            if (natural == 1) noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
+            else noteKernel(false, many && !byLevel ? "permutoTableGradKernel<D=%d,%u parts,positions beside>" : "permutoTableGradKernel<D=%d,%u parts,positions>", D, t.count);
             return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t, cus);
         }
         noteKernel(false, "permutoTableGradKernel<D=%d,%u parts>", D, t.count);

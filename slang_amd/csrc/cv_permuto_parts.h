@@ -28,12 +28,13 @@ constexpr uint64_t kPartHalf = 80 * 1024 / 8, kPartMost = 160 * 1024 / 8;
 // Levels may lie anywhere: with gaps between them (a sum that stays zero is not added to memory), in any order, on the same
 // entries (each part adds its sums to memory atomically).
 // False: more parts than that, or elements whose numbers exceed 32 bits.
-inline bool cutTable(const CvPermutoDesc& desc, TableParts& t)
+inline bool cutTable(const CvPermutoDesc& desc, TableParts& t, uint64_t together = kPartHalf)
 {
     const uint64_t F = (uint64_t)desc.featureDimensionPerEntry;
     t.count = 0;
     t.sliced = 0;
     bool whole = false;      // the part before this level is made of whole levels
+    // (together: the most elements that levels share a part up to)
     for (uint32_t l = 0; l < desc.maxLevels; ++l) {
         const CvPermutoLevelInfo& lv = desc.levelInfo[l];
         const uint64_t from = (uint64_t)lv.offsetOfFeatureTable * F, elems = (uint64_t)lv.featureTableSize * F, to = from + elems;
@@ -42,7 +43,7 @@ inline bool cutTable(const CvPermutoDesc& desc, TableParts& t)
             TablePart& last = t.part[t.count - 1];
             const uint64_t lastTo = (uint64_t)last.base + last.elems;
             const uint64_t lo = from < last.base ? from : last.base, hi = to > lastTo ? to : lastTo;
-            if (hi - lo <= kPartHalf) {
+            if (hi - lo <= together) {
                 last.base = (uint32_t)lo;
                 last.elems = (uint32_t)(hi - lo);
                 last.end = l + 1;
@@ -63,18 +64,40 @@ inline bool cutTable(const CvPermutoDesc& desc, TableParts& t)
     return t.count > 0;
 }
 
-// As many workgroups (of 1024 threads) as the compute units hold, dealt evenly to the parts, and none without positions.
+// As many workgroups (of 1024 threads) as the compute units hold, dealt evenly to the parts, and none without `share` positions.
 inline uint32_t largestPart(const TableParts& t)
 {
     uint32_t most = 0;
     for (uint32_t p = 0; p < t.count; ++p) most = t.part[p].elems > most ? t.part[p].elems : most;
     return most;
 }
-inline void dealGroups(TableParts& t, uint32_t batch, uint32_t cus)
+inline void dealGroups(TableParts& t, uint32_t batch, uint32_t cus, uint32_t share = 1024u)
 {
-    const uint32_t resident = cus * (largestPart(t) <= kPartHalf ? 2u : 1u), want = (batch - 1u) / 1024u + 1u;
+    const uint32_t resident = cus * (largestPart(t) <= kPartHalf ? 2u : 1u), want = (batch - 1u) / share + 1u;
     const uint32_t each = resident / t.count ? resident / t.count : 1u;
     t.groups = want < each ? want : each;
+}
+
+// One level to a part instead of several where the parts leave compute units without a workgroup of 1024 positions: a level's additions in LDS, not
+// its start, are what a workgroup takes its time for.  Several levels to a part against one (and position gradients beside), 3 dimensions, us: 6 levels of
+// 2^9 four-feature entries over 4096 / 2^14 / 2^16 positions 49.6, 50.4, 52.0 against 11.3, 11.3, 20.6; 8 levels of 2^10 two-feature entries over 20000
+// / 2^16 32.5, 33.0 against 12.0, 15.1; 2 dimensions, 8 levels of 2^8 of two over 20000 / 2^16 / 2^17 / 2^18 (one part) 21.8, 22.6, 23.6, 27.5
+// against 11.3, 11.4, 17.2, 28.3.  (Below kFewPositions there is little to spread.)
+constexpr uint32_t kFewPositions = 2048u;
+inline bool cutByLevel(const CvPermutoDesc& desc, uint32_t batch, uint32_t cus, TableParts& t)
+{
+    if (t.sliced || t.count >= desc.maxLevels || batch < kFewPositions || (uint64_t)t.count * ((batch - 1u) / 1024u + 1u) >= cus) return false;
+    return cutTable(desc, t, 0);      // (levels that were joined are whole ones, no more than a description has)
+}
+
+// Positions to a workgroup, of which it takes 1024 at a time: fewer where that leaves most compute units without one, and where a position
+// makes many additions (`adds` to a level).  1024 / 512 / 256 positions, us: 7 levels of 2^11 four-feature entries over 4096 16.8, 12.2, 12.4; 3 levels
+// of 2^12 17.9, 12.7, 11.1; 6 of 2^9 over 2^16 23.2, 20.7; but 8 levels of 2^12 two-feature entries over 2^14 11.9, 13.1, 15.3.
+inline uint32_t positionsShare(const TableParts& t, uint32_t batch, uint32_t adds, uint32_t cus)
+{
+    uint32_t share = adds > 8u ? 512u : 1024u;
+    while (share > 256u && 4ull * t.count * ((batch - 1u) / share + 1u) <= cus) share /= 2u;
+    return share;
 }
 
 // Whether position gradients go into the table's launch (of several parts; after dealGroups).  Not with too few positions for

@@ -539,3 +539,41 @@ def test_encoder_at_half_way_values(D):
     g = to_dev(rng.standard_normal((B, F)).astype(np.float32))
     got, want = enc.backward(pos, table, g)[0], enc.backward(far, table, g)[0]
     assert torch.equal(got[keep], want[keep]), pos[keep][(got != want)[keep].any(dim=1)][:8]
+
+
+@pytest.mark.parametrize("D,F,tables,B,kernel", [
+    # one part; several levels to a part, then one: from 2048 positions on a level to a part, and the positions in the same launch
+    (3, 4, [(512 * l, 512) for l in range(6)], 2047, "permutoTableGradKernel<D=3,2 parts> + permutoBackwardKernel<D=3,positions>"),
+    (3, 4, [(512 * l, 512) for l in range(6)], 2048, "permutoTableGradKernel<D=3,6 parts,positions>"),
+    (2, 1, [(64 * l, 64) for l in range(8)], 2049, "permutoTableGradKernel<D=2,positions>"),
+    (4, 2, [(300, 256), (0, 256), (700, 100), (700, 100)], 4097, "permutoTableGradKernel<D=4,positions>"),      # gaps, another order, shared entries
+    (2, 4, [(1024 * l, 1024) for l in range(3)], 20001, "permutoTableGradKernel<D=2,3 parts,positions>"),
+    # workgroups of 1024 positions on a quarter of 256 compute units, and on less
+    (3, 2, [(4096 * l, 4096) for l in range(8)], 7168, "permutoTableGradKernel<D=3,8 parts> + permutoBackwardKernel<D=3,positions>"),
+    (3, 2, [(4096 * l, 4096) for l in range(8)], 7169, "permutoTableGradKernel<D=3,8 parts,positions>"),
+    (3, 1, [(4096, 4096)], 3000, "permutoTableGradKernel<D=3,positions>"),                                     # one level: fewer positions to a workgroup
+])
+def test_permuto_backward_spread_over_levels(D, F, tables, B, kernel):
+    # the bounds are those of test_permuto_backward_table_parts
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the batches are those of 256 compute units")
+    rng = np.random.default_rng(F * 100 + B)
+    n = len(tables)
+    enc = cv.PermutoEncoder(D, F, 12, n, baseScale=3.0, log2PerLevelScale=0.5, maxLevelRatio=1.0, seed=11)
+    levels = ob.permuto_levels(D, 12, n, 3.0, 0.5, 11)
+    for l, (offset, size) in enumerate(tables):
+        for record in (enc.desc.levelInfo[l], levels[l]):
+            record.offsetOfFeatureTable, record.featureTableSize = offset, size
+    pos = rng.uniform(-1, 1, (B, D)).astype(np.float32)
+    table = rng.standard_normal(max(o + s for o, s in tables) * F).astype(np.float32)
+    g = rng.standard_normal((B, n * F)).astype(np.float32)
+    r_pos, r_table = ob.permuto_encode_backward(levels, F, float(n), pos, table, g)
+    d_table = torch.zeros(table.size, dtype=torch.float32, device=DEV)
+    d_pos, _ = enc.backward(to_dev(pos), to_dev(table), to_dev(g), dFeatureTable=d_table)
+    assert cv.lastKernelName() == kernel
+    assert np.linalg.norm(d_table.cpu().numpy() - r_table) <= 2.0 ** -16 * np.linalg.norm(r_table)
+    assert not d_table.cpu().numpy()[r_table == 0].any()
+    assert np.linalg.norm(d_pos.cpu().numpy() - r_pos) <= 1e-4 * np.linalg.norm(r_pos)
+    alone = torch.zeros_like(d_table)                                 # the table's gradient by itself
+    enc.backward(to_dev(pos), to_dev(table), to_dev(g), dFeatureTable=alone, wantPositionGrad=False)
+    assert np.linalg.norm(alone.cpu().numpy() - r_table) <= 2.0 ** -16 * np.linalg.norm(r_table)
