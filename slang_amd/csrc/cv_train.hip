@@ -75,9 +75,9 @@ hipError_t launchNet(hipStream_t stream, const TrainLaunch& t, int numCUs)
     const bool xy = t.mlp.inEncoding == kEncodeXYSquares;
     const bool dwords = !xy && t.mlp.layers[0].in % 2 == 0 && t.mlp.inAlign >= 4u;
     const int variant = !plain || !(xy || dwords) ? 0 : xy ? 2 : 1;
-    // Vectors of an odd number of halves (three or more: a dword is read), which lie at any half.  One-wave kernel against paired one: 23-64x4-1 over
-    // 697 samples 58.8 against 17 us, 27-32x3-6 over 14 110 31 against 16, 13-32-2 over 2^20 97 against 57, 21-64-4 148 against 78; a few hundred
-    // samples of one hidden layer the same.
+    // Vectors of an odd number of halves (three or more: a dword is read), which lie at any half.  One-wave kernel against paired one: 27-32x3-6
+    // over 14 110 samples 32 against 11 us, 13-32-2 over 2^20 94 against 54, 21-64-4 146 against 77; a few hundred samples of one hidden layer
+    // the same.
     const bool halves = kPairShape && t.mlp.inEncoding == kEncodeNone && t.mlp.layers[0].in % 2 == 1 && t.mlp.layers[0].in >= 3;
     const bool pairLeaky = kPairShape && leaky && (dwords || xy || halves), pairPlain = kPairShape && plain && halves;
     // a launch of one workgroup of the one-wave-per-SIMD kernel finishes the step itself
