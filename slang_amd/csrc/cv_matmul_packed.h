@@ -44,67 +44,6 @@ void forEach(F&& f)
     }
 }
 
-// 16-byte (8-byte) accesses of LDS and memory at the alignment of an element
-template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose16 { u32x4 v; };
-template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose8 { u32x2 v; };
-
-template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose4 { uint32_t v; };
-
-template <int ALIGN, int DW>
-__device__ __forceinline__ void loadLoose(const uint8_t* q, uint32_t (&x)[DW])
-{
-    if constexpr (DW % 4 == 0) {
-#pragma unroll
-        for (int d = 0; d < DW; d += 4) {
-            const u32x4 v = ((const Loose16<ALIGN>*)(q + 4 * d))->v;
-            x[d] = v.x; x[d + 1] = v.y; x[d + 2] = v.z; x[d + 3] = v.w;
-        }
-    } else {
-        const u32x2 v = ((const Loose8<ALIGN>*)q)->v;
-        x[0] = v.x; x[1] = v.y;
-    }
-}
-
-// The same where what is read may end beyond `end`, behind which nothing is read and zeros stand (at least 16 bytes lie before it).
-template <int ALIGN, int DW>
-__device__ __forceinline__ void loadUpTo(const uint8_t* q, const uint8_t* end, uint32_t (&x)[DW])
-{
-    constexpr int P = DW % 4 == 0 ? 4 : 2;      // dwords of a read
-#pragma unroll
-    for (int d0 = 0; d0 < DW; d0 += P) {
-        const uint8_t* at = q + 4 * d0;
-        const int64_t over = (at + 4 * P) - end;
-        const int shift = (int)(over < 0 ? 0 : over > 4 * P ? 4 * P : over), words = shift >> 2;
-        uint32_t v[2 * P + 1];
-        uint32_t part[P];
-        loadLoose<ALIGN>(over > 0 ? end - 4 * P : at, part);
-#pragma unroll
-        for (int i = 0; i < 2 * P + 1; ++i) v[i] = i < P ? part[i < P ? i : 0] : 0u;
-#pragma unroll
-        for (int i = 0; i < P; ++i) {
-            uint32_t lo = 0u, hi = 0u;
-#pragma unroll
-            for (int w = 0; w <= P; ++w) {
-                lo = words == w ? v[i + w] : lo;
-                hi = words == w ? v[i + w + 1 <= 2 * P ? i + w + 1 : 2 * P] : hi;
-            }
-            x[d0 + i] = __builtin_amdgcn_alignbyte(hi, lo, shift & 3);
-        }
-    }
-}
-
-// clears all but the first `bytes` bytes (none if that is negative)
-template <int ESZ, int DW>
-__device__ __forceinline__ void clearBehind(uint32_t (&x)[DW], int bytes)
-{
-#pragma unroll
-    for (int d = 0; d < DW; ++d) {
-        const int left = bytes - 4 * d;
-        if constexpr (ESZ == 4) x[d] = left > 0 ? x[d] : 0u;
-        else x[d] = left > 0 ? x[d] & (0xffffffffu >> max(32 - 8 * left, 0)) : 0u;
-    }
-}
-
 __device__ __forceinline__ void meetInWave()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -84,18 +84,28 @@ __device__ __forceinline__ CarrierCfg makeCarrierCfg(int act, float slope)
     return c;
 }
 
+// Leaky ReLU with such a slope may multiply packed halfs: the slope of a network of halfs is a half, so that the packed product rounds once,
+// as activateHalf's does.  (For any other slope that function chooses between z, NaN and zeros.)
+__device__ __forceinline__ bool packedSlope(float slope) { return slope > 0.f && slope < __builtin_inff(); }
+
 // accumulators (one 16-row tile, 4 values per lane) -> the carrier CoopVec<half>: round to
 // fp16 (v_cvt_pk_f16_f32, nearest even), then the activation, on packed pairs
 // SMOOTH: the kernel also serves the neural module's smooth activations (only the general kernel
 // does; the specialised ones would carry the transcendental code in every instantiation)
-template <bool SMOOTH = false>
+// PACKED_LEAKY: leaky ReLU with packedSlope(slope) on all layers that come here
+template <bool SMOOTH = false, bool PACKED_LEAKY = false>
 __device__ __forceinline__ void carrierFromAcc(const floatx4& acc, const CarrierCfg& c, halfx2& h01, halfx2& h23)
 {
     typedef float floatx2 __attribute__((ext_vector_type(2)));
     const floatx2 a01 = {acc[0], acc[1]}, a23 = {acc[2], acc[3]};
     h01 = __builtin_convertvector(a01, halfx2);
     h23 = __builtin_convertvector(a23, halfx2);
-    if (c.act == kActLeakyRelu || (SMOOTH && c.act >= kActSigmoid)) {   // leaky: max(z, z*slope) in half, fflayer.slang:64-65
+    if constexpr (PACKED_LEAKY) {
+        const half_t sl = (half_t)c.slope;
+        const halfx2 s2 = {sl, sl};
+        h01 = __builtin_elementwise_max(h01, h01 * s2);
+        h23 = __builtin_elementwise_max(h23, h23 * s2);
+    } else if (c.act == kActLeakyRelu || (SMOOTH && c.act >= kActSigmoid)) {   // leaky: max(z, z*slope) in half, fflayer.slang:64-65
         const int act = SMOOTH ? c.act : (int)kActLeakyRelu;      // without SMOOTH the transcendental code is not even compiled
         h01 = halfx2{activateHalf(h01.x, act, c.slope), activateHalf(h01.y, act, c.slope)};
         h23 = halfx2{activateHalf(h23.x, act, c.slope), activateHalf(h23.y, act, c.slope)};

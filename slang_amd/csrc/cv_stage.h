@@ -17,6 +17,89 @@
 
 namespace cv {
 
+// 16-byte (8-byte) accesses of LDS and memory at the alignment of an element
+template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose16 { u32x4 v; };
+template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose8 { u32x2 v; };
+template <int ALIGN> struct __attribute__((packed, aligned(ALIGN))) Loose4 { uint32_t v; };
+
+template <int ALIGN, int DW>
+__device__ __forceinline__ void loadLoose(const uint8_t* q, uint32_t (&x)[DW])
+{
+    if constexpr (DW % 4 == 0) {
+#pragma unroll
+        for (int d = 0; d < DW; d += 4) {
+            const u32x4 v = ((const Loose16<ALIGN>*)(q + 4 * d))->v;
+            x[d] = v.x; x[d + 1] = v.y; x[d + 2] = v.z; x[d + 3] = v.w;
+        }
+    } else {
+        const u32x2 v = ((const Loose8<ALIGN>*)q)->v;
+        x[0] = v.x; x[1] = v.y;
+    }
+}
+
+// The same where what is read may end beyond `end`, behind which nothing is read and zeros stand (at least 16 bytes lie before it).
+template <int ALIGN, int DW>
+__device__ __forceinline__ void loadUpTo(const uint8_t* q, const uint8_t* end, uint32_t (&x)[DW])
+{
+    constexpr int P = DW % 4 == 0 ? 4 : 2;      // dwords of a read
+#pragma unroll
+    for (int d0 = 0; d0 < DW; d0 += P) {
+        const uint8_t* at = q + 4 * d0;
+        const int64_t over = (at + 4 * P) - end;
+        const int shift = (int)(over < 0 ? 0 : over > 4 * P ? 4 * P : over), words = shift >> 2;
+        uint32_t v[2 * P + 1];
+        uint32_t part[P];
+        loadLoose<ALIGN>(over > 0 ? end - 4 * P : at, part);
+#pragma unroll
+        for (int i = 0; i < 2 * P + 1; ++i) v[i] = i < P ? part[i < P ? i : 0] : 0u;
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+            for (int w = 0; w <= P; ++w) {
+                lo = words == w ? v[i + w] : lo;
+                hi = words == w ? v[i + w + 1 <= 2 * P ? i + w + 1 : 2 * P] : hi;
+            }
+            x[d0 + i] = __builtin_amdgcn_alignbyte(hi, lo, shift & 3);
+        }
+    }
+}
+
+template <int W, int DW>
+__device__ __forceinline__ void downBy(uint32_t (&x)[DW], bool yes)
+{
+#pragma unroll
+    for (int i = 0; i < DW; ++i) {
+        const uint32_t own = x[i], above = i + W < DW ? x[i + W < DW ? i + W : i] : 0u;      // (values: a choice between elements would be one between addresses)
+        x[i] = yes ? above : own;
+    }
+}
+
+// moves what x holds down by `bytes` bytes (whole elements, fewer than x has); zeros come in
+template <int ESZ, int DW>
+__device__ __forceinline__ void shiftDown(uint32_t (&x)[DW], int bytes)
+{
+    if constexpr (DW > 4) downBy<4>(x, bytes & 16);
+    if constexpr (DW > 2) downBy<2>(x, bytes & 8);
+    downBy<1>(x, bytes & 4);
+    if constexpr (ESZ < 4) {
+#pragma unroll
+        for (int i = 0; i < DW; ++i) x[i] = __builtin_amdgcn_alignbyte(i + 1 < DW ? x[i + 1 < DW ? i + 1 : 0] : 0u, x[i], bytes & 3);
+    }
+}
+
+// clears all but the first `bytes` bytes (none if that is negative)
+template <int ESZ, int DW>
+__device__ __forceinline__ void clearBehind(uint32_t (&x)[DW], int bytes)
+{
+#pragma unroll
+    for (int d = 0; d < DW; ++d) {
+        const int left = bytes - 4 * d;
+        if constexpr (ESZ == 4) x[d] = left > 0 ? x[d] : 0u;
+        else x[d] = left > 0 ? x[d] & (0xffffffffu >> max(32 - 8 * left, 0)) : 0u;
+    }
+}
+
 // The EPL elements of lane-chunk c (chunk = 64 * fragment + lane) of that arrangement, fetched from memory into
 // CHUNK / 4 registers (zero where the matrix ends).  xorByte (1-byte types only): XORed into every valid element on the
 // way, used to re-bias unsigned bytes to signed ones (u ^ 0x80 == u - 128 as int8); padding stays zero.
@@ -263,5 +346,61 @@ struct FragmentStage {
         }
     }
 };
+
+// A matrix of up to 128 columns as it lies (not transposed, no block of rows), four lane-chunks of a thread requested together, a RowMajor one's
+// each in one read at whatever element it begins; store(c, v) takes chunk c.  For kernels that stage network after network, each
+// matrix of which then costs one trip to memory and not one for every chunk of a thread.
+template <int ESZ, int EPL, class Store>
+__device__ __forceinline__ void stageTogether(const uint8_t* w, const MatrixShape& shape, int MT, int KT, uint32_t rows, uint32_t cols, Store&& store)
+{
+    constexpr int CHUNK = ESZ * EPL, DW = CHUNK / 4, TOGETHER = 4;
+    const uint32_t gs = optGS(cols);
+    const int chunks = MT * KT * 64;
+    const bool direct = fragmentSourceIsDirect<ESZ, EPL>(shape, false, MT, KT, gs, rows, cols, 0, 0);
+    const size_t line = shape.stride ? shape.stride : (size_t)cols * ESZ, bytes = (size_t)(rows - 1) * line + (size_t)cols * ESZ;
+    if (!direct && (shape.layout != kRowMajor || bytes < (size_t)CHUNK || bytes > 0x7fffffffu)) {
+        for (int c = (int)threadIdx.x; c < chunks; c += (int)blockDim.x) {
+            uint32_t v[DW];
+            fetchFragmentChunk<ESZ, EPL>(v, w, shape, false, false, MT, KT, gs, rows, cols, 0, 0, c);
+            store(c, v);
+        }
+        return;
+    }
+    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
+    const uint32_t row0 = (uint32_t)((i >> 2) * 4 * MT + (i & 3)), col0 = (uint32_t)g * gs;
+    for (int c0 = (int)threadIdx.x; c0 < chunks; c0 += TOGETHER * (int)blockDim.x) {
+        uint32_t v[TOGETHER][DW];
+        int valid[TOGETHER];
+        uint32_t off[TOGETHER];
+#pragma unroll
+        for (int u = 0; u < TOGETHER; ++u) {
+            const int c = c0 + u * (int)blockDim.x;      // (whole waves: the branches are uniform)
+            if (__builtin_amdgcn_readfirstlane(c) >= chunks) break;
+            if (direct) {
+                valid[u] = CHUNK;
+                off[u] = (uint32_t)c * CHUNK;
+            } else {
+                // (KT is at most 4 and a matrix has no more than 32 fragments)
+                const int f = __builtin_amdgcn_readfirstlane(c >> 6), t = KT == 1 ? f : KT == 2 ? f >> 1 : KT == 4 ? f >> 2 : f * 171 >> 9, kt = f - t * KT;
+                const uint32_t row = row0 + 4 * t, col = col0 + (uint32_t)(kt * EPL);
+                const int have = (int)min((uint32_t)EPL, gs - min(gs, (uint32_t)(kt * EPL)));
+                valid[u] = row < rows ? max(min(have, (int)cols - (int)col), 0) * ESZ : 0;
+                off[u] = valid[u] ? row * (uint32_t)line + col * ESZ : 0u;
+            }
+            // (what would end behind the last row is read ending there and moved below)
+            loadLoose<ESZ>(w + (direct ? off[u] : min(off[u], (uint32_t)bytes - (uint32_t)CHUNK)), v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < TOGETHER; ++u) {
+            const int c = c0 + u * (int)blockDim.x;
+            if (__builtin_amdgcn_readfirstlane(c) >= chunks) break;
+            if (!direct) {
+                if (off[u] + CHUNK > (uint32_t)bytes) shiftDown<ESZ>(v[u], (int)(off[u] + CHUNK - (uint32_t)bytes));
+                clearBehind<ESZ>(v[u], valid[u]);
+            }
+            store(c, v[u]);
+        }
+    }
+}
 
 } // namespace cv

@@ -104,3 +104,56 @@ def test_rows_far_apart(ct, other):
         assert cv.lastKernelName().startswith(name), cv.lastKernelName()
         bits = torch.int32 if want.element_size() == 4 else torch.int16
         assert torch.equal(got.view(bits), want.view(bits))
+
+
+# Vectors that begin at any element: every number of k-slots beyond a whole fragment and half of one (inputs 1 to 40), results of one to
+# four rows beyond whole groups, matrices in rows that begin at any element; the last vector ends its buffer.
+@pytest.mark.parametrize("ct", [CT.Float16, CT.FloatE4M3, CT.Float32, CT.BFloat16])
+def test_chain_kernel_takes_vectors_at_any_element(ct):
+    floats = ct in TORCH
+    bits = torch.int32 if ct == CT.Float32 else torch.int16
+    for k in [1, 2, 5, 6, 7, 9, 15, 18, 31, 33, 34, 37, 39, 63, 97]:
+        rng = np.random.default_rng(1000 * int(ct) + k)
+        dims = [k, 19 if k < 64 else 70, 39, 24 + k % 4]      # (two sizes of hidden layer: not the kernel for equal ones)
+        acts = [Activation.LeakyReLU, Activation.NoActivation, Activation.NoActivation]
+        if floats:
+            layers, params = build(rng, dims, ct, acts, ML.RowMajor)
+        else:
+            specs = make_net(rng, dims, ct, act=Activation.LeakyReLU, slope=0.125, bias="rand", init="he" if ct == CT.Float16 else "half")
+            layers = gpu_layers(specs, ct, ML.RowMajor)
+        for B, pad in [(1, 0), (23, 0), (23, 3), (32785, 1)]:
+            x64 = rng.uniform(-1, 1, (B, k))
+            x = to_T(x64, ct) if floats else to_dev(x64.astype(np.float16))
+            if ct == CT.FloatE4M3:
+                x = x.to(torch.float8_e4m3fn)
+            want = chain(params, x, ct, acts) if floats else chain_of_single_layers(specs, x, ct)
+            # the last vector ends where its buffer does; NaN before the first and between them
+            size, each = x.element_size(), (k + pad) * x.element_size()
+            big = torch.full(((B - 1) * each + k * size + size,), 0xff, dtype=torch.uint8, device=DEV)
+            rows = big.view(x.dtype).as_strided((B, k), (k + pad, 1), 1)
+            rows.copy_(x)
+            out = torch.full((B * (dims[-1] + pad) + 1,), -7.0, dtype=want.dtype, device=DEV)
+            res = out[1:].view(B, dims[-1] + pad)
+            cv.mlpForward(layers, rows, weightType=ct, out=res[:, :dims[-1]])
+            name = cv.lastKernelName()
+            assert name.startswith("mlpChainKernel"), name
+            assert torch.equal(res[:, :dims[-1]].contiguous().view(bits), want.contiguous().view(bits)), (k, ct, B, pad, name)
+            assert out[0] == -7 and (res[:, dims[-1]:] == -7).all()
+
+
+@pytest.mark.parametrize("slope", [2.0 ** -24, 0.001, 1.0, 1.5, 0.0, -0.5])
+@pytest.mark.parametrize("ct", [CT.Float16, CT.FloatE4M3])
+def test_leaky_slopes(ct, slope):
+    # a positive slope takes the packed product, any other the choice element by element
+    rng = np.random.default_rng(5)
+    dims, B = [20, 48, 24, 5], 600
+    specs = make_net(rng, dims, ct, act=Activation.LeakyReLU, slope=slope, bias="rand", init="he" if ct == CT.Float16 else "half")
+    x = to_dev(rng.uniform(-1, 1, (B, dims[0])).astype(np.float16))
+    x[3] = 0.0
+    if ct == CT.FloatE4M3:
+        x = x.to(torch.float8_e4m3fn)
+    layers = gpu_layers(specs, ct, ML.InferencingOptimal)
+    got = cv.mlpForward(layers, x, weightType=ct)
+    assert cv.lastKernelName().startswith("mlpChainKernel")
+    want = chain_of_single_layers(specs, x, ct)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
