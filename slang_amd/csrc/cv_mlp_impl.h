@@ -171,9 +171,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const uint32_t gs0 = optGS((uint32_t)a.layers[0].in);
     const int colBase = (int)(g * gs0);
     const int validBytes = min((int)gs0, max(a.layers[0].in - colBase, 0)) * ESZ;
+    // (0: every lane's slice whole and aligned; 1: any other vector, in reads at whatever element a lane's slice begins)
     const int loadMode = a.inEncoding == kEncodeXYSquares ? 3 : a.inHalfAsE4M3 ? 4
-                       : (validBytes == IN_DW * 4 && a.inAlign >= (IN_DW % 4 == 0 ? 16u : 8u)) ? 0
-                       : ((validBytes & 3) == 0 && a.inAlign >= 4u) ? 1 : 2;
+                       : (a.layers[0].in == 32 * Net::KT0 && a.inAlign >= (IN_DW % 4 == 0 ? 16u : 8u)) ? 0 : 1;
+    const bool halfTail = gs0 <= 8 * Net::KT0 - 4;      // (then no lane has slots in the upper half of the last fragment)
+    uint32_t mask[LEAN == kChunkNone ? IN_DW : 1];      // the bytes of a lane's slice that exist (beyond them the other load modes leave zeros)
+    if constexpr (LEAN == kChunkNone) {
+#pragma unroll
+        for (int i = 0; i < IN_DW; ++i) mask[i] = 0xffffffffu;
+        if (loadMode == 1) clearBehind<ESZ>(mask, validBytes);
+    }
     constexpr int OROWS = 4 * Net::MTL;
     const int outDim = a.layers[L - 1].out;
     const int rowBase = g * OROWS;
@@ -191,7 +198,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     uint8_t* outLane = a.out + (size_t)rowBase * 2;
     const uint32_t lastSample = a.batch - 1;
 
+    // Load mode 1: a read takes the 16 (8) bytes at whatever element a lane's k-slots begin, and half of that where no lane has slots in the
+    // upper half of the last fragment.  What would end behind the last vector is read ending there and moved down when the tile is used, so that
+    // no load is waited for before the weights are staged.  (Dword or byte loads under a mask each before, us: 31-32-32-5 over 10^6 fp16 111 -> 36,
+    // 50-64-64-63 over 500 000 88 -> 41, 26-16-16-3 over 1 397 712 e4m3 76 -> 37, 3-16-16-1 over 500 8.6 -> 5.0.)
+    const uint64_t reach = (uint64_t)(TILE - 1) * a.inStride + (3 * gs0 + 8 * Net::KT0) * ESZ;      // from a super-tile's first vector
+    const uint64_t inEnd = (uint64_t)lastSample * a.inStride + (uint64_t)a.layers[0].in * ESZ;
+    const uint8_t* const inOwn = a.in + (validBytes > 0 ? colBase : 0) * ESZ;
+    auto readBytes = [&](int kt) { return kt + 1 == Net::KT0 && halfTail ? 2 * RAW : 4 * RAW; };
+    auto endsInside = [&](uint32_t t) { return (uint64_t)__builtin_amdgcn_readfirstlane(t) * TILE * a.inStride + reach <= inEnd; };
+    // (bytes by which such a read begins early)
+    auto early = [&](const uint8_t* q, int bytes) { return (int)min(max((int64_t)(q + bytes - (a.in + inEnd)), (int64_t)0), (int64_t)bytes); };
+    auto readSlots = [&](uint32_t* b, const uint8_t* q, int bytes) {
+        if (bytes == 2 * RAW) {
+            if constexpr (ESZ == 2) { const u32x2 v = ((const Loose8<ESZ>*)q)->v; b[0] = v.x; b[1] = v.y; }
+            else b[0] = ((const Loose4<ESZ>*)q)->v;
+        } else if constexpr (ESZ == 2) {
+            const u32x4 v = ((const Loose16<ESZ>*)q)->v; b[0] = v.x; b[1] = v.y; b[2] = v.z; b[3] = v.w;
+        } else {
+            const u32x2 v = ((const Loose8<ESZ>*)q)->v; b[0] = v.x; b[1] = v.y;
+        }
+    };
     auto loadTile = [&](uint32_t (&buf)[S][IN_DW], uint32_t t) {
+        if (LEAN == kChunkNone && loadMode == 1 && inEnd >= 16u) {
+            if (endsInside(t)) {
+                const uint8_t* p = inOwn + ((size_t)t * TILE + n) * a.inStride;
+#pragma unroll
+                for (int j = 0; j < S; ++j, p += (size_t)16 * a.inStride)
+#pragma unroll
+                    for (int kt = 0; kt < Net::KT0; ++kt) readSlots(&buf[j][kt * RAW], p + kt * 8 * ESZ, readBytes(kt));
+            } else {
+#pragma unroll
+                for (int j = 0; j < S; ++j) {
+                    const uint8_t* p = inOwn + (size_t)min(t * TILE + 16 * j + n, lastSample) * a.inStride;
+#pragma unroll
+                    for (int kt = 0; kt < Net::KT0; ++kt) {
+                        const uint8_t* q = p + kt * 8 * ESZ;
+                        readSlots(&buf[j][kt * RAW], q - early(q, readBytes(kt)), readBytes(kt));
+                    }
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < S; ++j) {
             const uint32_t s = min(t * TILE + 16 * j + n, lastSample);
@@ -246,10 +294,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
                         buf[j][2 * i] = v.x; buf[j][2 * i + 1] = v.y;
                     }
                 }
-            } else if (loadMode == 1) {
-#pragma unroll
-                for (int i = 0; i < IN_DW; ++i) buf[j][i] = (4 * i < validBytes) ? *(const uint32_t*)(p + 4 * i) : 0u;
-            } else {
+            } else {      // (a batch of less than 16 bytes)
 #pragma unroll
                 for (int i = 0; i < IN_DW; ++i) {
                     uint32_t v = 0;
@@ -375,6 +420,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     });
 
     auto computeStore = [&](const uint32_t (&buf)[S][IN_DW], uint32_t t0) {
+        const bool moved = LEAN == kChunkNone && loadMode == 1 && inEnd >= 16u && !endsInside(t0);
 #pragma unroll
         for (int r0 = 0; r0 < S; r0 += NT) {
             uint32_t act[NT][Net::KTMAX][FD];    // B fragments of the current layer's input
@@ -388,7 +434,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
                         for (int d = 0; d < RAW; ++d) own[d] = 4 * (kt * RAW + d) < validBytes ? buf[r0 + j][kt * RAW + d] : 0u;
                         Mma::decode(own, act[j][kt]);
                     } else {
-                        Mma::decode(&buf[r0 + j][kt * RAW], act[j][kt]);
+                        uint32_t own[RAW];
+#pragma unroll
+                        for (int d = 0; d < RAW; ++d) own[d] = buf[r0 + j][kt * RAW + d];
+                        if (moved) {
+                            const uint8_t* q = inOwn + (size_t)min(t0 * TILE + 16 * (r0 + j) + n, lastSample) * a.inStride + kt * 8 * ESZ;
+                            shiftDown<ESZ>(own, min(early(q, readBytes(kt)), 4 * RAW - ESZ));
+                        }
+#pragma unroll
+                        for (int d = 0; d < RAW; ++d) own[d] &= mask[kt * RAW + d];
+                        Mma::decode(own, act[j][kt]);
                     }
                 }
 
@@ -445,11 +500,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
                             }
                         } else {
 #pragma unroll
-                            for (int e = 0; e < OROWS; ++e)
-                                if (e < validRows) {
-                                    const uint16_t bits = (uint16_t)(pk[e / 2] >> (16 * (e & 1)));
-                                    o[e] = __builtin_bit_cast(half_t, bits);
+                            for (int t = 0; t < MT; ++t) {
+                                const int left = validRows - 4 * t;
+                                if (left >= 4) {
+                                    ((Loose8<2>*)(o + 4 * t))->v = u32x2{pk[2 * t], pk[2 * t + 1]};
+                                } else if (left > 0) {
+                                    if (left > 1) ((Loose4<2>*)(o + 4 * t))->v = pk[2 * t];
+                                    if (left != 2) ((uint16_t*)o)[4 * t + left - 1] = (uint16_t)(left == 1 ? pk[2 * t] : pk[2 * t + 1]);
                                 }
+                            }
                         }
                     }
                 }

@@ -683,3 +683,33 @@ def test_leaky_fp16_networks_on_32_sample_tiles(dims, B, bias):
         y = cv.mlpForward(gpu_layers(specs, CT.Float16, ML.RowMajor), xd, weightType=CT.Float16)
         assert not cv.lastKernelName().startswith("mlpWide16Kernel"), cv.lastKernelName()
         assert torch.equal(y.view(torch.int16), chain_of_single_layers(specs, xd, CT.Float16).view(torch.int16))
+
+
+# Vectors that begin at any element on the kernel of equal hidden layers (registers for all weights): every number of k-slots beyond a whole
+# fragment and half of one, results of one to four rows beyond whole groups, rows that end where their buffer does, NaN around and between
+# them, batches that end inside a tile and inside a round of tiles.
+@pytest.mark.parametrize("ct", [CT.Float16, CT.FloatE4M3])
+@pytest.mark.parametrize("hidden", [16, 64])
+def test_equal_layers_take_vectors_at_any_element(ct, hidden):
+    seen = set()
+    for k in [1, 2, 3, 5, 7, 11, 14, 15, 18, 30, 31, 33, 35, 37, 50, 63]:
+        rng = np.random.default_rng(1000 * int(ct) + k)
+        dims = [k, hidden, hidden, 1 + k % 16] if k <= 32 or hidden == 64 else [k % 32, hidden, hidden, 4]
+        specs = make_net(rng, dims, ct, act=Activation.ReLU, bias="rand", init="he" if ct == CT.Float16 else "half")
+        layers = gpu_layers(specs, ct, ML.RowMajor)
+        for B, pad in [(1, 0), (70, 0), (70, 3), (4099, 0), (300007, 1)]:
+            x = to_dev(rng.uniform(-1, 1, (B, dims[0])).astype(np.float16))
+            if ct == CT.FloatE4M3:
+                x = x.to(torch.float8_e4m3fn)
+            want = chain_of_single_layers(specs, x, ct)
+            pitch = dims[0] + pad
+            big = torch.full(((B - 1) * pitch + dims[0] + 1,), 0xff if ct == CT.FloatE4M3 else 0x7fff, dtype=torch.uint8 if ct == CT.FloatE4M3 else torch.int16, device=DEV)
+            rows = big.view(x.dtype).as_strided((B, dims[0]), (pitch, 1), 1)
+            rows.copy_(x)
+            out = torch.full((B * (dims[-1] + pad) + 1,), -7.0, dtype=torch.float16, device=DEV)
+            res = out[1:].view(B, dims[-1] + pad)
+            cv.mlpForward(layers, rows, weightType=ct, out=res[:, :dims[-1]])
+            seen.add(cv.lastKernelName().split("<")[0])
+            assert torch.equal(res[:, :dims[-1]].contiguous().view(torch.int16), want.view(torch.int16)), (dims, ct, B, pad, cv.lastKernelName())
+            assert out[0] == -7 and (res[:, dims[-1]:] == -7).all()
+    assert "mlpForwardKernel" in seen, seen
