@@ -34,6 +34,10 @@ namespace cv {
 namespace {
 
 constexpr int kRoundSamples = 64;
+// Networks of half wider than 64 whose weights leave no room for the vectors of 64 samples (8-128-128-128-128-4: 123 of 160 KB) take 32 to a
+// round: the same tiles of dW, and one row tile of the forward pass and of dX per wave instead of two.  A whole step, over the whole batch in
+// memory / in rounds of 32 (us): 8-128-128-128-128-4 over 1 024 samples 165 / 34, over 200 003 943 / 274; 128-128-128-128-9 146 / 30, 798 / 226.
+constexpr int kRoundFewSamples = 32;
 constexpr int kRoundThreads = 512;
 constexpr int kRoundMaxLayers = 5;
 
@@ -56,6 +60,7 @@ struct RoundArgs {
     const uint8_t* in; uint64_t inStride;
     const uint8_t* targets; uint64_t targetStride;
     uint32_t batch;
+    uint32_t samples;                // of a round
     int32_t inPieces;                // input rows of whole aligned 16-byte pieces: their number, else 0
     float lossScale;
     float* partials;
@@ -65,10 +70,10 @@ struct RoundArgs {
 };
 
 // Tiles per wave.  RT: half the 16-feature tiles of the widest layer, rounded up to 4 or 8 (RT = 2, 4).
-template <int RT>
+template <int RT, int SAMPLES>
 struct RoundSplit {
     // forward and dX: NS sample tiles x NT row tiles per wave; the waves of a sample group take every RG-th row tile
-    static constexpr int NS = RT == 4 ? 2 : 1, SG = 4 / NS, RG = 8 / SG, NT = 2;
+    static constexpr int NS = RT == 4 ? 2 : 1, SG = SAMPLES / 16 / NS, RG = 8 / SG, NT = SAMPLES / 32;
     // dW: WR x WC waves tile the matrix, KS of them the samples; RI x CJ tiles per wave
     static constexpr int WR = RT == 4 ? 4 : 2, WC = 2, KS = RT == 4 ? 1 : 2;
     static constexpr int RI = 2, CJ = RT == 2 ? 2 : 4;
@@ -90,6 +95,8 @@ template <> struct RoundMma<float> {
         const uint8_t* q = p + (uint32_t)(4 * g) * stride + 4 * i;
         return Op{*(const float*)q, *(const float*)(q + stride), *(const float*)(q + 2 * stride), *(const float*)(q + 3 * stride)};
     }
+    // the same of a matrix of sixteen rows (which a chunk has)
+    static __device__ __forceinline__ Op readColumnOf16(const uint8_t* p, uint32_t stride, int g, int i) { return readColumn(p, stride, g, i); }
     static __device__ __forceinline__ floatx4 mma(Op a, Op b, floatx4 c)
     {
 #pragma unroll
@@ -149,6 +156,14 @@ template <> struct RoundMma<half_t> {
         const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)q));
         const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)(q + 16 * stride)));
         return Op{lo.x, lo.y, hi.x, hi.y};
+    }
+    // the same of a matrix of sixteen rows
+    static __device__ __forceinline__ Op readColumnOf16(const uint8_t* p, uint32_t stride, int g, int i)
+    {
+        typedef short shortx4 __attribute__((ext_vector_type(4)));
+        typedef shortx4 __attribute__((address_space(3))) * LdsPtr;
+        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)(p + (uint32_t)(4 * g + (i >> 2)) * stride + 8 * (i & 3))));
+        return Op{lo.x, lo.y, 0u, 0u};
     }
     static __device__ __forceinline__ floatx4 mma(Op a, Op b, floatx4 c)
     {
@@ -275,11 +290,11 @@ __device__ __forceinline__ void stageRoundWeights(const RoundLayer (&layers)[kRo
 }
 
 // WAVES: per SIMD; 4 where two workgroups share a compute unit (128 registers a wave), else 2
-template <typename T, int NL, int RT, int WAVES>
+template <typename T, int NL, int RT, int WAVES, int SAMPLES>
 __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void trainRoundKernel(const RoundArgs a)
 {
     typedef RoundMma<T> M;
-    typedef RoundSplit<RT> S;
+    typedef RoundSplit<RT, SAMPLES> S;
     typedef typename M::Op Op;
     constexpr int KC = M::KC, ESZ = sizeof(T), NS = S::NS, NT = S::NT;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -315,22 +330,22 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
         }
     float lossAcc = 0.f, lossMaxAcc = 0.f;
 
-    const uint32_t lastSample = a.batch - 1, numRounds = lastSample / kRoundSamples + 1;
+    const uint32_t lastSample = a.batch - 1, numRounds = lastSample / SAMPLES + 1;
 
-    // ---- the network's input: eight threads to a sample, 16-byte pieces where rows are made of them, else elements.
+    // ---- the network's input: eight threads (sixteen) to a sample, 16-byte pieces where rows are made of them, else elements.
     //      Addresses always exist; what lies past the vector is not stored.
-    constexpr int PIECES = (2 * RT * 16 * ESZ / 16 + 7) / 8, ELEMS = 2 * RT * 16 / 8;
+    constexpr int PER = kRoundThreads / SAMPLES, PIECES = (2 * RT * 16 * ESZ / 16 + PER - 1) / PER, ELEMS = 2 * RT * 16 / PER;
     constexpr int IN_REGS = 4 * PIECES > ELEMS ? 4 * PIECES : ELEMS;
-    const int inRow = threadIdx.x >> 3;
+    const int inRow = threadIdx.x / PER;
     const int in0 = a.layers[0].in, topOut = a.layers[NL - 1].out;
     auto fetchInput = [&](uint32_t (&v)[IN_REGS], uint32_t r) {
-        int inCol = threadIdx.x & 7;
+        int inCol = threadIdx.x % PER;
         pinHere(inCol);                     // (the addresses are formed anew each round, see layer())
-        const uint8_t* row = a.in + (size_t)min(r * kRoundSamples + inRow, lastSample) * a.inStride;
+        const uint8_t* row = a.in + (size_t)min(r * SAMPLES + inRow, lastSample) * a.inStride;
         if (a.inPieces) {
 #pragma unroll
             for (int c = 0; c < PIECES; ++c) {
-                const u32x4 p = *(const u32x4*)(row + 16 * min(inCol + 8 * c, a.inPieces - 1));
+                const u32x4 p = *(const u32x4*)(row + 16 * min(inCol + PER * c, a.inPieces - 1));
                 v[4 * c] = p.x; v[4 * c + 1] = p.y; v[4 * c + 2] = p.z; v[4 * c + 3] = p.w;
             }
             asm volatile("");               // (the ends of the two branches differ: else their stores become one, to an address
@@ -338,26 +353,26 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
         } else {
 #pragma unroll
             for (int c = 0; c < ELEMS; ++c) {
-                const uint8_t* p = row + ESZ * min(inCol + 8 * c, in0 - 1);
+                const uint8_t* p = row + ESZ * min(inCol + PER * c, in0 - 1);
                 v[c] = ESZ == 4 ? *(const uint32_t*)p : *(const uint16_t*)p;
             }
         }
     };
     auto putInput = [&](const uint32_t (&v)[IN_REGS]) {
-        int inCol = threadIdx.x & 7;
+        int inCol = threadIdx.x % PER;
         pinHere(inCol);
         LayerInArgs& ly = layer(0);
         uint8_t* row = lds + ly.xOff + (uint32_t)inRow * ly.xStride;
         if (a.inPieces) {
 #pragma unroll
             for (int c = 0; c < PIECES; ++c)
-                if (inCol + 8 * c < a.inPieces) *(u32x4*)(row + 16 * (inCol + 8 * c)) = u32x4{v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]};
+                if (inCol + PER * c < a.inPieces) *(u32x4*)(row + 16 * (inCol + PER * c)) = u32x4{v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]};
         } else {
 #pragma unroll
             for (int c = 0; c < ELEMS; ++c)
-                if (inCol + 8 * c < in0) {
-                    if constexpr (ESZ == 4) *(uint32_t*)(row + 4 * (inCol + 8 * c)) = v[c];
-                    else *(uint16_t*)(row + 2 * (inCol + 8 * c)) = (uint16_t)v[c];
+                if (inCol + PER * c < in0) {
+                    if constexpr (ESZ == 4) *(uint32_t*)(row + 4 * (inCol + PER * c)) = v[c];
+                    else *(uint16_t*)(row + 2 * (inCol + PER * c)) = (uint16_t)v[c];
                 }
         }
     };
@@ -400,7 +415,7 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
     // ---- dW and db of layer l over this wave's samples of the round ------------------------------------------------------
     auto contract = [&](auto lc, auto rowsC, auto colsC, uint32_t dzOff, uint32_t dzStride) {
         constexpr int l = decltype(lc)::value, rows = decltype(rowsC)::value, cols = decltype(colsC)::value;
-        constexpr int chunks = kRoundSamples / S::KS / KC;
+        constexpr int chunks = SAMPLES / S::KS / KC;
         LayerInArgs& ly = layer(l);
         const uint8_t* dz = lds + dzOff + 16 * wr * ESZ;
         const uint8_t* x = lds + ly.xOff + 16 * wc * ESZ;
@@ -445,7 +460,7 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                 {
-                    const uint8_t* p = a.targets + (size_t)min(r * kRoundSamples + 16 * (NS * sg + s) + n, lastSample) * a.targetStride + ESZ * min(g4 + q, topOut - 1);
+                    const uint8_t* p = a.targets + (size_t)min(r * SAMPLES + 16 * (NS * sg + s) + n, lastSample) * a.targetStride + ESZ * min(g4 + q, topOut - 1);
                     tgt[s][q] = ESZ == 4 ? *(const uint32_t*)p : *(const uint16_t*)p;
                 }
         }
@@ -469,7 +484,7 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
             staticFor<0, NS>([&](auto sc) {
                 constexpr int s = decltype(sc)::value;
                 const int row = 16 * (NS * sg + s) + n;
-                const bool live = r * kRoundSamples + row < a.batch;
+                const bool live = r * SAMPLES + row < a.batch;
                 float tgtAll = 0.f;
                 if (!a.targets) {
                     // sin(sum of the inputs), each lane group a quarter of them, as the other steps form it
@@ -539,8 +554,11 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
                     for (int k = 0; k < ly.kOut; ++k) {
                         Op av[NT], bv[NS];
 #pragma unroll
-                        for (int t = 0; t < NT; ++t)
-                            av[t] = M::readColumn(lds + ly.wOff + (uint32_t)(k * KC) * ly.wStride + 16 * (rg + S::RG * (t < mine ? t : 0)) * ESZ, ly.wStride, g, n);
+                        for (int t = 0; t < NT; ++t) {
+                            const uint8_t* w = lds + ly.wOff + (uint32_t)(k * KC) * ly.wStride + 16 * (rg + S::RG * (t < mine ? t : 0)) * ESZ;
+                            if constexpr (SAMPLES == kRoundFewSamples && l + 1 == NL) av[t] = M::readColumnOf16(w, ly.wStride, g, n);
+                            else av[t] = M::readColumn(w, ly.wStride, g, n);
+                        }
 #pragma unroll
                         for (int s = 0; s < NS; ++s) bv[s] = M::readRowSplit(dz + (uint32_t)(16 * s) * dzStride + k * KC * ESZ, g);
 #pragma unroll
@@ -689,7 +707,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void trainRoundReduceKernel(cons
 
 // Lays the network out in LDS.  False where the kernel does not apply: more than five layers, more than 128 inputs or hidden
 // units, more than 16 outputs, an input encoding, or weights and a round that do not fit the LDS of a compute unit.
-inline bool planRound(const MlpArgs& m, int ct, RoundArgs& a, int& maxTiles)
+inline bool planRoundOf(uint32_t samples, const MlpArgs& m, int ct, RoundArgs& a, int& maxTiles)
 {
     const uint32_t esz = elemSize(ct), kc = ct == kF32 ? 16u : 32u;
     const int L = m.numLayers;
@@ -707,22 +725,28 @@ inline bool planRound(const MlpArgs& m, int ct, RoundArgs& a, int& maxTiles)
         ly.kIn = (int32_t)(up((uint32_t)src.in, kc) / kc); ly.kOut = (int32_t)(up((uint32_t)src.out, kc) / kc);
         if (ly.colTiles > maxTiles) maxTiles = ly.colTiles;
         ly.wStride = (uint32_t)ly.kIn * kc * esz + 16u;
-        ly.wOff = off; off += (uint32_t)ly.kOut * kc * ly.wStride;
+        ly.wOff = off; off += (samples == (uint32_t)kRoundFewSamples && l + 1 == L ? 16u : (uint32_t)ly.kOut * kc) * ly.wStride;      // (readColumnOf16)
         ly.tileBase = tiles; tiles += (uint32_t)(ly.rowTiles * ly.colTiles);
         ly.dbBase = groups; groups += (uint32_t)ly.rowTiles;
     }
     for (int l = 0; l < L; ++l) { a.layers[l].biasOff = off; off += (uint32_t)a.layers[l].rowTiles * 64u; }
     for (int l = 0; l < L; ++l) {
         a.layers[l].xStride = (uint32_t)a.layers[l].kIn * kc * esz + 16u;
-        a.layers[l].xOff = off; off += kRoundSamples * a.layers[l].xStride;
+        a.layers[l].xOff = off; off += samples * a.layers[l].xStride;
     }
     a.zStride = (uint32_t)a.layers[L - 1].kOut * kc * esz + 16u;
-    a.zOff = off; off += kRoundSamples * a.zStride;
+    a.zOff = off; off += samples * a.zStride;
     constexpr uint32_t kLeast = 17u * 1024u;      // the final sums of waves that share tiles
     a.ldsBytes = (off > kLeast ? off : kLeast) + 16u;
     a.dwTiles = tiles;
     a.partialFloats = tiles * 256u + groups * 16u + 16u;
+    a.samples = samples;
     return a.ldsBytes <= 160u * 1024u;
+}
+inline bool planRound(const MlpArgs& m, int ct, RoundArgs& a, int& maxTiles)
+{
+    if (planRoundOf(kRoundSamples, m, ct, a, maxTiles)) return true;
+    return ct == kF16 && m.numLayers >= 4 && planRoundOf(kRoundFewSamples, m, ct, a, maxTiles) && maxTiles > 4;
 }
 
 // Two workgroups to a compute unit where their LDS fits twice and a wave gets by with 128 registers.
@@ -733,23 +757,23 @@ inline uint32_t roundWorkgroups(const RoundArgs& a, int layers, int rt, int numC
 }
 inline int roundTiles(int maxTiles) { return maxTiles > 4 ? 4 : 2; }
 // workgroups of a launch: no more than the batch has rounds
-inline uint32_t roundBlocks(uint32_t batch, uint32_t resident)
+inline uint32_t roundBlocks(uint32_t batch, uint32_t samples, uint32_t resident)
 {
-    const uint32_t rounds = batch ? (batch - 1) / kRoundSamples + 1 : 1;
+    const uint32_t rounds = batch ? (batch - 1) / samples + 1 : 1;
     return rounds < resident ? rounds : resident;
 }
 
-template <typename T, int NL, int RT>
+template <typename T, int NL, int RT, int SAMPLES>
 hipError_t launchRoundSized(hipStream_t stream, const TrainLaunch& t, RoundArgs& a, int numCUs)
 {
     constexpr int WAVES = roundWavesPerSimd(NL, RT);
-    const hipError_t e = allowDynamicLds<trainRoundKernel<T, NL, RT, WAVES>>(160 * 1024);
+    const hipError_t e = allowDynamicLds<trainRoundKernel<T, NL, RT, WAVES, SAMPLES>>(160 * 1024);
     if (e != hipSuccess) return e;
-    const uint32_t blocks = roundBlocks(t.mlp.batch, roundWorkgroups(a, NL, RT, numCUs));
+    const uint32_t blocks = roundBlocks(t.mlp.batch, SAMPLES, roundWorkgroups(a, NL, RT, numCUs));
     a.finish.numPartials = blocks;
-    noteKernel(false, "trainRoundKernel<%s,%d layers,up to %d rows> + trainRoundReduceKernel",
-               sizeof(T) == 4 ? "f32" : "f16", NL, 32 * RT);
-    hipLaunchKernelGGL((trainRoundKernel<T, NL, RT, WAVES>), dim3(blocks), dim3(kRoundThreads), a.ldsBytes, stream, a);
+    noteKernel(false, "trainRoundKernel<%s,%d layers,up to %d rows%s> + trainRoundReduceKernel",
+               sizeof(T) == 4 ? "f32" : "f16", NL, 32 * RT, SAMPLES == kRoundFewSamples ? ",32 samples" : "");
+    hipLaunchKernelGGL((trainRoundKernel<T, NL, RT, WAVES, SAMPLES>), dim3(blocks), dim3(kRoundThreads), a.ldsBytes, stream, a);
     const hipError_t e1 = hipGetLastError();
     if (e1 != hipSuccess) return e1;
     hipLaunchKernelGGL(trainRoundReduceKernel, dim3((a.partialFloats - 16u) / 64u + 1u), dim3(64 * kReduceWaves), 0, stream, a);
@@ -787,9 +811,13 @@ hipError_t launchRoundTyped(hipStream_t stream, const TrainLaunch& t, int numCUs
     int maxTiles = 0;
     if (!fillRoundArgs<T>(t, a, maxTiles)) return hipErrorInvalidValue;
     const int L = t.mlp.numLayers;
+    if constexpr (sizeof(T) == 2) {
+        if (a.samples == (uint32_t)kRoundFewSamples)
+            return L == 4 ? launchRoundSized<T, 4, 4, kRoundFewSamples>(stream, t, a, numCUs) : launchRoundSized<T, 5, 4, kRoundFewSamples>(stream, t, a, numCUs);
+    }
     switch (roundTiles(maxTiles) * 8 + L) {
-#define CV_L(RT) case RT * 8 + 2: return launchRoundSized<T, 2, RT>(stream, t, a, numCUs); case RT * 8 + 3: return launchRoundSized<T, 3, RT>(stream, t, a, numCUs); \
-                 case RT * 8 + 4: return launchRoundSized<T, 4, RT>(stream, t, a, numCUs); case RT * 8 + 5: return launchRoundSized<T, 5, RT>(stream, t, a, numCUs);
+#define CV_L(RT) case RT * 8 + 2: return launchRoundSized<T, 2, RT, kRoundSamples>(stream, t, a, numCUs); case RT * 8 + 3: return launchRoundSized<T, 3, RT, kRoundSamples>(stream, t, a, numCUs); \
+                 case RT * 8 + 4: return launchRoundSized<T, 4, RT, kRoundSamples>(stream, t, a, numCUs); case RT * 8 + 5: return launchRoundSized<T, 5, RT, kRoundSamples>(stream, t, a, numCUs);
     CV_L(2) CV_L(4)
 #undef CV_L
     }

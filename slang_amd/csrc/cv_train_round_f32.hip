@@ -15,7 +15,7 @@ size_t trainRoundWorkspaceBytes(const MlpArgs& shapes, int numCUs, int carrierCt
     if (!planRound(shapes, carrierCt, a, maxTiles)) return 0;
     // a partial per workgroup: one per round of the batch, as long as they are all resident (trainWaveKernel: per two rounds and
     // per compute unit, never more)
-    return (size_t)roundBlocks(shapes.batch, roundWorkgroups(a, shapes.numLayers, roundTiles(maxTiles), numCUs)) * a.partialFloats * sizeof(float);
+    return (size_t)roundBlocks(shapes.batch, a.samples, roundWorkgroups(a, shapes.numLayers, roundTiles(maxTiles), numCUs)) * a.partialFloats * sizeof(float);
 }
 
 hipError_t launchTrainRound(hipStream_t stream, const TrainLaunch& t, int numCUs)

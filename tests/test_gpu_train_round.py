@@ -85,6 +85,8 @@ CASES = [
     ("f32", [31, 32, 32, 32, 31, 16], 129), ("f32", [1, 1, 1], 200), ("f32", [100, 128, 4], 130), ("f32", [65, 65, 20, 3], 77), ("f32", [16, 64, 64, 64, 64, 2], 300),
     ("f32", [64, 64, 64, 9], 4097), ("f32", [40, 32, 20, 32, 32, 16], 128), ("f32", [16, 10, 16, 16, 16, 1], 17), ("f32", [12, 50, 2], 2049), ("f32", [30, 40, 33, 64, 7], 190),
     ("f16", [16, 128, 128, 128, 8], 64), ("f16", [16, 128, 128, 128, 8], 40001), ("f16", [33, 16, 2], 1), ("f16", [64, 64, 64, 16], 65), ("f16", [40, 20, 49, 5], 127),
+    ("f16", [8, 128, 128, 128, 128, 4], 1), ("f16", [32, 128, 128, 128, 128, 16], 33), ("f16", [21, 128, 128, 128, 128, 5], 20011), ("f16", [7, 128, 113, 128, 97, 1], 1000),
+    ("f16", [128, 128, 128, 128, 9], 95),
     ("f16", [127, 33, 12], 300), ("f16", [48, 96, 80, 3], 200), ("f16", [10, 65, 33, 97, 16], 63), ("f16", [20, 129 - 1, 17, 64, 30, 7], 500), ("f16", [50, 30, 30, 30, 30, 1], 70),
 ]
 
