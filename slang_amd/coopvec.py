@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 import enum
+import struct
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
@@ -609,26 +610,39 @@ def _mlp_carrier_type(weightType: int) -> CoopVecComponentType:
     return CoopVecComponentType.Float16
 
 
+# CvMlpLayer and CvMlpDesc as struct formats: a structure written in one call instead of field by field, each by way of a proxy of its array
+# element (a description of two / four layers 8.5 / 14.9 us field by field, 6.0 / 10.0 us so; every training and optimiser step makes one).
+_MLP_LAYER = struct.Struct("=4QiiiIiIif")
+_MLP_DESC = struct.Struct("=Q6iIiQ")
+assert _MLP_LAYER.size == ctypes.sizeof(_lib.CvMlpLayer) and _MLP_DESC.size == ctypes.sizeof(_lib.CvMlpDesc)
+
+
 def _mlp_desc(layers: Sequence[FeedForwardLayer], weightType: int, gradType: int, flags: int,
               inputEncoding: int = 0):
+    """(CvMlpDesc, the array it points to: the caller keeps both until its call has returned)"""
     arr = (_lib.CvMlpLayer * len(layers))()
     for i, L in enumerate(layers):
-        arr[i].weights = _buffer_ptr(L.weights, "weights")
-        arr[i].weightsGrad = _buffer_ptr(L.weightsGrad, "weightsGrad") if L.weightsGrad is not None else None
-        arr[i].biases = _buffer_ptr(L.biases, "biases") if L.biases is not None else None
-        arr[i].biasesGrad = _buffer_ptr(L.biasesGrad, "biasesGrad") if L.biasesGrad is not None else None
-        arr[i].inputSize = L.inputSize; arr[i].outputSize = L.outputSize
-        arr[i].weightLayout = int(L.weightLayout); arr[i].weightStride = int(L.weightStride)
-        arr[i].gradLayout = int(L.gradLayout); arr[i].gradStride = int(L.gradStride)
-        arr[i].activation = int(L.activation); arr[i].leakySlope = float(L.leakySlope)
+        weights = _buffer_ptr(L.weights, "weights")
+        weightsGrad = _buffer_ptr(L.weightsGrad, "weightsGrad") if L.weightsGrad is not None else 0
+        biases = _buffer_ptr(L.biases, "biases") if L.biases is not None else 0
+        biasesGrad = _buffer_ptr(L.biasesGrad, "biasesGrad") if L.biasesGrad is not None else 0
+        try:
+            _MLP_LAYER.pack_into(arr, i * _MLP_LAYER.size, weights, weightsGrad, biases, biasesGrad, L.inputSize, L.outputSize,
+                                 L.weightLayout, L.weightStride, L.gradLayout, L.gradStride, L.activation, L.leakySlope)
+        except (struct.error, OverflowError, TypeError):      # (what only a conversion makes a number of the field's type)
+            arr[i] = _lib.CvMlpLayer(weights, weightsGrad, biases, biasesGrad, L.inputSize, L.outputSize, int(L.weightLayout), int(L.weightStride),
+                                     int(L.gradLayout), int(L.gradStride), int(L.activation), float(L.leakySlope))
+    carrier = int(_mlp_carrier_type(weightType))      # half, or T for networks of one type T = float / bfloat16
     d = _lib.CvMlpDesc()
-    d.layers = arr; d.numLayers = len(layers)
-    d.inputType = int(weightType); d.weightType = int(weightType)
-    carrier = _mlp_carrier_type(weightType)      # half, or T for networks of one type T = float / bfloat16
-    d.biasType = int(carrier); d.outputType = int(carrier)
-    d.gradType = int(gradType); d.flags = int(flags); d.inputEncoding = int(inputEncoding)
-    if inputEncoding:
-        d.inputType = int(CoopVecComponentType.Float32)
+    inputType = CoopVecComponentType.Float32 if inputEncoding else int(weightType)
+    try:
+        _MLP_DESC.pack_into(d, 0, ctypes.addressof(arr), len(layers), inputType, int(weightType), carrier, carrier, int(gradType), int(flags),
+                            int(inputEncoding), 0)
+    except struct.error:
+        d.layers = arr; d.numLayers = len(layers)
+        d.inputType = int(inputType); d.weightType = int(weightType)
+        d.biasType = carrier; d.outputType = carrier
+        d.gradType = int(gradType); d.flags = int(flags); d.inputEncoding = int(inputEncoding)
     return d, arr
 
 

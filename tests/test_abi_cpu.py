@@ -245,3 +245,28 @@ def test_bench_traffic_figures_come_from_the_profile_summaries():
         nbytes, path = traffic[key]
         assert nbytes > 100000 and os.path.exists(os.path.join(repo, path))
     assert set(bench.DEFAULT_RUN) <= set(bench.WORKLOADS) and bench.HEADLINE in bench.WORKLOADS
+
+
+@pytest.mark.parametrize("odd", [{}, dict(weightLayout=1.0, leakySlope=1), dict(leakySlope=1e39), dict(weightStride=-1), dict(gradStride=1 << 33)])
+def test_a_network_description_field_by_field(monkeypatch, odd):
+    # written in one call where the values are of the fields' types; what a field converts (or wraps) as before
+    import torch
+    from slang_amd import _lib, coopvec as cv
+    monkeypatch.setattr(cv, "_buffer_ptr", lambda t, what: t.data_ptr())
+    t = [torch.zeros(16, dtype=torch.uint8) for _ in range(4)]
+    base = dict(weightLayout=cv.CoopVecMatrixLayout.InferencingOptimal, weightStride=48, activation=cv.Activation.LeakyReLU, leakySlope=0.25, gradStride=96)
+    base.update(odd)
+    layers = [cv.FeedForwardLayer(20, 48, t[0], t[1], weightsGrad=t[2], biasesGrad=t[3], **base), cv.FeedForwardLayer(48, 5, t[0])]
+    d, arr = cv._mlp_desc(layers, cv.CoopVecComponentType.Float32, cv.CoopVecComponentType.Float32, 5, 1)
+    for at, L in enumerate(layers):
+        want = _lib.CvMlpLayer()
+        want.weights = L.weights.data_ptr()
+        for name in ("weightsGrad", "biases", "biasesGrad"):
+            setattr(want, name, getattr(L, name).data_ptr() if getattr(L, name) is not None else None)
+        want.inputSize, want.outputSize = L.inputSize, L.outputSize
+        want.leakySlope = float(L.leakySlope)
+        for name in ("weightLayout", "weightStride", "gradLayout", "gradStride", "activation"):
+            setattr(want, name, int(getattr(L, name)))
+        assert bytes(d.layers[at]) == bytes(want) == bytes(arr[at])
+    f32 = int(cv.CoopVecComponentType.Float32)
+    assert (d.numLayers, d.inputType, d.weightType, d.biasType, d.outputType, d.gradType, d.flags, d.inputEncoding, d.lossMax) == (2, f32, f32, f32, f32, f32, 5, 1, None)
