@@ -228,44 +228,68 @@ template <> struct RoundMma<half_t> {
 // every wave of the workgroup has finished its LDS accesses; loads from memory stay in flight
 __device__ __forceinline__ void meetInLds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Weights and biases of all layers to LDS.  A row-major matrix of whole aligned 16-byte pieces (what a program's own matrices
-// mostly are) goes in pieces, and the first kAhead pieces of a thread of every layer are requested before the first is stored: one
-// round trip to memory for all of them instead of one for every four elements.  16-128-128-128-8 (half), 64 samples to a
-// workgroup, see the head of this file.
+// Weights and biases of all layers to LDS.  A row-major matrix (what a program's own matrices mostly are) goes in 16-byte pieces, of
+// half at whatever element they begin, and the first kAhead pieces of a thread of every layer are requested before the first is stored:
+// one round trip to memory for all of them instead of one for every four elements.  16-128-128-128-8 (half), 64 samples to a workgroup, see
+// the head of this file.  Rows of half that are no whole aligned pieces, element by element / so (us): 7-67-16-67-123-1 over 5 923 samples
+// 35 / 24, 26-81-11-80-2 over 15 796 24.5 / 20, 12-128-128-128-15 over 1 819 26 / 23.  That is an instantiation of its own (ANY): the longer
+// code costs a network that does not need it 1 to 2 us (16-128-128-128-8 over 200 003 samples 151.7 / 154.2), and one of float whose rows do
+// (36-64-64-64-64-14 over 3 167 30.6 / 32.1), so that float stays element by element.
 template <typename T>
-__device__ __forceinline__ size_t roundWeightLine(const RoundLayer& ly) { return ly.shape.stride ? ly.shape.stride : (size_t)ly.shape.cols * sizeof(T); }
+__host__ __device__ __forceinline__ size_t roundWeightLine(const RoundLayer& ly) { return ly.shape.stride ? ly.shape.stride : (size_t)ly.shape.cols * sizeof(T); }
 template <typename T>
+__device__ __forceinline__ size_t roundWeightBytes(const RoundLayer& ly) { return (size_t)(ly.out - 1) * roundWeightLine<T>(ly) + (size_t)ly.in * sizeof(T); }
+// rows of whole aligned pieces
+template <typename T>
+__host__ __device__ __forceinline__ bool roundWeightWhole(const RoundLayer& ly)
+{
+    return ((size_t)ly.in * sizeof(T)) % 16u == 0 && (((uintptr_t)ly.w | roundWeightLine<T>(ly)) & 15u) == 0;
+}
+template <typename T, bool ANY>
 __device__ __forceinline__ bool roundWeightPieces(const RoundLayer& ly)
 {
-    return ly.shape.layout == kRowMajor && ((size_t)ly.in * sizeof(T)) % 16u == 0 && (((uintptr_t)ly.w | roundWeightLine<T>(ly)) & 15u) == 0;
+    return ly.shape.layout == kRowMajor && (ANY ? roundWeightBytes<T>(ly) >= 16u : roundWeightWhole<T>(ly));
 }
-template <typename T, int NL, int MAXT>
+template <typename T, int NL, int MAXT, bool ANY = false>
 __device__ __forceinline__ void stageRoundWeights(const RoundLayer (&layers)[kRoundMaxLayers], uint8_t* lds)
 {
     constexpr int kMost = MAXT * 16 * MAXT * 16 * (int)sizeof(T) / 16 / kRoundThreads, kUpTo = NL < 5 ? 4 : 2, kAhead = kMost < 1 ? 1 : kMost < kUpTo ? kMost : kUpTo;
     u32x4 v[NL][kAhead];
     auto piece = [&](const RoundLayer& ly, uint32_t c, uint32_t& row, uint32_t& at) {
-        const uint32_t perRow = (uint32_t)ly.in * sizeof(T) / 16u;
+        const uint32_t perRow = ((uint32_t)ly.in * sizeof(T) + 15u) / 16u;
         row = c / perRow;
         at = c - row * perRow;
         return row < (uint32_t)ly.out;
     };
-    auto load = [&](const RoundLayer& ly, uint32_t row, uint32_t at) {
-        return *(const u32x4*)(ly.w + row * roundWeightLine<T>(ly) + 16u * at);
+    // (a piece that would end behind the matrix is read ending there and moved down; what lies behind its row is cleared)
+    auto load = [&](const RoundLayer& ly, bool whole, uint32_t row, uint32_t at) {
+        if (whole) return *(const u32x4*)(ly.w + row * roundWeightLine<T>(ly) + 16u * at);
+        const size_t off = row * roundWeightLine<T>(ly) + 16u * at, last = roundWeightBytes<T>(ly) - 16u;
+        return ((const Loose16<(int)sizeof(T)>*)(ly.w + (off < last ? off : last)))->v;
     };
-    auto store = [&](const RoundLayer& ly, uint32_t row, uint32_t at, u32x4 x) { *(u32x4*)(lds + ly.wOff + row * ly.wStride + 16u * at) = x; };
+    auto store = [&](const RoundLayer& ly, bool whole, uint32_t row, uint32_t at, u32x4 v) {
+        if (!whole) {
+            const size_t off = row * roundWeightLine<T>(ly) + 16u * at, last = roundWeightBytes<T>(ly) - 16u;
+            uint32_t x[4] = {v.x, v.y, v.z, v.w};
+            if (off > last) shiftDown<(int)sizeof(T)>(x, (int)(off - last));
+            clearBehind<(int)sizeof(T)>(x, ly.in * (int)sizeof(T) - 16 * (int)at);
+            v = u32x4{x[0], x[1], x[2], x[3]};
+        }
+        *(u32x4*)(lds + ly.wOff + row * ly.wStride + 16u * at) = v;
+    };
     float bias[NL];
 #pragma unroll
     for (int l = 0; l < NL; ++l) {
         const RoundLayer& ly = layers[l];
         const int e = threadIdx.x;
         bias[l] = ly.bias && e < ly.out ? (float)((const T*)ly.bias)[e] : 0.f;      // (no layer has more rows than the workgroup threads)
-        if (!roundWeightPieces<T>(ly)) continue;
+        if (!roundWeightPieces<T, ANY>(ly)) continue;
+        const bool whole = !ANY || roundWeightWhole<T>(ly);
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) {
             uint32_t row, at;
             const bool on = piece(ly, threadIdx.x + (uint32_t)(i * kRoundThreads), row, at);
-            v[l][i] = load(ly, on ? row : 0u, on ? at : 0u);
+            v[l][i] = load(ly, whole, on ? row : 0u, on ? at : 0u);
         }
     }
 #pragma unroll
@@ -273,11 +297,12 @@ __device__ __forceinline__ void stageRoundWeights(const RoundLayer (&layers)[kRo
         const RoundLayer& ly = layers[l];
         if ((int)threadIdx.x < ly.out) *(float*)(lds + ly.biasOff + 4 * threadIdx.x) = bias[l];
         uint32_t row, at;
-        if (roundWeightPieces<T>(ly)) {
+        if (roundWeightPieces<T, ANY>(ly)) {
+            const bool whole = !ANY || roundWeightWhole<T>(ly);
 #pragma unroll
             for (int i = 0; i < kAhead; ++i)
-                if (piece(ly, threadIdx.x + (uint32_t)(i * kRoundThreads), row, at)) store(ly, row, at, v[l][i]);
-            for (uint32_t c = threadIdx.x + (uint32_t)(kAhead * kRoundThreads); piece(ly, c, row, at); c += kRoundThreads) store(ly, row, at, load(ly, row, at));
+                if (piece(ly, threadIdx.x + (uint32_t)(i * kRoundThreads), row, at)) store(ly, whole, row, at, v[l][i]);
+            for (uint32_t c = threadIdx.x + (uint32_t)(kAhead * kRoundThreads); piece(ly, c, row, at); c += kRoundThreads) store(ly, whole, row, at, load(ly, whole, row, at));
         } else {
             const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
             for (int col = lane; col < ly.in; col += 64) {
@@ -290,7 +315,8 @@ __device__ __forceinline__ void stageRoundWeights(const RoundLayer (&layers)[kRo
 }
 
 // WAVES: per SIMD; 4 where two workgroups share a compute unit (128 registers a wave), else 2
-template <typename T, int NL, int RT, int WAVES, int SAMPLES>
+// ANY (half): some matrix is row-major with rows that are no whole aligned pieces
+template <typename T, int NL, int RT, int WAVES, int SAMPLES, bool ANY>
 __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void trainRoundKernel(const RoundArgs a)
 {
     typedef RoundMma<T> M;
@@ -302,7 +328,7 @@ __global__ __launch_bounds__(kRoundThreads) __attribute__((amdgpu_waves_per_eu(W
 
     for (uint32_t i = threadIdx.x; i < a.ldsBytes / 16; i += kRoundThreads) ((u32x4*)lds)[i] = u32x4{0u, 0u, 0u, 0u};
     __syncthreads();
-    stageRoundWeights<T, NL, 2 * RT>(a.layers, lds);
+    stageRoundWeights<T, NL, 2 * RT, ANY>(a.layers, lds);
     __syncthreads();
 
     // The layers' sizes and places in LDS are read from the kernel's arguments where they are used (scalar loads): hoisted out
@@ -763,17 +789,22 @@ inline uint32_t roundBlocks(uint32_t batch, uint32_t samples, uint32_t resident)
     return rounds < resident ? rounds : resident;
 }
 
-template <typename T, int NL, int RT, int SAMPLES>
+template <typename T, int NL, int RT, int SAMPLES, bool ANY = false>
 hipError_t launchRoundSized(hipStream_t stream, const TrainLaunch& t, RoundArgs& a, int numCUs)
 {
+    if constexpr (sizeof(T) == 2 && !ANY) {
+        bool any = false;
+        for (int l = 0; l < NL; ++l) any = any || (a.layers[l].shape.layout == kRowMajor && !roundWeightWhole<T>(a.layers[l]));
+        if (any) return launchRoundSized<T, NL, RT, SAMPLES, true>(stream, t, a, numCUs);
+    }
     constexpr int WAVES = roundWavesPerSimd(NL, RT);
-    const hipError_t e = allowDynamicLds<trainRoundKernel<T, NL, RT, WAVES, SAMPLES>>(160 * 1024);
+    const hipError_t e = allowDynamicLds<trainRoundKernel<T, NL, RT, WAVES, SAMPLES, ANY>>(160 * 1024);
     if (e != hipSuccess) return e;
     const uint32_t blocks = roundBlocks(t.mlp.batch, SAMPLES, roundWorkgroups(a, NL, RT, numCUs));
     a.finish.numPartials = blocks;
     noteKernel(false, "trainRoundKernel<%s,%d layers,up to %d rows%s> + trainRoundReduceKernel",
                sizeof(T) == 4 ? "f32" : "f16", NL, 32 * RT, SAMPLES == kRoundFewSamples ? ",32 samples" : "");
-    hipLaunchKernelGGL((trainRoundKernel<T, NL, RT, WAVES, SAMPLES>), dim3(blocks), dim3(kRoundThreads), a.ldsBytes, stream, a);
+    hipLaunchKernelGGL((trainRoundKernel<T, NL, RT, WAVES, SAMPLES, ANY>), dim3(blocks), dim3(kRoundThreads), a.ldsBytes, stream, a);
     const hipError_t e1 = hipGetLastError();
     if (e1 != hipSuccess) return e1;
     hipLaunchKernelGGL(trainRoundReduceKernel, dim3((a.partialFloats - 16u) / 64u + 1u), dim3(64 * kReduceWaves), 0, stream, a);

@@ -87,6 +87,8 @@ CASES = [
     ("f16", [16, 128, 128, 128, 8], 64), ("f16", [16, 128, 128, 128, 8], 40001), ("f16", [33, 16, 2], 1), ("f16", [64, 64, 64, 16], 65), ("f16", [40, 20, 49, 5], 127),
     ("f16", [8, 128, 128, 128, 128, 4], 1), ("f16", [32, 128, 128, 128, 128, 16], 33), ("f16", [21, 128, 128, 128, 128, 5], 20011), ("f16", [7, 128, 113, 128, 97, 1], 1000),
     ("f16", [128, 128, 128, 128, 9], 95),
+    # (rows of weights that begin at any half: every remainder of a piece, matrices of few bytes)
+    ("f16", [33, 65, 1, 66, 2], 70), ("f16", [1, 67, 3, 68, 1], 70), ("f16", [34, 69, 5, 70, 16], 70), ("f16", [39, 71, 79, 2], 70), ("f16", [36, 73, 2, 6], 70),
     ("f16", [127, 33, 12], 300), ("f16", [48, 96, 80, 3], 200), ("f16", [10, 65, 33, 97, 16], 63), ("f16", [20, 129 - 1, 17, 64, 30, 7], 500), ("f16", [50, 30, 30, 30, 30, 1], 70),
 ]
 
