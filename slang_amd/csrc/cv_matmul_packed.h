@@ -1,8 +1,9 @@
 // cv_matmul_packed.h -- the batched matMul for vectors of any length and alignment.
 //
 // Vectors.  A wave takes 16 * NT samples at a time and a lane its k-slots of a sample in reads of 16 bytes at whatever element
-// they begin, a tile ahead; what lies behind the end of a vector (of the next one) is cleared in registers.  The samples whose reads
-// would leave the buffer, the last few of a batch, are read element by element.
+// they begin, a tile ahead; what lies behind the end of a vector (of the next one) is cleared in registers.  Reads that would leave the
+// buffer, of the last few samples of a batch, are made ending where it ends and moved down (loadUpTo; cv_reads.h says where reads lie);
+// element by element only where all vectors together are less than 16 bytes.
 // Results.  A tile's results meet in the wave's own part of the LDS, whole rows or segments of them, exactly as they lie in
 // memory, and leave in pieces of 16 bytes at whatever element these begin; packed vectors of any length are one block, 16 of which
 // are a whole number of pieces.
@@ -150,13 +151,13 @@ __device__ __forceinline__ void packedRows(const MatMulArgs& a, const PackedPlan
     uint32_t tile = blockIdx.x * waves + wave;
 
     // which of a lane's k-slots exist: in every lane all of the first wholeFragments fragments' ones
-    const int colBase = (int)(g * gs), validBytes = min((int)gs, max(a.k - colBase, 0)) * IESZ;
+    const int colBase = (int)(g * gs), validBytes = sliceBytes((uint32_t)a.k, gs, g, IESZ);
     const int wholeFragments = min((int)gs, max(a.k - 3 * (int)gs, 0)) / EPL;
     constexpr bool MASK = Fl::kIsFloat || Fl::kAnySign;      // (signed bytes: what has no weight adds nothing)
 
     // a tile whose lanes' reads, up to the last k-slot of the last lane group, end inside the buffer
-    const uint64_t inEnd = (uint64_t)(a.batch - 1) * a.inStride + (uint64_t)a.k * IESZ;
-    auto inside = [&](uint32_t t) { return ((uint64_t)t * S + S - 1) * a.inStride + (3 * gs + KT * EPL) * IESZ <= inEnd; };
+    const uint64_t inEnd = vectorsEnd(a.batch, a.inStride, (uint32_t)a.k, IESZ);
+    auto inside = [&](uint32_t t) { return tileReadsEnd((uint64_t)t * S, S, a.inStride, gs, KT * EPL, IESZ) <= inEnd; };
     const int tailSlots = (int)gs - (KT - 1) * EPL, tailDwords = tailSlots * IESZ == 12 ? 4 : tailSlots * IESZ / 4;
     uint32_t raw[NT][KT][IRAW] = {};
     auto request = [&](uint32_t t) {
@@ -229,11 +230,11 @@ __device__ __forceinline__ void packedRows(const MatMulArgs& a, const PackedPlan
         } else {
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                const uint8_t* q = a.in + min((uint64_t)tile * S + 16 * j + n, (uint64_t)(a.batch - 1)) * a.inStride + colBase * IESZ;
+                const uint64_t at = min((uint64_t)tile * S + 16 * j + n, (uint64_t)(a.batch - 1)) * a.inStride + colBase * IESZ;
 #pragma unroll
                 for (int kt = 0; kt < KT; ++kt) {
-                    if (inEnd >= 16) loadUpTo<IESZ>(q + kt * EPL * IESZ, a.in + inEnd, raw[j][kt]);
-                    else loadSlots<IRAW>(raw[j][kt], q + kt * EPL * IESZ, validBytes - kt * EPL * IESZ, 2);
+                    if (inEnd >= 16) loadUpTo<IESZ>(a.in, at + kt * EPL * IESZ, inEnd, raw[j][kt]);
+                    else loadSlots<IRAW>(raw[j][kt], a.in + at + kt * EPL * IESZ, validBytes - kt * EPL * IESZ, 2);
                 }
             }
         }

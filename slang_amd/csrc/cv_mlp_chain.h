@@ -343,9 +343,9 @@ __global__ __launch_bounds__((chainThreads<Mma, MAXT>()), Mma::kEsz == 4 ? (MAXT
     const int g = lane >> 4, n = lane & 15;
     const int in0 = a.layers[0].in, gs0 = (int)optGS((uint32_t)in0);
     // which of a lane's k-slots exist: in every lane all of the first wholeFragments fragments' ones
-    const int colBase = g * gs0, validBytes = min(gs0, max(in0 - colBase, 0)) * ESZ;
+    const int colBase = g * gs0, validBytes = sliceBytes((uint32_t)in0, (uint32_t)gs0, (uint32_t)g, ESZ);
     const int wholeFragments = min(gs0, max(in0 - 3 * gs0, 0)) / 8;
-    const uint64_t inEnd = (uint64_t)(a.batch - 1) * a.inStride + (uint64_t)in0 * ESZ;
+    const uint64_t inEnd = vectorsEnd(a.batch, a.inStride, (uint32_t)in0, ESZ);
     const int kt0 = ga.gl[0].kt;
     const uint32_t laneOffset = (uint32_t)n * (uint32_t)a.inStride + (uint32_t)colBase * ESZ;
     // offsets of a lane's groups of four, the same for every tile (of float, where registers are scarce, formed for each)
@@ -402,8 +402,8 @@ __global__ __launch_bounds__((chainThreads<Mma, MAXT>()), Mma::kEsz == 4 ? (MAXT
                 continue;
             }
             const uint32_t first = min(tile + nt, numTiles - 1) * 16u;      // (beyond the batch: the last tile, whose results nobody stores)
-            // reads of 16 bytes (8) at whatever element a lane's slots begin; those that would end behind the last vector one by one
-            if ((uint64_t)(first + 15u) * a.inStride + (uint64_t)((3 * gs0 + 8 * kt0) * ESZ) <= inEnd) {
+            // reads of 16 bytes (8) at whatever element a lane's slots begin; what would end behind the last vector is read ending there and moved down (loadUpTo)
+            if (tileReadsEnd(first, 16u, a.inStride, (uint32_t)gs0, (uint32_t)(8 * kt0), ESZ) <= inEnd) {
                 const uint8_t* base = a.in + (uint64_t)first * a.inStride;
 #pragma unroll
                 for (int kt = 0; kt < INKT; ++kt) {
@@ -418,12 +418,12 @@ __global__ __launch_bounds__((chainThreads<Mma, MAXT>()), Mma::kEsz == 4 ? (MAXT
                     }
                 }
             } else {
-                const uint8_t* q = a.in + (uint64_t)min(first + n, a.batch - 1u) * a.inStride + colBase * ESZ;
+                const uint64_t at = (uint64_t)min(first + n, a.batch - 1u) * a.inStride + (uint64_t)(colBase * ESZ);
 #pragma unroll
                 for (int kt = 0; kt < INKT; ++kt) {
                     if (kt > 0 && kt >= kt0) continue;
-                    if (inEnd >= 16u) loadUpTo<ESZ>(q + kt * 8 * ESZ, a.in + inEnd, raw[nt][kt]);
-                    else loadSlots<RAW>(raw[nt][kt], q + kt * 8 * ESZ, validBytes - kt * 8 * ESZ, 2);
+                    if (inEnd >= 16u) loadUpTo<ESZ>(a.in, at + kt * 8 * ESZ, inEnd, raw[nt][kt]);
+                    else loadSlots<RAW>(raw[nt][kt], a.in + at + kt * 8 * ESZ, validBytes - kt * 8 * ESZ, 2);
                 }
             }
         }
@@ -475,7 +475,7 @@ __global__ __launch_bounds__((chainThreads<Mma, MAXT>()), Mma::kEsz == 4 ? (MAXT
             }
         const uint64_t following = (uint64_t)tile + step;
         const uint32_t next = following < numTiles ? (uint32_t)following : numTiles;
-        if constexpr (AHEAD) fetch(next);                     // (beyond the batch: an empty descriptor, nothing is read)
+        if constexpr (AHEAD) fetch(next);                     // (beyond the batch: QUAD's descriptor is empty and nothing is read; else the last tile again)
 
         const uint32_t sample = tile * 16u + n;
         for (int l = 0; l < L; ++l) {

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     // ---- per-lane constants ----------------------------------------------------------------
     const uint32_t gs0 = optGS((uint32_t)a.layers[0].in);
     const int colBase = (int)(g * gs0);
-    const int validBytes = min((int)gs0, max(a.layers[0].in - colBase, 0)) * ESZ;
+    const int validBytes = sliceBytes((uint32_t)a.layers[0].in, gs0, (uint32_t)g, ESZ);
     // (0: every lane's slice whole and aligned; 1: any other vector, in reads at whatever element a lane's slice begins)
     const int loadMode = a.inEncoding == kEncodeXYSquares ? 3 : a.inHalfAsE4M3 ? 4
                        : (a.layers[0].in == 32 * Net::KT0 && a.inAlign >= (IN_DW % 4 == 0 ? 16u : 8u)) ? 0 : 1;
@@ -199,16 +199,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const uint32_t lastSample = a.batch - 1;
 
     // Load mode 1: a read takes the 16 (8) bytes at whatever element a lane's k-slots begin, and half of that where no lane has slots in the
-    // upper half of the last fragment.  What would end behind the last vector is read ending there and moved down when the tile is used, so that
-    // no load is waited for before the weights are staged.  (Dword or byte loads under a mask each before, us: 31-32-32-5 over 10^6 fp16 111 -> 36,
+    // upper half of the last fragment.  What would end behind the last vector is read ending there, also where it begins behind it (placeRead,
+    // cv_reads.h), and moved down when the tile is used, so that no load is waited for before the weights are staged.  (Dword or byte loads under a mask each before, us: 31-32-32-5 over 10^6 fp16 111 -> 36,
     // 50-64-64-63 over 500 000 88 -> 41, 26-16-16-3 over 1 397 712 e4m3 76 -> 37, 3-16-16-1 over 500 8.6 -> 5.0.)
-    const uint64_t reach = (uint64_t)(TILE - 1) * a.inStride + (3 * gs0 + 8 * Net::KT0) * ESZ;      // from a super-tile's first vector
-    const uint64_t inEnd = (uint64_t)lastSample * a.inStride + (uint64_t)a.layers[0].in * ESZ;
-    const uint8_t* const inOwn = a.in + (validBytes > 0 ? colBase : 0) * ESZ;
+    const uint64_t inEnd = vectorsEnd(a.batch, a.inStride, (uint32_t)a.layers[0].in, ESZ);
+    const uint32_t own0 = (uint32_t)(validBytes > 0 ? colBase : 0) * ESZ;
     auto readBytes = [&](int kt) { return kt + 1 == Net::KT0 && halfTail ? 2 * RAW : 4 * RAW; };
-    auto endsInside = [&](uint32_t t) { return (uint64_t)__builtin_amdgcn_readfirstlane(t) * TILE * a.inStride + reach <= inEnd; };
-    // (bytes by which such a read begins early)
-    auto early = [&](const uint8_t* q, int bytes) { return (int)min(max((int64_t)(q + bytes - (a.in + inEnd)), (int64_t)0), (int64_t)bytes); };
+    auto endsInside = [&](uint32_t t) { return tileReadsEnd((uint64_t)__builtin_amdgcn_readfirstlane(t) * TILE, TILE, a.inStride, gs0, 8 * Net::KT0, ESZ) <= inEnd; };
+    // (of super-tiles that do not: sample 16 j + n of the tile, the last one instead of those beyond the batch)
+    auto edge = [&](uint32_t t, int j, int kt) {
+        return placeRead((uint64_t)min(t * TILE + 16 * j + n, lastSample) * a.inStride + own0 + kt * 8 * ESZ, (uint32_t)readBytes(kt), inEnd);
+    };
     auto readSlots = [&](uint32_t* b, const uint8_t* q, int bytes) {
         if (bytes == 2 * RAW) {
             if constexpr (ESZ == 2) { const u32x2 v = ((const Loose8<ESZ>*)q)->v; b[0] = v.x; b[1] = v.y; }
@@ -222,21 +223,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     auto loadTile = [&](uint32_t (&buf)[S][IN_DW], uint32_t t) {
         if (LEAN == kChunkNone && loadMode == 1 && inEnd >= 16u) {
             if (endsInside(t)) {
-                const uint8_t* p = inOwn + ((size_t)t * TILE + n) * a.inStride;
+                const uint8_t* p = a.in + own0 + ((size_t)t * TILE + n) * a.inStride;
 #pragma unroll
                 for (int j = 0; j < S; ++j, p += (size_t)16 * a.inStride)
 #pragma unroll
                     for (int kt = 0; kt < Net::KT0; ++kt) readSlots(&buf[j][kt * RAW], p + kt * 8 * ESZ, readBytes(kt));
             } else {
 #pragma unroll
-                for (int j = 0; j < S; ++j) {
-                    const uint8_t* p = inOwn + (size_t)min(t * TILE + 16 * j + n, lastSample) * a.inStride;
+                for (int j = 0; j < S; ++j)
 #pragma unroll
-                    for (int kt = 0; kt < Net::KT0; ++kt) {
-                        const uint8_t* q = p + kt * 8 * ESZ;
-                        readSlots(&buf[j][kt * RAW], q - early(q, readBytes(kt)), readBytes(kt));
-                    }
-                }
+                    for (int kt = 0; kt < Net::KT0; ++kt) readSlots(&buf[j][kt * RAW], a.in + edge(t, j, kt).at, readBytes(kt));
             }
             return;
         }
@@ -437,10 +433,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
                         uint32_t own[RAW];
 #pragma unroll
                         for (int d = 0; d < RAW; ++d) own[d] = buf[r0 + j][kt * RAW + d];
-                        if (moved) {
-                            const uint8_t* q = inOwn + (size_t)min(t0 * TILE + 16 * (r0 + j) + n, lastSample) * a.inStride + kt * 8 * ESZ;
-                            shiftDown<ESZ>(own, min(early(q, readBytes(kt)), 4 * RAW - ESZ));
-                        }
+                        if (moved) shiftDown<ESZ>(own, min((int)edge(t0, r0 + j, kt).down, 4 * RAW - ESZ));
 #pragma unroll
                         for (int d = 0; d < RAW; ++d) own[d] &= mask[kt * RAW + d];
                         Mma::decode(own, act[j][kt]);

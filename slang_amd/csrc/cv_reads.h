@@ -1,0 +1,34 @@
+// cv_reads.h -- which bytes a kernel reads of a batch of vectors of any length.  A lane reads its k-slots 16, 8 or 4 bytes at a time at
+// whatever element they begin; what it gets of the elements behind its slice is cleared in registers, but no read may touch a byte behind the
+// last vector.  Without HIP, so that every read can be checked against its buffer on the host.  Offsets are bytes from the first vector.
+#pragma once
+#include "cv_layout.h"
+
+namespace cv {
+
+// bytes from the first vector's first to the last one's last
+CV_HD uint64_t vectorsEnd(uint32_t batch, uint64_t stride, uint32_t in, uint32_t esz) { return (uint64_t)(batch - 1u) * stride + (uint64_t)in * esz; }
+
+// bytes of lane group g's slice (gs k-slots to a group) that exist
+CV_HD int32_t sliceBytes(uint32_t in, uint32_t gs, uint32_t g, uint32_t esz)
+{
+    const uint32_t col = g * gs, left = col < in ? in - col : 0u;
+    return (int32_t)((left < gs ? left : gs) * esz);
+}
+
+// Where the reads of `samples` vectors from vector `first` on end at most: those of the last lane group, whose fragments hold `slots` k-slots.
+CV_HD uint64_t tileReadsEnd(uint64_t first, uint32_t samples, uint64_t stride, uint32_t gs, uint32_t slots, uint32_t esz)
+{
+    return (first + samples - 1u) * stride + (uint64_t)(3u * gs + slots) * esz;
+}
+
+// A read of `bytes` bytes that is wanted at offset `want` of vectors that end at `end` (at least `bytes`): it is made at `at`, and what it
+// brings belongs `down` bytes further down (all of it, where nothing that is wanted exists).
+struct PlacedRead { uint64_t at; uint32_t down; };
+CV_HD PlacedRead placeRead(uint64_t want, uint32_t bytes, uint64_t end)
+{
+    const uint64_t at = want + bytes <= end ? want : end - bytes, down = want - at;
+    return PlacedRead{at, down < bytes ? (uint32_t)down : bytes};
+}
+
+} // namespace cv

@@ -14,6 +14,7 @@
 // with 8-byte loads, else element by element with zero fill.
 #pragma once
 #include "cv_device.h"
+#include "cv_reads.h"
 
 namespace cv {
 
@@ -37,19 +38,18 @@ __device__ __forceinline__ void loadLoose(const uint8_t* q, uint32_t (&x)[DW])
     }
 }
 
-// The same where what is read may end beyond `end`, behind which nothing is read and zeros stand (at least 16 bytes lie before it).
+// The same at offset `want` of vectors that end `end` bytes (16 at least) behind `base`: behind them nothing is read and zeros stand.
 template <int ALIGN, int DW>
-__device__ __forceinline__ void loadUpTo(const uint8_t* q, const uint8_t* end, uint32_t (&x)[DW])
+__device__ __forceinline__ void loadUpTo(const uint8_t* base, uint64_t want, uint64_t end, uint32_t (&x)[DW])
 {
     constexpr int P = DW % 4 == 0 ? 4 : 2;      // dwords of a read
 #pragma unroll
     for (int d0 = 0; d0 < DW; d0 += P) {
-        const uint8_t* at = q + 4 * d0;
-        const int64_t over = (at + 4 * P) - end;
-        const int shift = (int)(over < 0 ? 0 : over > 4 * P ? 4 * P : over), words = shift >> 2;
+        const PlacedRead r = placeRead(want + 4u * d0, 4u * P, end);
+        const int words = (int)(r.down >> 2);
         uint32_t v[2 * P + 1];
         uint32_t part[P];
-        loadLoose<ALIGN>(over > 0 ? end - 4 * P : at, part);
+        loadLoose<ALIGN>(base + r.at, part);
 #pragma unroll
         for (int i = 0; i < 2 * P + 1; ++i) v[i] = i < P ? part[i < P ? i : 0] : 0u;
 #pragma unroll
@@ -60,7 +60,7 @@ __device__ __forceinline__ void loadUpTo(const uint8_t* q, const uint8_t* end, u
                 lo = words == w ? v[i + w] : lo;
                 hi = words == w ? v[i + w + 1 <= 2 * P ? i + w + 1 : 2 * P] : hi;
             }
-            x[d0 + i] = __builtin_amdgcn_alignbyte(hi, lo, shift & 3);
+            x[d0 + i] = __builtin_amdgcn_alignbyte(hi, lo, r.down & 3u);
         }
     }
 }

@@ -686,8 +686,8 @@ def test_leaky_fp16_networks_on_32_sample_tiles(dims, B, bias):
 
 
 # Vectors that begin at any element on the kernel of equal hidden layers (registers for all weights): every number of k-slots beyond a whole
-# fragment and half of one, results of one to four rows beyond whole groups, rows that end where their buffer does, NaN around and between
-# them, batches that end inside a tile and inside a round of tiles.
+# fragment and half of one, results of one to four rows beyond whole groups, NaN around and between them, batches that end inside a tile and inside
+# a round of tiles.  (What is read behind the last vector does not show in the results: test_vector_reads.py checks that nothing is.)
 @pytest.mark.parametrize("ct", [CT.Float16, CT.FloatE4M3])
 @pytest.mark.parametrize("hidden", [16, 64])
 def test_equal_layers_take_vectors_at_any_element(ct, hidden):

@@ -107,7 +107,8 @@ def test_rows_far_apart(ct, other):
 
 
 # Vectors that begin at any element: every number of k-slots beyond a whole fragment and half of one (inputs 1 to 40), results of one to
-# four rows beyond whole groups, matrices in rows that begin at any element; the last vector ends its buffer.
+# four rows beyond whole groups, matrices in rows that begin at any element; the last vector ends its buffer.  (What is read
+# behind it does not show in the results: test_vector_reads.py checks that nothing is.)
 @pytest.mark.parametrize("ct", [CT.Float16, CT.FloatE4M3, CT.Float32, CT.BFloat16])
 def test_chain_kernel_takes_vectors_at_any_element(ct):
     floats = ct in TORCH
