@@ -210,6 +210,9 @@ CV_API CvResult cvConvertMatrices(void* stream, void* dstBuffer, const CvMatrixD
  * type is accepted and changes nothing: the stored elements are cast to the result type.
  * accumulate != 0 gives the member forms matMulAccum / matMulAddAccum
  * (hlsl.meta.slang:31476-31650): output += result (activation must be NONE).
+ * The results may lie on the vectors they come from (sample s's on no other sample's vector) up to m = k = 128 for elements of 8 and 16
+ * bits and m = k = 64 for FLOAT32, where the combination has a matrix instruction.  Otherwise, and for larger matrices, output and
+ * input must have no byte in common.
  */
 typedef struct CvMatMulDesc {
     /* vectors */

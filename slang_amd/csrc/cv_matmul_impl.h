@@ -792,9 +792,9 @@ template <class Fl, int MT, int KT, typename OutT>
 hipError_t launchRest(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append)
 {
     if constexpr (kPackedRows<Fl>) {
-        // (a block of a larger matrix does not come here: its rows would begin inside the matrix)
+        // (what is left of a streaming call: at most four k-tiles and 128 rows, which launchPacked always takes)
         hipError_t e = hipErrorInvalidValue;
-        return a.rowOff == 0 && launchPacked<Fl, OutT>(stream, a, numCUs, append, e) ? e : hipErrorInvalidValue;
+        return launchPacked<Fl, OutT>(stream, a, numCUs, append, e) ? e : hipErrorInvalidValue;
     } else {
         return launchOne<Fl, MT, KT, OutT, false>(stream, a, numCUs, append);
     }
@@ -881,32 +881,47 @@ hipError_t dispatchBlock(hipStream_t stream, const MatMulArgs& a, int numCUs, bo
     return hipErrorInvalidValue;
 }
 
-// Splits m into blocks of rows that one workgroup can hold: 128 rows while the fragments stay in
-// registers (at most four k-tiles), else as many 16-row tiles (8, 4, 2 or 1) as fit the LDS budget.
-// hipErrorInvalidValue when even one 16-row tile of k columns does not fit.
+// Row tiles to a block of matmulLargeKernel and the k-tiles it walks: as many 16-row tiles (8, 4, 2 or 1) as fit the LDS budget, 0 where not
+// even one does.
+template <class Fl>
+int largeBlockTiles(uint32_t kt, int& largeKT)
+{
+    constexpr uint32_t kSteps = LargeShape<Fl>::kSteps;
+    largeKT = (int)((kt + kSteps - 1) / kSteps * kSteps);
+    const size_t tileBytes = (size_t)largeKT * LargeShape<Fl>::kTileBytes, most = LargeShape<Fl>::kLdsBytes;
+    int tiles = 8;
+    while (tiles > 1 && tiles * tileBytes > most) tiles /= 2;
+    return tiles * tileBytes > most ? 0 : tiles;
+}
+
+// The common flavours (kPackedRows): the streaming form where it applies, else cv_matmul_packed.h, else matmulLargeKernel.  The others: blocks
+// of 128 rows on matmulKernel while the fragments stay in registers (at most four k-tiles), else matmulLargeKernel.
+// hipErrorInvalidValue when not even one 16-row tile of k columns fits the LDS.
 template <class Fl, typename OutT>
 hipError_t dispatchShape(hipStream_t stream, const MatMulArgs& a, int numCUs)
 {
+    const uint32_t kt = optKT((uint32_t)a.k, Fl::kEpl);
+    int largeKT = 0;
+    int blockTiles = largeBlockTiles<Fl>(kt, largeKT);
     if constexpr (kPackedRows<Fl>) {
-        hipError_t packed;
+        if (streamingApplies<Fl, OutT>(a)) return dispatchBlock<Fl, OutT>(stream, a, numCUs, false, 0);
         // fp32 vectors of many aligned elements: six and more k-tiles of pieces leave no registers to read ahead with, and matmulLargeKernel reads
         // aligned vectors as well.  Packed against large: 27 x 256 over 34 000 samples 21.8, 14.5 us, 64 x 256 over 200 000 94, 64 us; 8 x 188
         // over 3 000 10.3, 8.2 us, 27 x 188 over 34 000 12.6, 11.2 us; but 100 x 256 over 3 000 16.5, 27.9 us and 27 x 188 over 200 000 39, 50 us.
         const bool many = Fl::kWideFragments && a.inAlign >= 16u &&
                           (a.k > 224 ? a.m <= 64 || a.batch >= 16384u : a.k > 160 && a.batch < 65536u && (a.m <= 32 || (a.m <= 64 && a.batch >= 16384u)));
-        if (!many && !(a.m <= 128 && streamingApplies<Fl, OutT>(a)) && launchPacked<Fl, OutT>(stream, a, numCUs, false, packed)) return packed;
+        // Results on top of the vectors: one wave forms all rows of a sample and reads nothing of it afterwards, here or in matmulLargeKernel
+        // where a block of that holds them all (for larger matrices such calls are not defined).
+        const bool onVectors = rowsOverlap(Rows{(uint64_t)(uintptr_t)a.in, a.inStride, (uint64_t)a.k * Fl::kInEsz},
+                                           Rows{(uint64_t)(uintptr_t)a.out, a.outStride, (uint64_t)a.m * sizeof(OutT)}, a.batch);
+        hipError_t packed;
+        if (!many && launchPacked<Fl, OutT>(stream, a, numCUs, false, packed, onVectors)) return packed;
+        if (!many && onVectors && a.m > 16 * blockTiles && launchPacked<Fl, OutT>(stream, a, numCUs, false, packed)) return packed;
+    } else if (Fl::kWideFragments ? (kt <= 2 && a.m <= 64) : kt <= 4) {
+        largeKT = 0;
+        blockTiles = Fl::kWideFragments ? 4 : 8;
     }
-    const uint32_t kt = optKT((uint32_t)a.k, Fl::kEpl);
-    int blockTiles = 8, largeKT = 0;
-    const bool inRegisters = Fl::kWideFragments ? (kt <= 2 && a.m <= 64) : kt <= 4;
-    if (Fl::kWideFragments && inRegisters) blockTiles = 4;
-    if (!inRegisters) {
-        constexpr uint32_t kSteps = LargeShape<Fl>::kSteps;
-        largeKT = (int)((kt + kSteps - 1) / kSteps * kSteps);
-        const size_t tileBytes = (size_t)largeKT * LargeShape<Fl>::kTileBytes, most = LargeShape<Fl>::kLdsBytes;
-        while (blockTiles > 1 && blockTiles * tileBytes > most) blockTiles /= 2;
-        if (blockTiles * tileBytes > most) return hipErrorInvalidValue;
-    }
+    if (!blockTiles) return hipErrorInvalidValue;
     const int blockRows = 16 * blockTiles;
     const uint32_t biasEsz = a.bias ? elemSize(a.biasCt) : 0;
     for (int r0 = 0; r0 < a.m; r0 += blockRows) {

@@ -20,20 +20,10 @@
 // vectors are requested together), those between by the trip of a tile while few waves find registers or LDS.
 // Vectors staged through LDS in whole pieces took as long as read directly, 1.2 to 1.6 times for fp32 of many terms, and need the LDS.
 #pragma once
+#include "cv_matmul_plan.h"
 
 namespace cv {
 namespace {
-
-struct PackedPlan {
-    int32_t mt, tb;                  // row tiles of the matrix, of a workgroup's block (blockIdx.y)
-    int32_t segment;                 // row tiles whose results wait in LDS together
-    uint32_t outRow;                 // bytes from one sample's results to the next in LDS
-    uint32_t stageBytes;             // a wave's part of the LDS
-    uint32_t outPieces, outMagic;    // 16-byte pieces of a row of results (a segment) and 2^20 / outPieces, rounded up; 0: one block
-    int32_t outElements;             // the results leave element by element
-    int32_t outLines;                // rows and segments of results are whole 128-byte lines: they pass by the caches (storeStream16)
-    uint64_t matBytes;               // RowMajor matrices at least a lane-chunk long: their bytes, else 0
-};
 
 // f(integral_constant<int, B>) ... f(integral_constant<int, E - 1>)
 template <int B, int E, class F>
@@ -407,7 +397,6 @@ __device__ __forceinline__ void packedRows(const MatMulArgs& a, const PackedPlan
     }
 }
 
-constexpr uint32_t kPackedLds = 159u * 1024u;      // (__syncthreads_or has some of its own)
 // waves of a workgroup: eight, of which two workgroups find the registers on a compute unit; twelve of one where fp32 operands take more
 template <class Fl, int KT>
 constexpr int kPackedWaves = kInPieces<Fl> && KT > 2 ? 12 : 8;
@@ -449,79 +438,31 @@ hipError_t launchPackedSized(hipStream_t stream, const MatMulArgs& a, const Pack
     return hipGetLastError();
 }
 
-// How rows of `bytes` bytes leave: as one block (pieces = 0) where they lie one behind the other, or in pieces of every row.  False: rows
-// shorter than a piece that are not packed.
-inline bool rowsInPieces(const void* base, uint64_t stride, uint32_t bytes, PackedPlan& p)
-{
-    p.outPieces = p.outMagic = 0u;
-    p.outRow = bytes % 16u ? bytes : bytes + 16u;      // (so that the 16 rows of a tile lie on different banks)
-    if (((uintptr_t)base & 15u) == 0 && stride == bytes && bytes % 16u) return true;
-    if (bytes < 16u || stride >= (1u << 26)) return false;
-    p.outPieces = (bytes + 15u) / 16u;
-    p.outMagic = ((1u << 20) + p.outPieces - 1u) / p.outPieces;
-    return true;
-}
-
-// false where the k-tiles are beyond the registers
+// false where the k-tiles are beyond the registers, and (whole) where the rows of a sample's results would not come from one wave at once
 template <class Fl, typename OutT>
-bool launchPacked(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append, hipError_t& result)
+bool launchPacked(hipStream_t stream, const MatMulArgs& a, int numCUs, bool append, hipError_t& result, bool whole = false)
 {
-    const uint32_t kt = optKT((uint32_t)a.k, Fl::kEpl), mt = optMT((uint32_t)a.m);
+    const uint32_t kt = optKT((uint32_t)a.k, Fl::kEpl);
     constexpr int kMostKT = Fl::kEpl == 16 ? 4 : 8;
     if (kt > kMostKT) return false;
-    PackedPlan p = {};
-    p.mt = (int32_t)mt;
+    constexpr int kMostPairs = Fl::kEsz == 4 ? 2 : 4;
+    const int waves = kt > 2 ? kPackedWaves<Fl, 3> : kPackedWaves<Fl, 1>;
+    const PackedCall call = {(uint32_t)a.m, kt, a.batch, (uint64_t)(uintptr_t)a.in, a.inStride, (uint64_t)a.k * Fl::kInEsz, (uint64_t)(uintptr_t)a.out, a.outStride,
+                             (uint32_t)sizeof(OutT), 64u * 4u * (uint32_t)(kInPieces<Fl> ? Fl::kFD : Fl::kRawDW), kMostPairs, (uint32_t)waves, a.accumulate != 0, (uint32_t)numCUs};
+    PackedLaunch l = planPacked(call);
+    if (!l.fits || (whole && l.split)) return false;
+    PackedPlan& p = l.plan;
     if (a.shape.layout == kRowMajor && !a.transpose) {
         p.matBytes = matrixSize(a.shape);
         if (p.matBytes < Fl::kEpl * Fl::kEsz) p.matBytes = 0;
     }
-    const uint32_t fragment = 64u * 4u * (uint32_t)(kInPieces<Fl> ? Fl::kFD : Fl::kRawDW);
-    constexpr int kMostPairs = Fl::kEsz == 4 ? 2 : 4;      // k-tiles up to which a wave takes two tiles (registers)
-    const int mostWaves = kt > 2 ? kPackedWaves<Fl, 3> : kPackedWaves<Fl, 1>;
-    int nt = kt <= kMostPairs && a.batch / 32u >= (uint32_t)(numCUs * 8) ? 2 : 1;
-    uint32_t ldsBytes = 0;
-    int waves = mostWaves;
-    bool fits = false;
-    const uint32_t rowBytes = (uint32_t)a.m * (uint32_t)sizeof(OutT);
-    auto plan = [&](uint32_t blocks, uint32_t mostStage) {
-        p.tb = (int32_t)((mt + blocks - 1) / blocks);
-        const uint32_t tileBytes = 16u * nt * 16u * (uint32_t)sizeof(OutT);
-        p.outElements = a.accumulate;
-        p.segment = p.tb;
-        if (blocks == 1 && mt * tileBytes <= mostStage) {
-            if (!rowsInPieces(a.out, a.outStride, rowBytes, p)) p.outElements = 1;
-        } else {
-            const int most = (int)(mostStage / tileBytes);
-            if (most < p.tb) p.segment = most;
-            p.outPieces = (uint32_t)p.segment * (uint32_t)sizeof(OutT);
-            p.outRow = 16u * p.outPieces + 16u;
-            p.outMagic = ((1u << 20) + p.outPieces - 1u) / p.outPieces;
-            if (a.outStride >= (1u << 26)) p.outElements = 1;
-        }
-        p.stageBytes = (16u * nt * p.outRow + 15u) / 16u * 16u;
-        ldsBytes = (uint32_t)p.tb * (kt * fragment + 64u) + (uint32_t)waves * p.stageBytes;
-        fits = ldsBytes <= kPackedLds;
-        const uint32_t segmentBytes = p.segment == (int32_t)mt ? rowBytes : (uint32_t)p.segment * 16u * (uint32_t)sizeof(OutT);
-        p.outLines = (((uintptr_t)a.out | a.outStride | rowBytes | segmentBytes) & 127u) == 0;
-    };
-    // a batch that leaves compute units idle: the rows are split between them, down to a lane-chunk of the matrix a thread
-    const uint32_t groups = (uint32_t)(((uint64_t)a.batch + 16 * nt * mostWaves - 1) / (16 * nt * mostWaves));
-    uint32_t blocks = 1;
-    while (blocks < mt && groups * (blocks + 1) <= (uint32_t)numCUs && (mt + blocks - 1) / blocks * kt > 8u) ++blocks;
-    // where the LDS is short, fewer results wait, then a wave takes one tile, then the rows are split
-    const int wanted = nt;
-    for (; !fits && blocks <= mt; ++blocks)
-        for (int n = wanted; !fits && n >= 1; --n) {
-            nt = n;
-            for (uint32_t stage = 8192u; !fits && stage >= 2048u; stage /= 2u) plan(blocks, stage);
-        }
-    if (!fits) return false;
+    const int nt = (int)l.nt;
     bool done = false;
     forEach<1, kMostKT + 1>([&](auto kc) {
         constexpr int K = decltype(kc)::value;
         if ((int)kt != K) return;
         auto launch = [&](auto nc, auto large) {
-            result = launchPackedSized<Fl, K, decltype(nc)::value, OutT, decltype(large)::value>(stream, a, p, ldsBytes, waves, numCUs, append);
+            result = launchPackedSized<Fl, K, decltype(nc)::value, OutT, decltype(large)::value>(stream, a, p, l.ldsBytes, waves, numCUs, append);
             done = true;
         };
         auto sized = [&](auto nc) {

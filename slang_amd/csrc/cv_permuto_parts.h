@@ -4,6 +4,7 @@
 #include <cstdint>
 
 #include "coopvec.h"
+#include "cv_rows.h"
 
 namespace cv {
 namespace {
@@ -109,15 +110,6 @@ inline uint32_t positionsShare(const TableParts& t, uint32_t batch, uint32_t add
 inline bool positionsBeside(const TableParts& t, uint32_t batch, uint32_t cus)
 {
     return (uint64_t)t.count * ((batch - 1u) / 1024u + 1u) >= cus && !(t.groups <= 2u && batch > 65536u * t.groups);
-}
-
-// Whether two regions of `rows` rows each, `stride` bytes apart and `width` bytes wide, may have a byte in common (between their first
-// and their last byte: rows of one in the gaps of the other count as well).
-struct Rows { uint64_t at, stride, width; };
-inline bool rowsMeet(const Rows& a, const Rows& b, uint32_t rows)
-{
-    const uint64_t aEnd = a.at + (rows - 1ull) * a.stride + a.width, bEnd = b.at + (rows - 1ull) * b.stride + b.width;
-    return a.at < bEnd && b.at < aEnd;
 }
 
 } // namespace

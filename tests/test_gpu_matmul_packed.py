@@ -109,3 +109,39 @@ def test_activations_are_those_of_aligned_vectors(act):
         # fp32 functions to a few of their own units, then one rounding to half
         tolerance = (2.0 ** -20 if kind == "f32" else 2.0 ** -11 * 1.01) * want.abs() + 2.0 ** -21
         assert ((y.double() - want).abs() <= tolerance).all(), (kind, cv.lastKernelName())
+
+
+# Results on top of the vectors.  Small batches, whose rows would otherwise be split between workgroups; more samples than a round of tiles; whole
+# aligned rows (streaming, and what it leaves), odd ones, results longer and shorter than the vectors.
+@pytest.mark.parametrize("kind", list(TYPES))
+@pytest.mark.parametrize("M,K,B", [(72, 72, 1000), (120, 120, 300), (128, 128, 2000), (64, 64, 1003), (33, 128, 517), (128, 17, 70), (1, 1, 40), (57, 59, 70003)])
+def test_results_on_their_vectors(kind, M, K, B):
+    if kind == "f32":
+        M, K = min(M, 64), min(K, 64)
+    rng = np.random.default_rng(M * 1000 + K)
+    dt, ct, odt, oct = TYPES[kind]
+    x, W = values(kind, rng, B, K), values(kind, rng, M, K)
+    b = torch.from_numpy(rng.integers(-65536, 65537, M).astype(np.int32)).to(DEV) if oct == CT.SignedInt32 else values(kind, rng, M)
+
+    def run(xs, out, accumulate=False):
+        if accumulate:
+            return cv.coopVecMatMul(xs, ct, as_bytes(W), 0, ct, ML.RowMajor, False, K * W.element_size(), M=M, resultType=oct, out=out, accumulate=True)
+        return cv.coopVecMatMulAdd(xs, ct, as_bytes(W), 0, ct, as_bytes(b), 0, oct if oct == CT.SignedInt32 else ct, ML.RowMajor, False, K * W.element_size(),
+                                   M=M, resultType=oct, out=out)
+
+    isz, osz = x.element_size(), torch.empty(0, dtype=odt).element_size()
+    pitch = -(-max(K * isz, M * osz) // osz) * osz
+    for values_ in (x, x * 2 ** 16 if kind == "f32" else x):      # (fp32 from 2^32 on: the sums are formed again from the vectors)
+        if kind == "f32" and values_ is not x:
+            values_ = values_.clone()
+            values_[::3, K // 2] = 2.0 ** 33
+        for accumulate in (False, True):
+            raw = torch.zeros(B * pitch, dtype=torch.uint8, device=DEV)
+            vectors = raw.view(dt).as_strided((B, K), (pitch // isz, 1))
+            vectors.copy_(values_)
+            results = raw.view(odt).as_strided((B, M), (pitch // osz, 1))
+            before = results.clone()
+            want = run(values_, before if accumulate else torch.empty(B, M, dtype=odt, device=DEV), accumulate)
+            run(vectors, results, accumulate)
+            bits = torch.int16 if osz == 2 else torch.int32
+            assert torch.equal(results.contiguous().view(bits), want.view(bits)), (accumulate, cv.lastKernelName())
