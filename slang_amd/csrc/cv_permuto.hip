@@ -504,7 +504,6 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     const Rows dPos{(uint64_t)(uintptr_t)a.dPos, a.dPosStride, D * 4ull}, pos{(uint64_t)(uintptr_t)a.pos, a.posStride, D * 4ull},
         dOut{(uint64_t)(uintptr_t)a.dOut, a.dOutStride, features * 4ull};
     const bool apart = a.dPos && !rowsMeet(dPos, pos, a.batch) && !rowsMeet(dPos, dOut, a.batch);
-    const uint32_t natural = cut ? t.count : 0u;
     const bool byLevel = cut && FT > 0 && (apart || !a.dPos) && cutByLevel(a.desc, a.batch, (uint32_t)cus, t);
     if (cut) {
         if (FT > 0 && !t.sliced && a.batch >= kFewPositions) dealGroups(t, a.batch, (uint32_t)cus, positionsShare(t, a.batch, (uint32_t)(FT * (D + 1)), (uint32_t)cus));
@@ -526,8 +525,7 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
         // 11.9 us, in two launches 19.4, and 11.9 against 16.0 over 4096, where calls keep the two launches they had).
         const bool many = positionsBeside(t, a.batch, (uint32_t)cus), quarter = FT > 0 && !t.sliced && (uint64_t)t.count * ((a.batch - 1u) / 1024u + 1u) >= (uint32_t)cus / 4u;
         if (apart && (byLevel || many || quarter)) {
-            if (natural == 1) noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
-            else noteKernel(false, many && !byLevel ? "permutoTableGradKernel<D=%d,%u parts,positions beside>" : "permutoTableGradKernel<D=%d,%u parts,positions>", D, t.count);
+            noteKernel(false, "permutoTableGradKernel<D=%d,%u parts,positions beside>", D, t.count);
             return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t, cus);
         }
         noteKernel(false, "permutoTableGradKernel<D=%d,%u parts>", D, t.count);

@@ -186,7 +186,8 @@ def test_permuto_encoder_kernel_choices(D, F, levels_n, log2):
 
 
 @pytest.mark.parametrize("D,F,levels_n,log2,B,kernel", [
-    (2, 2, 4, 8, 5000, "permutoTableGradKernel<D=2,positions>"),           # the whole table in one workgroup's LDS
+    (2, 2, 4, 8, 2047, "permutoTableGradKernel<D=2,positions>"),           # the whole table in one workgroup's LDS
+    (2, 2, 4, 8, 5000, "permutoTableGradKernel<D=2,4 parts,positions beside>"),   # the same table, a level to a part
     (3, 1, 2, 6, 1, "permutoTableGradKernel<D=3,positions>"),
     (2, 4, 3, 10, 1025, "permutoTableGradKernel<D=2,2 parts> + permutoBackwardKernel<D=2,positions>"),   # two levels, then one
     (3, 2, 8, 12, 4099, "permutoTableGradKernel<D=3,8 parts> + permutoBackwardKernel<D=3,positions>"),   # a level to a part
@@ -229,10 +230,13 @@ def test_permuto_backward_table_parts(D, F, levels_n, log2, B, kernel):
     (15, [(0, 4096), (4096, 4096)], 700, "permutoTableGradKernel<D=2,8 parts> + permutoBackwardKernel<D=2,positions>"),
     (30, [(0, 2048)], 500, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),
     (3, [(0, 20480)], 900, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),
-    # small tables with gaps, in reverse order, on shared entries, all of them a single part
-    (2, [(3, 256), (267, 256), (531, 100), (700, 256)], 5000, "permutoTableGradKernel<D=2,positions>"),
-    (4, [(384, 128), (256, 128), (128, 128), (0, 128)], 4097, "permutoTableGradKernel<D=2,positions>"),
-    (2, [(0, 256), (0, 256), (128, 256)], 4500, "permutoTableGradKernel<D=2,positions>"),
+    # small tables with gaps, in reverse order, on shared entries: up to 2047 positions all of them a single part, beyond a level to a part
+    (2, [(3, 256), (267, 256), (531, 100), (700, 256)], 2000, "permutoTableGradKernel<D=2,positions>"),
+    (4, [(384, 128), (256, 128), (128, 128), (0, 128)], 2047, "permutoTableGradKernel<D=2,positions>"),
+    (2, [(0, 256), (0, 256), (128, 256)], 1500, "permutoTableGradKernel<D=2,positions>"),
+    (2, [(3, 256), (267, 256), (531, 100), (700, 256)], 5000, "permutoTableGradKernel<D=2,4 parts,positions beside>"),
+    (4, [(384, 128), (256, 128), (128, 128), (0, 128)], 4097, "permutoTableGradKernel<D=2,4 parts,positions beside>"),
+    (2, [(0, 256), (0, 256), (128, 256)], 4500, "permutoTableGradKernel<D=2,3 parts,positions beside>"),
     # larger ones, a part to a level or in slices
     (2, [(20000, 4096), (3000, 8192), (3000, 8192)], 3000, "permutoTableGradKernel<D=2,3 parts> + permutoBackwardKernel<D=2,positions>"),
     (1, [(50, 40000), (0, 60), (45, 9000)], 2500, "permutoTableGradKernel<D=2,3 parts> + permutoBackwardKernel<D=2,positions>"),
@@ -286,9 +290,9 @@ def test_permuto_backward_positions_beside_the_table(D, F, tables, B, parts):
     d_pos, _ = enc.backward(pos, table, g, dFeatureTable=d_table)
     assert cv.lastKernelName() == "permutoTableGradKernel<D=%d,%d parts,positions beside>" % (D, parts)
     want_table, want_pos = torch.zeros(table.numel(), dtype=torch.float64, device=DEV), []
-    for i in range(0, B, 16384):
+    for i in range(0, B, 2000):                                   # (two launches, or one part's pass)
         part = torch.zeros_like(table)
-        d, _ = enc.backward(pos[i:i + 16384], table, g[i:i + 16384], dFeatureTable=part)
+        d, _ = enc.backward(pos[i:i + 2000], table, g[i:i + 2000], dFeatureTable=part)
         assert "beside" not in cv.lastKernelName()
         want_pos.append(d)
         want_table += part
@@ -336,11 +340,12 @@ def test_permuto_backward_of_many_parts():
     assert torch.linalg.norm((d_table - d_table2).double()) <= 2.0 ** -16 * torch.linalg.norm(d_table.double())
 
 
-@pytest.mark.parametrize("D,F,tables,B,kernel", [(3, 2, [1 << 12] * 8, 1 << 16, "permutoTableGradKernel<D=3,8 parts>"), (2, 4, [1 << 8] * 4, 4099, "permutoTableGradKernel<D=2,positions>"),
-                                                  (3, 1, [1 << 15] * 3, 70001, "permutoTableGradKernel<D=3,6 parts>")])
+@pytest.mark.parametrize("D,F,tables,B,parts,kernel", [(3, 2, [1 << 12] * 8, 1 << 16, 8, "permutoTableGradKernel<D=3,8 parts> + permutoBackwardKernel<D=3,positions>"),
+                                                        (2, 4, [1 << 8] * 4, 4099, 4, "permutoTableGradKernel<D=2,positions>"),
+                                                        (3, 1, [1 << 15] * 3, 70001, 6, "permutoTableGradKernel<D=3,6 parts> + permutoBackwardKernel<D=3,positions>")])
 @pytest.mark.parametrize("where", ["positions", "dOut"])
-def test_permuto_backward_positions_on_top_of_inputs(D, F, tables, B, kernel, where):
-    # dPositions row on row of positions, or of the gradients that come in: as into a buffer of its own
+def test_permuto_backward_positions_on_top_of_inputs(D, F, tables, B, parts, kernel, where):
+    # dPositions row on row of positions, or of the gradients that come in: as into a buffer of its own (beside the table's `parts` there)
     rng = np.random.default_rng(B)
     enc = cv.PermutoEncoder(D, F, 4, len(tables), baseScale=2.0, log2PerLevelScale=0.5, seed=5)
     for l, n in enumerate(tables):
@@ -349,12 +354,12 @@ def test_permuto_backward_positions_on_top_of_inputs(D, F, tables, B, kernel, wh
     table = to_dev(rng.standard_normal(sum(tables) * F).astype(np.float32))
     g = to_dev(rng.integers(-4, 5, (B, len(tables) * F)).astype(np.float32))
     want_pos, want_table = enc.backward(pos, table, g)
-    assert cv.lastKernelName() == (kernel if "positions" in kernel else kernel[:-1] + ",positions beside>"), cv.lastKernelName()
+    assert cv.lastKernelName() == "permutoTableGradKernel<D=%d,%d parts,positions beside>" % (D, parts), cv.lastKernelName()
     d_table, into = torch.zeros_like(table), pos if where == "positions" else g
     lib = cv._lib.load()
     rc = lib.cvPermutoEncodeBackward(torch.cuda.current_stream().cuda_stream, cv.ctypes.byref(enc.desc), pos.data_ptr(), 4 * D, table.data_ptr(), g.data_ptr(),
                                      4 * g.shape[1], into.data_ptr(), 4 * into.shape[1], d_table.data_ptr(), B)
-    assert rc == 0 and cv.lastKernelName().startswith(kernel), cv.lastKernelName()
+    assert rc == 0 and cv.lastKernelName() == kernel, cv.lastKernelName()
     assert torch.equal(into[:, :D], want_pos)
     assert torch.allclose(d_table, want_table, rtol=1e-6, atol=1e-4)
 
@@ -544,13 +549,13 @@ def test_encoder_at_half_way_values(D):
 @pytest.mark.parametrize("D,F,tables,B,kernel", [
     # one part; several levels to a part, then one: from 2048 positions on a level to a part, and the positions in the same launch
     (3, 4, [(512 * l, 512) for l in range(6)], 2047, "permutoTableGradKernel<D=3,2 parts> + permutoBackwardKernel<D=3,positions>"),
-    (3, 4, [(512 * l, 512) for l in range(6)], 2048, "permutoTableGradKernel<D=3,6 parts,positions>"),
-    (2, 1, [(64 * l, 64) for l in range(8)], 2049, "permutoTableGradKernel<D=2,positions>"),
-    (4, 2, [(300, 256), (0, 256), (700, 100), (700, 100)], 4097, "permutoTableGradKernel<D=4,positions>"),      # gaps, another order, shared entries
-    (2, 4, [(1024 * l, 1024) for l in range(3)], 20001, "permutoTableGradKernel<D=2,3 parts,positions>"),
+    (3, 4, [(512 * l, 512) for l in range(6)], 2048, "permutoTableGradKernel<D=3,6 parts,positions beside>"),
+    (2, 1, [(64 * l, 64) for l in range(8)], 2049, "permutoTableGradKernel<D=2,8 parts,positions beside>"),
+    (4, 2, [(300, 256), (0, 256), (700, 100), (700, 100)], 4097, "permutoTableGradKernel<D=4,4 parts,positions beside>"),      # gaps, another order, shared entries
+    (2, 4, [(1024 * l, 1024) for l in range(3)], 20001, "permutoTableGradKernel<D=2,3 parts,positions beside>"),
     # workgroups of 1024 positions on a quarter of 256 compute units, and on less
     (3, 2, [(4096 * l, 4096) for l in range(8)], 7168, "permutoTableGradKernel<D=3,8 parts> + permutoBackwardKernel<D=3,positions>"),
-    (3, 2, [(4096 * l, 4096) for l in range(8)], 7169, "permutoTableGradKernel<D=3,8 parts,positions>"),
+    (3, 2, [(4096 * l, 4096) for l in range(8)], 7169, "permutoTableGradKernel<D=3,8 parts,positions beside>"),
     (3, 1, [(4096, 4096)], 3000, "permutoTableGradKernel<D=3,positions>"),                                     # one level: fewer positions to a workgroup
 ])
 def test_permuto_backward_spread_over_levels(D, F, tables, B, kernel):
