@@ -497,18 +497,14 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
     const dim3 grid((a.batch - 1u) / 256u + 1u), block(256);
-    TableParts t;
-    const bool cut = a.dTable && cutTable(a.desc, t);
     const uint64_t features = (uint64_t)a.desc.featureDimensionPerEntry * a.desc.maxLevels;
     // Where position gradients are written on top of what is read (rows on rows), other workgroups of one launch would still read it.
     const Rows dPos{(uint64_t)(uintptr_t)a.dPos, a.dPosStride, D * 4ull}, pos{(uint64_t)(uintptr_t)a.pos, a.posStride, D * 4ull},
         dOut{(uint64_t)(uintptr_t)a.dOut, a.dOutStride, features * 4ull};
     const bool apart = a.dPos && !rowsMeet(dPos, pos, a.batch) && !rowsMeet(dPos, dOut, a.batch);
-    const bool byLevel = cut && FT > 0 && (apart || !a.dPos) && cutByLevel(a.desc, a.batch, (uint32_t)cus, t);
-    if (cut) {
-        if (FT > 0 && !t.sliced && a.batch >= kFewPositions) dealGroups(t, a.batch, (uint32_t)cus, positionsShare(t, a.batch, (uint32_t)(FT * (D + 1)), (uint32_t)cus));
-        else dealGroups(t, a.batch, (uint32_t)cus);
-    }
+    TableParts t;
+    bool byLevel = FT > 0 && (apart || !a.dPos);
+    const bool cut = a.dTable && planTable(a.desc, a.batch, (uint32_t)cus, t, byLevel);
     if (cut && t.count == 1 && a.dPos) {
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
         return launchTableGrad<D, FT, kPosInPass, false, PLAIN>(stream, a, t, cus);

@@ -65,40 +65,54 @@ inline bool cutTable(const CvPermutoDesc& desc, TableParts& t, uint64_t together
     return t.count > 0;
 }
 
-// As many workgroups (of 1024 threads) as the compute units hold, dealt evenly to the parts, and none without `share` positions.
+// As many workgroups (of 1024 threads) as the compute units hold, dealt evenly to the parts, and none without 1024 positions.
 inline uint32_t largestPart(const TableParts& t)
 {
     uint32_t most = 0;
     for (uint32_t p = 0; p < t.count; ++p) most = t.part[p].elems > most ? t.part[p].elems : most;
     return most;
 }
-inline void dealGroups(TableParts& t, uint32_t batch, uint32_t cus, uint32_t share = 1024u)
+inline void dealGroups(TableParts& t, uint32_t batch, uint32_t cus)
 {
-    const uint32_t resident = cus * (largestPart(t) <= kPartHalf ? 2u : 1u), want = (batch - 1u) / share + 1u;
+    const uint32_t resident = cus * (largestPart(t) <= kPartHalf ? 2u : 1u), want = (batch - 1u) / 1024u + 1u;
     const uint32_t each = resident / t.count ? resident / t.count : 1u;
     t.groups = want < each ? want : each;
 }
 
 // One level to a part instead of several where the parts leave compute units without a workgroup of 1024 positions: a level's additions in LDS, not
 // its start, are what a workgroup takes its time for.  Several levels to a part against one (and position gradients beside), 3 dimensions, us: 6 levels of
-// 2^9 four-feature entries over 4096 / 2^14 / 2^16 positions 49.6, 50.4, 52.0 against 11.3, 11.3, 20.6; 8 levels of 2^10 two-feature entries over 20000
-// / 2^16 32.5, 33.0 against 12.0, 15.1; 2 dimensions, 8 levels of 2^8 of two over 20000 / 2^16 / 2^17 / 2^18 (one part) 21.8, 22.6, 23.6, 27.5
-// against 11.3, 11.4, 17.2, 28.3.  (Below kFewPositions there is little to spread.)
+// 2^9 four-feature entries over 4096 / 2^14 / 2^16 positions 48.5, 48.5, 49.1 against 14.1, 14.4, 21.1; 8 levels of 2^10 two-feature entries over 20000
+// / 2^16 30.8, 31.9 against 8.9, 12.7; 2 dimensions, 8 levels of 2^8 of two over 20000 / 2^16 / 2^17 (one part) 19.7, 20.4, 21.9 against 7.1, 9.5,
+// 14.6, and over 2^18 25.1 against 28.3.  (Below kFewPositions there is little to spread.)
+// Each workgroup of a part rounds its sums to float once, on their way to memory.  A part of one level has no more workgroups than the part of several it
+// came from, so no entry's sum is rounded more often; levels on the same entries, whose addends one part sums in double, stay together.  (Fewer
+// positions to a workgroup, 512 or 256, would halve the time over 4096 positions, 6 levels of 2^9 four-feature entries 14.1 -> 6.9 us, but put the gradient
+// 8.3e-8 of its norm off the 64-bit one instead of 5.3e-8.)
 constexpr uint32_t kFewPositions = 2048u;
+inline bool levelsApart(const CvPermutoDesc& desc)
+{
+    for (uint32_t l = 0; l < desc.maxLevels; ++l)
+        for (uint32_t m = 0; m < l; ++m) {
+            const CvPermutoLevelInfo &a = desc.levelInfo[l], &b = desc.levelInfo[m];
+            if ((uint64_t)a.offsetOfFeatureTable < (uint64_t)b.offsetOfFeatureTable + b.featureTableSize &&
+                (uint64_t)b.offsetOfFeatureTable < (uint64_t)a.offsetOfFeatureTable + a.featureTableSize) return false;
+        }
+    return true;
+}
 inline bool cutByLevel(const CvPermutoDesc& desc, uint32_t batch, uint32_t cus, TableParts& t)
 {
-    if (t.sliced || t.count >= desc.maxLevels || batch < kFewPositions || (uint64_t)t.count * ((batch - 1u) / 1024u + 1u) >= cus) return false;
+    if (t.sliced || t.count >= desc.maxLevels || batch < kFewPositions || (uint64_t)t.count * ((batch - 1u) / 1024u + 1u) >= cus || !levelsApart(desc)) return false;
     return cutTable(desc, t, 0);      // (levels that were joined are whole ones, no more than a description has)
 }
 
-// Positions to a workgroup, of which it takes 1024 at a time: fewer where that leaves most compute units without one, and where a position
-// makes many additions (`adds` to a level).  1024 / 512 / 256 positions, us: 7 levels of 2^11 four-feature entries over 4096 16.8, 12.2, 12.4; 3 levels
-// of 2^12 17.9, 12.7, 11.1; 6 of 2^9 over 2^16 23.2, 20.7; but 8 levels of 2^12 two-feature entries over 2^14 11.9, 13.1, 15.3.
-inline uint32_t positionsShare(const TableParts& t, uint32_t batch, uint32_t adds, uint32_t cus)
+// The parts and workgroups of a launch; byLevel: cutByLevel may be asked (entries of 1, 2 or 4 features, gradients that do not lie on what is
+// read), and then whether it cut.  False: no parts.
+inline bool planTable(const CvPermutoDesc& desc, uint32_t batch, uint32_t cus, TableParts& t, bool& byLevel)
 {
-    uint32_t share = adds > 8u ? 512u : 1024u;
-    while (share > 256u && 4ull * t.count * ((batch - 1u) / share + 1u) <= cus) share /= 2u;
-    return share;
+    if (!cutTable(desc, t)) return byLevel = false;
+    byLevel = byLevel && cutByLevel(desc, batch, cus, t);
+    dealGroups(t, batch, cus);
+    return true;
 }
 
 // Whether position gradients go into the table's launch (of several parts; after dealGroups).  Not with too few positions for

@@ -230,13 +230,14 @@ def test_permuto_backward_table_parts(D, F, levels_n, log2, B, kernel):
     (15, [(0, 4096), (4096, 4096)], 700, "permutoTableGradKernel<D=2,8 parts> + permutoBackwardKernel<D=2,positions>"),
     (30, [(0, 2048)], 500, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),
     (3, [(0, 20480)], 900, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),
-    # small tables with gaps, in reverse order, on shared entries: up to 2047 positions all of them a single part, beyond a level to a part
+    # small tables with gaps, in reverse order, on shared entries: up to 2047 positions all of them a single part, beyond a level to a part, but for
+    # levels on the same entries
     (2, [(3, 256), (267, 256), (531, 100), (700, 256)], 2000, "permutoTableGradKernel<D=2,positions>"),
     (4, [(384, 128), (256, 128), (128, 128), (0, 128)], 2047, "permutoTableGradKernel<D=2,positions>"),
     (2, [(0, 256), (0, 256), (128, 256)], 1500, "permutoTableGradKernel<D=2,positions>"),
     (2, [(3, 256), (267, 256), (531, 100), (700, 256)], 5000, "permutoTableGradKernel<D=2,4 parts,positions beside>"),
     (4, [(384, 128), (256, 128), (128, 128), (0, 128)], 4097, "permutoTableGradKernel<D=2,4 parts,positions beside>"),
-    (2, [(0, 256), (0, 256), (128, 256)], 4500, "permutoTableGradKernel<D=2,3 parts,positions beside>"),
+    (2, [(0, 256), (0, 256), (128, 256)], 4500, "permutoTableGradKernel<D=2,positions>"),
     # larger ones, a part to a level or in slices
     (2, [(20000, 4096), (3000, 8192), (3000, 8192)], 3000, "permutoTableGradKernel<D=2,3 parts> + permutoBackwardKernel<D=2,positions>"),
     (1, [(50, 40000), (0, 60), (45, 9000)], 2500, "permutoTableGradKernel<D=2,3 parts> + permutoBackwardKernel<D=2,positions>"),
@@ -551,12 +552,13 @@ def test_encoder_at_half_way_values(D):
     (3, 4, [(512 * l, 512) for l in range(6)], 2047, "permutoTableGradKernel<D=3,2 parts> + permutoBackwardKernel<D=3,positions>"),
     (3, 4, [(512 * l, 512) for l in range(6)], 2048, "permutoTableGradKernel<D=3,6 parts,positions beside>"),
     (2, 1, [(64 * l, 64) for l in range(8)], 2049, "permutoTableGradKernel<D=2,8 parts,positions beside>"),
-    (4, 2, [(300, 256), (0, 256), (700, 100), (700, 100)], 4097, "permutoTableGradKernel<D=4,4 parts,positions beside>"),      # gaps, another order, shared entries
+    (4, 2, [(300, 256), (0, 256), (700, 100), (800, 100)], 4097, "permutoTableGradKernel<D=4,4 parts,positions beside>"),      # gaps, another order
+    (4, 2, [(300, 256), (0, 256), (700, 100), (700, 100)], 4097, "permutoTableGradKernel<D=4,positions>"),                     # levels on the same entries stay together
     (2, 4, [(1024 * l, 1024) for l in range(3)], 20001, "permutoTableGradKernel<D=2,3 parts,positions beside>"),
     # workgroups of 1024 positions on a quarter of 256 compute units, and on less
     (3, 2, [(4096 * l, 4096) for l in range(8)], 7168, "permutoTableGradKernel<D=3,8 parts> + permutoBackwardKernel<D=3,positions>"),
     (3, 2, [(4096 * l, 4096) for l in range(8)], 7169, "permutoTableGradKernel<D=3,8 parts,positions beside>"),
-    (3, 1, [(4096, 4096)], 3000, "permutoTableGradKernel<D=3,positions>"),                                     # one level: fewer positions to a workgroup
+    (3, 1, [(4096, 4096)], 3000, "permutoTableGradKernel<D=3,positions>"),                                     # one level
 ])
 def test_permuto_backward_spread_over_levels(D, F, tables, B, kernel):
     # the bounds are those of test_permuto_backward_table_parts

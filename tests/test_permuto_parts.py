@@ -35,6 +35,15 @@ extern "C" int beside(uint32_t count, uint32_t elems, uint32_t batch, uint32_t c
     *groups = t.groups;
     return cv::positionsBeside(t, batch, cus);
 }
+// parts and workgroups of a launch (out[4 n ..]: as cut's; returned: n * 65536 + workgroups), spread: cutByLevel may be asked
+extern "C" int plan(const CvPermutoDesc* d, uint32_t batch, uint32_t cus, int spread, uint32_t* out)
+{
+    cv::TableParts t{};
+    bool byLevel = spread != 0;
+    if (!cv::planTable(*d, batch, cus, t, byLevel)) return -1;
+    for (uint32_t p = 0; p < t.count; ++p) { out[4 * p] = t.part[p].base; out[4 * p + 1] = t.part[p].elems; out[4 * p + 2] = t.part[p].first; out[4 * p + 3] = t.part[p].end; }
+    return (int)(t.count * 65536u + t.groups);
+}
 extern "C" int meet(const uint64_t* a, const uint64_t* b, uint32_t rows) { return cv::rowsMeet({a[0], a[1], a[2]}, {b[0], b[1], b[2]}, rows); }
 """
 
@@ -152,3 +161,35 @@ def test_rows_that_meet(built):
 def test_one_launch_for_table_and_positions(built, count, elems, batch, groups, one):
     got = ctypes.c_uint32()
     assert (bool(built.beside(count, elems, batch, 256, ctypes.byref(got))), got.value) == (one, groups)
+
+
+@pytest.mark.parametrize("F", [1, 2, 4])
+def test_sums_are_rounded_no_more_often_where_levels_are_spread(built, F):
+    """A workgroup rounds the sum of an entry once on its way to memory: cutting by level must not put more of them on an entry than parts
+    of several levels and 1024 positions to a workgroup do."""
+    rng = random.Random(F)
+    for _ in range(400):
+        n = rng.randint(1, 16)
+        sizes = [1 << rng.randint(4, 12)] * n if rng.random() < 0.6 else [rng.randint(1, 5000) for _ in range(n)]
+        tables = behind_one_another(sizes)
+        if rng.random() < 0.3:
+            tables = [(rng.randint(0, 8000), s) for s in sizes]                    # gaps, any order, shared entries
+        desc = _lib.CvPermutoDesc(dimensions=3, featureDimensionPerEntry=F, maxLevels=n, maxLevel=99.0)
+        for l, (offset, size) in enumerate(tables):
+            lv = desc.levelInfo[l]
+            lv.currentLevelIndex, lv.offsetOfFeatureTable, lv.featureTableSize = l, offset, size
+        batch = round(2 ** rng.uniform(6, 18))
+
+        def additions(spread):
+            out = (ctypes.c_uint32 * (4 * 144))()
+            r = built.plan(ctypes.byref(desc), batch, 256, int(spread), out)
+            assert r > 0
+            parts = [tuple(out[4 * p:4 * p + 4]) for p in range(r >> 16)]
+            check(parts, 0, F, tables)
+            # workgroups that may add to an entry, at the first entry and in the middle of every level
+            return [(r & 65535) * sum(base <= at * F < base + elems and any(o <= at < o + s for o, s in tables[first:end]) for base, elems, first, end in parts)
+                    for o_, s_ in tables for at in (o_, o_ + s_ // 2)], len(parts), r & 65535
+        before, parts, groups = additions(False)
+        after, _, _ = additions(True)
+        assert groups <= (batch - 1) // 1024 + 1
+        assert all(x <= y for x, y in zip(after, before)), (F, tables, batch, before, after)
