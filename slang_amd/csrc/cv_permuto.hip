@@ -503,24 +503,21 @@ hipError_t launchBackwardLevels(hipStream_t stream, const PermutoArgs& a)
         dOut{(uint64_t)(uintptr_t)a.dOut, a.dOutStride, features * 4ull};
     const bool apart = a.dPos && !rowsMeet(dPos, pos, a.batch) && !rowsMeet(dPos, dOut, a.batch);
     TableParts t;
-    bool byLevel = FT > 0 && (apart || !a.dPos);
-    const bool cut = a.dTable && planTable(a.desc, a.batch, (uint32_t)cus, t, byLevel);
+    const bool cut = a.dTable && planTable(a.desc, a.batch, (uint32_t)cus, FT > 0 && (apart || !a.dPos), t);
     if (cut && t.count == 1 && a.dPos) {
         noteKernel(false, "permutoTableGradKernel<D=%d,positions>", D);
         return launchTableGrad<D, FT, kPosInPass, false, PLAIN>(stream, a, t, cus);
     }
-    // Two launches against one: a handful of positions whose few additions hardly meet is done sooner by the one kernel that adds
-    // in memory.  It takes 7.4 to 8.1 us per call back to back and the pair 11.5 to 13.5 (16 positions on 3 levels of 2^10
-    // four-feature entries, 4 of 2^12 two-feature ones, ...); its time grows with the additions and reaches the pair's at 1300 to
-    // 2000 of them (one to five and eight dimensions, 2 to 8 levels).  Where a position has more than 16 features it is the slower
-    // one from the first position (16 levels of 4 features: 34.8 against 25.3 us).
+    // A handful of positions whose few additions hardly meet is done sooner by the one kernel that adds in memory: 4.1 to 4.7 us where the
+    // table in slices, which takes two launches, has 7.9 (4 levels of 2^15 entries, 1 to 64 positions).  Its time grows with the additions and
+    // reaches the two launches' at 1300 to 2000 of them.  Against one launch it is the sooner one up to 580 to 860 additions (3 levels of 2^10
+    // four-feature entries, 16 / 24 / 32 positions 4.7, 6.8, 8.3 against 5.8, 5.7, 5.7; 2 of 2^12 two-feature ones, 24 / 32 / 48 4.2, 5.1, 6.7 against 5.2),
+    // or beyond 1440 where they spread over more entries (4 dimensions, 6 levels of 2^12, 48 positions 7.4 against 8.4; 4 levels of 2^12
+    // four-feature entries, 16 positions 6.2 against 7.8): no line by their number serves both, so there is one for all.  Where a position has more than 16 features it
+    // is the slower one from the first position (16 levels of 4 features: 34.8 against 14.5 us).
     const bool few = FT > 0 && a.batch <= 64u && features <= 16u && a.batch * (uint64_t)(D + 1) * features <= 1440u;
     if (cut && !(a.dPos && few)) {
-        // One launch where that is sooner: always behind cutByLevel; else for workgroups on every compute unit (positionsBeside), or on a quarter of
-        // them where levels are no slices and entries of 1, 2 or 4 features (8 levels of 2^12 two-feature entries, 3 dimensions, 2^14 positions:
-        // 11.9 us, in two launches 19.4, and 11.9 against 16.0 over 4096, where calls keep the two launches they had).
-        const bool many = positionsBeside(t, a.batch, (uint32_t)cus), quarter = FT > 0 && !t.sliced && (uint64_t)t.count * ((a.batch - 1u) / 1024u + 1u) >= (uint32_t)cus / 4u;
-        if (apart && (byLevel || many || quarter)) {
+        if (apart && positionsBeside(t, a.batch, (uint32_t)cus)) {      // (one launch)
             noteKernel(false, "permutoTableGradKernel<D=%d,%u parts,positions beside>", D, t.count);
             return t.sliced ? launchTableGrad<D, FT, kPosBeside, true, PLAIN>(stream, a, t, cus) : launchTableGrad<D, FT, kPosBeside, false, PLAIN>(stream, a, t, cus);
         }

@@ -105,25 +105,28 @@ inline bool cutByLevel(const CvPermutoDesc& desc, uint32_t batch, uint32_t cus, 
     return cutTable(desc, t, 0);      // (levels that were joined are whole ones, no more than a description has)
 }
 
-// The parts and workgroups of a launch; byLevel: cutByLevel may be asked (entries of 1, 2 or 4 features, gradients that do not lie on what is
-// read), and then whether it cut.  False: no parts.
-inline bool planTable(const CvPermutoDesc& desc, uint32_t batch, uint32_t cus, TableParts& t, bool& byLevel)
+// The parts and workgroups of a launch; spread: cutByLevel may be asked (entries of 1, 2 or 4 features, position gradients that do not lie on what
+// is read).  False: no parts.
+inline bool planTable(const CvPermutoDesc& desc, uint32_t batch, uint32_t cus, bool spread, TableParts& t)
 {
-    if (!cutTable(desc, t)) return byLevel = false;
-    byLevel = byLevel && cutByLevel(desc, batch, cus, t);
+    if (!cutTable(desc, t)) return false;
+    if (spread) cutByLevel(desc, batch, cus, t);
     dealGroups(t, batch, cus);
     return true;
 }
 
-// Whether position gradients go into the table's launch (of several parts; after dealGroups).  Not with too few positions for
-// workgroups on every compute unit: spread by a kernel of their own they are done sooner.  And not where a part has but one or two
-// workgroups and many positions: a table of 91 parts or more, whose grid leaves compute units without one or deals some of them twice the
+// Whether position gradients go into the table's launch (of several parts; after dealGroups).  Always where parts are whole levels; two launches against one,
+// us: 3 dimensions, 8 levels of 2^12 two-feature entries over 65 / 1024 / 4096 / 2^14 positions 11.1, 16.6, 17.2, 19.4 against 8.9, 10.0, 9.5, 9.7; 5 levels of
+// 2^11 three-feature ones over 65 / 4096 / 24000 18.8, 28.1, 28.2 against 14.9, 16.5, 16.9; 2 levels of 2^12 over 65 / 30000 6.9, 12.8 against 5.2, 10.1; 4
+// dimensions, 8 levels of 2^9 four-feature entries over one position 17.4 against 12.2.
+// Slices: not with too few positions for workgroups on every compute unit: spread by a kernel of their own they are done sooner.  And not where a part has but
+// one or two workgroups and many positions: a table of 91 parts or more, whose grid leaves compute units without one or deals some of them twice the
 // work.  One launch against two, 3 dimensions, 9 or 7 levels of two-feature entries, 2^14 / 2^16 / 2^18 positions: 144 parts (144
 // workgroups) 41.7, 149, 606 us against 53.9, 150, 542; 126 parts (252) 24.0, 79.2, 304 against 36.6, 86.5, 288; 105 parts (210) 23.7,
 // 77.2, 297 against 33.2, 81.7, 276; 64 parts (256) 62.5 and 258 against 84.6 and 273 over 2^16 and 2^18, and still 1063 against 1108 over 2^20.
 inline bool positionsBeside(const TableParts& t, uint32_t batch, uint32_t cus)
 {
-    return (uint64_t)t.count * ((batch - 1u) / 1024u + 1u) >= cus && !(t.groups <= 2u && batch > 65536u * t.groups);
+    return !t.sliced || ((uint64_t)t.count * ((batch - 1u) / 1024u + 1u) >= cus && !(t.groups <= 2u && batch > 65536u * t.groups));
 }
 
 } // namespace

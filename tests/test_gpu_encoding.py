@@ -189,10 +189,10 @@ def test_permuto_encoder_kernel_choices(D, F, levels_n, log2):
     (2, 2, 4, 8, 2047, "permutoTableGradKernel<D=2,positions>"),           # the whole table in one workgroup's LDS
     (2, 2, 4, 8, 5000, "permutoTableGradKernel<D=2,4 parts,positions beside>"),   # the same table, a level to a part
     (3, 1, 2, 6, 1, "permutoTableGradKernel<D=3,positions>"),
-    (2, 4, 3, 10, 1025, "permutoTableGradKernel<D=2,2 parts> + permutoBackwardKernel<D=2,positions>"),   # two levels, then one
-    (3, 2, 8, 12, 4099, "permutoTableGradKernel<D=3,8 parts> + permutoBackwardKernel<D=3,positions>"),   # a level to a part
-    (3, 4, 2, 12, 1023, "permutoTableGradKernel<D=3,2 parts> + permutoBackwardKernel<D=3,positions>"),   # beyond half a unit's LDS
-    (2, 5, 2, 12, 300, "permutoTableGradKernel<D=2,2 parts> + permutoBackwardKernel<D=2,positions>"),    # the LDS full to the byte
+    (2, 4, 3, 10, 1025, "permutoTableGradKernel<D=2,2 parts,positions beside>"),   # two levels, then one
+    (3, 2, 8, 12, 4099, "permutoTableGradKernel<D=3,8 parts,positions beside>"),   # a level to a part
+    (3, 4, 2, 12, 1023, "permutoTableGradKernel<D=3,2 parts,positions beside>"),   # beyond half a unit's LDS
+    (2, 5, 2, 12, 300, "permutoTableGradKernel<D=2,2 parts,positions beside>"),    # the LDS full to the byte
     (2, 3, 2, 13, 2000, "permutoTableGradKernel<D=2,4 parts> + permutoBackwardKernel<D=2,positions>"),   # two slices to a level
     (3, 2, 2, 17, 3000, "permutoTableGradKernel<D=3,26 parts> + permutoBackwardKernel<D=3,positions>"),  # thirteen slices
     (2, 2, 1, 18, 2000, "permutoBackwardKernel<D=2,positions,table>"),     # too many slices: added in memory
@@ -239,7 +239,7 @@ def test_permuto_backward_table_parts(D, F, levels_n, log2, B, kernel):
     (4, [(384, 128), (256, 128), (128, 128), (0, 128)], 4097, "permutoTableGradKernel<D=2,4 parts,positions beside>"),
     (2, [(0, 256), (0, 256), (128, 256)], 4500, "permutoTableGradKernel<D=2,positions>"),
     # larger ones, a part to a level or in slices
-    (2, [(20000, 4096), (3000, 8192), (3000, 8192)], 3000, "permutoTableGradKernel<D=2,3 parts> + permutoBackwardKernel<D=2,positions>"),
+    (2, [(20000, 4096), (3000, 8192), (3000, 8192)], 3000, "permutoTableGradKernel<D=2,3 parts,positions beside>"),
     (1, [(50, 40000), (0, 60), (45, 9000)], 2500, "permutoTableGradKernel<D=2,3 parts> + permutoBackwardKernel<D=2,positions>"),
 ])
 def test_permuto_backward_of_other_tables(F, tables, B, kernel):
@@ -274,8 +274,9 @@ def test_permuto_backward_of_other_tables(F, tables, B, kernel):
     (2, 5, [(2048 * l, 2048) for l in range(4)], 65000, 4),
 ])
 def test_permuto_backward_positions_beside_the_table(D, F, tables, B, parts):
-    # One launch for both gradients where the batch fills the chip: the position gradients are those of batches that do not, bit
-    # for bit, the table's the sum of theirs (in another order: bound as in test_permuto_backward_table_parts).
+    # One launch for both gradients: the position gradients are those of a launch of their own, bit for bit, which they have where they
+    # are written on top of the positions; the table's the sum of parts of the batch by itself (in another order: bound as in
+    # test_permuto_backward_table_parts).
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the batches are those of 256 compute units")
     rng = np.random.default_rng(D * 100 + F * 10 + len(tables))
@@ -290,14 +291,17 @@ def test_permuto_backward_positions_beside_the_table(D, F, tables, B, parts):
     d_table = torch.zeros_like(table)
     d_pos, _ = enc.backward(pos, table, g, dFeatureTable=d_table)
     assert cv.lastKernelName() == "permutoTableGradKernel<D=%d,%d parts,positions beside>" % (D, parts)
-    want_table, want_pos = torch.zeros(table.numel(), dtype=torch.float64, device=DEV), []
-    for i in range(0, B, 2000):                                   # (two launches, or one part's pass)
+    into, both = pos.clone(), torch.zeros_like(table)
+    rc = cv._lib.load().cvPermutoEncodeBackward(torch.cuda.current_stream().cuda_stream, cv.ctypes.byref(enc.desc), into.data_ptr(), 4 * D, table.data_ptr(),
+                                                g.data_ptr(), 4 * n * F, into.data_ptr(), 4 * D, both.data_ptr(), B)
+    assert rc == 0 and cv.lastKernelName().endswith(" + permutoBackwardKernel<D=%d,positions>" % D), cv.lastKernelName()
+    assert torch.equal(d_pos, into)
+    want_table = torch.zeros(table.numel(), dtype=torch.float64, device=DEV)
+    for i in range(0, B, 16384):
         part = torch.zeros_like(table)
-        d, _ = enc.backward(pos[i:i + 2000], table, g[i:i + 2000], dFeatureTable=part)
-        assert "beside" not in cv.lastKernelName()
-        want_pos.append(d)
+        enc.backward(pos[i:i + 16384], table, g[i:i + 16384], dFeatureTable=part, wantPositionGrad=False)
         want_table += part
-    assert torch.equal(d_pos, torch.cat(want_pos))
+    assert torch.linalg.norm(both - want_table) <= 2.0 ** -16 * torch.linalg.norm(want_table)
     assert torch.linalg.norm(d_table - want_table) <= 2.0 ** -16 * torch.linalg.norm(want_table)
 
 
@@ -548,16 +552,19 @@ def test_encoder_at_half_way_values(D):
 
 
 @pytest.mark.parametrize("D,F,tables,B,kernel", [
-    # one part; several levels to a part, then one: from 2048 positions on a level to a part, and the positions in the same launch
-    (3, 4, [(512 * l, 512) for l in range(6)], 2047, "permutoTableGradKernel<D=3,2 parts> + permutoBackwardKernel<D=3,positions>"),
+    # one part; several levels to a part, then one: from 2048 positions on a level to a part
+    (3, 4, [(512 * l, 512) for l in range(6)], 2047, "permutoTableGradKernel<D=3,2 parts,positions beside>"),
     (3, 4, [(512 * l, 512) for l in range(6)], 2048, "permutoTableGradKernel<D=3,6 parts,positions beside>"),
     (2, 1, [(64 * l, 64) for l in range(8)], 2049, "permutoTableGradKernel<D=2,8 parts,positions beside>"),
     (4, 2, [(300, 256), (0, 256), (700, 100), (800, 100)], 4097, "permutoTableGradKernel<D=4,4 parts,positions beside>"),      # gaps, another order
     (4, 2, [(300, 256), (0, 256), (700, 100), (700, 100)], 4097, "permutoTableGradKernel<D=4,positions>"),                     # levels on the same entries stay together
     (2, 4, [(1024 * l, 1024) for l in range(3)], 20001, "permutoTableGradKernel<D=2,3 parts,positions beside>"),
-    # workgroups of 1024 positions on a quarter of 256 compute units, and on less
-    (3, 2, [(4096 * l, 4096) for l in range(8)], 7168, "permutoTableGradKernel<D=3,8 parts> + permutoBackwardKernel<D=3,positions>"),
-    (3, 2, [(4096 * l, 4096) for l in range(8)], 7169, "permutoTableGradKernel<D=3,8 parts,positions beside>"),
+    # fewer units of positions than waves, one, and as many of them as waves; entries of three features
+    (3, 2, [(4096 * l, 4096) for l in range(8)], 7168, "permutoTableGradKernel<D=3,8 parts,positions beside>"),
+    (3, 2, [(4096 * l, 4096) for l in range(8)], 65, "permutoTableGradKernel<D=3,8 parts,positions beside>"),
+    (4, 4, [(512 * l, 512) for l in range(8)], 1, "permutoTableGradKernel<D=4,2 parts,positions beside>"),
+    (3, 2, [(4096 * l, 4096) for l in range(2)], 2048, "permutoTableGradKernel<D=3,2 parts,positions beside>"),
+    (3, 3, [(2048 * l, 2048) for l in range(5)], 4096, "permutoTableGradKernel<D=3,5 parts,positions beside>"),
     (3, 1, [(4096, 4096)], 3000, "permutoTableGradKernel<D=3,positions>"),                                     # one level
 ])
 def test_permuto_backward_spread_over_levels(D, F, tables, B, kernel):

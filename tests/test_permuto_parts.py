@@ -26,10 +26,11 @@ extern "C" int cut(const CvPermutoDesc* d, uint32_t* out, uint32_t* sliced)
     *sliced = ok ? t.sliced : 0;
     return ok ? (int)t.count : -1;
 }
-extern "C" int beside(uint32_t count, uint32_t elems, uint32_t batch, uint32_t cus, uint32_t* groups)
+extern "C" int beside(uint32_t count, uint32_t elems, uint32_t batch, uint32_t cus, int sliced, uint32_t* groups)
 {
     cv::TableParts t{};
     t.count = count;
+    t.sliced = sliced;
     for (uint32_t p = 0; p < count; ++p) t.part[p].elems = p + 1 < count ? 1u : elems;
     cv::dealGroups(t, batch, cus);
     *groups = t.groups;
@@ -39,8 +40,7 @@ extern "C" int beside(uint32_t count, uint32_t elems, uint32_t batch, uint32_t c
 extern "C" int plan(const CvPermutoDesc* d, uint32_t batch, uint32_t cus, int spread, uint32_t* out)
 {
     cv::TableParts t{};
-    bool byLevel = spread != 0;
-    if (!cv::planTable(*d, batch, cus, t, byLevel)) return -1;
+    if (!cv::planTable(*d, batch, cus, spread != 0, t)) return -1;
     for (uint32_t p = 0; p < t.count; ++p) { out[4 * p] = t.part[p].base; out[4 * p + 1] = t.part[p].elems; out[4 * p + 2] = t.part[p].first; out[4 * p + 3] = t.part[p].end; }
     return (int)(t.count * 65536u + t.groups);
 }
@@ -159,8 +159,10 @@ def test_rows_that_meet(built):
     (129, 10241, 1 << 18, 1, False), (128, 20480, 1 << 17, 2, True), (128, 20480, (1 << 17) + 1, 2, False), (64, 20480, 1 << 20, 4, True),
     (144, 20480, 1, 1, False), (144, 20480, (1 << 32) - 1, 1, False), (85, 20480, (1 << 32) - 1, 3, True)])
 def test_one_launch_for_table_and_positions(built, count, elems, batch, groups, one):
+    # slices; parts that are whole levels take one launch for any batch
     got = ctypes.c_uint32()
-    assert (bool(built.beside(count, elems, batch, 256, ctypes.byref(got))), got.value) == (one, groups)
+    assert (bool(built.beside(count, elems, batch, 256, 1, ctypes.byref(got))), got.value) == (one, groups)
+    assert built.beside(count, elems, batch, 256, 0, ctypes.byref(got)) and got.value == groups
 
 
 @pytest.mark.parametrize("F", [1, 2, 4])
