@@ -19,11 +19,12 @@
 //
 // This kernel serves the shapes it streams best (FAST: full-width aligned vectors, at most 128
 // rows and four k-tiles, both powers of two, no leaky ReLU, no accumulate form: a branch-free loop).
-// Everything else up to eight k-tiles (ragged shapes, unaligned vectors, `this += ...`, every
-// activation, more rows) runs on cv_matmul_packed.h, and what has more k-tiles on
-// matmulLargeKernel, which keeps a block of rows in LDS and walks the k-tiles in a loop (one launch
-// per block, MatMulArgs::rowOff).  The less common flavours (kPackedRows) have a general
-// instantiation of this kernel instead.
+// Everything else of the common flavours (kPackedRows) up to eight k-tiles, four of 8-bit integers
+// (ragged shapes, unaligned vectors, `this += ...`, every activation, more rows), runs on
+// matmulPackedKernel (cv_matmul_packed.h), and what has more k-tiles, or is fp32 of many aligned
+// elements, on matmulLargeKernel, which keeps a block of rows in LDS and walks the k-tiles in a loop
+// (one launch per block, MatMulArgs::rowOff).  The other flavours have a general instantiation of
+// this kernel for up to four k-tiles, in blocks of 128 rows, and matmulLargeKernel beyond.
 #pragma once
 #include <type_traits>
 
@@ -46,8 +47,8 @@ struct VecAsMatrix : Mma {
     // kStreaming: the flavour also gets the branch-free streaming instantiations (the less common
     // ones run every shape on the general kernel)
     static constexpr bool kStreaming = !std::is_same<Mma, Bf8AsF16Mma>::value;
-    // kWideFragments: fp32 fragments are twice as wide; a block of the matrix stays in registers up to 64 rows and two
-    // k-tiles (64 columns), everything larger runs on matmulLargeKernel
+    // kWideFragments: fp32 fragments are twice as wide; the streaming form, whose fragments stay in registers, goes up to 64 rows and two
+    // k-tiles (64 columns)
     static constexpr bool kWideFragments = Mma::kEsz == 4;
     static __device__ __forceinline__ void decodeIn(const uint32_t* raw, uint32_t* frag) { Mma::decode(raw, frag); }
 };
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(256, kInPieces<Fl> ? 2 : 1) void matmulKernel(const
     const int reluFloorI = a.act == kActRelu ? 0 : (int)0x80000000;
 
     constexpr uint32_t TILE = 16 * NT;
-    // FAST handles whole tiles only (the launcher sends the ragged tail to the general kernel),
+    // FAST handles whole tiles only (launchRest takes the ragged tail),
     // so its loop has no per-lane predicates and the prefetch below is unconditional: with a
     // fixed number of loads and stores per iteration the compiler can wait for exactly the
     // current tile's loads while the next tile's stay in flight.

@@ -10,12 +10,12 @@
 // Matrix.  The whole of it lies in LDS in fragment order, one copy to a workgroup of eight waves; the row tiles are a loop, so
 // that one kernel serves every number of rows (tile t: rows 16t .. 16t+15).  A matrix beyond the LDS is split by row tiles
 // (blockIdx.y).
-// Sums are formed as in matmulKernel and matmulLargeKernel on MatMulArgs alone (the same k-slots in the same instructions): the same bits.
+// Sums are formed as in matmulKernel and matmulLargeKernel (the same k-slots in the same instructions): the same bits.
 //
 // What it replaced: loads and stores of single elements wherever k, m or an address was no multiple of 16 bytes, one launch for every 128
-// rows, and a matrix gathered element by element for every such launch (before, now; us): half 79 x 29 over 221 953 samples 110, 18.8;
-// bfloat16 18 x 221 over 129 870 245, 26.7; int8 221 x 9 over 292 087 306, 60 (5.1 TB/s; floor 52); fp32 18 x 238 over 60 333 74, 16.9;
-// bfloat16 156 x 211 over 16 447 144, 15; half 256 x 256 over 400 000 213, 141.  200 sizes between 8 and 256 over 2^10 to 2^22 samples: 2.26
+// rows, and a matrix gathered element by element for every such launch (before, now; us): half 79 x 29 over 221 953 samples 110, 18.6;
+// bfloat16 18 x 221 over 129 870 245, 22.6; int8 221 x 9 over 292 087 306, 60 (5.1 TB/s; floor 52); fp32 18 x 238 over 60 333 74, 32;
+// bfloat16 156 x 211 over 16 447 144, 17.8; half 256 x 256 over 400 000 213, 119.  200 sizes between 8 and 256 over 2^10 to 2^22 samples: 2.26
 // times as fast (geometric mean).  The largest are bound by HBM, small batches by launching and two trips to memory (matrix and
 // vectors are requested together), those between by the trip of a tile while few waves find registers or LDS.
 // Vectors staged through LDS in whole pieces took as long as read directly, 1.2 to 1.6 times for fp32 of many terms, and need the LDS.
@@ -119,6 +119,7 @@ __device__ __forceinline__ void stageRowTiles(const MatMulArgs& a, const PackedP
     }
 }
 
+// (a function that the kernel takes in: written as the kernel itself the compiler lays out its loops otherwise, 256 x 256 over 400 000 half samples 119 -> 124 us)
 template <class Fl, int KT, int NT, typename OutT>
 __device__ __forceinline__ void packedRows(const MatMulArgs& a, const PackedPlan& p, uint8_t* lds)
 {
@@ -402,28 +403,16 @@ template <class Fl, int KT>
 constexpr int kPackedWaves = kInPieces<Fl> && KT > 2 ? 12 : 8;
 template <class Fl, int KT>
 constexpr int kPackedResident = kInPieces<Fl> ? 2 : Fl::kEsz == 4 && KT > 4 ? 2 : 4;      // waves of a SIMD at least
-// fp32 blocks beyond 64 rows or two k-tiles keep the name of the kernel that serves such blocks otherwise
 template <class Fl, int KT, int NT, typename OutT>
-__global__ __launch_bounds__((64 * kPackedWaves<Fl, KT>), (kPackedResident<Fl, KT>)) void matmulKernel(const MatMulArgs a, const PackedPlan p)
+__global__ __launch_bounds__((64 * kPackedWaves<Fl, KT>), (kPackedResident<Fl, KT>)) void matmulPackedKernel(const MatMulArgs a, const PackedPlan p)
 {
-    extern __shared__ __attribute__((aligned(16))) uint8_t ldsPacked[];
-    packedRows<Fl, KT, NT, OutT>(a, p, ldsPacked);
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    packedRows<Fl, KT, NT, OutT>(a, p, lds);
 }
 template <class Fl, int KT, int NT, typename OutT>
-__global__ __launch_bounds__((64 * kPackedWaves<Fl, KT>), (kPackedResident<Fl, KT>)) void matmulLargeKernel(const MatMulArgs a, const PackedPlan p)
-{
-    extern __shared__ __attribute__((aligned(16))) uint8_t ldsPacked[];
-    packedRows<Fl, KT, NT, OutT>(a, p, ldsPacked);
-}
-
-template <class Fl, int KT, int NT, typename OutT, bool LARGE>
 hipError_t launchPackedSized(hipStream_t stream, const MatMulArgs& a, const PackedPlan& p, uint32_t ldsBytes, int waves, int numCUs, bool append)
 {
-    constexpr auto kernel = [] {
-        typedef void (*Kernel)(const MatMulArgs, const PackedPlan);
-        if constexpr (LARGE) return (Kernel)matmulLargeKernel<Fl, KT, NT, OutT>;
-        else return (Kernel)matmulKernel<Fl, KT, NT, OutT>;
-    }();
+    constexpr auto kernel = matmulPackedKernel<Fl, KT, NT, OutT>;
     const hipError_t e = allowDynamicLds<kernel>((int)kPackedLds);
     if (e != hipSuccess) return e;
     int perCU = residentBlocksPerCU<kernel>(64 * kPackedWaves<Fl, KT>) * kPackedWaves<Fl, KT> / waves;
@@ -433,7 +422,7 @@ hipError_t launchPackedSized(hipStream_t stream, const MatMulArgs& a, const Pack
     const uint32_t tiles = (uint32_t)(((uint64_t)a.batch + 16 * NT - 1) / (16 * NT)), need = (tiles + waves - 1) / waves;
     uint32_t cap = (uint32_t)numCUs * (uint32_t)perCU / blocksY;
     if (cap < 1) cap = 1;
-    noteKernel(append, "matmul%sKernel<%s,KT=%d,NT=%d,out=%dB,packed>", LARGE ? "Large" : "", Fl::kName, KT, NT, (int)sizeof(OutT));
+    noteKernel(append, "matmulPackedKernel<%s,KT=%d,NT=%d,out=%dB>", Fl::kName, KT, NT, (int)sizeof(OutT));
     hipLaunchKernelGGL(kernel, dim3(need < cap ? need : cap, blocksY), dim3(64 * waves), ldsBytes, stream, a, p);
     return hipGetLastError();
 }
@@ -456,25 +445,18 @@ bool launchPacked(hipStream_t stream, const MatMulArgs& a, int numCUs, bool appe
         p.matBytes = matrixSize(a.shape);
         if (p.matBytes < Fl::kEpl * Fl::kEsz) p.matBytes = 0;
     }
-    const int nt = (int)l.nt;
     bool done = false;
     forEach<1, kMostKT + 1>([&](auto kc) {
         constexpr int K = decltype(kc)::value;
         if ((int)kt != K) return;
-        auto launch = [&](auto nc, auto large) {
-            result = launchPackedSized<Fl, K, decltype(nc)::value, OutT, decltype(large)::value>(stream, a, p, l.ldsBytes, waves, numCUs, append);
+        auto launch = [&](auto nc) {
+            result = launchPackedSized<Fl, K, decltype(nc)::value, OutT>(stream, a, p, l.ldsBytes, waves, numCUs, append);
             done = true;
         };
-        auto sized = [&](auto nc) {
-            if constexpr (Fl::kWideFragments) {
-                if (K > 2 || a.m > 64) return launch(nc, std::true_type{});
-            }
-            if constexpr (!Fl::kWideFragments || K <= 2) launch(nc, std::false_type{});
-        };
         if constexpr (K <= kMostPairs) {
-            if (nt == 2) return sized(std::integral_constant<int, 2>{});
+            if (l.nt == 2) return launch(std::integral_constant<int, 2>{});
         }
-        sized(std::integral_constant<int, 1>{});
+        launch(std::integral_constant<int, 1>{});
     });
     return done;
 }

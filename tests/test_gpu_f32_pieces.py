@@ -27,7 +27,7 @@ def bound(x, W, b):
     return (K / 32 + 4) * 2.0 ** -24 * mag
 
 
-# registers up to 64 x 64, then LDS: remainders of tiles; from 20 x 1664 on the fp32 instruction, whose roundings, one for every term,
+# remainders of tiles; 16 x 32 and 64 x 64 in the streaming form; from 20 x 1664 on the fp32 instruction, whose roundings, one for every term,
 # mostly cancel
 @pytest.mark.parametrize("M,K,B", [(1, 1, 1), (16, 32, 64), (17, 33, 100), (64, 64, 1027), (65, 64, 500), (128, 192, 400), (130, 200, 300),
                                    (20, 1664, 60), (20, 1680, 60), (33, 2048, 50)])
@@ -40,22 +40,24 @@ def test_products_against_64_bits(M, K, B):
     assert (np.abs(matmul(x, W, b) - ref) <= bound(x, W, b)).all()
 
 
-# the rule between the pieces and the fp32 instruction (one rounding for every term and for the bias), at its edges
-@pytest.mark.parametrize("M,K,whole", [(16, 192, False), (16, 193, True), (17, 193, False), (32, 320, False), (32, 321, True), (33, 321, False),
-                                       (130, 384, False), (33, 385, True), (100, 1025, True), (3, 2048, True)])
+# the rule between the pieces and the fp32 instruction (one rounding for every term and for the bias), at its edges; up to 256 terms of vectors that
+# are no aligned groups of four the packed kernel, else matmulLargeKernel
+@pytest.mark.parametrize("M,K,whole", [(16, 192, False), (16, 193, True), (17, 193, False), (16, 200, True), (17, 200, False), (32, 320, False), (32, 321, True),
+                                       (33, 321, False), (130, 384, False), (33, 385, True), (100, 1025, True), (3, 2048, True)])
 def test_large_products_take_the_faster_instruction(M, K, whole):
     rng = np.random.default_rng(M * 5000 + K)
     for B in (1, 37, 4000):
         x, W, b = (rng.standard_normal(s).astype(np.float32) for s in ((B, K), (M, K), (M,)))
         got = matmul(x, W, b)
-        assert cv.lastKernelName().startswith("matmulLargeKernel<%s," % ("f32-whole" if whole else "f32")), cv.lastKernelName()
+        kernel = "matmulPackedKernel<%s,KT=7," if K == 193 else "matmulLargeKernel<%s,"
+        assert cv.lastKernelName().startswith(kernel % ("f32-whole" if whole else "f32")), cv.lastKernelName()
         ref = x.astype(np.float64) @ W.astype(np.float64).T + b
         mag = np.abs(x.astype(np.float64)) @ np.abs(W.astype(np.float64)).T + np.abs(b)
         assert (np.abs(got - ref) <= ((K + 1) * 2.0 ** -24 * mag if whole else bound(x, W, b))).all()
 
 
-# (63 x 64: the kernel in registers; its streaming form for 64 x 64 takes NaN through a maximum)
-@pytest.mark.parametrize("M,K", [(24, 40), (63, 64), (100, 96), (8, 1700)])
+# (the packed kernel; the streaming form of 64 x 64 takes NaN through a maximum; then matmulLargeKernel on pieces and on the fp32 instruction)
+@pytest.mark.parametrize("M,K", [(24, 40), (63, 64), (100, 96), (40, 300), (8, 1700)])
 def test_values_at_the_ends_of_the_range(M, K):
     rng = np.random.default_rng(M + K)
     B = 200
@@ -99,8 +101,9 @@ def large(rng, *shape):
     return (10.0 ** rng.uniform(22, 30, shape) * rng.choice([-1.0, 1.0], shape)).astype(np.float32)
 
 
-# (64 x 64: the streaming kernel, 37 samples beyond its whole tiles on the general one; then LDS, and the fp32 instruction)
-@pytest.mark.parametrize("M,K", [(64, 64), (24, 40), (100, 96), (8, 1700)])
+# (64 x 64: the streaming kernel, 37 samples beyond its whole tiles on the packed one, as the next two; then matmulLargeKernel on pieces and on the fp32
+# instruction)
+@pytest.mark.parametrize("M,K", [(64, 64), (24, 40), (100, 96), (40, 300), (8, 1700)])
 def test_products_of_finite_operands_that_overflow(M, K):
     rng = np.random.default_rng(M * 7 + K)
     B = 293

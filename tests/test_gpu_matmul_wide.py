@@ -342,11 +342,11 @@ def test_query_lists_what_matmul_accepts():
 
 
 def test_float32_blocks_in_registers_and_in_lds():
-    # Up to 64 rows and 64 columns an fp32 block stays in registers (the kernels of the 16-bit types, their streaming form
-    # for whole aligned vectors); anything larger is staged in LDS.  Large and ragged batches, padded vector rows, `+=`.
+    # 64 x 64 in whole aligned vectors stays in registers (the streaming form of the 16-bit types), other sizes up to 256 columns run on the
+    # packed form and what lies beyond on matmulLargeKernel, both from LDS.  Large and ragged batches, padded vector rows, `+=`.
     rng = np.random.default_rng(4242)
     for M, K, B, pad in ((64, 64, 70001, 0), (64, 32, 4096, 0), (8, 64, 1000, 4), (33, 17, 999, 0), (64, 64, 513, 3), (128, 64, 2000, 0),
-                         (64, 128, 2000, 0)):
+                         (64, 128, 2000, 0), (64, 320, 2000, 0), (128, 257, 999, 0), (40, 384, 513, 3)):
         x = rng.standard_normal((B, K)).astype(np.float32)
         W = (rng.standard_normal((M, K)) / np.sqrt(K)).astype(np.float32)
         b = rng.uniform(-0.5, 0.5, M).astype(np.float32)
@@ -357,8 +357,9 @@ def test_float32_blocks_in_registers_and_in_lds():
         y = cv.coopVecMatMulAdd(wide[:, :K], CT.Float32, as_bytes(to_dev(W)), 0, CT.Float32, as_bytes(to_dev(b)), 0, CT.Float32,
                                 ML.RowMajor, False, 4 * K, M=M, resultType=CT.Float32)
         name = cv.lastKernelName()
-        assert name.startswith("matmulKernel<f32" if M <= 64 and K <= 64 else "matmulLargeKernel<f32"), (M, K, name)
-        if (M, K, pad) == (64, 64, 0):
+        streams = (M, K, pad) in ((64, 64, 0), (64, 32, 0))
+        assert name.startswith("matmulLargeKernel<f32" if K > 256 else "matmulKernel<f32" if streams else "matmulPackedKernel<f32"), (M, K, name)
+        if streams:
             assert "streaming" in name, name
         assert (np.abs(y.cpu().numpy() - ref64) <= bound).all(), (M, K, B)
         # the member form: this += W x (no bias)
