@@ -221,11 +221,11 @@ __device__ __forceinline__ void packedRows(const MatMulArgs& a, const PackedPlan
         } else {
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                const uint64_t at = min((uint64_t)tile * S + 16 * j + n, (uint64_t)(a.batch - 1)) * a.inStride + colBase * IESZ;
+                const uint8_t* q = a.in + min((uint64_t)tile * S + 16 * j + n, (uint64_t)(a.batch - 1)) * a.inStride + colBase * IESZ;
 #pragma unroll
                 for (int kt = 0; kt < KT; ++kt) {
-                    if (inEnd >= 16) loadUpTo<IESZ>(a.in, at + kt * EPL * IESZ, inEnd, raw[j][kt]);
-                    else loadSlots<IRAW>(raw[j][kt], a.in + at + kt * EPL * IESZ, validBytes - kt * EPL * IESZ, 2);
+                    if (inEnd >= 16) loadUpTo<IESZ>(q + kt * EPL * IESZ, a.in + inEnd, raw[j][kt]);
+                    else loadSlots<IRAW>(raw[j][kt], q + kt * EPL * IESZ, validBytes - kt * EPL * IESZ, 2);
                 }
             }
         }

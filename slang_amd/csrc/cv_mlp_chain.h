@@ -418,12 +418,12 @@ __global__ __launch_bounds__((chainThreads<Mma, MAXT>()), Mma::kEsz == 4 ? (MAXT
                     }
                 }
             } else {
-                const uint64_t at = (uint64_t)min(first + n, a.batch - 1u) * a.inStride + (uint64_t)(colBase * ESZ);
+                const uint8_t* q = a.in + (uint64_t)min(first + n, a.batch - 1u) * a.inStride + colBase * ESZ;
 #pragma unroll
                 for (int kt = 0; kt < INKT; ++kt) {
                     if (kt > 0 && kt >= kt0) continue;
-                    if (inEnd >= 16u) loadUpTo<ESZ>(a.in, at + kt * 8 * ESZ, inEnd, raw[nt][kt]);
-                    else loadSlots<RAW>(raw[nt][kt], a.in + at + kt * 8 * ESZ, validBytes - kt * 8 * ESZ, 2);
+                    if (inEnd >= 16u) loadUpTo<ESZ>(q + kt * 8 * ESZ, a.in + inEnd, raw[nt][kt]);
+                    else loadSlots<RAW>(raw[nt][kt], q + kt * 8 * ESZ, validBytes - kt * 8 * ESZ, 2);
                 }
             }
         }

@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const uint32_t lastSample = a.batch - 1;
 
     // Load mode 1: a read takes the 16 (8) bytes at whatever element a lane's k-slots begin, and half of that where no lane has slots in the
-    // upper half of the last fragment.  What would end behind the last vector is read ending there, also where it begins behind it (placeRead,
+    // upper half of the last fragment.  What would end behind the last vector is read ending there, also where it begins behind it (readAt,
     // cv_reads.h), and moved down when the tile is used, so that no load is waited for before the weights are staged.  (Dword or byte loads under a mask each before, us: 31-32-32-5 over 10^6 fp16 111 -> 36,
     // 50-64-64-63 over 500 000 88 -> 41, 26-16-16-3 over 1 397 712 e4m3 76 -> 37, 3-16-16-1 over 500 8.6 -> 5.0.)
     const uint64_t inEnd = vectorsEnd(a.batch, a.inStride, (uint32_t)a.layers[0].in, ESZ);
@@ -207,9 +207,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     auto readBytes = [&](int kt) { return kt + 1 == Net::KT0 && halfTail ? 2 * RAW : 4 * RAW; };
     auto endsInside = [&](uint32_t t) { return tileReadsEnd((uint64_t)__builtin_amdgcn_readfirstlane(t) * TILE, TILE, a.inStride, gs0, 8 * Net::KT0, ESZ) <= inEnd; };
     // (of super-tiles that do not: sample 16 j + n of the tile, the last one instead of those beyond the batch)
-    auto edge = [&](uint32_t t, int j, int kt) {
-        return placeRead((uint64_t)min(t * TILE + 16 * j + n, lastSample) * a.inStride + own0 + kt * 8 * ESZ, (uint32_t)readBytes(kt), inEnd);
-    };
+    auto edge = [&](uint32_t t, int j, int kt) { return a.in + own0 + (uint64_t)min(t * TILE + 16 * j + n, lastSample) * a.inStride + kt * 8 * ESZ; };
     auto readSlots = [&](uint32_t* b, const uint8_t* q, int bytes) {
         if (bytes == 2 * RAW) {
             if constexpr (ESZ == 2) { const u32x2 v = ((const Loose8<ESZ>*)q)->v; b[0] = v.x; b[1] = v.y; }
@@ -232,7 +230,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 #pragma unroll
                 for (int j = 0; j < S; ++j)
 #pragma unroll
-                    for (int kt = 0; kt < Net::KT0; ++kt) readSlots(&buf[j][kt * RAW], a.in + edge(t, j, kt).at, readBytes(kt));
+                    for (int kt = 0; kt < Net::KT0; ++kt) readSlots(&buf[j][kt * RAW], readAt(edge(t, j, kt), (uint32_t)readBytes(kt), a.in + inEnd), readBytes(kt));
             }
             return;
         }
@@ -433,7 +431,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
                         uint32_t own[RAW];
 #pragma unroll
                         for (int d = 0; d < RAW; ++d) own[d] = buf[r0 + j][kt * RAW + d];
-                        if (moved) shiftDown<ESZ>(own, min((int)edge(t0, r0 + j, kt).down, 4 * RAW - ESZ));
+                        if (moved) shiftDown<ESZ>(own, min((int)readDown(edge(t0, r0 + j, kt), (uint32_t)readBytes(kt), a.in + inEnd), 4 * RAW - ESZ));
 #pragma unroll
                         for (int d = 0; d < RAW; ++d) own[d] &= mask[kt * RAW + d];
                         Mma::decode(own, act[j][kt]);

@@ -1,6 +1,6 @@
 // cv_reads.h -- which bytes a kernel reads of a batch of vectors of any length.  A lane reads its k-slots 16, 8 or 4 bytes at a time at
 // whatever element they begin; what it gets of the elements behind its slice is cleared in registers, but no read may touch a byte behind the
-// last vector.  Without HIP, so that every read can be checked against its buffer on the host.  Offsets are bytes from the first vector.
+// last vector.  Without HIP, so that every read can be checked against its buffer on the host.  Offsets and ends are bytes from the first vector.
 #pragma once
 #include "cv_layout.h"
 
@@ -12,8 +12,8 @@ CV_HD uint64_t vectorsEnd(uint32_t batch, uint64_t stride, uint32_t in, uint32_t
 // bytes of lane group g's slice (gs k-slots to a group) that exist
 CV_HD int32_t sliceBytes(uint32_t in, uint32_t gs, uint32_t g, uint32_t esz)
 {
-    const uint32_t col = g * gs, left = col < in ? in - col : 0u;
-    return (int32_t)((left < gs ? left : gs) * esz);
+    const int32_t left = (int32_t)in - (int32_t)(g * gs), some = left > 0 ? left : 0;
+    return (some < (int32_t)gs ? some : (int32_t)gs) * (int32_t)esz;
 }
 
 // Where the reads of `samples` vectors from vector `first` on end at most: those of the last lane group, whose fragments hold `slots` k-slots.
@@ -22,13 +22,15 @@ CV_HD uint64_t tileReadsEnd(uint64_t first, uint32_t samples, uint64_t stride, u
     return (first + samples - 1u) * stride + (uint64_t)(3u * gs + slots) * esz;
 }
 
-// A read of `bytes` bytes that is wanted at offset `want` of vectors that end at `end` (at least `bytes`): it is made at `at`, and what it
-// brings belongs `down` bytes further down (all of it, where nothing that is wanted exists).
-struct PlacedRead { uint64_t at; uint32_t down; };
-CV_HD PlacedRead placeRead(uint64_t want, uint32_t bytes, uint64_t end)
+// A read of `bytes` bytes that is wanted at `want`, of vectors that end at `end` (at least `bytes` behind the first; addresses or offsets): where it is
+// made, and by how many bytes what it brings is moved down then (all of it, where nothing that is wanted exists).
+template <typename At>
+CV_HD At readAt(At want, uint32_t bytes, At end) { return (int64_t)(want + bytes - end) > 0 ? end - bytes : want; }
+template <typename At>
+CV_HD uint32_t readDown(At want, uint32_t bytes, At end)
 {
-    const uint64_t at = want + bytes <= end ? want : end - bytes, down = want - at;
-    return PlacedRead{at, down < bytes ? (uint32_t)down : bytes};
+    const int64_t over = (int64_t)(want + bytes - end);
+    return over < 0 ? 0u : over > (int64_t)bytes ? bytes : (uint32_t)over;
 }
 
 } // namespace cv

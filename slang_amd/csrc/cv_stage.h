@@ -38,18 +38,19 @@ __device__ __forceinline__ void loadLoose(const uint8_t* q, uint32_t (&x)[DW])
     }
 }
 
-// The same at offset `want` of vectors that end `end` bytes (16 at least) behind `base`: behind them nothing is read and zeros stand.
+// The same where what is read may end, or begin, behind the vectors' `end`: behind it nothing is read and zeros stand (at least 16 bytes lie before it).
 template <int ALIGN, int DW>
-__device__ __forceinline__ void loadUpTo(const uint8_t* base, uint64_t want, uint64_t end, uint32_t (&x)[DW])
+__device__ __forceinline__ void loadUpTo(const uint8_t* q, const uint8_t* end, uint32_t (&x)[DW])
 {
     constexpr int P = DW % 4 == 0 ? 4 : 2;      // dwords of a read
 #pragma unroll
     for (int d0 = 0; d0 < DW; d0 += P) {
-        const PlacedRead r = placeRead(want + 4u * d0, 4u * P, end);
-        const int words = (int)(r.down >> 2);
+        const uint8_t* at = q + 4 * d0;
+        const uint32_t shift = readDown(at, 4u * P, end);
+        const int words = (int)(shift >> 2);
         uint32_t v[2 * P + 1];
         uint32_t part[P];
-        loadLoose<ALIGN>(base + r.at, part);
+        loadLoose<ALIGN>(readAt(at, 4u * P, end), part);
 #pragma unroll
         for (int i = 0; i < 2 * P + 1; ++i) v[i] = i < P ? part[i < P ? i : 0] : 0u;
 #pragma unroll
@@ -60,7 +61,7 @@ __device__ __forceinline__ void loadUpTo(const uint8_t* base, uint64_t want, uin
                 lo = words == w ? v[i + w] : lo;
                 hi = words == w ? v[i + w + 1 <= 2 * P ? i + w + 1 : 2 * P] : hi;
             }
-            x[d0 + i] = __builtin_amdgcn_alignbyte(hi, lo, r.down & 3u);
+            x[d0 + i] = __builtin_amdgcn_alignbyte(hi, lo, shift & 3u);
         }
     }
 }

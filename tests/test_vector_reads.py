@@ -44,8 +44,7 @@ void readUpTo(uint64_t want, uint32_t dwords, uint8_t* x)
 {
     const uint32_t part = dwords % 4 == 0 ? 16 : 8;
     for (uint32_t d = 0; d < 4 * dwords; d += part) {
-        const PlacedRead r = placeRead(want + d, part, end);
-        read(r.at, part, r.down, x + d);
+        read(readAt(want + d, part, end), part, readDown(want + d, part, end), x + d);
     }
 }
 }
@@ -66,8 +65,8 @@ extern "C" uint64_t equalLayers(uint32_t in, uint32_t esz, uint32_t batch, uint6
                     const uint64_t s = inside ? t * samples + i : least(t * samples + i, batch - 1);
                     const uint64_t want = s * stride + (valid > 0 ? g * gs * esz : 0) + kt * 8 * esz;
                     uint8_t x[16] = {};
-                    const PlacedRead r = inside ? PlacedRead{want, 0} : placeRead(want, bytes, end);
-                    read(r.at, bytes, r.down, x);
+                    if (inside) read(want, bytes, 0, x);
+                    else read(readAt(want, bytes, end), bytes, readDown(want, bytes, end), x);
                     expect(x, want, valid - (int)(kt * 8 * esz), (int)bytes);
                 }
     }
