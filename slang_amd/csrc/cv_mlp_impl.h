@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     // Load mode 1: a read takes the 16 (8) bytes at whatever element a lane's k-slots begin, and half of that where no lane has slots in the
     // upper half of the last fragment.  What would end behind the last vector is read ending there, also where it begins behind it (readAt,
     // cv_reads.h), and moved down when the tile is used, so that no load is waited for before the weights are staged.  (Dword or byte loads under a mask each before, us: 31-32-32-5 over 10^6 fp16 111 -> 36,
-    // 50-64-64-63 over 500 000 88 -> 41, 26-16-16-3 over 1 397 712 e4m3 76 -> 37, 3-16-16-1 over 500 8.6 -> 5.0.)
+    // 50-64-64-63 over 500 000 88 -> 43, 26-16-16-3 over 1 397 712 e4m3 76 -> 37, 3-16-16-1 over 500 8.6 -> 5.0.)
     const uint64_t inEnd = vectorsEnd(a.batch, a.inStride, (uint32_t)a.layers[0].in, ESZ);
     const uint32_t own0 = (uint32_t)(validBytes > 0 ? colBase : 0) * ESZ;
     auto readBytes = [&](int kt) { return kt + 1 == Net::KT0 && halfTail ? 2 * RAW : 4 * RAW; };

@@ -295,8 +295,8 @@ __device__ __forceinline__ void stageTrainingWeights(const MlpArgs& a, uint32_t*
 // LOADS selects how the network input is fetched.  kLoadDwords (every lane's slice is whole, 4-byte
 // aligned dwords) and kLoadXY (float2 samples of the example's encoding) are straight-line code: every
 // lane loads from an address that is always valid and masks afterwards, so the requests of the next
-// round stay in flight during the whole current round.  So is kLoadHalves (the paired kernel: vectors of at least two
-// elements at any element): dwords read at whatever half they begin, the last one of a slice of odd length ending where the
+// round stay in flight during the whole current round.  So is kLoadHalves (the paired kernel: vectors of an odd number of
+// elements, three or more, at any element): dwords read at whatever half they begin, the last one of a slice of odd length ending where the
 // slice does.  kLoadAny covers everything else with predicated loads, which the round has to wait for.
 enum : int { kLoadDwords = 0, kLoadAny = 1, kLoadXY = 2, kLoadHalves = 3 };
 
