@@ -25,10 +25,15 @@ CV_HD uint64_t tileReadsEnd(uint64_t first, uint32_t samples, uint64_t stride, u
 // A read of `bytes` bytes that is wanted at `want`, of vectors that end at `end` (at least `bytes` behind the first; addresses or offsets): where it is
 // made, and by how many bytes what it brings is moved down then (all of it, where nothing that is wanted exists).
 template <typename At>
-CV_HD At readAt(At want, uint32_t bytes, At end) { return (int64_t)(want + bytes - end) > 0 ? end - bytes : want; }
+CV_HD At readAt(At want, uint32_t bytes, At end)
+{
+    static_assert(sizeof(At) == 8, "differences are taken as signed 64-bit numbers");
+    return (int64_t)(want + bytes - end) > 0 ? end - bytes : want;
+}
 template <typename At>
 CV_HD uint32_t readDown(At want, uint32_t bytes, At end)
 {
+    static_assert(sizeof(At) == 8, "differences are taken as signed 64-bit numbers");
     const int64_t over = (int64_t)(want + bytes - end);
     return over < 0 ? 0u : over > (int64_t)bytes ? bytes : (uint32_t)over;
 }

@@ -145,3 +145,24 @@ def test_results_on_their_vectors(kind, M, K, B):
             run(vectors, results, accumulate)
             bits = torch.int16 if osz == 2 else torch.int32
             assert torch.equal(results.contiguous().view(bits), want.view(bits)), (accumulate, cv.lastKernelName())
+
+
+# The same of the flavours that matmulKernel's general instantiation serves: half vectors taken as e4m3, e5m2 vectors, e4m3 ones on the e4m3 pipeline.
+@pytest.mark.parametrize("vector,interpretation,flags", [(torch.float16, CT.FloatE4M3, 0), (torch.uint8, CT.FloatE5M2, 0), (torch.uint8, CT.FloatE4M3, 0),
+                                                         (torch.uint8, CT.FloatE4M3, cv.FLAG_FP8_MATRIX_PIPELINE)])
+@pytest.mark.parametrize("M,K,B", [(100, 100, 1000), (128, 128, 517), (17, 128, 40)])
+def test_eight_bit_float_results_on_their_vectors(vector, interpretation, flags, M, K, B):
+    rng = np.random.default_rng(M + K + int(interpretation))
+    W = torch.from_numpy(rng.integers(0, 0x41, (M, K)).astype(np.uint8)).to(DEV)      # moderate values of either type
+    x = torch.from_numpy(rng.standard_normal((B, K)).astype(np.float16)).to(DEV) if vector == torch.float16 else torch.from_numpy(rng.integers(0, 0x41, (B, K)).astype(np.uint8)).to(DEV)
+
+    def run(xs, out):
+        return cv.coopVecMatMul(xs, interpretation, W.flatten(), 0, interpretation, ML.RowMajor, False, K, M=M, resultType=CT.Float16, out=out, flags=flags)
+
+    pitch = max(K * x.element_size(), 2 * M)
+    raw = torch.zeros(B * pitch, dtype=torch.uint8, device=DEV)
+    vectors, results = raw.view(vector).as_strided((B, K), (pitch // x.element_size(), 1)), raw.view(torch.float16).as_strided((B, M), (pitch // 2, 1))
+    vectors.copy_(x)
+    want = run(x, torch.empty(B, M, dtype=torch.float16, device=DEV))
+    run(vectors, results)
+    assert torch.equal(results.contiguous().view(torch.int16), want.view(torch.int16)), cv.lastKernelName()
